@@ -26,13 +26,13 @@
 //     10 % slower) and moved to the matrix instruction's lanes by one lane permutation per register.
 //   * The four waves of a workgroup take every fourth 256-element block of the same 16 rows and meet
 //     in LDS at the end; blocks are requested one iteration ahead, across row tiles.
-//   * Q4_K, Q5_K and Q6_K matrices made of whole 16-row tiles -- every matrix of a model -- take a second
-//     kernel with the same arithmetic and another way to the bytes (gemv_rows_kernel, further down): rows
-//     read in lane-linear runs of two blocks with streaming loads and laid out for the matrix instruction
-//     through a wave's own LDS buffer, which this machine's memory path serves a quarter faster.  The
-//     kernel described above remains for Q8_0 and for matrices with a ragged last tile.
-#include "layer_common.hpp"
-#include "fa_common.hpp"
+//   * Matrices made of whole 16-row tiles -- every matrix of a model -- take a second kernel with the same
+//     arithmetic and another way to the bytes (gemv_rows_kernel, further down): rows read in lane-linear
+//     runs with streaming loads and laid out for the matrix instruction through a wave's own LDS buffer,
+//     which this machine's memory path serves a quarter faster.  The kernel described above remains for
+//     matrices with a ragged last tile, for Q8_0 matrices that do not start on a 16-byte boundary, and for
+//     rows whose digits and buffers do not fit LDS together.
+#include "gemv_blocks.hpp"
 
 // Stage marks of the kernel that reads rows in long runs: wall-clock stamps in the timeline build (waves 0-3 of a
 // workgroup), nothing otherwise (fa_common.hpp).  ROWS_ITEM_STAMP marks an item's arrival in LDS and waits for the
@@ -66,68 +66,6 @@ __device__ long long g_gemv_stamps[kStampWgs * 4 * kStampSlots];
 
 namespace orin_fa {
 namespace {
-
-constexpr int kMaxWaves = 8; // waves per workgroup: 4, or 8 where a matrix has few 16-row tiles and long rows
-constexpr float kDigitRange = 8388608.0f - 65536.0f; // largest |integer| the three signed digits hold
-
-struct XPair {
-    float scale, sum; // of one sub-block of the activation
-};
-
-// LDS: digit planes [3][n_in] | XPair [n_in / G] | 16 zero bytes | partial row sums [kMaxWaves][2][16]
-template <int G>
-struct Lds {
-    static __host__ __device__ int pairs_off(int n_in) { return 3 * n_in; }
-    static __host__ __device__ int zero_off(int n_in) { return 3 * n_in + n_in / G * 8; }
-    static __host__ __device__ int red_off(int n_in) { return zero_off(n_in) + 16; }
-    static __host__ __device__ size_t bytes(int n_in) { return (size_t)red_off(n_in) + kMaxWaves * 2 * 16 * 4; }
-};
-
-// Eight consecutive elements (x, already multiplied by the norm's weights) of a group of G into the digit planes;
-// the G / 8 threads of a group sit in one quad (n_in is a multiple of 32, so a quad is never split) and meet
-// by DPP moves.
-template <int G>
-__device__ __forceinline__ void digits8(const float (&x)[8], int e, int n_in, unsigned char* smem, XPair* pairs, int tid) {
-    float mx = 0.0f, sum = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        mx = fmaxf(mx, fabsf(x[i]));
-        sum += x[i];
-    }
-    mx = fmaxf(mx, dpp_xor_step(mx, 0));
-    sum += dpp_xor_step(sum, 0);
-    if constexpr (G == 32) {
-        mx = fmaxf(mx, dpp_xor_step(mx, 1));
-        sum += dpp_xor_step(sum, 1);
-    }
-    // A group that holds an infinity or a NaN gets a NaN scale, so that every row sum it enters is NaN, as the
-    // products of the vector-ALU kernel are (fmaxf above drops a NaN and (int)rintf would turn it into 0; the sum
-    // does not lose it: a sum of floats is finite only if every term is).
-    const float scale = sum - sum == 0.0f ? (mx > 0.0f ? mx / kDigitRange : 1.0f) : __builtin_nanf("");
-    const float inv = 1.0f / scale;
-    // X + 0x808080 carries 128 into each of the three byte positions, so its bytes are the signed
-    // digits plus 128 (byte k of X + 0x808080 is ((X >> 8 k) + 128) & 255 with the lower digits'
-    // carries already taken out); the exclusive-or takes the 128 off again, byte by byte.
-    unsigned z[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) z[i] = ((unsigned)((int)rintf(x[i] * inv)) + 0x808080u) ^ 0x808080u;
-    // byte k of four consecutive elements into one word of plane 2 - k (plane 0 holds the top digits)
-    u32x2 plane[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const unsigned pick = (unsigned)k | ((unsigned)(4 + k) << 8); // byte k of the second operand, then of the first
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-            const unsigned t01 = __builtin_amdgcn_perm(z[4 * w + 1], z[4 * w + 0], pick);
-            const unsigned t23 = __builtin_amdgcn_perm(z[4 * w + 3], z[4 * w + 2], pick);
-            plane[2 - k][w] = __builtin_amdgcn_perm(t23, t01, 0x05040100u);
-        }
-    }
-    *reinterpret_cast<u32x2*>(smem + e) = plane[0];
-    *reinterpret_cast<u32x2*>(smem + n_in + e) = plane[1];
-    *reinterpret_cast<u32x2*>(smem + 2 * n_in + e) = plane[2];
-    if ((tid & (G / 8 - 1)) == 0) pairs[e / G] = XPair{scale, sum};
-}
 
 // Digits of the (optionally normalised) activation into LDS, in groups of G elements.  Thread t takes
 // elements 8 t .. 8 t + 7 of every kWaves * 512.
@@ -171,316 +109,6 @@ __device__ float stage_digits(const GemvArgs& a, int first, int n_in, unsigned c
     __syncthreads(); // (red is reused for the row sums)
     return 1.0f / sqrtf(ss / (float)n_in + a.eps);
 }
-
-// A workgroup barrier that waits for this wave's LDS traffic only: weight requests in flight stay in flight.
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-// 16-byte loads of the kernels that fetch 64 bytes of each of 16 rows per instruction: ordinary ones, because the
-// neighbouring pieces of a line are fetched by other instructions and meet in the CU's cache (as streaming loads,
-// which pass that cache, these kernels take half as long again).  p may be 2-byte aligned.
-typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
-__device__ __forceinline__ u32x4 load16(const unsigned char* p) { return *reinterpret_cast<const u32x4_a2*>(p); }
-__device__ __forceinline__ u32x4 load16_aligned(const unsigned char* p) { return *reinterpret_cast<const u32x4*>(p); }
-__device__ __forceinline__ float half_of(unsigned bits) { return (float)__builtin_bit_cast(_Float16, (uint16_t)bits); }
-__device__ __forceinline__ unsigned from_lane(int src_lane4, unsigned v) {
-    return (unsigned)__builtin_amdgcn_ds_bpermute(src_lane4, (int)v);
-}
-// (the upper two digits' sums are put together as integers: below 2^30 for every block type, and rounded once on
-// conversion where the fused multiply-add of the converted parts would round, to the same value)
-__device__ __forceinline__ float digits_sum(const i32x4& acc) {
-    return (float)(acc[0] * 256 + acc[1]) * 256.0f + (float)acc[2];
-}
-// Every byte's low nibble from a, its high nibble from b, in one instruction (spelled out, since the compiler, which
-// knows which bits of b can be set, narrows the mask and then needs an AND and an AND-OR).
-__device__ __forceinline__ unsigned low_nibbles_of(unsigned a, unsigned b) {
-    unsigned r;
-    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(r) : "v"(0x0f0f0f0fu), "v"(a), "v"(b));
-    return r;
-}
-// LDS byte offset of a lane's A operand: base + x for a lane that holds digits (step 1), base (the zero bytes) for
-// one whose rows are zero (step 0); x is the same in every lane.  One 24-bit multiply-add.
-__device__ __forceinline__ int operand_at(int base, int step, int x) {
-    return (int)(__umul24((unsigned)x, (unsigned)step) + (unsigned)base);
-}
-// (the step as a value the compiler knows nothing of: told that it is 0 or 1, it replaces the multiply-add by a
-// move, a select and an add)
-__device__ __forceinline__ int opaque_step(bool on) {
-    int step = on ? 1 : 0;
-    asm volatile("" : "+v"(step));
-    return step;
-}
-
-// What a lane needs to know of itself: as a loader (row ln of the tile, 16-byte piece lg), as a lane of
-// the matrix instruction (weight row / column n, element group g; the loader of its data is lane
-// 4 n + g, whose piece is g as well), and as a lane of the A operand (accumulator row am = 4 p + digit).
-struct LaneCtx {
-    int n, g, ln, lg, src_lane4, am;
-    const unsigned char* smem;
-    const XPair* pairs;
-    int n_in, zero_off;
-};
-
-template <int T>
-struct MF;
-
-// Q4_K and Q5_K (reference: src/quant.h:14-31): per 128-element half of a block, the lane's 16 bytes of
-// nibbles are 16 elements of sub-block 2 (g / 2) (low nibbles) and of 2 (g / 2) + 1 (high nibbles); the two
-// matrix instructions of a half add into one accumulator whose row group p is sub-block p of the half.
-// Q5_K keeps a fifth bit per element in 32 bytes behind the header: bit p of byte e belongs to element e of
-// sub-block p.
-template <bool FIVE>
-struct MFK45 {
-    static constexpr int kGroup = 32, kBlockBytes = FIVE ? 176 : 144, kQs = FIVE ? 48 : 16;
-    struct Raw {
-        u32x4 hdr, q1, q2; // a block's header and this lane's 16 bytes of each half of its nibbles
-        u32x4 qh;          // (Q5_K) the 16 bytes of fifth bits that cover this lane's elements
-    };
-    struct Addr {
-        int lo_base, hi_base, lo_step, hi_step; // LDS byte offsets of this lane's A operands and whether they move with the block (1); a lane whose row is zero reads the 16 zero bytes (0)
-    };
-    static __device__ __forceinline__ void load(const unsigned char* blk, int lg, Raw& r) {
-        r.hdr = load16_aligned(blk);
-        if constexpr (FIVE) r.qh = load16_aligned(blk + 16 + 16 * (lg & 1));
-        r.q1 = load16_aligned(blk + kQs + 16 * lg);
-        r.q2 = load16_aligned(blk + kQs + 64 + 16 * lg);
-    }
-    static __device__ __forceinline__ Addr addr(const LaneCtx& c) {
-        const int ap = c.am >> 2, ad = c.am & 3, g = c.g;
-        const bool live = ad < 3 && (ap >> 1) == (g >> 1);
-        const int elem = 64 * (g >> 1) + 16 * (g & 1);
-        const bool lo = live && (ap & 1) == 0, hi = live && (ap & 1) == 1;
-        return Addr{lo ? ad * c.n_in + elem : c.zero_off, hi ? ad * c.n_in + elem + 32 : c.zero_off, opaque_step(lo), opaque_step(hi)};
-    }
-    static __device__ __forceinline__ float block(const Raw& r, const LaneCtx& c, const Addr& ad, int b) {
-        // (the loading lane holds piece lg of its row, and lane (n, g) wants piece g of row n: the bytes of
-        // the packed pairs it needs are bytes lg of the loading lane's three words)
-        const unsigned mine = ((r.hdr.y >> (8 * c.lg)) & 0xffu) | (((r.hdr.z >> (8 * c.lg)) & 0xffu) << 8) |
-                              (((r.hdr.w >> (8 * c.lg)) & 0xffu) << 16);
-        const unsigned dd = from_lane(c.src_lane4, r.hdr.x), bb = from_lane(c.src_lane4, mine);
-        u32x4 fifth = {0u, 0u, 0u, 0u}, q1, q2;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            if constexpr (FIVE) fifth[i] = from_lane(c.src_lane4, r.qh[i]) >> (2 * (c.g >> 1));
-            q1[i] = from_lane(c.src_lane4, r.q1[i]);
-            q2[i] = from_lane(c.src_lane4, r.q2[i]);
-        }
-        const unsigned b0 = bb & 0xffu, b1 = (bb >> 8) & 0xffu, b2 = (bb >> 16) & 0xffu;
-        // pairs g (first half of the block) and 4 + g (second half) of the twelve packed bytes
-        const float sc[2] = {(float)(b0 & 63u), (float)((b2 & 0x0fu) | ((b0 >> 6) << 4))};
-        const float mn[2] = {(float)(b1 & 63u), (float)((b2 >> 4) | ((b1 >> 6) << 4))};
-        return math(dd, sc, mn, q1, q2, fifth, c, ad, b);
-    }
-    // A block laid out in LDS piece after piece (the kernel that reads rows in long runs): piece k is the block's
-    // bytes 16 k ...
-    static constexpr int kPieces = kBlockBytes / 16;
-    static constexpr bool kAligned = true;
-    static __host__ __device__ constexpr int piece_off(int k) { return 16 * k; }
-    static __device__ __forceinline__ float from_lds(const unsigned char* blk, const LaneCtx& c, const Addr& ad, int b) {
-        const u32x4 hdr = *reinterpret_cast<const u32x4*>(blk);
-        const u32x4 q1 = *reinterpret_cast<const u32x4*>(blk + kQs + 16 * c.g);
-        const u32x4 q2 = *reinterpret_cast<const u32x4*>(blk + kQs + 64 + 16 * c.g);
-        u32x4 fifth = {0u, 0u, 0u, 0u};
-        if constexpr (FIVE) fifth = *reinterpret_cast<const u32x4*>(blk + 16 + 16 * (c.g & 1)) >> (unsigned)(2 * (c.g >> 1));
-        // the six-bit pairs straight out of the three words (bit fields at 8 g: no byte is put together first)
-        const unsigned s8 = 8 * c.g;
-        const float sc[2] = {(float)__builtin_amdgcn_ubfe(hdr.y, s8, 6), (float)(__builtin_amdgcn_ubfe(hdr.w, s8, 4) | ((hdr.y >> (s8 + 2)) & 0x30u))};
-        const float mn[2] = {(float)__builtin_amdgcn_ubfe(hdr.z, s8, 6), (float)(__builtin_amdgcn_ubfe(hdr.w, s8 + 4, 4) | ((hdr.z >> (s8 + 2)) & 0x30u))};
-        return math(hdr.x, sc, mn, q1, q2, fifth, c, ad, b);
-    }
-    // In lane (n, g): dd = the block's two fp16 scales, sc / mn = the six-bit scales and minima of sub-blocks g (first
-    // half of the block) and 4 + g (second half), q1 / q2 = piece g of each half of the nibbles, fifth = the fifth
-    // bits of this lane's elements shifted down to bit 0 (Q5_K).
-    static __device__ __forceinline__ float math(unsigned dd, const float (&sc)[2], const float (&mn)[2], const u32x4& q1, const u32x4& q2,
-                                                 const u32x4& fifth, const LaneCtx& c, const Addr& ad, int b) {
-        const float d = half_of(dd & 0xffffu), dmin = half_of(dd >> 16);
-        float scaled[2], offset[2]; // sum of sc * q * x and of mn * x over a sub-block pair; the block's two scales come last
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const i32x4 alo = *reinterpret_cast<const i32x4*>(c.smem + operand_at(ad.lo_base, ad.lo_step, 256 * b + 128 * h));
-            const i32x4 ahi = *reinterpret_cast<const i32x4*>(c.smem + operand_at(ad.hi_base, ad.hi_step, 256 * b + 128 * h));
-            const XPair xp = c.pairs[8 * b + 4 * h + c.g];
-            const u32x4 qs = h ? q2 : q1;
-            i32x4 lo, hi;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const unsigned q = qs[i];
-                unsigned l = q & 0x0f0f0f0fu, u = (q >> 4) & 0x0f0f0f0fu;
-                if constexpr (FIVE) { // sub-blocks 4 h + 2 (g / 2) and + 1: bits 4 h and 4 h + 1 of the shifted bytes
-                    const unsigned f = fifth[i] >> (4 * h);
-                    l |= (f & 0x01010101u) << 4;
-                    u |= (f & 0x02020202u) << 3;
-                }
-                lo[i] = (int)l;
-                hi[i] = (int)u;
-            }
-            i32x4 acc = {0, 0, 0, 0};
-            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(alo, lo, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(ahi, hi, acc, 0, 0, 0);
-            scaled[h] = sc[h] * (digits_sum(acc) * xp.scale);
-            offset[h] = mn[h] * xp.sum;
-        }
-        return d * (scaled[0] + scaled[1]) - dmin * (offset[0] + offset[1]);
-    }
-};
-template <>
-struct MF<kQ4_K> : MFK45<false> {};
-template <>
-struct MF<kQ5_K> : MFK45<true> {};
-
-// Q8_0 (reference: src/quant.h:42-45; blocks of 34 bytes, 2-byte aligned): eight blocks make up the 256
-// elements the kernel walks at a time.  Per 128-element half, the lane's 16 bytes are half of block
-// 2 run + g / 2 of the half, for run = 0, 1: one matrix instruction per run, both adding into one accumulator
-// whose row group p is block p of the half.
-template <>
-struct MF<kQ8_0> {
-    static constexpr int kGroup = 32, kBlockBytes = 272;
-    struct Raw {
-        u32x4 q[2][2]; // [half][run]
-        unsigned d[2]; // scales of blocks lg and 4 + lg
-    };
-    typedef MFK45<false>::Addr Addr;
-    template <typename V>
-    struct __attribute__((packed, aligned(2))) Loose {
-        V v;
-    };
-    static __device__ __forceinline__ void load(const unsigned char* blk, int lg, Raw& r) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-#pragma unroll
-            for (int run = 0; run < 2; ++run)
-                r.q[h][run] = load16(blk + 34 * (4 * h + 2 * run + (lg >> 1)) + 2 + 16 * (lg & 1));
-            r.d[h] = *reinterpret_cast<const uint16_t*>(blk + 34 * (4 * h + lg));
-        }
-    }
-    static __device__ __forceinline__ Addr addr(const LaneCtx& c) {
-        const int ap = c.am >> 2, ad = c.am & 3, g = c.g;
-        const bool live = ad < 3 && (ap & 1) == (g >> 1);
-        const int elem = 32 * ap + 16 * (g & 1);
-        const bool r0 = live && (ap >> 1) == 0, r1 = live && (ap >> 1) == 1;
-        return Addr{r0 ? ad * c.n_in + elem : c.zero_off, r1 ? ad * c.n_in + elem : c.zero_off, opaque_step(r0), opaque_step(r1)};
-    }
-    static __device__ __forceinline__ float block(const Raw& r, const LaneCtx& c, const Addr& ad, int b) {
-        float out[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const i32x4 a0 = *reinterpret_cast<const i32x4*>(c.smem + operand_at(ad.lo_base, ad.lo_step, 256 * b + 128 * h));
-            const i32x4 a1 = *reinterpret_cast<const i32x4*>(c.smem + operand_at(ad.hi_base, ad.hi_step, 256 * b + 128 * h));
-            const XPair xp = c.pairs[8 * b + 4 * h + c.g];
-            const float d = half_of(from_lane(c.src_lane4, r.d[h]));
-            i32x4 w0, w1;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                w0[i] = (int)from_lane(c.src_lane4, r.q[h][0][i]);
-                w1[i] = (int)from_lane(c.src_lane4, r.q[h][1][i]);
-            }
-            i32x4 acc = {0, 0, 0, 0};
-            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, w0, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, w1, acc, 0, 0, 0);
-            out[h] = d * (digits_sum(acc) * xp.scale);
-        }
-        return out[0] + out[1];
-    }
-};
-
-// Q6_K (reference: src/quant.h:34-40; blocks of 210 bytes, 2-byte aligned): per 128-element half, piece g
-// of the half's 64 low-nibble bytes holds sub-block g (elements 16 g .. 16 g + 15 of the half) in its low
-// nibbles and sub-block 4 + g in its high nibbles; their high bit pairs sit in high byte 16 (g & 1) + i at
-// bits 2 (g / 2) and 4 + 2 (g / 2).  One matrix instruction and one accumulator per nibble; the element
-// group g of the instruction is sub-block g (or 4 + g), so the A operand's row group p is live in group p.
-template <>
-struct MF<kQ6_K> {
-    static constexpr int kGroup = 16, kBlockBytes = 210;
-    struct Raw {
-        u32x4 ql[2], qh[2], sc;
-        unsigned d;
-    };
-    struct Addr {
-        int base, step;
-    };
-    template <typename V>
-    struct __attribute__((packed, aligned(2))) Loose {
-        V v;
-    };
-    static __device__ __forceinline__ void load(const unsigned char* blk, int lg, Raw& r) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            r.ql[h] = load16(blk + 64 * h + 16 * lg);
-            r.qh[h] = load16(blk + 128 + 32 * h + 16 * (lg & 1));
-        }
-        r.sc = load16(blk + 192);
-        r.d = *reinterpret_cast<const uint16_t*>(blk + 208);
-    }
-    static __device__ __forceinline__ Addr addr(const LaneCtx& c) {
-        const int ap = c.am >> 2, ad = c.am & 3;
-        const bool live = ad < 3 && ap == c.g;
-        return Addr{live ? ad * c.n_in + 16 * c.g : c.zero_off, opaque_step(live)};
-    }
-    static __device__ __forceinline__ float block(const Raw& r, const LaneCtx& c, const Addr& ad, int b) {
-        // scales 8 h + g and 8 h + 4 + g of both halves: byte lg of each of the loading lane's four words
-        const unsigned mine = ((r.sc.x >> (8 * c.lg)) & 0xffu) | (((r.sc.y >> (8 * c.lg)) & 0xffu) << 8) |
-                              (((r.sc.z >> (8 * c.lg)) & 0xffu) << 16) | (((r.sc.w >> (8 * c.lg)) & 0xffu) << 24);
-        const unsigned ss = from_lane(c.src_lane4, mine);
-        const unsigned dd = from_lane(c.src_lane4, r.d);
-        u32x4 ql[2], qh[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                ql[h][i] = from_lane(c.src_lane4, r.ql[h][i]);
-                qh[h][i] = from_lane(c.src_lane4, r.qh[h][i]);
-            }
-        }
-        return math(ss, dd, ql, qh, c, ad, b);
-    }
-    // A block laid out in LDS piece after piece (the kernel that reads rows in long runs): pieces 0 ... 12 are the
-    // block's bytes 16 k ..., piece 13 its last 16 bytes (194 ... 209: the fp16 scale in its last two), so that no
-    // piece reaches past the block.
-    static constexpr int kPieces = 14;
-    static constexpr bool kAligned = false;
-    static __host__ __device__ constexpr int piece_off(int k) { return k < 13 ? 16 * k : 194; }
-    static __device__ __forceinline__ float from_lds(const unsigned char* blk, const LaneCtx& c, const Addr& ad, int b) {
-        const u32x4 sc = *reinterpret_cast<const u32x4*>(blk + 192);
-        const unsigned ss = ((sc.x >> (8 * c.g)) & 0xffu) | (((sc.y >> (8 * c.g)) & 0xffu) << 8) | (((sc.z >> (8 * c.g)) & 0xffu) << 16) |
-                            (((sc.w >> (8 * c.g)) & 0xffu) << 24);
-        const unsigned dd = *reinterpret_cast<const unsigned*>(blk + 13 * 16 + 12) >> 16;
-        u32x4 ql[2], qh[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            ql[h] = *reinterpret_cast<const u32x4*>(blk + 64 * h + 16 * c.g);
-            qh[h] = *reinterpret_cast<const u32x4*>(blk + 128 + 32 * h + 16 * (c.g & 1));
-        }
-        return math(ss, dd, ql, qh, c, ad, b);
-    }
-    // In lane (n, g): ss = the scales 8 h + g and 8 h + 4 + g of both halves (a byte each), dd = the block's fp16
-    // scale, ql / qh = piece g of each half's low nibbles and the piece of high bit pairs that covers it.
-    static __device__ __forceinline__ float math(unsigned ss, unsigned dd, const u32x4 (&ql)[2], const u32x4 (&qh)[2], const LaneCtx& c,
-                                                 const Addr& ad, int b) {
-        const float d = half_of(dd & 0xffffu);
-        const int s1 = 2 * (c.g >> 1);
-        float out[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const i32x4 alo = *reinterpret_cast<const i32x4*>(c.smem + operand_at(ad.base, ad.step, 256 * b + 128 * h));
-            const i32x4 ahi = *reinterpret_cast<const i32x4*>(c.smem + operand_at(ad.base, ad.step, 256 * b + 128 * h + 64));
-            const XPair xlo = c.pairs[16 * b + 8 * h + c.g], xhi = c.pairs[16 * b + 8 * h + 4 + c.g];
-            i32x4 lo, hi;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                // u: this lane's two bit pairs of every byte at bits 0, 1 and 4, 5, nothing else; each lands in the
-                // high nibble of its element by one bit-field insert
-                const unsigned l = ql[h][i], u = (qh[h][i] >> s1) & 0x33333333u;
-                lo[i] = (int)low_nibbles_of(l, u << 4);
-                hi[i] = (int)low_nibbles_of(l >> 4, u);
-            }
-            const i32x4 zero = {0, 0, 0, 0};
-            const i32x4 acc_lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(alo, lo, zero, 0, 0, 0);
-            const i32x4 acc_hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(ahi, hi, zero, 0, 0, 0);
-            const float sc_lo = (float)((int)(ss << (24 - 16 * h)) >> 24), sc_hi = (float)((int)(ss << (16 - 16 * h)) >> 24);
-            out[h] = sc_lo * (digits_sum(acc_lo) * xlo.scale - 32.0f * xlo.sum) + sc_hi * (digits_sum(acc_hi) * xhi.scale - 32.0f * xhi.sum);
-        }
-        return d * (out[0] + out[1]);
-    }
-};
 
 // T: weight type.  DUAL: two matrices (gate, up) and SiLU(gate) * up.  Grid: (workgroups, matrices); a
 // workgroup walks the 16-row tiles blockIdx.x, + gridDim.x, ...
@@ -609,21 +237,6 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_mfma_kernel(const GemvArgs a
 // Requires whole 16-row tiles.  (Deeper request queues, three and four items a wave, were slower in both kernels,
 // and so were four-block items: what bounds the kernels after the loads is the vector ALU, about 74 instructions
 // per block and wave for the nibbles, the six-bit pairs and the digit sums.)
-constexpr int kRowsMaxCb = 2; // blocks of a row in an item, at most
-constexpr int kRowsRedBytes = 2 * kMaxWaves * 2 * 16 * 4 + 64; // two sets of partial row sums (tiles alternate: one barrier a tile), the waves' sums of squares
-
-template <int T, int CB>
-struct RowsGeom {
-    static constexpr int P = MF<T>::kPieces;                 // pieces of a block
-    static constexpr int kRowPieces = CB * P;                // pieces of a row in an item
-    static constexpr int R = kRowPieces | 1;                 // LDS row stride, pieces
-    static constexpr int NL = (16 * kRowPieces + 63) / 64;   // load instructions an item
-    static constexpr int kWaveBytes = (16 * R + 1) * 16;     // (one more piece: where lanes past the item's end write)
-    static __host__ __device__ size_t lds_bytes(int n_in, int waves) {
-        return (size_t)Lds<MF<T>::kGroup>::red_off(n_in) + kRowsRedBytes + (size_t)waves * kWaveBytes;
-    }
-};
-
 template <int T, bool DUAL, int kWaves, int CB, bool kShortPrologue = false>
 __device__ __forceinline__ void gemv_rows_body(const GemvArgs& a) {
     using F = MF<T>;
@@ -905,7 +518,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_mfma_mixed_kernel(const Gemv
     }
 }
 
-// The same for the kernel that reads rows in long runs (no Q8_0 there).
+// The same for the kernel that reads rows in long runs (no Q8_0 there: a file of that format has no other beside it).
 template <int kWaves, int CB>
 __global__ __launch_bounds__(kWaves * 64) void gemv_rows_mixed_kernel(const GemvArgs a) {
     switch (a.seg[blockIdx.y].type) {
@@ -920,7 +533,8 @@ constexpr size_t kMfmaLdsMax = 96u * 1024u;
 template <int T>
 size_t lds_bytes(int n_in) { return Lds<MF<T>::kGroup>::bytes(n_in); }
 
-// The long-run kernel where it applies: Q4_K / Q5_K / Q6_K, whole 16-row tiles, LDS within the limit.
+// The long-run kernel where it applies: whole 16-row tiles, LDS within the limit, and of Q8_0 only matrices that start on
+// a 16-byte boundary.
 bool rows_enabled() {
     static const bool on = getenv("ORIN_GEMV_NO_ROWS") == nullptr;
     return on;
@@ -953,12 +567,23 @@ bool launch_rows_as(const GemvArgs& a, dim3 grid, int n_in_wg, hipStream_t strea
     return true;
 }
 
+// Q8_0's 34-byte blocks: 256 elements are seventeen whole 16-byte pieces where the matrix starts on one, and the loads are
+// then aligned and the runs go through LDS as they are (MF<kQ8_0>::from_lds).  Llama-3.2-1B's shapes, per launch with 64
+// bytes of each of 16 rows per instruction -> in long runs: gate/up 13.7 -> 9.8 us (35.7 MB, 3.65 TB/s), down 8.6 -> 6.8,
+// q, k, v 8.4 -> 6.5, output projection 6.5 -> 4.5, logits 63.4 -> 45.8 us (279 MB, 6.1 TB/s).
+bool rows_base_ok(int type, const void* w) { return type != kQ8_0 || (reinterpret_cast<uintptr_t>(w) & 15u) == 0; }
+
 template <int T>
 bool launch_rows(const GemvArgs& a, dim3 grid, bool wide, int nb_wg, hipStream_t stream) {
     if (!rows_enabled()) return false;
     for (int i = 0; i < a.n_seg; ++i)
-        if (a.seg[i].n_out % 16 != 0) return false;
+        if (a.seg[i].n_out % 16 != 0 || !rows_base_ok(T, a.seg[i].w)) return false;
+    if (a.w_up && !rows_base_ok(T, a.w_up)) return false;
     const int n_in_wg = nb_wg * 256;
+    if constexpr (T == kQ8_0) { // (272 bytes are a long run already)
+        if (wide) return launch_rows_as<T, false, 8, 1>(a, grid, n_in_wg, stream);
+        return a.w_up ? launch_rows_as<T, true, 4, 1>(a, grid, n_in_wg, stream) : launch_rows_as<T, false, 4, 1>(a, grid, n_in_wg, stream);
+    }
     if (wide) { // (eight waves: never two matrices)
         return (nb_wg + 7) / 8 <= 1 ? launch_rows_as<T, false, 8, 1>(a, grid, n_in_wg, stream)
                                     : launch_rows_as<T, false, 8, 2>(a, grid, n_in_wg, stream);
@@ -989,7 +614,7 @@ hipError_t launch(const GemvArgs& a, int cu_count, hipStream_t stream) {
     // Eight waves a workgroup where a row has the blocks to share out and a workgroup has one tile only (a
     // second tile would have amortised the staging instead).
     const bool wide = ks == 1 && nb_row >= 16 && !a.w_up && (int)grid.x == (max_out + 15) / 16;
-    if constexpr (T == kQ4_K || T == kQ5_K || T == kQ6_K) {
+    {
         const int per_cu = rows_wgs_per_cu(a.mfma_wgs_per_cu);
         g_rows_resident = cu_count * 3;
         dim3 gr = g3;
@@ -1121,6 +746,9 @@ hipError_t gemv_mfma_allow_lds() {
     if ((e = allow_rows_all<kQ4_K>()) != hipSuccess) return e;
     if ((e = allow_rows_all<kQ5_K>()) != hipSuccess) return e;
     if ((e = allow_rows_all<kQ6_K>()) != hipSuccess) return e;
+    if ((e = allow_rows<kQ8_0, false, 8, 1>()) != hipSuccess) return e;
+    if ((e = allow_rows<kQ8_0, false, 4, 1>()) != hipSuccess) return e;
+    if ((e = allow_rows<kQ8_0, true, 4, 1>()) != hipSuccess) return e;
     if ((e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemv_rows_mixed_kernel<8, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMfmaLdsMax)) != hipSuccess) return e;
     if ((e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemv_rows_mixed_kernel<8, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMfmaLdsMax)) != hipSuccess) return e;
     if ((e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemv_rows_mixed_kernel<4, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMfmaLdsMax)) != hipSuccess) return e;

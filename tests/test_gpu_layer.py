@@ -378,6 +378,36 @@ def test_whole_tiles_in_long_runs(ly, wtype, n_in, n_out):
         assert e < TOL_OP, what
 
 
+@pytest.mark.parametrize("offset", [0, 2])
+@pytest.mark.parametrize("n_in,n_out", [(256, 16), (512, 48), (1792, 64), (2048, 4112), (8192, 2048), (18944, 32)])
+def test_q8_0_in_long_runs(ly, n_in, n_out, offset):
+    """Q8_0 matrices that start on a 16-byte boundary are read in long runs, others are not: one block group a row to
+    seventy-four, one tile to several a workgroup, a share of a row per workgroup, every epilogue."""
+    import torch
+
+    ly.use_matrix_cores(True)
+    rs = lm.Stream(7700 + n_in + n_out)
+    t, up = lm.make_tensor(rs, lm.Q8_0, n_in, n_out), lm.make_tensor(rs, lm.Q8_0, n_in, n_out)
+    x, nw = rs.sym(n_in, 1.0), (1.0 + rs.sym(n_in, 0.3)).astype(np.float32)
+    bias, y0 = rs.sym(n_out, 0.5), rs.sym(n_out, 1.0)
+    w, wu, dx = dev_bytes(t[1], offset=offset), dev_bytes(up[1], offset=offset), _dev(x)
+    xn = ref.rms_norm(x, nw, 1e-5)
+    plain = ref.gemv(lm.Q8_0, t[1], x, n_in, n_out).astype(np.float64)
+    normed = ref.gemv(lm.Q8_0, t[1], xn, n_in, n_out)
+    yb, yg, ya = out_buf(n_out), out_buf(n_out), _dev(np.concatenate([y0, np.full(4, 12345.0, np.float32)]))
+    ly.gemv_multi(lm.Q8_0, [w], [_dev(bias)], [yb], [n_out], dx, _dev(nw), 1e-5, n_in)
+    ly.gemv_norm_gate_up_swiglu(lm.Q8_0, w, wu, dx, _dev(nw), 1e-5, yg, n_in, n_out)
+    ly.gemv_multi(lm.Q8_0, [w], None, [ya], [n_out], dx, None, 0.0, n_in, True)
+    torch.cuda.synchronize()
+    act = ref.swiglu(normed, ref.gemv(lm.Q8_0, up[1], xn, n_in, n_out)).astype(np.float64)
+    for what, y, want in (("norm + bias", yb, normed.astype(np.float64) + bias), ("gate/up", yg, act), ("accumulate", ya, plain + y0)):
+        got = y.cpu().numpy()
+        assert (got[n_out:] == 12345.0).all(), f"{what}: rows past n_out were written"
+        e = vec_err(got[:n_out], want)
+        print(f"Q8_0 {n_in} x {n_out} at {offset} {what}: err {e:.2e}", flush=True)
+        assert e < TOL_OP, what
+
+
 def test_rms_norm_rows_swiglu_and_in_place(ly):
     import torch
 
