@@ -11,7 +11,7 @@
 //   * Unit of work ("slot"): 32 elements of a row, chosen per weight type so that one lane's
 //     loads are whole 16- or 8-byte pieces of a block (Q4_K/Q5_K: one 16-byte piece of nibbles,
 //     i.e. 16 low-nibble and 16 high-nibble elements; Q6_K: 8 columns of the block's four
-//     32-element strips; Q8_0: one block; F16/F32: 32 consecutive elements).  A lane keeps the
+//     32-element strips; Q8_0: one block; F32: 32 consecutive elements).  A lane keeps the
 //     same slots for every row it works on, so its 32 activations per slot -- and their sums,
 //     which the minimum / offset terms of the block formats multiply -- sit in registers for
 //     the whole kernel: the vector cache and LDS carry weight bytes only.
@@ -24,6 +24,7 @@
 //     prologue (every workgroup needs the whole activation anyway), a bias or the accumulation
 //     into y in the epilogue, two matrices with SiLU(gate) * up, and up to three matrices of one
 //     type that share the activation (the q, k, v projections).
+//   * F16 matrices have a kernel of their own (gemv_f16.hip).
 #include "layer_common.hpp"
 
 #include <stdlib.h>
@@ -211,27 +212,6 @@ struct Fmt<kQ8_0> {
                 a += sb(w.b[i], k) * x[16 + 4 * i + k];
             }
         return half_bits(w.d) * a;
-    }
-};
-
-template <>
-struct Fmt<kF16> {
-    static constexpr int kRuns = 1, kRunLen = 32, kAlign = 16;
-    struct Raw {
-        h8 v[4];
-    };
-    static __device__ __forceinline__ int run_start(int s, int) { return s * 32; }
-    static __device__ __forceinline__ void load(const unsigned char* row, int s, Raw& w) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) w.v[i] = *reinterpret_cast<const h8*>(row + (size_t)s * 64 + i * 16);
-    }
-    static __device__ __forceinline__ float dot(const Raw& w, int, const float* x, const float*) {
-        float a = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int k = 0; k < 8; ++k) a += (float)w.v[i][k] * x[8 * i + k];
-        return a;
     }
 };
 
@@ -520,7 +500,7 @@ hipError_t gemv_launch(int type, GemvArgs a, int cu_count, hipStream_t stream) {
     if (gemv_use_mfma() && gemv_mfma_ok(type, a)) return gemv_mfma_launch(type, a, cu_count, stream);
     switch (type) {
     case kF32: return launch_type<kF32>(a, cu_count, stream);
-    case kF16: return launch_type<kF16>(a, cu_count, stream);
+    case kF16: return gemv_f16_launch(a, cu_count, stream);
     case kQ8_0: return launch_type<kQ8_0>(a, cu_count, stream);
     case kQ4_K: return launch_type<kQ4_K>(a, cu_count, stream);
     case kQ5_K: return launch_type<kQ5_K>(a, cu_count, stream);

@@ -48,6 +48,7 @@ hipError_t gemv_mfma_allow_lds();
 // Up to three matrices, each Q4_K or Q6_K (GemvSeg::type), in one launch on the matrix cores.
 hipError_t gemv_mixed_launch(GemvArgs args, int cu_count, hipStream_t stream);
 hipError_t gemv_mfma_mixed_launch(GemvArgs args, int cu_count, hipStream_t stream);
+hipError_t gemv_f16_launch(const GemvArgs& args, int cu_count, hipStream_t stream); // F16 (gemv_f16.hip)
 bool gemv_use_mfma();
 void gemv_set_use_mfma(bool on);
 int gemv_row_shares();          // 0: chosen by shape; 1: accumulating projections never cut a row into shares

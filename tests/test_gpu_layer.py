@@ -408,6 +408,34 @@ def test_q8_0_in_long_runs(ly, n_in, n_out, offset):
         assert e < TOL_OP, what
 
 
+@pytest.mark.parametrize("n_in", [32, 544, 2080, 10272, 16416, 32768])
+def test_f16_rows_in_runs(ly, n_in):
+    """F16 products: rows that end inside a run, one run per wave to eight, four and eight waves a workgroup; three matrices
+    of different heights (batches that end inside a matrix) as one launch, the pair, and the accumulating form."""
+    import torch
+
+    rs, heights = lm.Stream(7800 + n_in), (37, 1, 130)
+    ts = [lm.make_tensor(rs, lm.F16, n_in, n) for n in heights]
+    x, nw = rs.sym(n_in, 1.0), (1.0 + rs.sym(n_in, 0.3)).astype(np.float32)
+    bias, y0 = [rs.sym(n, 0.5) for n in heights], rs.sym(heights[0], 1.0)
+    up = lm.make_tensor(rs, lm.F16, n_in, heights[0])
+    xn = ref.rms_norm(x, nw, 1e-5)
+    ws, wu, dx = [dev_bytes(t[1]) for t in ts], dev_bytes(up[1]), _dev(x)
+    ys, yg, ya = [out_buf(n) for n in heights], out_buf(heights[0]), _dev(np.concatenate([y0, np.full(4, 12345.0, np.float32)]))
+    ly.gemv_multi(lm.F16, ws, [_dev(b) for b in bias], ys, list(heights), dx, _dev(nw), 1e-5, n_in)
+    ly.gemv_norm_gate_up_swiglu(lm.F16, ws[0], wu, dx, _dev(nw), 1e-5, yg, n_in, heights[0])
+    ly.gemv_multi(lm.F16, [ws[0]], None, [ya], [heights[0]], dx, None, 0.0, n_in, True)
+    torch.cuda.synchronize()
+    gate = ref.gemv(lm.F16, ts[0][1], xn, n_in, heights[0])
+    checks = [(f"matrix {i}", y, ref.gemv(lm.F16, t[1], xn, n_in, n).astype(np.float64) + b, n) for i, (y, t, b, n) in enumerate(zip(ys, ts, bias, heights))]
+    checks.append(("gate/up", yg, ref.swiglu(gate, ref.gemv(lm.F16, up[1], xn, n_in, heights[0])).astype(np.float64), heights[0]))
+    checks.append(("accumulate", ya, ref.gemv(lm.F16, ts[0][1], x, n_in, heights[0]).astype(np.float64) + y0, heights[0]))
+    for what, y, want, n in checks:
+        got = y.cpu().numpy()
+        assert (got[n:] == 12345.0).all(), f"{what}: rows past n_out were written"
+        assert vec_err(got[:n], want) < TOL_OP, what
+
+
 def test_rms_norm_rows_swiglu_and_in_place(ly):
     import torch
 
