@@ -263,8 +263,9 @@ int decode_impl(const float* q, const uint16_t* kc, const uint16_t* vc, float* o
     a.q = q; a.kc = kc; a.vc = vc; a.out = out; a.d_pos = d_pos;
     a.k_new = k_new; a.v_new = v_new;
     if (rope) {
-        a.n_rot = rope->n_rot; a.theta = rope->theta; a.freq_factors = rope->freq_factors; a.neox = rope->neox;
+        a.n_rot = rope->n_rot; a.freq_factors = rope->freq_factors; a.neox = rope->neox;
         a.rope_angles = rope->angles;
+        if (!rope->angles) a.freq = rope_freq_plan(rope->n_rot, rope->theta);
     }
     a.n_head = n_head; a.n_kv = n_kv; a.n_ctx = n_ctx; a.batch = 1;
     a.r = n_head / n_kv;

@@ -3,6 +3,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <stdint.h>
 
 namespace orin_fa {
@@ -29,6 +30,26 @@ constexpr float kPShift = 7.0f;
 constexpr int kMaxSplits = 256;                 // decode KV splits per KV head, at most
 constexpr size_t kWorkspaceBytes = 8u << 20;    // split-KV partial results
 
+// The rotary frequencies theta^(-2 i / n_rot), as kernels take them: where -2 i / n_rot is exact in fp32 (n_rot a power of
+// two: every model shape) by the doubles theta^(-2 2^k / n_rot), a frequency being the product over the bits k of i -- within
+// a few of a double's ulps of the power, so the same float, for 20 instructions instead of 300.  Else by theta itself.
+struct RopeFreq {
+    double step[8];
+    float theta;
+    int n_rot, by_steps;
+};
+inline RopeFreq rope_freq_plan(int n_rot, float theta) {
+    RopeFreq f{};
+    f.theta = theta;
+    f.n_rot = n_rot;
+    f.by_steps = n_rot > 0 && (n_rot & (n_rot - 1)) == 0 && n_rot <= 512;
+    if (f.by_steps) {
+        double s = pow((double)theta, -2.0 / n_rot);
+        for (int k = 0; k < 8; ++k, s *= s) f.step[k] = s;
+    }
+    return f;
+}
+
 struct FaArgs {
     const float* q;
     const uint16_t* kc;
@@ -42,7 +63,7 @@ struct FaArgs {
     const float* freq_factors; // decode with rotary embedding of q and k_new (n_rot > 0), as rope_launch takes them
     const float* rope_angles;  // optional: (cos, sin) of every pair at this token's position, [n_rot/2][2], from rope_angles_launch
     int n_rot, neox;
-    float theta;
+    RopeFreq freq;
     int n_head, n_kv, n_ctx;
     int n_past, batch; // prefill only
     int r;             // query heads per KV head
@@ -205,15 +226,22 @@ __device__ __forceinline__ void wave_lds_sync() {
 // multiply-adds; the frequency is the double-precision power rounded to fp32, which is what a
 // correctly rounded powf returns (at position 32768 one ulp of the frequency moves the angle by
 // 2e-3 rad).
-__device__ __forceinline__ float rope_freq_base(int i, int n_rot, float theta) {
+__device__ __forceinline__ float rope_freq_of(const RopeFreq& f, int i) {
+    if (!f.by_steps) {
 #pragma clang fp contract(off)
-    const float expo = -2.0f * (float)i / (float)n_rot;
-    return (float)pow((double)theta, (double)expo);
+        const float expo = -2.0f * (float)i / (float)f.n_rot;
+        return (float)pow((double)f.theta, (double)expo);
+    }
+    double r = 1.0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) r *= (i >> k) & 1 ? f.step[k] : 1.0;
+    return (float)r;
 }
-__device__ __forceinline__ float rope_freq(int i, int n_rot, float theta, const float* freq_factors) {
-    float f = rope_freq_base(i, n_rot, theta);
-    if (freq_factors) f /= freq_factors[i];
-    return f;
+__device__ __forceinline__ float rope_freq(int i, const RopeFreq& f, const float* freq_factors) {
+#pragma clang fp contract(off)
+    float r = rope_freq_of(f, i);
+    if (freq_factors) r /= freq_factors[i];
+    return r;
 }
 __device__ __forceinline__ void rope_rotate(float& x0, float& x1, float c, float s) {
 #pragma clang fp contract(off)

@@ -344,7 +344,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
         const int half = a.n_rot / 2;
         if (!rot_early && lane < half) {
             if (!a.rope_angles) {
-                float freq = rope_freq_base(lane, a.n_rot, a.theta);
+                float freq = rope_freq_of(a.freq, lane);
                 if (a.freq_factors) freq /= ff_given;
                 const float ang = (float)pos * freq;
                 cs_given.x = cosf(ang);

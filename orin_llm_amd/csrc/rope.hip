@@ -7,7 +7,7 @@
 // with i + n_rot/2, "normal" pairs 2i with 2i + 1; elements at or past n_rot are left alone.
 // pos = n_past + row / heads (batch form) or *d_pos (single-token form, read on the device).
 //
-// Two kernels: rope4_kernel for the shapes models have (n_rot a multiple of 8, 16-byte aligned
+// Two kernels: rope_pieces_kernel for the shapes models have (n_rot a multiple of 8, 16-byte aligned
 // rows), all 128-bit accesses, and rope_kernel for any even n_rot.  In rope_kernel,
 // every head of a token shares the token's angles, so one thread owns (token, pair, group of up
 // to 8 heads): the block's first threads compute the frequency of each pair once into LDS, each
@@ -23,6 +23,7 @@ namespace orin_fa {
 namespace {
 
 constexpr int kHeadsPerThread = 8;
+typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 
 // The rotated rows and the cache rows are read next by another kernel, on other compute units:
 // streaming stores send them on instead of leaving them dirty in this die's cache until the
@@ -32,12 +33,11 @@ __device__ __forceinline__ void store_stream(float* p, const float4& v) {
 }
 
 template <bool NEOX, bool IND>
-__global__ __launch_bounds__(256) void rope_kernel(float* x, int tokens, int heads, int head_dim, int n_rot,
-                                                   float theta, int n_past, const int* d_pos,
-                                                   const float* freq_factors) {
+__global__ __launch_bounds__(256) void rope_kernel(float* x, int tokens, int heads, int head_dim, const RopeFreq f, int n_past,
+                                                   const int* d_pos, const float* freq_factors) {
 #pragma clang fp contract(off)
     __shared__ float sh_freq[128];
-    const int half = n_rot / 2;
+    const int half = f.n_rot / 2;
     const int n_hgroups = (heads + kHeadsPerThread - 1) / kHeadsPerThread;
     // pair index fastest, then head group, then token; a block covers whole runs of pairs when
     // half divides 256, otherwise every thread computes its own frequency
@@ -61,7 +61,7 @@ __global__ __launch_bounds__(256) void rope_kernel(float* x, int tokens, int hea
         }
     const int pos = IND ? *d_pos : n_past + token;
     if (shared_freq && (int)threadIdx.x < half) {
-        sh_freq[threadIdx.x] = rope_freq(threadIdx.x, n_rot, theta, freq_factors);
+        sh_freq[threadIdx.x] = rope_freq(threadIdx.x, f, freq_factors);
     }
     if (shared_freq) __syncthreads();
     if (!active) return;
@@ -69,7 +69,7 @@ __global__ __launch_bounds__(256) void rope_kernel(float* x, int tokens, int hea
     if (shared_freq) {
         freq = sh_freq[i];
     } else {
-        freq = rope_freq(i, n_rot, theta, freq_factors);
+        freq = rope_freq(i, f, freq_factors);
     }
     const float ang = (float)pos * freq;
     const float c = cosf(ang), s = sinf(ang);
@@ -82,165 +82,144 @@ __global__ __launch_bounds__(256) void rope_kernel(float* x, int tokens, int hea
         }
 }
 
-// The same rotation for the common shapes (n_rot a multiple of 8, rows 16-byte aligned), moved in
-// 16-byte pieces: a thread owns four adjacent pairs of (token, group of up to 4 heads) -- "neox":
-// elements 4j..4j+3 and the four n_rot/2 further on; "normal": elements 8j..8j+7 -- so every
-// load and store is a full 128-bit access that a wave makes on whole cache lines, all of a
-// thread's loads are in flight before its four sines and cosines are formed, and an angle is
-// computed once per four heads.  The frequencies come from a table the block's first n_rot/2
-// threads fill.  Arithmetic per element as in rope_kernel.
-constexpr int kHeadsPerThread4 = 4;
+// The same rotation for the shapes models have (n_rot a multiple of 8, rows 16-byte aligned), and with it, in one launch,
+// the whole of what a prefill layer does ahead of its attention (reference call sites: src/model_gpu.cu:378-382): K rows
+// are also stored to the cache as fp16 (rounded from the rotated fp32 value, as the store kernel rounds what the rotary
+// kernel wrote), V rows are stored.
+//
+// A piece is four adjacent pairs of one head -- "neox": elements 4j..4j+3 and the four n_rot/2 further on; "normal":
+// elements 8j..8j+7 -- so every load and store is a full 128-bit access that a wave makes on whole cache lines.  A block
+// takes a few tokens (as many as it has threads for their angles) and a few heads, of Q, K and V in that order: its
+// threads ask for their pieces, form one (cos, sin) each for the block's table in LDS, and rotate.  These launches are
+// short chains, not bandwidth: a wave issues an instruction every 2 ns, so what counts is how many stand between a
+// thread's start and its stores.  Per thread that is one sine and cosine (four, when a thread formed the angles of its own
+// pieces), no power (a product of doubles the host prepares; 300 instructions) and 32-bit index arithmetic by
+// multiplication (64-bit divisions: 500).  Measured, per launch: 45 tokens
+// of Qwen2.5-1.5B (Q, K and V rows) 4.3 -> 3.0 us, a single token's Q rows 4.0 -> 2.9 us, 301 tokens of Llama-3.2-1B's Q rows
+// 4.1 -> 3.9; 512 tokens of Llama-3-8B (25 MB) stay at the memory's 7.5 us.
+constexpr int kRopeThreads = 256;
 
-template <bool NEOX, bool IND>
-__global__ __launch_bounds__(256) void rope4_kernel(float* x, int tokens, int heads, int head_dim, int n_rot,
-                                                    float theta, int n_past, const int* d_pos,
-                                                    const float* freq_factors) {
+struct RopeArgs {
+    float *q, *k;
+    const float* v;
+    uint16_t *kc, *vc;
+    const int* d_pos;
+    const float* freq_factors;
+    RopeFreq freq;
+    int tokens, n_past, n_ctx, head_dim, n_q, n_k, n_heads; // n_heads = n_q + n_k + V heads
+    int half, quads, block_tokens, block_heads_log2;
+    unsigned half_magic, quads_magic; // x / half = x * magic >> 16, x < 256 (quads: x < 1024)
+};
+
+template <bool NEOX, int U>
+__global__ __launch_bounds__(kRopeThreads) void rope_pieces_kernel(const RopeArgs a) {
 #pragma clang fp contract(off)
-    __shared__ float sh_freq[256];
-    const int half = n_rot / 2, quads = half / 4;
-    const int n_hgroups = (heads + kHeadsPerThread4 - 1) / kHeadsPerThread4;
-    const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
-    const bool active = t < (long long)tokens * n_hgroups * quads;
-    const int qi = (int)(t % quads);
-    const long long th = t / quads;
-    const int hgroup = (int)(th % n_hgroups), token = (int)(th / n_hgroups);
-    const int h0 = hgroup * kHeadsPerThread4;
-    float* row = x + ((size_t)token * heads + h0) * head_dim;
-    const int o0 = NEOX ? 4 * qi : 8 * qi, o1 = NEOX ? 4 * qi + half : 8 * qi + 4;
-    float4 a[kHeadsPerThread4], b[kHeadsPerThread4];
+    __shared__ float2 sh_cs[kRopeThreads];
+    const int tid = threadIdx.x, token0 = (int)blockIdx.x * a.block_tokens, head0 = (int)blockIdx.y << a.block_heads_log2;
+    const int o1 = NEOX ? a.half : 4;
+    float4 lo[U], hi[U];
+    int token[U], head[U], quad[U];
+    bool live[U];
 #pragma unroll
-    for (int u = 0; u < kHeadsPerThread4; ++u)
-        if (active && h0 + u < heads) {
-            a[u] = *reinterpret_cast<const float4*>(row + (size_t)u * head_dim + o0);
-            b[u] = *reinterpret_cast<const float4*>(row + (size_t)u * head_dim + o1);
+    for (int u = 0; u < U; ++u) {
+        const int s = tid + kRopeThreads * u, rest = (int)((unsigned)s * a.quads_magic >> 16);
+        quad[u] = s - rest * a.quads;
+        head[u] = head0 + (rest & ((1 << a.block_heads_log2) - 1));
+        const int t = rest >> a.block_heads_log2;
+        token[u] = token0 + t;
+        live[u] = t < a.block_tokens && token[u] < a.tokens && head[u] < a.n_heads;
+        if (live[u]) {
+            const bool is_q = head[u] < a.n_q, is_k = head[u] < a.n_q + a.n_k;
+            const float* const row = is_q ? a.q + ((size_t)token[u] * a.n_q + head[u]) * a.head_dim
+                                          : (is_k ? a.k : a.v) + ((size_t)token[u] * a.n_k + (head[u] - a.n_q - (is_k ? 0 : a.n_k))) * a.head_dim;
+            const float* const p = row + quad[u] * (NEOX ? 4 : 8);
+            lo[u] = *reinterpret_cast<const float4*>(p);
+            hi[u] = *reinterpret_cast<const float4*>(p + o1);
         }
-    const int pos = IND ? *d_pos : n_past + token;
-    if ((int)threadIdx.x < half) sh_freq[threadIdx.x] = rope_freq(threadIdx.x, n_rot, theta, freq_factors);
-    __syncthreads();
-    if (!active) return;
-    float c[4], sn[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const float ang = (float)pos * sh_freq[4 * qi + e];
-        c[e] = cosf(ang);
-        sn[e] = sinf(ang);
     }
-#pragma unroll
-    for (int u = 0; u < kHeadsPerThread4; ++u)
-        if (h0 + u < heads) {
-            if (NEOX) {
-                rope_rotate(a[u].x, b[u].x, c[0], sn[0]);
-                rope_rotate(a[u].y, b[u].y, c[1], sn[1]);
-                rope_rotate(a[u].z, b[u].z, c[2], sn[2]);
-                rope_rotate(a[u].w, b[u].w, c[3], sn[3]);
-            } else {
-                rope_rotate(a[u].x, a[u].y, c[0], sn[0]);
-                rope_rotate(a[u].z, a[u].w, c[1], sn[1]);
-                rope_rotate(b[u].x, b[u].y, c[2], sn[2]);
-                rope_rotate(b[u].z, b[u].w, c[3], sn[3]);
-            }
-            store_stream(row + (size_t)u * head_dim + o0, a[u]);
-            store_stream(row + (size_t)u * head_dim + o1, b[u]);
+    {
+        const int t = (int)((unsigned)tid * a.half_magic >> 16), i = tid - t * a.half;
+        if (t < a.block_tokens) {
+            const float ang = (float)(a.d_pos ? *a.d_pos : a.n_past + token0 + t) * rope_freq(i, a.freq, a.freq_factors);
+            sh_cs[tid] = float2{cosf(ang), sinf(ang)};
         }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        if (!live[u]) continue;
+        const bool is_q = head[u] < a.n_q, is_k = !is_q && head[u] < a.n_q + a.n_k;
+        if (is_q || is_k) {
+            const float4* const cs = reinterpret_cast<const float4*>(sh_cs + (token[u] - token0) * a.half + 4 * quad[u]);
+            const float4 c01 = cs[0], c23 = cs[1];
+            float4 &x = lo[u], &y = hi[u];
+            if (NEOX) {
+                rope_rotate(x.x, y.x, c01.x, c01.y);
+                rope_rotate(x.y, y.y, c01.z, c01.w);
+                rope_rotate(x.z, y.z, c23.x, c23.y);
+                rope_rotate(x.w, y.w, c23.z, c23.w);
+            } else {
+                rope_rotate(x.x, x.y, c01.x, c01.y);
+                rope_rotate(x.z, x.w, c01.z, c01.w);
+                rope_rotate(y.x, y.y, c23.x, c23.y);
+                rope_rotate(y.z, y.w, c23.z, c23.w);
+            }
+            float* const row = is_q ? a.q + ((size_t)token[u] * a.n_q + head[u]) * a.head_dim : a.k + ((size_t)token[u] * a.n_k + (head[u] - a.n_q)) * a.head_dim;
+            float* const p = row + quad[u] * (NEOX ? 4 : 8);
+            store_stream(p, x);
+            store_stream(p + o1, y);
+        }
+        if (!is_q && a.kc) {
+            const int h = head[u] - a.n_q - (is_k ? 0 : a.n_k);
+            uint16_t* const p = (is_k ? a.kc : a.vc) + ((size_t)h * a.n_ctx + a.n_past + token[u]) * a.head_dim + quad[u] * (NEOX ? 4 : 8);
+            half4_t l, m;
+            l[0] = (_Float16)lo[u].x; l[1] = (_Float16)lo[u].y; l[2] = (_Float16)lo[u].z; l[3] = (_Float16)lo[u].w;
+            m[0] = (_Float16)hi[u].x; m[1] = (_Float16)hi[u].y; m[2] = (_Float16)hi[u].z; m[3] = (_Float16)hi[u].w;
+            __builtin_nontemporal_store(l, reinterpret_cast<half4_t*>(p));
+            __builtin_nontemporal_store(m, reinterpret_cast<half4_t*>(p + o1));
+        }
+    }
 }
 
-// The three launches a prefill layer makes ahead of its attention (reference call sites:
-// src/model_gpu.cu:378-382) in one: blocks [0, nbq) rotate the Q rows as rope4_kernel does,
-// blocks [nbq, nbq + nbk) rotate the K rows, write them back and store them to the cache as
-// fp16 (rounded from the rotated fp32 value, as the store kernel rounds what the rotary kernel
-// wrote), the remaining blocks store the V rows.  n_rot = head_dim, a multiple of 8.
-typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-
-template <bool NEOX>
-__global__ __launch_bounds__(256) void rope_store_kernel(float* q, float* k, const float* v, uint16_t* kc, uint16_t* vc,
-                                                         int tokens, int n_head, int n_kv, int head_dim, int n_ctx,
-                                                         int n_past, float theta, const float* freq_factors,
-                                                         unsigned nbq, unsigned nbk) {
-#pragma clang fp contract(off)
-    __shared__ float sh_freq[256];
-    if (blockIdx.x >= nbq + nbk) { // ---- V rows -> cache ----
-        const int per_row = head_dim / 8;
-        const long long j = (long long)(blockIdx.x - nbq - nbk) * 256 + threadIdx.x;
-        if (j >= (long long)tokens * n_kv * per_row) return;
-        const long long row = j / per_row; // = token * n_kv + head
-        const int piece = (int)(j % per_row), head = (int)(row % n_kv), pos = n_past + (int)(row / n_kv);
-        const float* src = v + row * head_dim + piece * 8;
-        const float4 x0 = *reinterpret_cast<const float4*>(src);
-        const float4 x1 = *reinterpret_cast<const float4*>(src + 4);
-        half8_t h;
-        h[0] = (_Float16)x0.x; h[1] = (_Float16)x0.y; h[2] = (_Float16)x0.z; h[3] = (_Float16)x0.w;
-        h[4] = (_Float16)x1.x; h[5] = (_Float16)x1.y; h[6] = (_Float16)x1.z; h[7] = (_Float16)x1.w;
-        __builtin_nontemporal_store(h, reinterpret_cast<half8_t*>(vc + ((size_t)head * n_ctx + pos) * head_dim + piece * 8));
-        return;
+// n_k, n_v: heads behind the n_q ones that go to the cache (0: the rotation alone).
+hipError_t pieces_launch(RopeArgs a, int n_rot, float theta, int n_v, bool neox, hipStream_t stream) {
+    a.freq = rope_freq_plan(n_rot, theta);
+    a.half = n_rot / 2;
+    a.quads = n_rot / 8;
+    a.n_heads = a.n_q + a.n_k + n_v;
+    a.half_magic = 65536u / a.half + 1;
+    a.quads_magic = 65536u / a.quads + 1;
+    a.block_tokens = kRopeThreads / a.half;
+    if (a.block_tokens > a.tokens) a.block_tokens = a.tokens;
+    // Heads of a block: as many as give every thread a piece, more where that would be over four blocks a CU (the angles
+    // are formed once per block).
+    const int groups = (a.tokens + a.block_tokens - 1) / a.block_tokens, slots = a.block_tokens * a.quads;
+    int u = 1, log2 = 0;
+    auto fill = [&](int pieces) { log2 = 0; while ((slots << (log2 + 1)) <= pieces && (1 << log2) < a.n_heads) ++log2; };
+    for (;; u *= 2) {
+        fill(kRopeThreads * u);
+        if (u == 4 || groups * ((a.n_heads + (1 << log2) - 1) >> log2) <= 1024) break;
     }
-    const bool is_k = blockIdx.x >= nbq;
-    float* const x = is_k ? k : q;
-    const int heads = is_k ? n_kv : n_head;
-    const int n_rot = head_dim, half = n_rot / 2, quads = half / 4;
-    const int n_hgroups = (heads + kHeadsPerThread4 - 1) / kHeadsPerThread4;
-    const long long t = (long long)(blockIdx.x - (is_k ? nbq : 0u)) * 256 + threadIdx.x;
-    const bool active = t < (long long)tokens * n_hgroups * quads;
-    const int qi = (int)(t % quads);
-    const long long th = t / quads;
-    const int hgroup = (int)(th % n_hgroups), token = (int)(th / n_hgroups);
-    const int h0 = hgroup * kHeadsPerThread4;
-    float* row = x + ((size_t)token * heads + h0) * head_dim;
-    const int o0 = NEOX ? 4 * qi : 8 * qi, o1 = NEOX ? 4 * qi + half : 8 * qi + 4;
-    float4 a[kHeadsPerThread4], b[kHeadsPerThread4];
-#pragma unroll
-    for (int u = 0; u < kHeadsPerThread4; ++u)
-        if (active && h0 + u < heads) {
-            a[u] = *reinterpret_cast<const float4*>(row + (size_t)u * head_dim + o0);
-            b[u] = *reinterpret_cast<const float4*>(row + (size_t)u * head_dim + o1);
-        }
-    const int pos = n_past + token;
-    if ((int)threadIdx.x < half) sh_freq[threadIdx.x] = rope_freq(threadIdx.x, n_rot, theta, freq_factors);
-    __syncthreads();
-    if (!active) return;
-    float c[4], sn[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const float ang = (float)pos * sh_freq[4 * qi + e];
-        c[e] = cosf(ang);
-        sn[e] = sinf(ang);
-    }
-#pragma unroll
-    for (int u = 0; u < kHeadsPerThread4; ++u)
-        if (h0 + u < heads) {
-            if (NEOX) {
-                rope_rotate(a[u].x, b[u].x, c[0], sn[0]);
-                rope_rotate(a[u].y, b[u].y, c[1], sn[1]);
-                rope_rotate(a[u].z, b[u].z, c[2], sn[2]);
-                rope_rotate(a[u].w, b[u].w, c[3], sn[3]);
-            } else {
-                rope_rotate(a[u].x, a[u].y, c[0], sn[0]);
-                rope_rotate(a[u].z, a[u].w, c[1], sn[1]);
-                rope_rotate(b[u].x, b[u].y, c[2], sn[2]);
-                rope_rotate(b[u].z, b[u].w, c[3], sn[3]);
-            }
-            store_stream(row + (size_t)u * head_dim + o0, a[u]);
-            store_stream(row + (size_t)u * head_dim + o1, b[u]);
-            if (is_k) {
-                uint16_t* dst = kc + ((size_t)(h0 + u) * n_ctx + pos) * head_dim;
-                half4_t ha, hb;
-                ha[0] = (_Float16)a[u].x; ha[1] = (_Float16)a[u].y; ha[2] = (_Float16)a[u].z; ha[3] = (_Float16)a[u].w;
-                hb[0] = (_Float16)b[u].x; hb[1] = (_Float16)b[u].y; hb[2] = (_Float16)b[u].z; hb[3] = (_Float16)b[u].w;
-                __builtin_nontemporal_store(ha, reinterpret_cast<half4_t*>(dst + o0));
-                __builtin_nontemporal_store(hb, reinterpret_cast<half4_t*>(dst + o1));
-            }
-        }
+    a.block_heads_log2 = log2;
+    const dim3 grid(groups, (a.n_heads + (1 << log2) - 1) >> log2);
+#define ORIN_ROPE_PIECES(U) \
+    if (neox) hipLaunchKernelGGL((rope_pieces_kernel<true, U>), grid, dim3(kRopeThreads), 0, stream, a); \
+    else hipLaunchKernelGGL((rope_pieces_kernel<false, U>), grid, dim3(kRopeThreads), 0, stream, a)
+    if (u == 1) { ORIN_ROPE_PIECES(1); }
+    else if (u == 2) { ORIN_ROPE_PIECES(2); }
+    else { ORIN_ROPE_PIECES(4); }
+#undef ORIN_ROPE_PIECES
+    return hipGetLastError();
 }
 
 // (cos, sin) of every pair at the position *d_pos: what each thread of rope_kernel forms for
 // itself, written out once for callers that rotate several rows of one token (every layer of a
 // decode step rotates by the same angles).
-__global__ __launch_bounds__(64) void rope_angles_kernel(float* angles, int n_rot, float theta, const int* d_pos,
-                                                         const float* freq_factors) {
+__global__ __launch_bounds__(64) void rope_angles_kernel(float* angles, RopeFreq f, const int* d_pos, const float* freq_factors) {
 #pragma clang fp contract(off)
     const int i = blockIdx.x * 64 + threadIdx.x;
-    if (i >= n_rot / 2) return;
-    const float ang = (float)*d_pos * rope_freq(i, n_rot, theta, freq_factors);
+    if (i >= f.n_rot / 2) return;
+    const float ang = (float)*d_pos * rope_freq(i, f, freq_factors);
     angles[2 * i] = cosf(ang);
     angles[2 * i + 1] = sinf(ang);
 }
@@ -252,7 +231,7 @@ hipError_t rope_angles_launch(float* angles, int n_rot, float theta, const int* 
     drop_stale_error();
     const unsigned grid = (unsigned)((n_rot / 2 + 63) / 64);
     if (grid == 0) return hipSuccess;
-    hipLaunchKernelGGL(rope_angles_kernel, dim3(grid), dim3(64), 0, stream, angles, n_rot, theta, d_pos, freq_factors);
+    hipLaunchKernelGGL(rope_angles_kernel, dim3(grid), dim3(64), 0, stream, angles, rope_freq_plan(n_rot, theta), d_pos, freq_factors);
     return hipGetLastError();
 }
 
@@ -267,19 +246,11 @@ hipError_t rope_store_launch(float* q, float* k, const float* v, uint16_t* kc, u
                              int n_kv, int head_dim, int n_ctx, int n_past, float theta, const float* freq_factors,
                              bool neox, hipStream_t stream) {
     drop_stale_error();
-    const int quads = head_dim / 8;
-    auto blocks = [](long long threads) { return (unsigned)((threads + 255) / 256); };
-    const unsigned nbq = blocks((long long)tokens * ((n_head + kHeadsPerThread4 - 1) / kHeadsPerThread4) * quads);
-    const unsigned nbk = blocks((long long)tokens * ((n_kv + kHeadsPerThread4 - 1) / kHeadsPerThread4) * quads);
-    const unsigned nbv = blocks((long long)tokens * n_kv * (head_dim / 8));
-    if (nbq + nbk + nbv == 0) return hipSuccess;
-    if (neox)
-        hipLaunchKernelGGL(rope_store_kernel<true>, dim3(nbq + nbk + nbv), dim3(256), 0, stream, q, k, v, kc, vc, tokens,
-                           n_head, n_kv, head_dim, n_ctx, n_past, theta, freq_factors, nbq, nbk);
-    else
-        hipLaunchKernelGGL(rope_store_kernel<false>, dim3(nbq + nbk + nbv), dim3(256), 0, stream, q, k, v, kc, vc, tokens,
-                           n_head, n_kv, head_dim, n_ctx, n_past, theta, freq_factors, nbq, nbk);
-    return hipGetLastError();
+    if (tokens == 0) return hipSuccess;
+    RopeArgs a{};
+    a.q = q; a.k = k; a.v = v; a.kc = kc; a.vc = vc; a.freq_factors = freq_factors;
+    a.tokens = tokens; a.n_past = n_past; a.n_ctx = n_ctx; a.head_dim = head_dim; a.n_q = n_head; a.n_k = n_kv;
+    return pieces_launch(a, head_dim, theta, n_kv, neox, stream);
 }
 
 hipError_t rope_launch(float* x, int rows, int head_dim, int n_rot, float theta, int n_past, int heads,
@@ -288,18 +259,12 @@ hipError_t rope_launch(float* x, int rows, int head_dim, int n_rot, float theta,
     // batch form: rows = tokens * heads; single-token form: every row belongs to the one token
     const int tokens = d_pos ? 1 : rows / heads;
     const int heads_per_token = d_pos ? rows : heads;
+    if (tokens == 0 || heads_per_token == 0) return hipSuccess;
     if (n_rot % 8 == 0 && n_rot / 2 <= 256 && head_dim % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0) {
-        const int n_hgroups4 = (heads_per_token + kHeadsPerThread4 - 1) / kHeadsPerThread4;
-        const long long threads4 = (long long)tokens * n_hgroups4 * (n_rot / 8);
-        const unsigned grid4 = (unsigned)((threads4 + 255) / 256);
-        if (grid4 == 0) return hipSuccess;
-#define ORIN_ROPE4_LAUNCH(NEOX, IND) \
-    hipLaunchKernelGGL((rope4_kernel<NEOX, IND>), dim3(grid4), dim3(256), 0, stream, x, tokens, heads_per_token, \
-                       head_dim, n_rot, theta, n_past, d_pos, freq_factors)
-        if (neox) { if (d_pos) ORIN_ROPE4_LAUNCH(true, true); else ORIN_ROPE4_LAUNCH(true, false); }
-        else      { if (d_pos) ORIN_ROPE4_LAUNCH(false, true); else ORIN_ROPE4_LAUNCH(false, false); }
-#undef ORIN_ROPE4_LAUNCH
-        return hipGetLastError();
+        RopeArgs a{};
+        a.q = x; a.d_pos = d_pos; a.freq_factors = freq_factors;
+        a.tokens = tokens; a.n_past = n_past; a.head_dim = head_dim; a.n_q = heads_per_token;
+        return pieces_launch(a, n_rot, theta, 0, neox, stream);
     }
     const int n_hgroups = (heads_per_token + kHeadsPerThread - 1) / kHeadsPerThread;
     const long long threads = (long long)tokens * n_hgroups * (n_rot / 2);
@@ -307,7 +272,7 @@ hipError_t rope_launch(float* x, int rows, int head_dim, int n_rot, float theta,
     if (grid == 0) return hipSuccess;
 #define ORIN_ROPE_LAUNCH(NEOX, IND) \
     hipLaunchKernelGGL((rope_kernel<NEOX, IND>), dim3(grid), dim3(256), 0, stream, x, tokens, heads_per_token, \
-                       head_dim, n_rot, theta, n_past, d_pos, freq_factors)
+                       head_dim, rope_freq_plan(n_rot, theta), n_past, d_pos, freq_factors)
     if (neox) { if (d_pos) ORIN_ROPE_LAUNCH(true, true); else ORIN_ROPE_LAUNCH(true, false); }
     else      { if (d_pos) ORIN_ROPE_LAUNCH(false, true); else ORIN_ROPE_LAUNCH(false, false); }
 #undef ORIN_ROPE_LAUNCH

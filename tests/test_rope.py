@@ -108,6 +108,25 @@ def test_rope_batch(fa, case, neox):
     _check(dx.cpu().numpy(), want, x, n_rot, f"rope batch neox={neox} {case}")
 
 
+# how a chunk is cut into blocks: one to thirty-two tokens' angles a block, pieces that do not divide its threads, heads that do
+# not fill its last group, one, two and four pieces a thread, lengths that take the power instead of the steps
+@pytest.mark.gpu
+@pytest.mark.parametrize("neox", [True, False])
+@pytest.mark.parametrize("head_dim,n_rot,heads,tokens", [(16, 16, 3, 33), (128, 40, 5, 7), (96, 96, 1, 301), (128, 128, 14, 1), (128, 128, 33, 511),
+                                                         (128, 128, 40, 513), (256, 256, 7, 3), (512, 512, 2, 2)])
+def test_rope_batch_at_the_edges_of_its_blocks(fa, head_dim, n_rot, heads, tokens, neox):
+    import torch
+    rng = np.random.default_rng(head_dim + tokens)
+    x = rng.standard_normal((tokens * heads, head_dim)).astype(np.float32)
+    want = ref.rope_batch(x, head_dim, n_rot, 1.0e6, 1234, heads, None, neox)
+    guard = torch.full((tokens * heads + 1, head_dim), 7.0, device="cuda")
+    guard[:-1].copy_(torch.from_numpy(x))
+    (fa.rope_neox_batch if neox else fa.rope_normal_batch)(guard, tokens * heads, head_dim, n_rot, 1.0e6, 1234, heads, None)
+    torch.cuda.synchronize()
+    assert (guard[-1] == 7.0).all()
+    _check(guard[:-1].cpu().numpy(), want, x, n_rot, f"rope blocks neox={neox} {head_dim} {n_rot} {heads} {tokens}")
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("neox", [True, False])
 def test_rope_ind_reads_the_position_on_the_device_and_replays(fa, neox):
