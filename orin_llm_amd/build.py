@@ -1,7 +1,9 @@
-"""Builds liborin_fa.so (HIP kernels + C ABI + llm::cuda shim) for gfx950, in-tree, and beside it the two
+"""Builds liborin_fa.so (HIP kernels + C ABI + llm::cuda shim) for gfx950, in-tree, with the extension module that calls it
+from Python (_fastcall.so), and beside it the two
 measurement-aid libraries that bench.py and one GPU test load (liborin_fa_stamps.so, liborin_fa_bench.so)."""
 import os
 import subprocess
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -13,6 +15,9 @@ STAMPED = ("fa_prefill.hip", "fa_decode.hip", "gemv_mfma.hip", "fa_api.hip")
 # Read-only stand-ins and a do-nothing kernel (csrc/bench_aids.hip), a library of their own: the product exports none of them.
 BENCH_LIB = os.path.join(HERE, "liborin_fa_bench.so")
 BENCH_SOURCE = os.path.join(HERE, "csrc", "bench_aids.hip")
+# The eager calls of kernels.py as a CPython extension on top of LIB (csrc/fastcall.c).
+FASTCALL = os.path.join(HERE, "_fastcall.so")
+FASTCALL_SOURCE = os.path.join(HERE, "csrc", "fastcall.c")
 # The cut-off builds: the decode split kernel with parts taken out (-DORIN_FA_DECODE_PROBE=flags, see fa_decode.hip;
 # results wrong by design), one library per flag set, for bench.py's cut-off workloads.  Measurement aids, built
 # only on request: build(probes=True), `python -m orin_llm_amd.build --probes`, or the cut-off workloads themselves.
@@ -86,6 +91,8 @@ def build(verbose=False, probes=False):
     lines.append(_run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC"] + [stamped.get(s, o) for s, o in zip(SOURCES, objs)]
                       + ["-o", STAMPS_LIB]))
     lines.append(_run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", bench_obj, "-o", BENCH_LIB]))
+    lines.append(_run(["gcc", "-O2", "-Wall", "-shared", "-fPIC", "-I" + sysconfig.get_paths()["include"], FASTCALL_SOURCE,
+                       "-L" + HERE, "-l:" + os.path.basename(LIB), "-Wl,-rpath,$ORIGIN", "-o", FASTCALL]))
     for f, o in probes.items():
         lines.append(_run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC"] + [o if s == dec else x for s, x in zip(SOURCES, objs)]
                           + ["-o", PROBE_LIB.format(f)]))

@@ -1,5 +1,5 @@
-"""ctypes mirror of the operator API, same names and argument order as the reference's
-src/kernels.h:8-12,77-81.  Pointer arguments accept torch tensors (device memory) or raw
+"""Python mirror of the operator API, same names and argument order as the reference's src/kernels.h:8-12,77-81: ctypes,
+and an extension module for the calls a program makes eagerly.  Pointer arguments accept torch tensors (device memory) or raw
 integer addresses.  A non-zero return code from the library raises, the Python analogue of
 the reference's print-and-abort (src/common.h:14-22).  There is no fallback: a missing
 library is an ImportError.
@@ -20,6 +20,7 @@ BENCH_LIB_PATH = os.path.join(_HERE, "liborin_fa_bench.so")
 _lib = None
 _stamps_lib = None
 _bench_lib = None
+_fastcall = None
 _stream = None  # what set_stream was last given: the measurement aids launch on it too
 
 
@@ -82,6 +83,20 @@ def lib():
     return _lib
 
 
+def _calls():
+    """The eager calls as an extension module (csrc/fastcall.c): what ctypes spends on a call's arguments is a quarter of
+    a small launch."""
+    global _fastcall
+    if _fastcall is None:
+        lib()  # (says what is missing, if it is)
+        try:
+            from . import _fastcall as m
+        except ImportError as e:
+            raise ImportError(f"{os.path.join(_HERE, '_fastcall.so')} is missing or does not load ({e}): build it with __graft_entry__.build()") from e
+        _fastcall = m
+    return _fastcall
+
+
 def _ptr(x):
     if x is None:
         return None
@@ -119,8 +134,7 @@ def set_workspace(dev_ptr, nbytes):
 
 
 def flash_attention(q, kc, vc, out, n_head, n_kv, head_dim, n_ctx, n_past, batch, scale):
-    rc = lib().orin_fa_prefill(_ptr(q), _ptr(kc), _ptr(vc), _ptr(out), n_head, n_kv, head_dim, n_ctx,
-                               n_past, batch, scale)
+    rc = (_fastcall or _calls()).prefill(q, kc, vc, out, n_head, n_kv, head_dim, n_ctx, n_past, batch, scale)
     if rc != 0:
         raise OrinFaError("flash_attention", rc)
 
@@ -169,8 +183,8 @@ def flash_attention_decode_rope_store_ind(q, k_new, v_new, kc, vc, out, n_head, 
 def rope_store_batch(q, k, v, kc, vc, batch, n_head, n_kv, head_dim, n_ctx, n_past, n_rot, theta, freq_factors=None,
                      neox=True):
     """rope_*_batch on the Q rows and on the K rows, then kv_store_batch, as one call (no counterpart in the reference)."""
-    rc = lib().orin_fa_rope_store_batch(_ptr(q), _ptr(k), _ptr(v), _ptr(kc), _ptr(vc), batch, n_head, n_kv, head_dim,
-                                        n_ctx, n_past, n_rot, theta, _ptr(freq_factors), 1 if neox else 0)
+    rc = (_fastcall or _calls()).rope_store_batch(q, k, v, kc, vc, batch, n_head, n_kv, head_dim, n_ctx, n_past, n_rot, theta,
+                                                  freq_factors, 1 if neox else 0)
     if rc != 0:
         raise OrinFaError("rope_store_batch", rc)
 
@@ -183,13 +197,13 @@ def rope_angles_ind(angles, n_rot, theta, d_pos, freq_factors=None):
 
 
 def rope_neox_batch(x, rows, head_dim, n_rot, theta, n_past, heads, freq_factors=None):
-    rc = lib().orin_fa_rope_batch(_ptr(x), rows, head_dim, n_rot, theta, n_past, heads, _ptr(freq_factors), 1)
+    rc = (_fastcall or _calls()).rope_batch(x, rows, head_dim, n_rot, theta, n_past, heads, freq_factors, 1)
     if rc != 0:
         raise OrinFaError("rope_neox_batch", rc)
 
 
 def rope_normal_batch(x, rows, head_dim, n_rot, theta, n_past, heads, freq_factors=None):
-    rc = lib().orin_fa_rope_batch(_ptr(x), rows, head_dim, n_rot, theta, n_past, heads, _ptr(freq_factors), 0)
+    rc = (_fastcall or _calls()).rope_batch(x, rows, head_dim, n_rot, theta, n_past, heads, freq_factors, 0)
     if rc != 0:
         raise OrinFaError("rope_normal_batch", rc)
 
@@ -207,7 +221,7 @@ def rope_normal_ind(x, rows, head_dim, n_rot, theta, d_pos, freq_factors=None):
 
 
 def kv_store_batch(kc, vc, k, v, heads, head_dim, n_ctx, pos_base, batch):
-    rc = lib().orin_fa_kv_store_batch(_ptr(kc), _ptr(vc), _ptr(k), _ptr(v), heads, head_dim, n_ctx, pos_base, batch)
+    rc = (_fastcall or _calls()).kv_store_batch(kc, vc, k, v, heads, head_dim, n_ctx, pos_base, batch)
     if rc != 0:
         raise OrinFaError("kv_store_batch", rc)
 

@@ -221,3 +221,31 @@ int main(int argc, char**) {
                         "-Wl,--allow-shlib-undefined", "-Wl,-rpath," + os.path.dirname(LIB)],
                        capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
+
+
+def test_eager_calls_take_what_the_wrappers_document():
+    """The extension module behind the eager calls: integers, None and objects with data_ptr() as pointers, keywords, and
+    errors that are not swallowed (the library itself refuses every call here: it has not been initialised)."""
+    from orin_llm_amd import kernels as k
+
+    class Tensor:
+        def data_ptr(self):
+            return 4096
+
+    class Broken:
+        def data_ptr(self):
+            raise ValueError("no storage")
+
+    for call in (lambda: k.flash_attention(Tensor(), 4096, 4096, Tensor(), 12, 2, 128, 4096, n_past=0, batch=45, scale=0.1),
+                 lambda: k.rope_store_batch(1, 2, 3, 4, 5, 45, 12, 2, 128, 4096, 0, 128, 1.0e6, freq_factors=None, neox=False),
+                 lambda: k.rope_neox_batch(Tensor(), 24, 128, 128, 1.0e6, 0, 12), lambda: k.rope_normal_batch(Tensor(), 24, 128, 128, 1.0e6, 0, 12, None),
+                 lambda: k.kv_store_batch(4096, 4096, 4096, 4096, 2, 128, 4096, 0, 45)):
+        with pytest.raises(k.OrinFaError) as e:
+            call()
+        assert e.value.code == -4
+    with pytest.raises(ValueError):
+        k.flash_attention(Broken(), 1, 1, 1, 12, 2, 128, 4096, 0, 45, 0.1)
+    with pytest.raises(TypeError):
+        k.flash_attention(1, 1, 1, 1, 12, 2, 128, 4096, 0, "45", 0.1)
+    with pytest.raises(AttributeError):
+        k.kv_store_batch("cache", 1, 1, 1, 2, 128, 4096, 0, 45)
