@@ -42,28 +42,30 @@ __device__ __forceinline__ void digits8(const float (&x)[8], int e, int n_in, un
         mx = fmaxf(mx, dpp_xor_step(mx, 1));
         sum += dpp_xor_step(sum, 1);
     }
-    // A group that holds an infinity or a NaN gets a NaN scale, so that every row sum it enters is NaN, as the
-    // products of the vector-ALU kernel are (fmaxf above drops a NaN and (int)rintf would turn it into 0; the sum
-    // does not lose it: a sum of floats is finite only if every term is).
-    const float scale = sum - sum == 0.0f ? (mx > 0.0f ? mx / kDigitRange : 1.0f) : __builtin_nanf("");
-    const float inv = 1.0f / scale;
+    // A group that holds an infinity or a NaN gets a NaN scale (sum - sum), so that every row sum it enters is NaN, as the
+    // products of the vector-ALU kernel are (fmaxf above drops a NaN and the conversion would turn it into 0; the sum
+    // does not lose it: a sum of floats is finite only if every term is).  The smallest normal number stands in for a
+    // scale below it (a group of zeros, too): the reciprocal stays finite.  One Newton step on the hardware's
+    // reciprocal: x inv scale = x to the rounding of a division.  (Divisions spelled "/" are ten instructions each, and
+    // every wave of a product passes here with each of its chunks: 135 vector instructions a pass with them, 109 without.)
+    const float scale = fmaxf(mx * (1.0f / kDigitRange), 1.17549435e-38f) + (sum - sum);
+    float inv = __builtin_amdgcn_rcpf(scale);
+    inv = __builtin_fmaf(__builtin_fmaf(-scale, inv, 1.0f), inv, inv);
     // X + 0x808080 carries 128 into each of the three byte positions, so its bytes are the signed
     // digits plus 128 (byte k of X + 0x808080 is ((X >> 8 k) + 128) & 255 with the lower digits'
     // carries already taken out); the exclusive-or takes the 128 off again, byte by byte.
     unsigned z[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) z[i] = ((unsigned)((int)rintf(x[i] * inv)) + 0x808080u) ^ 0x808080u;
+    for (int i = 0; i < 8; ++i) z[i] = (unsigned)((int)rintf(x[i] * inv)) + 0x808080u; // (to even: most of these are halves or quarters, and halves rounded up add up over a row of weights of one sign)
     // byte k of four consecutive elements into one word of plane 2 - k (plane 0 holds the top digits)
     u32x2 plane[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const unsigned pick = (unsigned)k | ((unsigned)(4 + k) << 8); // byte k of the second operand, then of the first
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-            const unsigned t01 = __builtin_amdgcn_perm(z[4 * w + 1], z[4 * w + 0], pick);
-            const unsigned t23 = __builtin_amdgcn_perm(z[4 * w + 3], z[4 * w + 2], pick);
-            plane[2 - k][w] = __builtin_amdgcn_perm(t23, t01, 0x05040100u);
-        }
+    for (int w = 0; w < 2; ++w) {
+        const unsigned lo01 = __builtin_amdgcn_perm(z[4 * w + 1], z[4 * w + 0], 0x05010400u), lo23 = __builtin_amdgcn_perm(z[4 * w + 3], z[4 * w + 2], 0x05010400u); // bytes 0, 0, 1, 1 of two elements
+        const unsigned hi01 = __builtin_amdgcn_perm(z[4 * w + 1], z[4 * w + 0], 0x0c0c0602u), hi23 = __builtin_amdgcn_perm(z[4 * w + 3], z[4 * w + 2], 0x0c0c0602u); // bytes 2, 2
+        plane[2][w] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u) ^ 0x80808080u;
+        plane[1][w] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u) ^ 0x80808080u;
+        plane[0][w] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u) ^ 0x80808080u;
     }
     *reinterpret_cast<u32x2*>(smem + e) = plane[0];
     *reinterpret_cast<u32x2*>(smem + n_in + e) = plane[1];
