@@ -63,9 +63,16 @@ __device__ long long g_gemv_stamps[kStampWgs * 4 * kStampSlots];
 #endif
 
 #include <stdlib.h>
+#include <type_traits>
 
 namespace orin_fa {
 namespace {
+
+// Lane i of a row of 16: lane (i + 8) % 16's value.
+__device__ __forceinline__ float dpp_row_ror8(float v) {
+    const int x = __float_as_int(v);
+    return __int_as_float(__builtin_amdgcn_update_dpp(x, x, 0x128, 0xF, 0xF, false));
+}
 
 // Digits of the (optionally normalised) activation into LDS, in groups of G elements.  Thread t takes
 // elements 8 t .. 8 t + 7 of every kWaves * 512.
@@ -237,228 +244,308 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_mfma_kernel(const GemvArgs a
 // Requires whole 16-row tiles.  (Deeper request queues, three and four items a wave, were slower in both kernels,
 // and so were four-block items: what bounds the kernels after the loads is the vector ALU, about 74 instructions
 // per block and wave for the nibbles, the six-bit pairs and the digit sums.)
-template <int T, bool DUAL, int kWaves, int CB, bool kShortPrologue = false>
-__device__ __forceinline__ void gemv_rows_body(const GemvArgs& a) {
+// Two matrices that become one product (gate, up) share a tile: eight rows of each.  Tiles of sixteen rows of each are
+// half as many, and 896 of them on 256 CUs leave half the CUs with a fourth; 1792 are seven a CU (Llama-3-8B's pair in Q6_K
+// 22.7 -> 20.9 us, Qwen2.5-1.5B's in Q4_K 7.2 -> 6.5 us).
+// The matrices of a launch (q, k, v) have their own stretches of workgroups, one grid row: as grid rows, the shorter
+// ones' empty workgroups were two of three (Llama-3.2-1B's q, k, v in Q8_0 5.9 -> 4.7 us).
+// A launch smaller than the chip is a chain of latencies -- arguments, activation, digits, weights, products, sums, at 2 ns an
+// instruction of a wave -- and this kernel's was cut where it could be: the arguments of the first requests come with the
+// wave (below), the slots are stepped through without a division, the digits are made with one reciprocal and wait for the activation
+// alone, and every wave has one item where the launcher can arrange it.  Per launch, before -> now: output projection of
+// Qwen2.5-1.5B in Q4_K 3.9 -> 3.0 us and of Llama-3-8B 5.6 -> 4.4, q projections 4.3 -> 3.3 and 5.8 -> 4.7, down projections 5.7
+// -> 4.4 and 10.8 -> 8.6 (33 MB, 3.85 TB/s), Qwen2.5-7B's down projection in Q5_K 14.5 -> 11.5 us (47 MB, 4.05 TB/s).
+
+// What a launch's first requests need, in the kernel's leading argument words, which are in a wave's registers when it
+// starts (kernel-argument preload): behind a trip to the argument block and the launch description, and with the
+// divisions that the grid leaves to the kernel, the first weight request left a microsecond after the wave's start.
+struct RowsHead {
+    const void *w0, *w1, *w2; // the launch's matrices (two matrices that become one product: gate, up)
+    const float *x, *norm_w;
+    // of each matrix: tiles a workgroup takes at least | << 6 how many of its workgroups take one more | << 19 its first workgroup
+    unsigned turns0, turns1, turns2;
+    unsigned shape; // blocks of a row - 1 | blocks of a share of it - 1 << 7 | shares that take one more << 14 | workgroups of a share << 18
+};
+constexpr unsigned kMostRowsWgs = 8190, kMostRowsTurns = 62; // what these words have room for
+constexpr int kMostRowsOneTurn = 16383; // (workgroups with one tile each of one matrix)
+constexpr int kMostRowsShares = 16;
+constexpr unsigned kNoMatrix = 8191; // as the first workgroup of a matrix that is not there
+__device__ __forceinline__ int rows_seg(const RowsHead& h, int wg) {
+    const unsigned first1 = h.turns1 >> 19, first2 = h.turns2 >> 19;
+    return wg >= (int)first2 && first2 != kNoMatrix ? 2 : wg >= (int)first1 && first1 != kNoMatrix ? 1 : 0;
+}
+
+// What a launch says of every wave's share, so that nothing between the loads and their uses is under a condition and the
+// compiler's waits are exact: the digits wait for the activation, not for the weights behind it.
+//   kRowsOneItem    every wave has one item (or none): requested, digits, multiplied out, done.  The output and the q, k,
+//                   v projections of most models.
+//   kRowsOnePass, kRowsTwoPasses   several items, over one or two passes of digits: the first item is used as soon as it is
+//                   there.  Only for launches that leave resident places empty, or whose workgroups have one tile or
+//                   two: one that fills the chip with work runs longer this way (Llama-3-8B's gate/up by 1 us), its second
+//                   round of requests getting in the way of the first.
+//   kRowsAny        anything: the digits come behind the wave's first two items.
+enum : int { kRowsAny = 0, kRowsOnePass = 1, kRowsTwoPasses = 2, kRowsOneItem = 3 };
+
+template <int T, bool DUAL, int kWaves, int CB, int kMode>
+__device__ __forceinline__ void gemv_rows_body(const RowsHead h, const GemvArgs& a) {
     using F = MF<T>;
     using L = Lds<F::kGroup>;
     using G = RowsGeom<T, CB>;
-    constexpr int M = DUAL ? 2 : 1, P = G::P, R = G::R, NL = G::NL;
+    constexpr int P = G::P, R = G::R, NL = G::NL;
+    constexpr int kTileOut = DUAL ? 8 : 16; // outputs of a tile: two matrices give eight rows each to its sixteen
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     ROWS_STAMP(0);
-    const GemvSeg seg = a.seg[blockIdx.y];
-    {
-        // Every argument word the kernel reads, asked for here in one batch: left to the compiler the scalar loads
-        // sit ahead of their uses, four dependent trips to the argument block before the first weight request.
-        const int grid_x = gridDim.x;
-        asm volatile("" ::"s"(seg.w), "s"(seg.bias), "s"(seg.y), "s"(seg.n_out), "s"(seg.row_bytes), "s"(a.w_up), "s"(a.x), "s"(a.norm_w),
-                     "s"(a.eps), "s"(a.accumulate), "s"(a.row_bytes), "s"(a.n_seg_types), "s"(a.share_blocks), "s"(a.share_extra), "s"(grid_x));
-    }
-    // (this share's blocks of a row, from what the launcher divided: no division ahead of the first requests)
-    const int b0 = (int)blockIdx.z * a.share_blocks + min((int)blockIdx.z, a.share_extra);
-    const int nb = a.share_blocks + ((int)blockIdx.z < a.share_extra ? 1 : 0);
+    const void* w_mine = h.w0;
+    unsigned turns = h.turns0;
+    unsigned next = h.turns1;
+    const int seg = DUAL ? 0 : rows_seg(h, (int)blockIdx.x);
+    if (seg == 1) w_mine = h.w1, turns = h.turns1, next = h.turns2;
+    if (seg == 2) w_mine = h.w2, turns = h.turns2, next = ~0u;
+    const int seg_wg = (int)blockIdx.x - (int)(turns >> 19), grid_x = (int)min(next >> 19, h.shape >> 18) - (int)(turns >> 19); // among the matrix's workgroups
+    const int nb_row = (int)(h.shape & 0x7fu) + 1, share_blocks = (int)((h.shape >> 7) & 0x7fu) + 1, share_extra = (int)((h.shape >> 14) & 15u);
+    const int n_mine = (int)(turns & 63u) + (seg_wg < (int)((turns >> 6) & 0x1fffu) ? 1 : 0); // tiles of this workgroup, one at least
+    const int b0 = (int)blockIdx.z * share_blocks + min((int)blockIdx.z, share_extra);
+    const int nb = share_blocks + ((int)blockIdx.z < share_extra ? 1 : 0);
     const int n_in = nb << 8;
+    const unsigned row_bytes = (unsigned)nb_row * F::kBlockBytes;
     float* const red = reinterpret_cast<float*>(smem + L::red_off(n_in));
-    const unsigned row_bytes = (unsigned)(a.n_seg_types ? seg.row_bytes : a.row_bytes);
-    const int n_tiles = seg.n_out >> 4;
-    if ((int)blockIdx.x >= n_tiles) return; // (whole workgroup: a shorter matrix of a shared launch)
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); // (scalar: what follows from it stays in scalar registers)
     unsigned char* const transit = smem + L::red_off(n_in) + kRowsRedBytes + wave * G::kWaveBytes;
-    LaneCtx c;
-    c.n = lane & 15; c.g = lane >> 4; c.ln = 0; c.lg = 0; c.src_lane4 = 0;
-    c.am = lane & 15;
-    c.smem = smem;
-    c.pairs = reinterpret_cast<const XPair*>(smem + L::pairs_off(n_in));
-    c.n_in = n_in;
-    c.zero_off = L::zero_off(n_in);
-    const unsigned char* const wbase[2] = {static_cast<const unsigned char*>(seg.w),
-                                           static_cast<const unsigned char*>(DUAL ? a.w_up : seg.w)};
-    const int n_chunks = (nb + CB - 1) / CB;
-    const int my_chunks = wave < n_chunks ? (n_chunks - wave + kWaves - 1) / kWaves : 0;
-    const int n_mine = n_tiles <= (int)gridDim.x ? 1 : (n_tiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
-    const int total = n_mine * my_chunks * M;
-    // slot 64 i + lane of an item: (row, piece), row-major
-    unsigned goff[NL];
-    int loff[NL];
-#pragma unroll
-    for (int i = 0; i < NL; ++i) {
-        const int s = 64 * i + lane, row = s / G::kRowPieces, piece = s - row * G::kRowPieces, blk = piece / P;
-        goff[i] = row < 16 ? (unsigned)row * row_bytes + (unsigned)(blk * F::kBlockBytes + F::piece_off(piece - blk * P)) : 0xffffffffu; // (past the end: cut to the item's last piece below)
-        loff[i] = row < 16 ? (row * R + piece) * 16 : 16 * R * 16;
+    const int n_chunks = (int)((unsigned)(nb + CB - 1) / CB);
+    const int my_chunks = (int)((unsigned)(n_chunks + kWaves - 1 - wave) / kWaves);
+    const int total = n_mine * my_chunks;
+    const bool has_norm = h.norm_w != nullptr;
+    float* const wave_ss = red + 2 * kMaxWaves * 2 * 16;
+    if (kMode != kRowsAny && total == 0) { // (fewer chunks than waves: this wave only leaves its zeros and keeps the barriers' count)
+        if (lane == 0) wave_ss[wave] = 0.0f;
+        for (int t = 0; t < n_mine; ++t) {
+            if (lane < 16) red[(t & 1) * (kMaxWaves * 2 * 16) + wave * 16 + lane] = 0.0f;
+            lds_barrier();
+        }
+        return;
     }
 
     // ---- requests ----
-    int rq_tile = blockIdx.x, rq_c = wave;
-    constexpr int kRing = 2; // items on their way or in use (M divides it: an item's matrix is its slot's)
-    u32x4 buf[kRing][NL];
-    float bias_v[kRing];
-    auto request = [&](u32x4 (&r)[NL], float& bias, int m) {
-        const int cb = min(CB, nb - rq_c * CB);
-        // pieces past the chunk's end in rows above the last are the row's next blocks or the next row's first (fetched,
-        // never used); in the last row they are cut to the last piece
-        const unsigned limit = 15u * row_bytes + (unsigned)((cb - 1) * F::kBlockBytes + F::piece_off(P - 1));
-        const unsigned char* const base = wbase[m] + (size_t)rq_tile * 16 * row_bytes + (size_t)(b0 + rq_c * CB) * F::kBlockBytes;
+    // slot 64 i + lane of an item: (row, piece), row-major
+    unsigned goff[NL];
+    int loff[NL];
+    auto slots = [&] {
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
+            const unsigned s = 64u * i + (unsigned)lane, row = s / G::kRowPieces;
+            const unsigned r = DUAL ? row & 7u : row; // (of its matrix)
+            // (slots past the sixteenth row: cut to the item's last piece by the request -- or some row's first of two matrices --
+            // and to the buffer's spare piece here)
+            if constexpr (F::kBlockBytes == 16 * P) {
+                if constexpr (DUAL) goff[i] = __umul24(r, row_bytes) + 16u * (s - __umul24(row, G::kRowPieces));
+                else goff[i] = __umul24(row, row_bytes - 16u * G::kRowPieces) + 16u * s;
+            } else {
+                const unsigned piece = s - __umul24(row, G::kRowPieces), k = piece >= (unsigned)P ? piece - P : piece;
+                goff[i] = __umul24(r, row_bytes) + (piece >= (unsigned)P ? F::kBlockBytes : 0u) + (unsigned)F::piece_off((int)k);
+            }
+            const unsigned l = 16u * (R == G::kRowPieces ? s : s + row);
+            loff[i] = (int)(64 * i + 63 >= 16 * G::kRowPieces ? min(l, 16u * R * 16u) : l);
+        }
+    };
+    const unsigned char *const w_first = static_cast<const unsigned char*>(w_mine), *const w_second = static_cast<const unsigned char*>(h.w1);
+    int rq_tile = seg_wg, rq_c = wave;
+    size_t rq_off = (size_t)((unsigned)seg_wg * (unsigned)kTileOut) * row_bytes + (size_t)((unsigned)(b0 + wave * CB) * (unsigned)F::kBlockBytes);
+    const size_t next_tile = (size_t)((unsigned)grid_x * (unsigned)kTileOut) * row_bytes - (size_t)((unsigned)(my_chunks * (kWaves * CB)) * (unsigned)F::kBlockBytes);
+    constexpr int kRing = kMode == kRowsOneItem ? 1 : 2; // items on their way or in use
+    u32x4 buf[kRing][NL];
+    float bias_v[kRing];
+    auto request = [&](u32x4 (&r)[NL], bool real = true) {
+        // pieces past the chunk's end in rows above the last are the row's next blocks or the next row's first (fetched,
+        // never used); in the last row they are cut to the last piece
+        unsigned limit = (kTileOut - 1u) * row_bytes + (unsigned)((min(CB, nb - rq_c * CB) - 1) * F::kBlockBytes + F::piece_off(P - 1));
+        if (!real) limit = 0; // (one address for all: the same count of loads on every path)
+        const unsigned char *const first = w_first + rq_off, *const second = w_second + rq_off;
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            // slots 8 * kRowPieces ... are the second matrix's: one instruction at most has both
+            constexpr int kFirst = DUAL ? 8 * G::kRowPieces : 64 * NL;
+            const unsigned char* const base = 64 * i + 63 < kFirst ? first : 64 * i >= kFirst ? second : 64 * i + lane < kFirst ? first : second;
             // whole runs, read once: streaming loads
             if constexpr (F::kAligned) r[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(base + min(goff[i], limit)));
             else r[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_a2*>(base + min(goff[i], limit)));
         }
-        bias = *(seg.bias ? seg.bias + rq_tile * 16 + c.n : a.x); // (always a load: the same count on every path)
-        if (m == M - 1) {
-            rq_c += kWaves;
-            if (rq_c >= n_chunks) {
-                rq_c = wave;
-                rq_tile += (int)gridDim.x;
-            }
+    };
+    auto advance = [&] { // to the next item
+        rq_c += kWaves;
+        rq_off += kWaves * CB * F::kBlockBytes;
+        if (rq_c >= n_chunks) {
+            rq_c = wave;
+            rq_tile += grid_x;
+            rq_off += next_tile;
         }
     };
     // ---- the activation's digits: every wave makes those of its own chunks (it multiplies no others), so
     // nothing waits for another wave before the first tile's end; the norm's sum of squares is put together
-    // there.  The first chunk's loads go out ahead of the weight requests (loads return in order). ----
-    float* const wave_ss = red + 2 * kMaxWaves * 2 * 16;
-    {
-        const float* const ax = a.x + (b0 << 8);
-        const float* const aw = a.norm_w ? a.norm_w + (b0 << 8) : nullptr;
-        XPair* const pairs = reinterpret_cast<XPair*>(smem + L::pairs_off(n_in));
-        float ss = 0.0f;
-        auto fetch = [&](const float* p, int e, float (&v)[8]) {
-            *reinterpret_cast<float4*>(v) = *reinterpret_cast<const float4*>(p + e);
-            *reinterpret_cast<float4*>(v + 4) = *reinterpret_cast<const float4*>(p + e + 4);
-        };
-        auto digits = [&](float (&x)[8], const float (&g)[8], int e) {
-            if (aw) {
+    // there.  A pass is 512 elements: a chunk of two blocks, or two chunks of one.  The first passes' loads go
+    // out ahead of the weight requests (loads return in order). ----
+    const float* const ax = h.x + (b0 << 8);
+    const float* const aw = has_norm ? h.norm_w + (b0 << 8) : ax; // (always a load)
+    XPair* const pairs = reinterpret_cast<XPair*>(smem + L::pairs_off(n_in));
+    const int n_passes = CB == 2 ? my_chunks : (int)((unsigned)(my_chunks + 1) / 2u);
+    const int pass_lane = CB == 2 ? lane * 8 : (lane >> 5) * (kWaves * 256) + (lane & 31) * 8;
+    auto elem = [&](int ps) { return (CB == 2 ? (wave + ps * kWaves) * 512 : (wave + 2 * ps * kWaves) * 256) + pass_lane; };
+    auto fetch = [&](const float* p, int e, float (&v)[8]) {
+        const float4* const q = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(p) + (unsigned)e * 4u); // (scalar base, 32-bit offset)
+        *reinterpret_cast<float4*>(v) = q[0];
+        *reinterpret_cast<float4*>(v + 4) = q[1];
+    };
+    float ss = 0.0f;
+    auto digits = [&](float (&x)[8], const float (&g)[8], int e) {
+        if (has_norm) {
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    ss += x[i] * x[i];
-                    x[i] *= g[i];
-                }
-            }
-            digits8<F::kGroup>(x, e, n_in, smem, pairs, lane);
-        };
-        constexpr int kPasses = (CB * 256 + 511) / 512; // 512 elements a pass
-        // The wave's first kPre chunks are fetched ahead of the weight requests: loads return in order, so fetched
-        // behind them a chunk's few floats wait for two items of weights, and the wave's first item for all its
-        // digits (the stage marks below, read in the timeline build: first digits 1.4 us after the requests, the second chunk's 2.1 us
-        // later, the first item 0.5 us after that).
-        constexpr int kPre = kWaves == 8 ? 2 : 4; // (eight-wave workgroups: fewer chunks a wave, and registers for four waves a SIMD)
-        float xs[kPre][kPasses][8], gs[kPre][kPasses][8]; // (read under the conditions they are loaded under)
-        if (kShortPrologue && kPasses == 1 && total >= kRing && my_chunks <= 2) {
-            // One or two chunks and at least two items: nothing between the loads and their uses is under a
-            // condition (a second chunk the wave does not have is fetched from the row's end and dropped), so the
-            // compiler's waits are exact: the digits wait for the activation, not for the weights behind it, and
-            // the first item is used as soon as it is there.  Only in the kernel for launches that leave resident places empty
-            // (Qwen2.5-1.5B's gate/up 8.1 -> 7.4 us, its down projection 7.25 -> 6.9): a launch that fills the chip
-            // runs 1.5 us longer this way, its second round of requests getting in the way of the first.  Not in
-            // the kernels of eight waves and of mixed types either.
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int e = min((wave + i * kWaves) * CB * 256 + lane * 8, n_in - 8);
-                fetch(ax, e, xs[i][0]);
-                fetch(aw ? aw : ax, e, gs[i][0]);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int j = 0; j < kRing; ++j) request(buf[j], bias_v[j], j % M);
-            __builtin_amdgcn_sched_barrier(0);
-            {
-                const int e = wave * CB * 256 + lane * 8;
-                if (e < min((wave + 1) * CB * 256, n_in)) digits(xs[0][0], gs[0][0], e);
-            }
-            if (my_chunks == 2) {
-                const int e = (wave + kWaves) * CB * 256 + lane * 8;
-                if (e < min((wave + kWaves + 1) * CB * 256, n_in)) digits(xs[1][0], gs[1][0], e);
-            }
-        } else {
-#pragma unroll
-        for (int i = 0; i < kPre; ++i) {
-            const int ch = wave + i * kWaves, end = min((ch + 1) * CB * 256, n_in);
-#pragma unroll
-            for (int ps = 0; ps < kPasses; ++ps) {
-                const int e = ch * CB * 256 + ps * 512 + lane * 8;
-                if (e < end) { // (a chunk past the row's end starts past it)
-                    fetch(ax, e, xs[i][ps]);
-                    if (aw) fetch(aw, e, gs[i][ps]);
-                }
+            for (int i = 0; i < 8; ++i) {
+                ss += x[i] * x[i];
+                x[i] *= g[i];
             }
         }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int j = 0; j < kRing; ++j)
-            if (j < total) request(buf[j], bias_v[j], j % M);
+        digits8<F::kGroup>(x, e, n_in, smem, pairs, lane);
+    };
+    // The wave's first kPre passes are fetched ahead of the weight requests: fetched behind them a chunk's few floats
+    // wait for two items of weights, and the wave's first item for all its digits (the stage marks below, read in the
+    // timeline build: first digits 1.4 us after the requests, the second chunk's 2.1 us later, the first item 0.5 us after
+    // that).
+    constexpr int kPre = kWaves == 8 ? 2 : 4; // (eight-wave workgroups: fewer chunks a wave, and registers for four waves a SIMD)
+    float xs[kPre][8], gs[kPre][8]; // (read under the conditions they are loaded under)
+    // (what follows the requests: the other arguments, in one batch, and what a lane needs to know of itself)
+    float* seg_y;
+    const float* seg_bias;
+    float norm_eps;
+    bool adds;
+    LaneCtx c;
+    typename F::Addr addr;
+    auto request_bias = [&](float& bias, int tile) {
+        if constexpr (!DUAL) bias = *(seg_bias ? seg_bias + tile * 16 + c.n : h.x); // (always a load: the same count on every path)
+    };
+    auto behind_requests = [&] {
         __builtin_amdgcn_sched_barrier(0);
         ROWS_STAMP(1);
+        seg_y = a.seg[seg].y;
+        seg_bias = a.seg[seg].bias;
+        norm_eps = a.eps;
+        adds = a.accumulate || share_blocks != nb_row;
+        asm volatile("" ::"s"(seg_y), "s"(seg_bias), "s"(norm_eps), "s"(a.accumulate));
+        c.n = lane & 15; c.g = lane >> 4; c.ln = 0; c.lg = 0; c.src_lane4 = 0;
+        c.am = lane & 15;
+        c.smem = smem;
+        c.pairs = pairs;
+        c.n_in = n_in;
+        c.zero_off = L::zero_off(n_in);
+        addr = F::addr(c);
+        // (the first items' bias values: the first tile's, except where every item is a tile's last)
+        request_bias(bias_v[0], seg_wg);
+        if constexpr (kRing == 2) request_bias(bias_v[1], my_chunks == 1 && n_mine > 1 ? seg_wg + grid_x : seg_wg);
+        if (lane < 4) reinterpret_cast<unsigned*>(smem + L::zero_off(n_in))[lane] = 0u; // (every wave writes the same zeros)
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if constexpr (kMode != kRowsAny) {
+        constexpr int kPasses = kMode == kRowsTwoPasses ? 2 : 1;
 #pragma unroll
-        for (int i = 0; i < kPre; ++i) {
-            const int ch = wave + i * kWaves, end = min((ch + 1) * CB * 256, n_in);
-#pragma unroll
-            for (int ps = 0; ps < kPasses; ++ps) {
-                const int e = ch * CB * 256 + ps * 512 + lane * 8;
-                if (e < end) digits(xs[i][ps], gs[i][ps], e);
-            }
+        for (int i = 0; i < kPasses; ++i) {
+            const int e = min(elem(i), n_in - 8);
+            fetch(ax, e, xs[i]);
+            fetch(aw, e, gs[i]);
         }
-        for (int ch = wave + kPre * kWaves; ch < n_chunks; ch += kWaves) { // (rows longer still: these loads queue behind the weights)
-            const int end = min((ch + 1) * CB * 256, n_in);
-            for (int e = ch * CB * 256 + lane * 8; e < end; e += 512) {
-                float x[8], g[8] = {};
+        __builtin_amdgcn_sched_barrier(0);
+        slots();
+        request(buf[0]);
+        if constexpr (kRing == 2) {
+            if (total > 1) advance();
+            request(buf[1], total > 1);
+            advance();
+        }
+        behind_requests();
+#pragma unroll
+        for (int i = 0; i < kPasses; ++i) {
+            const int e = elem(i);
+            if (e < n_in) digits(xs[i], gs[i], e);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < kPre; ++i)
+            if (i < n_passes) {
+                const int e = min(elem(i), n_in - 8);
+                fetch(ax, e, xs[i]);
+                fetch(aw, e, gs[i]);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+        slots();
+        if (total > 0) {
+            request(buf[0]);
+            advance();
+        }
+        if (total > 1) {
+            request(buf[1]);
+            advance();
+        }
+        behind_requests();
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // (both items, see above)
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < kPre; ++i)
+            if (i < n_passes) {
+                const int e = elem(i);
+                if (e < n_in) digits(xs[i], gs[i], e);
+            }
+        for (int ps = kPre; ps < n_passes; ++ps) { // (rows longer still: these loads queue behind the weights)
+            const int e = elem(ps);
+            if (e < n_in) {
+                float x[8], g[8];
                 fetch(ax, e, x);
-                if (aw) fetch(aw, e, g);
+                fetch(aw, e, g);
                 digits(x, g, e);
             }
         }
-        }
-        if (lane < 4) reinterpret_cast<unsigned*>(smem + L::zero_off(n_in))[lane] = 0u; // (every wave writes the same zeros)
+    }
+    if (has_norm) {
         ss = wave_sum(ss);
         if (lane == 0) wave_ss[wave] = ss;
     }
     ROWS_STAMP(2);
     [[maybe_unused]] int n_consumed = 0;
-    const bool has_norm = a.norm_w != nullptr;
-    const float norm_n = (float)n_in, norm_eps = a.eps;
-
-    const typename F::Addr addr = F::addr(c);
+    const float norm_n = (float)n_in;
     int set = 0;
-    auto tile_end = [&](int tile, const float (&rowacc)[M], float bias) {
+    auto tile_end = [&](int tile, float rowacc, float bias) {
         float* const mine = red + set * (kMaxWaves * 2 * 16);
         set ^= 1;
-#pragma unroll
-        for (int m = 0; m < M; ++m) {
-            const float t = xor_sum(rowacc[m]);
-            if (c.g == 0) mine[(wave * M + m) * 16 + c.n] = t;
-        }
+        const float t = xor_sum(rowacc);
+        if (c.g == 0) mine[wave * 16 + c.n] = t;
         lds_barrier();
         if (threadIdx.x < 16) {
-            const int r = tile * 16 + (int)threadIdx.x;
-            float rinv = 1.0f;
+            float y = 0.0f;
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) y += mine[w * 16 + threadIdx.x];
             if (has_norm) { // (every wave has left its sum of squares before its first barrier here)
                 float ss = 0.0f;
 #pragma unroll
                 for (int w = 0; w < kWaves; ++w) ss += wave_ss[w];
-                rinv = 1.0f / sqrtf(ss / norm_n + norm_eps);
+                y *= 1.0f / sqrtf(ss / norm_n + norm_eps);
             }
-            float v[M];
-#pragma unroll
-            for (int m = 0; m < M; ++m) {
-                v[m] = 0.0f;
-#pragma unroll
-                for (int w = 0; w < kWaves; ++w) v[m] += mine[(w * M + m) * 16 + threadIdx.x];
-                v[m] *= rinv;
+            if constexpr (DUAL) { // SiLU(gate) * up: rows 0-7 and 8-15
+                const float up = dpp_row_ror8(y);
+                y = y / (1.0f + expf(-y)) * up;
+            } else if (seg_bias && blockIdx.z == 0) {
+                y += bias;
             }
-            float y = v[0];
-            if constexpr (DUAL) y = y / (1.0f + expf(-y)) * v[1]; // SiLU(gate) * up
-            if (seg.bias && blockIdx.z == 0) y += bias;
-            if (gridDim.z > 1 || a.accumulate) atomicAdd(seg.y + r, y); // (one writer a row and share: with one share the sum is the plain one)
-            else seg.y[r] = y;
+            const int r = tile * kTileOut + (int)threadIdx.x;
+            if (!DUAL || threadIdx.x < 8) {
+                if (adds) atomicAdd(seg_y + r, y); // (one writer a row and share: with one share the sum is the plain one)
+                else seg_y[r] = y;
+            }
         }
         ROWS_STAMP(13);
     };
-    if (my_chunks == 0) { // (fewer chunks than waves: this wave only keeps the barriers' count)
-        const float zero[M] = {};
-        for (int t = 0; t < n_mine; ++t) tile_end((int)blockIdx.x + t * (int)gridDim.x, zero, 0.0f);
+    if (kMode == kRowsAny && total == 0) { // (here and not ahead of the requests: the loads' order and waits as they are cost 4 % less)
+        for (int t = 0; t < n_mine; ++t) tile_end(seg_wg + t * grid_x, 0.0f, 0.0f);
         return;
     }
-    int cs_tile = blockIdx.x, cs_c = wave;
-    float rowacc[M] = {};
-    auto consume = [&](const u32x4 (&r)[NL], float bias, int m) {
+    int cs_tile = seg_wg, cs_c = wave;
+    float rowacc = 0.0f;
+    auto consume = [&](const u32x4 (&r)[NL], float bias) {
 #pragma unroll
         for (int i = 0; i < NL; ++i) *reinterpret_cast<u32x4*>(transit + loff[i]) = r[i];
         ROWS_ITEM_STAMP(3 + n_consumed);
@@ -469,41 +556,46 @@ __device__ __forceinline__ void gemv_rows_body(const GemvArgs& a) {
 #pragma unroll
         for (int j = 1; j < CB; ++j)
             if (j < cb) v += F::from_lds(transit + (c.n * R + j * P) * 16, c, addr, cs_c * CB + j);
-        rowacc[m] += v;
-        if (m == M - 1) {
-            cs_c += kWaves;
-            if (cs_c >= n_chunks) {
-                tile_end(cs_tile, rowacc, bias);
-                cs_c = wave;
-                cs_tile += (int)gridDim.x;
-#pragma unroll
-                for (int mm = 0; mm < M; ++mm) rowacc[mm] = 0.0f;
-            }
+        rowacc += v;
+        cs_c += kWaves;
+        if (cs_c >= n_chunks) {
+            tile_end(cs_tile, rowacc, bias);
+            cs_c = wave;
+            cs_tile += grid_x;
+            rowacc = 0.0f;
         }
     };
-    // Steady state: every item consumed is followed by the request kRing items on, which exists: no branch around
-    // a load, so the compiler's wait counts are exact.
-    int k = 0;
-    for (; k + 2 * kRing <= total; k += kRing) {
+    auto request_next = [&](int j) {
+        request_bias(bias_v[j], rq_tile);
+        request(buf[j]);
+        advance();
+    };
+    if constexpr (kRing == 1) {
+        consume(buf[0], bias_v[0]);
+    } else {
+        // Steady state: every item consumed is followed by the request kRing items on, which exists: no branch around
+        // a load, so the compiler's wait counts are exact.
+        int k = 0;
+        for (; k + 2 * kRing <= total; k += kRing) {
 #pragma unroll
-        for (int j = 0; j < kRing; ++j) {
-            consume(buf[j], bias_v[j], j % M);
-            request(buf[j], bias_v[j], j % M);
+            for (int j = 0; j < kRing; ++j) {
+                consume(buf[j], bias_v[j]);
+                request_next(j);
+            }
         }
+        // the last two or three items (or the only one)
+        if (k < total) consume(buf[0], bias_v[0]);
+        if (k + 2 < total) request_next(0);
+        if (k + 1 < total) consume(buf[1], bias_v[1]);
+        if (k + 2 < total) consume(buf[0], bias_v[0]);
     }
-    // the last two or three items (or the only one)
-    if (k < total) consume(buf[0], bias_v[0], 0);
-    if (k + 2 < total) request(buf[0], bias_v[0], 0);
-    if (k + 1 < total) consume(buf[1], bias_v[1], M - 1);
-    if (k + 2 < total) consume(buf[0], bias_v[0], 0);
     ROWS_STAMP(14);
 }
 
-// kShortPrologue: the kernel for launches that leave resident places empty (see the body's prologue): a kernel of
-// its own, because the second path's code alone costs the launches that do not take it a microsecond.
-template <int T, bool DUAL, int kWaves, int CB, bool kShortPrologue = false>
-__global__ __launch_bounds__(kWaves * 64) void gemv_rows_kernel(const GemvArgs a) {
-    gemv_rows_body<T, DUAL, kWaves, CB, kShortPrologue>(a);
+#define ROWS_HEAD_ARGS const void *w0, const void *w1, const void *w2, const float *x, const float *norm_w, unsigned turns0, unsigned turns1, unsigned turns2, unsigned shape
+template <int T, bool DUAL, int kWaves, int CB, int kMode>
+__global__ __launch_bounds__(kWaves * 64) void gemv_rows_kernel(ROWS_HEAD_ARGS, const GemvArgs a) {
+    gemv_rows_body<T, DUAL, kWaves, CB, kMode>(RowsHead{w0, w1, w2, x, norm_w, turns0, turns1, turns2, shape}, a);
 }
 
 // Matrices of different block types in one launch (the q, k, v projections of a file that keeps attn_v in
@@ -519,14 +611,38 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_mfma_mixed_kernel(const Gemv
 }
 
 // The same for the kernel that reads rows in long runs (no Q8_0 there: a file of that format has no other beside it).
-template <int kWaves, int CB>
-__global__ __launch_bounds__(kWaves * 64) void gemv_rows_mixed_kernel(const GemvArgs a) {
-    switch (a.seg[blockIdx.y].type) {
-    case kQ4_K: gemv_rows_body<kQ4_K, false, kWaves, CB>(a); break;
-    case kQ5_K: gemv_rows_body<kQ5_K, false, kWaves, CB>(a); break;
-    default: gemv_rows_body<kQ6_K, false, kWaves, CB>(a); break;
+// (nothing is cut into shares here: RowsHead::shape's bits for those carry the types, two bits each)
+constexpr unsigned rows_type_code(int type) { return type == kQ4_K ? 0u : type == kQ5_K ? 1u : 2u; }
+template <int kWaves, int CB, int kMode>
+__global__ __launch_bounds__(kWaves * 64) void gemv_rows_mixed_kernel(ROWS_HEAD_ARGS, const GemvArgs a) {
+    const RowsHead h{w0, w1, w2, x, norm_w, turns0, turns1, turns2, (shape & ~0x3ff80u) | (shape & 0x7fu) << 7};
+    switch ((shape >> (7 + 2 * rows_seg(h, (int)blockIdx.x))) & 3u) {
+    case rows_type_code(kQ4_K): gemv_rows_body<kQ4_K, false, kWaves, CB, kMode>(h, a); break;
+    case rows_type_code(kQ5_K): gemv_rows_body<kQ5_K, false, kWaves, CB, kMode>(h, a); break;
+    default: gemv_rows_body<kQ6_K, false, kWaves, CB, kMode>(h, a); break;
     }
 }
+
+// The leading arguments of a launch of `wgs` workgroups for every share of a row (as many as the matrices have tiles, or
+// fewer, which then divide over the matrices as the tiles do), and whether they hold it.
+bool rows_head(const GemvArgs& a, int wgs, int shares, RowsHead& h) {
+    const int nb = a.n_in / 256;
+    const void* w[3] = {};
+    unsigned tiles[3] = {}, turns[3] = {kNoMatrix << 19, kNoMatrix << 19, kNoMatrix << 19}, total = 0, first = 0;
+    for (int i = 0; i < a.n_seg; ++i) total += tiles[i] = (unsigned)a.seg[i].n_out / (a.w_up ? 8 : 16);
+    for (int i = 0; i < a.n_seg; ++i) {
+        const unsigned rest = (unsigned)wgs - first, more = (unsigned)(a.n_seg - 1 - i); // (one for every matrix behind this one)
+        const unsigned mine = i + 1 == a.n_seg ? min(rest, tiles[i]) : min(rest - more, max(1u, (unsigned)((size_t)tiles[i] * (unsigned)wgs / total)));
+        if (mine < 1 || tiles[i] / mine > kMostRowsTurns) return false;
+        w[i] = a.seg[i].w;
+        turns[i] = tiles[i] / mine | tiles[i] % mine << 6 | first << 19;
+        first += mine;
+    }
+    h = RowsHead{w[0], a.w_up ? a.w_up : w[1], w[2], a.x, a.norm_w, turns[0], turns[1], turns[2],
+                 (unsigned)(nb - 1) | (unsigned)(nb / shares - 1) << 7 | (unsigned)(nb % shares) << 14 | first << 18};
+    return (first <= kMostRowsWgs || (a.n_seg == 1 && first == tiles[0] && first <= (unsigned)kMostRowsOneTurn)) && shares <= kMostRowsShares && shares <= nb && nb <= 128;
+}
+#define ROWS_HEAD_OF(h) (h).w0, (h).w1, (h).w2, (h).x, (h).norm_w, (h).turns0, (h).turns1, (h).turns2, (h).shape
 
 constexpr size_t kMfmaLdsMax = 96u * 1024u;
 
@@ -546,24 +662,40 @@ int rows_wgs_per_cu(int given) {
     return env ? given : 3;
 }
 
+// Tiles of a launch's matrices: 16 rows, or 8 of each of two.
+int rows_tiles(const GemvArgs& a) {
+    int n = 0;
+    for (int i = 0; i < a.n_seg; ++i) n += a.seg[i].n_out / (a.w_up ? 8 : 16);
+    return n;
+}
+
 int g_rows_resident = 768; // workgroups of four waves the chip holds at once (three a CU; set by the launcher)
 
 template <int T, bool DUAL, int kWaves, int CB>
-bool launch_rows_as(const GemvArgs& a, dim3 grid, int n_in_wg, hipStream_t stream) {
+bool launch_rows_as(const GemvArgs& a, int wgs, int shares, int n_in_wg, hipStream_t stream) {
     const size_t lds = RowsGeom<T, CB>::lds_bytes(n_in_wg, kWaves);
     if (lds > kMfmaLdsMax) return false;
-    GemvArgs b = a;
-    b.share_blocks = (a.n_in / 256) / (int)grid.z;
-    b.share_extra = (a.n_in / 256) % (int)grid.z;
-    // (... and gives a wave one or two chunks: the other kernel's prologue serves more)
-    b.few_workgroups = kWaves == 4 && (int)(grid.x * grid.y * grid.z) <= g_rows_resident * 3 / 4 && (n_in_wg / 256 + CB - 1) / CB <= 2 * kWaves;
+    RowsHead h;
+    if (!rows_head(a, wgs, shares, h)) return false;
+    const dim3 grid(h.shape >> 18, 1, shares);
+    const int per_wave = ((n_in_wg / 256 + CB - 1) / CB + kWaves - 1) / kWaves, passes = CB == 2 ? per_wave : (per_wave + 1) / 2; // of a tile, at most
+    auto go = [&](auto mode) {
+        hipLaunchKernelGGL((gemv_rows_kernel<T, DUAL, kWaves, CB, decltype(mode)::value>), grid, dim3(kWaves * 64), lds, stream, ROWS_HEAD_OF(h), a);
+    };
+    if (per_wave == 1 && wgs == rows_tiles(a)) {
+        go(std::integral_constant<int, kRowsOneItem>());
+        return true;
+    }
     if constexpr (kWaves == 4) {
-        if (b.few_workgroups) {
-            hipLaunchKernelGGL((gemv_rows_kernel<T, DUAL, kWaves, CB, true>), grid, dim3(kWaves * 64), lds, stream, b);
+        // (two matrices' tiles are half as large: up to three tiles for two workgroups)
+        const bool few = DUAL ? wgs * 3 >= rows_tiles(a) * 2 : wgs * shares <= g_rows_resident * 3 / 4;
+        if (few && passes <= 2) {
+            if (passes == 1) go(std::integral_constant<int, kRowsOnePass>());
+            else go(std::integral_constant<int, kRowsTwoPasses>());
             return true;
         }
     }
-    hipLaunchKernelGGL((gemv_rows_kernel<T, DUAL, kWaves, CB>), grid, dim3(kWaves * 64), lds, stream, b);
+    go(std::integral_constant<int, kRowsAny>());
     return true;
 }
 
@@ -574,27 +706,27 @@ bool launch_rows_as(const GemvArgs& a, dim3 grid, int n_in_wg, hipStream_t strea
 bool rows_base_ok(int type, const void* w) { return type != kQ8_0 || (reinterpret_cast<uintptr_t>(w) & 15u) == 0; }
 
 template <int T>
-bool launch_rows(const GemvArgs& a, dim3 grid, bool wide, int nb_wg, hipStream_t stream) {
+bool launch_rows(const GemvArgs& a, int wgs, int shares, bool wide, int nb_wg, hipStream_t stream) {
     if (!rows_enabled()) return false;
     for (int i = 0; i < a.n_seg; ++i)
         if (a.seg[i].n_out % 16 != 0 || !rows_base_ok(T, a.seg[i].w)) return false;
     if (a.w_up && !rows_base_ok(T, a.w_up)) return false;
     const int n_in_wg = nb_wg * 256;
-    if constexpr (T == kQ8_0) { // (272 bytes are a long run already)
-        if (wide) return launch_rows_as<T, false, 8, 1>(a, grid, n_in_wg, stream);
-        return a.w_up ? launch_rows_as<T, true, 4, 1>(a, grid, n_in_wg, stream) : launch_rows_as<T, false, 4, 1>(a, grid, n_in_wg, stream);
+    if constexpr (T == kQ8_0) { // (272 bytes are a long run already: two blocks only where they make one item of a wave's share)
+        if (wide) return nb_wg <= 16 ? launch_rows_as<T, false, 8, 2>(a, wgs, shares, n_in_wg, stream) : launch_rows_as<T, false, 8, 1>(a, wgs, shares, n_in_wg, stream);
+        if (!a.w_up && nb_wg > 4 && nb_wg <= 8 && wgs == rows_tiles(a)) return launch_rows_as<T, false, 4, 2>(a, wgs, shares, n_in_wg, stream);
+        return a.w_up ? launch_rows_as<T, true, 4, 1>(a, wgs, shares, n_in_wg, stream) : launch_rows_as<T, false, 4, 1>(a, wgs, shares, n_in_wg, stream);
     }
-    if (wide) { // (eight waves: never two matrices)
-        return (nb_wg + 7) / 8 <= 1 ? launch_rows_as<T, false, 8, 1>(a, grid, n_in_wg, stream)
-                                    : launch_rows_as<T, false, 8, 2>(a, grid, n_in_wg, stream);
-    }
+    else { // (the other branch returned)
+    if (wide) return launch_rows_as<T, false, 8, 2>(a, wgs, shares, n_in_wg, stream); // (sixteen blocks at least; never two matrices)
     // runs of 288 (352) bytes read within a few percent of longer ones, and the wave's last item, which nothing
     // overlaps, is half as long as with four blocks
     const int cb = min(kRowsMaxCb, (nb_wg + 3) / 4);
     if (a.w_up) {
-        return cb == 1 ? launch_rows_as<T, true, 4, 1>(a, grid, n_in_wg, stream) : launch_rows_as<T, true, 4, 2>(a, grid, n_in_wg, stream);
+        return cb == 1 ? launch_rows_as<T, true, 4, 1>(a, wgs, shares, n_in_wg, stream) : launch_rows_as<T, true, 4, 2>(a, wgs, shares, n_in_wg, stream);
     }
-    return cb == 1 ? launch_rows_as<T, false, 4, 1>(a, grid, n_in_wg, stream) : launch_rows_as<T, false, 4, 2>(a, grid, n_in_wg, stream);
+    return cb == 1 ? launch_rows_as<T, false, 4, 1>(a, wgs, shares, n_in_wg, stream) : launch_rows_as<T, false, 4, 2>(a, wgs, shares, n_in_wg, stream);
+    }
 }
 
 template <int T>
@@ -617,17 +749,28 @@ hipError_t launch(const GemvArgs& a, int cu_count, hipStream_t stream) {
     {
         const int per_cu = rows_wgs_per_cu(a.mfma_wgs_per_cu);
         g_rows_resident = cu_count * 3;
-        dim3 gr = g3;
-        gr.x = min((max_out + 15) / 16, per_cu > 0 ? cu_count * per_cu : (max_out + 15) / 16);
-        // (its LDS buffers let three workgroups of four waves share a CU: no more shares of a row than are resident at once)
+        const int tiles = rows_tiles(a);
+        // One item a wave where a row is short enough: as many workgroups as there are tiles, for the chip to hand out, and
+        // no second turn.  Of two matrices up to 8 blocks (Qwen2.5-1.5B's gate/up in Q4_K 6.5 -> 6.1 us; 16 blocks in workgroups
+        // of eight waves: Llama-3-8B's 15.0 -> 17.4), in Q8_0 up to 4 (its items of two blocks: 9.9 -> 10.2 us); of one
+        // matrix up to 6, which would leave a fourth of the waves of long-lived workgroups without a chunk
+        // (Qwen2.5-1.5B's logits in Q6_K 38.4 -> 35.7 us; 8 blocks: Llama-3.2-1B's in Q5_K 32.6 -> 34.4).
+        const bool one_item = nb_row <= (!a.w_up ? 6 : T == kQ8_0 ? 4 : 8) && tiles <= kMostRowsOneTurn;
+        const int wgs = one_item || per_cu <= 0 ? tiles : min(tiles, cu_count * per_cu);
+        // Shares of a row of a matrix that is accumulated into: up to 8 blocks, so that every wave has one item.  Digits
+        // are each share's own, so more shares make no more of them, and the chip evens out what workgroups of two long
+        // shares a CU did not (Qwen2.5-7B's down projection in Q5_K 13.9 -> 11.5 us, Llama-3-8B's in Q4_K 10.0 -> 8.6).  Smaller
+        // ones where that still leaves CUs empty (output projection of Qwen2.5-1.5B: 3.15 -> 3.0 us).
         int ks_r = ks;
         if (a.k_split_override <= 0) {
-            if (ks == 1 && nb_row >= 6 && a.accumulate && !a.w_up && !a.norm_w && (int)(grid.x * grid.y) <= cu_count) ks_r = 2; // (shorter rows too: a share is cheap here)
-            while (ks_r > 1 && (int)(gr.x * gr.y) * ks_r > cu_count * 3) ks_r /= 2;
+            ks_r = 1;
+            if (a.accumulate && !a.w_up && !a.norm_w && tiles <= cu_count) {
+                ks_r = min((nb_row + 7) / 8, kMostRowsShares);
+                while (tiles * ks_r * 2 <= cu_count && ks_r * 2 <= kMostRowsShares && nb_row >= ks_r * 4) ks_r *= 2;
+            }
         }
-        gr.z = ks_r;
-        const bool wide_r = ks_r == 1 && nb_row >= 16 && !a.w_up && (int)gr.x == (max_out + 15) / 16;
-        if (launch_rows<T>(a, gr, wide_r, (nb_row + ks_r - 1) / ks_r, stream)) return hipGetLastError();
+        const bool wide_r = ks_r == 1 && nb_row >= 16 && !a.w_up && wgs == tiles;
+        if (launch_rows<T>(a, wgs, ks_r, wide_r, (nb_row + ks_r - 1) / ks_r, stream)) return hipGetLastError();
     }
     const size_t lds = lds_bytes<T>((nb_row + ks - 1) / ks * 256);
     if (a.w_up) {
@@ -649,21 +792,28 @@ hipError_t allow() {
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMfmaLdsMax);
 }
 
+hipError_t allow_lds(const void* kernel) { return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMfmaLdsMax); }
+
 template <int T, bool DUAL, int kWaves, int CB>
 hipError_t allow_rows() {
+    hipError_t e;
     if constexpr (kWaves == 4) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemv_rows_kernel<T, DUAL, kWaves, CB, true>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMfmaLdsMax);
-        if (e != hipSuccess) return e;
+        if ((e = allow_lds(reinterpret_cast<const void*>(&gemv_rows_kernel<T, DUAL, kWaves, CB, kRowsOnePass>))) != hipSuccess) return e;
+        if ((e = allow_lds(reinterpret_cast<const void*>(&gemv_rows_kernel<T, DUAL, kWaves, CB, kRowsTwoPasses>))) != hipSuccess) return e;
     }
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(&gemv_rows_kernel<T, DUAL, kWaves, CB>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMfmaLdsMax);
+    if ((e = allow_lds(reinterpret_cast<const void*>(&gemv_rows_kernel<T, DUAL, kWaves, CB, kRowsOneItem>))) != hipSuccess) return e;
+    return allow_lds(reinterpret_cast<const void*>(&gemv_rows_kernel<T, DUAL, kWaves, CB, kRowsAny>));
+}
+
+template <int kWaves, int CB>
+hipError_t allow_mixed() {
+    const hipError_t e = allow_lds(reinterpret_cast<const void*>(&gemv_rows_mixed_kernel<kWaves, CB, kRowsOneItem>));
+    return e != hipSuccess ? e : allow_lds(reinterpret_cast<const void*>(&gemv_rows_mixed_kernel<kWaves, CB, kRowsAny>));
 }
 
 template <int T>
 hipError_t allow_rows_all() {
     hipError_t e;
-    if ((e = allow_rows<T, false, 8, 1>()) != hipSuccess) return e;
     if ((e = allow_rows<T, false, 8, 2>()) != hipSuccess) return e;
     if ((e = allow_rows<T, false, 4, 1>()) != hipSuccess) return e;
     if ((e = allow_rows<T, false, 4, 2>()) != hipSuccess) return e;
@@ -683,28 +833,30 @@ hipError_t gemv_mfma_mixed_launch(GemvArgs a, int cu_count, hipStream_t stream) 
     a.n_seg_types = 1;
     bool rows = rows_enabled();
     for (int i = 0; i < a.n_seg; ++i) rows = rows && a.seg[i].n_out % 16 == 0 && a.seg[i].type != kQ8_0;
-    a.share_blocks = a.n_in / 256; // (one share: whole rows)
-    a.share_extra = 0;
-    a.few_workgroups = 0;
     if (rows) {
         const int per_cu = rows_wgs_per_cu(a.mfma_wgs_per_cu), nb = a.n_in / 256;
-        const dim3 gr(min((max_out + 15) / 16, per_cu > 0 ? cu_count * per_cu : (max_out + 15) / 16), a.n_seg);
-        const bool wide_r = nb >= 16 && (int)gr.x == (max_out + 15) / 16;
-        // (the largest of the types' layouts: Q6_K's digits in groups of 16, Q5_K's 11 pieces a block are within Q6_K's 14)
-        if (wide_r) {
-            const size_t lds = RowsGeom<kQ6_K, 2>::lds_bytes(a.n_in, 8);
-            if (lds <= kMfmaLdsMax) {
-                if ((nb + 7) / 8 <= 1) hipLaunchKernelGGL((gemv_rows_mixed_kernel<8, 1>), gr, dim3(512), lds, stream, a);
-                else hipLaunchKernelGGL((gemv_rows_mixed_kernel<8, 2>), gr, dim3(512), lds, stream, a);
-                return hipGetLastError();
-            }
-        } else {
-            const size_t lds = RowsGeom<kQ6_K, 2>::lds_bytes(a.n_in, 4);
-            if (lds <= kMfmaLdsMax) {
-                if ((nb + 3) / 4 <= 1) hipLaunchKernelGGL((gemv_rows_mixed_kernel<4, 1>), gr, dim3(256), lds, stream, a);
-                else hipLaunchKernelGGL((gemv_rows_mixed_kernel<4, 2>), gr, dim3(256), lds, stream, a);
-                return hipGetLastError();
-            }
+        const int tiles = rows_tiles(a);
+        const int wgs = per_cu > 0 ? min(tiles, cu_count * per_cu) : tiles;
+        const bool wide_r = nb >= 16 && wgs == tiles;
+        RowsHead h;
+        if (rows_head(a, wgs, 1, h)) {
+            h.shape &= ~0x3ff80u;
+            for (int i = 0; i < a.n_seg; ++i) h.shape |= rows_type_code(a.seg[i].type) << (7 + 2 * i);
+            auto go = [&](auto waves, auto blocks) {
+                constexpr int W = decltype(waves)::value, CB = decltype(blocks)::value;
+                // (the largest of the types' layouts: Q6_K's digits in groups of 16, Q5_K's 11 pieces a block are within Q6_K's 14)
+                const size_t lds = RowsGeom<kQ6_K, CB>::lds_bytes(a.n_in, W);
+                if (lds > kMfmaLdsMax) return false;
+                const dim3 gr(h.shape >> 18), block(W * 64);
+                if (nb <= W * CB && wgs == tiles) hipLaunchKernelGGL((gemv_rows_mixed_kernel<W, CB, kRowsOneItem>), gr, block, lds, stream, ROWS_HEAD_OF(h), a);
+                else hipLaunchKernelGGL((gemv_rows_mixed_kernel<W, CB, kRowsAny>), gr, block, lds, stream, ROWS_HEAD_OF(h), a);
+                return true;
+            };
+            using One = std::integral_constant<int, 1>;
+            using Two = std::integral_constant<int, 2>;
+            const bool done = wide_r ? go(std::integral_constant<int, 8>(), Two())
+                                     : (nb <= 4 ? go(std::integral_constant<int, 4>(), One()) : go(std::integral_constant<int, 4>(), Two()));
+            if (done) return hipGetLastError();
         }
     }
     const size_t lds = max(lds_bytes<kQ4_K>(a.n_in), lds_bytes<kQ6_K>(a.n_in));
@@ -747,12 +899,13 @@ hipError_t gemv_mfma_allow_lds() {
     if ((e = allow_rows_all<kQ5_K>()) != hipSuccess) return e;
     if ((e = allow_rows_all<kQ6_K>()) != hipSuccess) return e;
     if ((e = allow_rows<kQ8_0, false, 8, 1>()) != hipSuccess) return e;
+    if ((e = allow_rows<kQ8_0, false, 8, 2>()) != hipSuccess) return e;
+    if ((e = allow_rows<kQ8_0, false, 4, 2>()) != hipSuccess) return e;
     if ((e = allow_rows<kQ8_0, false, 4, 1>()) != hipSuccess) return e;
     if ((e = allow_rows<kQ8_0, true, 4, 1>()) != hipSuccess) return e;
-    if ((e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemv_rows_mixed_kernel<8, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMfmaLdsMax)) != hipSuccess) return e;
-    if ((e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemv_rows_mixed_kernel<8, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMfmaLdsMax)) != hipSuccess) return e;
-    if ((e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemv_rows_mixed_kernel<4, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMfmaLdsMax)) != hipSuccess) return e;
-    if ((e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemv_rows_mixed_kernel<4, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMfmaLdsMax)) != hipSuccess) return e;
+    if ((e = allow_mixed<8, 2>()) != hipSuccess) return e;
+    if ((e = allow_mixed<4, 1>()) != hipSuccess) return e;
+    if ((e = allow_mixed<4, 2>()) != hipSuccess) return e;
     if ((e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemv_mfma_mixed_kernel<8>),
                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMfmaLdsMax)) != hipSuccess) return e;
     return hipFuncSetAttribute(reinterpret_cast<const void*>(&gemv_mfma_mixed_kernel<4>),

@@ -613,3 +613,53 @@ def test_whole_model_against_reference_logits(fa, ly, name, how):
         worst_g = max(worst_g, vec_err(got, golden["logits_" + name][t].astype(np.float64)))
     print(f"{name} {how}: vs oracle (fp16 cache) {worst_o:.2e}, vs reference logits (fp32 cache) {worst_g:.2e}", flush=True)
     assert worst_o < TOL_OP * 50 and worst_g < TOL_MODEL
+
+
+@pytest.mark.parametrize("types", [(4, 4, 4), (5, 5, 5), (6, 6, 6), (8, 8, 8), (4, 4, 6), (6, 5, 4)])
+@pytest.mark.parametrize("n_in,heights", [(256, (16, 16, 32)), (1280, (16, 4128, 32)), (2048, (3088, 48, 16)), (2304, (64, 16, 16)),
+                                          (3584, (48, 16, 8240)), (4096, (2064, 1024, 1024)), (4352, (96, 48, 16)), (9472, (48, 32, 16))])
+def test_workgroups_and_shares_of_rows_in_runs(ly, types, n_in, heights):
+    """Matrices of whole row tiles: one item a wave, several over one pass of digits or two, and whatever is longer; workgroups
+    with one tile and with more, three matrices of a launch that get different numbers of workgroups (in one block type
+    and in several), the pair's tiles of eight rows of each, and shares of a row."""
+    import torch
+
+    ly.use_matrix_cores(True)
+    wt = [{4: lm.Q4_K, 5: lm.Q5_K, 6: lm.Q6_K, 8: lm.Q8_0}[t] for t in types]
+    rs = lm.Stream(7900 + n_in + sum(heights) + sum(types))
+    ts = [lm.make_tensor(rs, t, n_in, n) for t, n in zip(wt, heights)]
+    up = lm.make_tensor(rs, wt[0], n_in, heights[0])
+    x, nw, eps = rs.sym(n_in, 1.0), (1.0 + rs.sym(n_in, 0.3)).astype(np.float32), 1e-5
+    bias, y0 = [rs.sym(n, 0.5) for n in heights], rs.sym(heights[0], 1.0)
+    ws, wu, dx, dnw = [dev_bytes(t[1]) for t in ts], dev_bytes(up[1]), _dev(x), _dev(nw)
+    ys, yg, ya = [out_buf(n) for n in heights], out_buf(heights[0]), _dev(np.concatenate([y0, np.full(4, 12345.0, np.float32)]))
+    ly.gemv_multi_types(wt, ws, [_dev(b) for b in bias], ys, list(heights), dx, dnw, eps, n_in)
+    ly.gemv_norm_gate_up_swiglu(wt[0], ws[0], wu, dx, dnw, eps, yg, n_in, heights[0])
+    ly.gemv_multi(wt[0], [ws[0]], None, [ya], [heights[0]], dx, None, 0.0, n_in, True)
+    torch.cuda.synchronize()
+    xn = ref.rms_norm(x, nw, eps)
+    normed = [ref.gemv(t, m[1], xn, n_in, n) for t, m, n in zip(wt, ts, heights)]
+    act = ref.swiglu(normed[0], ref.gemv(wt[0], up[1], xn, n_in, heights[0])).astype(np.float64)
+    added = ref.gemv(wt[0], ts[0][1], x, n_in, heights[0]).astype(np.float64) + y0
+    checks = [(f"matrix {i}", ys[i], normed[i].astype(np.float64) + bias[i], heights[i]) for i in range(3)]
+    for what, y, want, n in checks + [("gate/up", yg, act, heights[0]), ("accumulate", ya, added, heights[0])]:
+        got = y.cpu().numpy()
+        assert (got[n:] == 12345.0).all(), f"{what}: rows past n_out were written"
+        e = vec_err(got[:n], want)
+        print(f"{types} {n_in} x {heights} {what}: err {e:.2e}", flush=True)
+        assert e < TOL_OP, what
+
+
+@pytest.mark.parametrize("n_in", [256, 1792])
+def test_more_row_tiles_than_a_launch_counts_workgroups_for(ly, n_in):
+    """A vocabulary's worth of rows: 8200 tiles, one workgroup each or several tiles a workgroup."""
+    import torch
+
+    n_out, rs = 131200, lm.Stream(7950 + n_in)
+    t, x = lm.make_tensor(rs, lm.Q4_K, n_in, n_out), rs.sym(n_in, 1.0)
+    y = out_buf(n_out)
+    ly.gemv_multi(lm.Q4_K, [dev_bytes(t[1])], None, [y], [n_out], _dev(x), None, 0.0, n_in)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy()
+    assert (got[n_out:] == 12345.0).all()
+    assert vec_err(got[:n_out], ref.gemv(lm.Q4_K, t[1], x, n_in, n_out).astype(np.float64)) < TOL_OP
