@@ -20,11 +20,14 @@
 //     so the launch can be captured in a graph and replayed after the position changes.  The
 //     position and the query heads are requested together, first thing; a split that the
 //     position leaves without a tile exits without having touched the cache (at a short
-//     position in a long cache that is nearly all of them).  Tiles are fetched whole: rows at
+//     position in a long cache that is nearly all of them), and so does a wave without one, on its
+//     way to the merge.  Tiles are fetched whole: rows at
 //     or past the position are masked (K) or zeroed on their way into LDS (V).
 //   * Partials (reference maximum, row sum, O) of the 8 waves are merged through LDS and
 //     written per split; the combine kernel merges the splits that were active.
 #include "fa_common.hpp"
+
+#include <type_traits>
 
 // Stage marks: wall-clock stamps in the timeline build, nothing otherwise (fa_common.hpp).
 #ifdef ORIN_FA_STAMPS
@@ -104,7 +107,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
     FA_STAMP(0);
 
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15; // MFMA column (query head of the group) / row (KV row or head_dim index) of the lane
     const int grp = lane >> 4; // lane-group: 8-wide k slice of an operand, 4-row slice of an accumulator
 
@@ -116,6 +119,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
     float* const part_ml = dst + (size_t)n_splits * n_head * D; // [n_head][split][2]
 
     unsigned char* const vs = smem + wave * G::kWaveB;
+
     const __amdgpu_buffer_rsrc_t krs = make_rsrc(kc + (size_t)kvh * n_ctx * D, (unsigned)n_ctx * D * 2);
     const __amdgpu_buffer_rsrc_t vrs = make_rsrc(vc + (size_t)kvh * n_ctx * D, (unsigned)n_ctx * D * 2);
 
@@ -221,7 +225,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
     int tile = tile_first;
     float* const qs = reinterpret_cast<float*>(smem + G::kQOff);
     __shared__ __attribute__((aligned(16))) float sh_cs_all[ROPE ? kWaves : 1][D / 2][2];
-    __shared__ __attribute__((aligned(16))) float sh_krow_all[STORE ? kWaves : 1][D];
+    __shared__ __attribute__((aligned(16))) _Float16 sh_krow_all[STORE ? kWaves : 1][D];
     float (*const sh_cs)[2] = sh_cs_all[ROPE ? wave : 0];
     const bool rot_early = ROPE && !a.neox && a.rope_angles != nullptr; // (the query is rotated piece by piece before it is parked)
     if (id * wu < n_tiles) {
@@ -261,10 +265,6 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
         }
         *reinterpret_cast<float4*>(qs + col * G::kQStride + (q_piece >> 1) * 32 + grp * 8 + (q_piece & 1) * 4) = q_park;
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        fetch_k(tile);
-        fetch_v(tile);
-        asm volatile("" ::: "memory"); // (as above: ahead of the conversions that follow, not behind them)
-        __builtin_amdgcn_sched_barrier(0);
     }
     if (id * wu >= n_tiles) {
         // Inactive split: it leaves "no row seen" for its heads, so that the combine kernel can tell
@@ -278,280 +278,305 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
         return;
     }
 
-    FA_STAMP(1);
-    if constexpr (kProbeCutOff) { // (cut-off build: wait for the tile, keep every load alive, leave)
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        unsigned acc = __float_as_uint(q_share.x) ^ __float_as_uint(q_share.w);
-#pragma unroll
-        for (int i = 0; i < 2 * G::kSteps; ++i) acc ^= kreg[i].x ^ kreg[i].y ^ kreg[i].z ^ kreg[i].w;
-#pragma unroll
-        for (int i = 0; i < G::kLoads; ++i) acc ^= vreg[i].x ^ vreg[i].y ^ vreg[i].z ^ vreg[i].w;
-        if (acc == 0x9E3779B9u) part_ml[0] = 1.0f;
-        if (acc != 0x9E3779BAu) return;
-    }
-    // (the query pieces met ahead of the tile requests; the operands are picked up while the first tile is on its way)
-    float qf[G::kSteps][8]; // this lane's 8 elements of every k-step: head_dim indices kk*32 + grp*8 + 0..7
-#pragma unroll
-    for (int kk = 0; kk < G::kSteps; ++kk) {
-        const float4 x0 = *reinterpret_cast<const float4*>(qs + col * G::kQStride + kk * 32 + grp * 8);
-        const float4 x1 = *reinterpret_cast<const float4*>(qs + col * G::kQStride + kk * 32 + grp * 8 + 4);
-        qf[kk][0] = x0.x; qf[kk][1] = x0.y; qf[kk][2] = x0.z; qf[kk][3] = x0.w;
-        qf[kk][4] = x1.x; qf[kk][5] = x1.y; qf[kk][6] = x1.z; qf[kk][7] = x1.w;
-    }
-    // (rotate + store) the rotation of this lane's 8 elements of every k-step, by the wave's table
-    // x0, x1: this lane's elements of k-steps kk and kk + kSteps/2 (head_dim indices kk*32 + grp*8 + e
-    // and the same + head_dim/2)
-    auto rotate2 = [&](float (&x0)[8], float (&x1)[8], int kk) {
-        if (a.neox) { // n_rot == D (checked by the host): element e pairs with e + D/2
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int i = kk * 32 + grp * 8 + e;
-                rope_rotate(x0[e], x1[e], sh_cs[i][0], sh_cs[i][1]);
-            }
-        } else {      // elements 2i and 2i + 1, below n_rot
-            // No branch per pair: el0 differs from lane to lane, and a branch around each pair's table
-            // read makes the wave wait out sixteen LDS round trips one after the other (1.7 us of a
-            // Llama-3-8B launch).  Every lane reads an entry (its own, or the table's last), all reads
-            // go out together, and a pair past n_rot keeps its values by a select.
-            const int last = max(a.n_rot / 2 - 1, 0); // (n_rot = 0: nothing is rotated, entry 0 is read and not used)
-            float2 cs0[4], cs1[4];
-#pragma unroll
-            for (int e = 0; e < 8; e += 2) {
-                const int el0 = kk * 32 + grp * 8 + e, el1 = el0 + D / 2;
-                cs0[e / 2] = *reinterpret_cast<const float2*>(sh_cs[min(el0 / 2, last)]);
-                cs1[e / 2] = *reinterpret_cast<const float2*>(sh_cs[min(el1 / 2, last)]);
-            }
-#pragma unroll
-            for (int e = 0; e < 8; e += 2) {
-                const int el0 = kk * 32 + grp * 8 + e, el1 = el0 + D / 2;
-                float a0 = x0[e], a1 = x0[e + 1], b0 = x1[e], b1 = x1[e + 1];
-                rope_rotate(a0, a1, cs0[e / 2].x, cs0[e / 2].y);
-                rope_rotate(b0, b1, cs1[e / 2].x, cs1[e / 2].y);
-                x0[e] = el0 < a.n_rot ? a0 : x0[e];
-                x0[e + 1] = el0 < a.n_rot ? a1 : x0[e + 1];
-                x1[e] = el1 < a.n_rot ? b0 : x1[e];
-                x1[e + 1] = el1 < a.n_rot ? b1 : x1[e + 1];
-            }
-        }
-    };
-    if constexpr (ROPE) {
-        // (cos, sin) of pair i at the raw position, as the rotary kernel forms them
-        // A table per wave (head_dim <= 128: a wave's 64 lanes cover the pairs), so that no wave
-        // waits here for the others: the waves of a workgroup get their loads out at very
-        // different times when the whole chip is requesting its first tiles.  Write and reads
-        // are the same wave's, and a wave's LDS operations complete in order.
-        static_assert(D / 2 <= 64, "one lane per pair");
-        const int half = a.n_rot / 2;
-        if (!rot_early && lane < half) {
-            if (!a.rope_angles) {
-                float freq = rope_freq_of(a.freq, lane);
-                if (a.freq_factors) freq /= ff_given;
-                const float ang = (float)pos * freq;
-                cs_given.x = cosf(ang);
-                cs_given.y = sinf(ang);
-            }
-            sh_cs[lane][0] = cs_given.x;
-            sh_cs[lane][1] = cs_given.y;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (!rot_early) {
-#pragma unroll
-            for (int kk = 0; kk < G::kSteps / 2; ++kk) rotate2(qf[kk], qf[kk + G::kSteps / 2], kk);
-        }
-    }
-    // ---- query heads -> B operands, fp16 hi + lo ----
-    h8 qhi[G::kSteps], qlo[G::kSteps];
-#pragma unroll
-    for (int kk = 0; kk < G::kSteps; ++kk) {
-        const float* x = qf[kk];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const float xe = x[e] * qmul;
-            qhi[kk][e] = (_Float16)xe;
-            qlo[kk][e] = (_Float16)(xe - (float)qhi[kk][e]);
-        }
-    }
-
-    __builtin_amdgcn_sched_barrier(0);
-    FA_STAMP(2);
     // m_ref: reference maximum of the raw scores (before the scale); l_run: this lane's share of
     // the row sum; o: O^T accumulators, lane (col, grp) holds head_dim rows db*16 + grp*4 + i.
     float m_ref = -INFINITY, l_run = 0.0f;
     f4 o[G::kDBlk];
 #pragma unroll
     for (int db = 0; db < G::kDBlk; ++db) o[db] = f4{0.f, 0.f, 0.f, 0.f};
-    const int v_rd = (grp * 4 + (col >> 2)) * G::kRowBV + (col & 3) * 8; // + h*16 rows, + db*32 bytes
-
-    // (store, rotate + store) The new row is made ready here, while the tiles travel, by the one wave whose tiles
-    // include the row's (the last visible tile: the wave's own last): converted -- and the K row rotated -- as the
-    // store kernel and the rotary kernel would, the pieces this lane is to substitute and to write kept in
-    // registers.  At that tile only the substitution and the two cache writes are left.  (Made ready at the tile
-    // itself, as it used to be, the LDS round trips and the rotation sat between the arrival of the launch's last
-    // tile and its products: 0.7 us of a Qwen2.5-1.5B launch pair at 32k.)  The row's loads went out ahead of the
-    // tile requests, so waiting for them waits for no tile.
-    const int own_tile = n_tiles - 1;
-    [[maybe_unused]] bool owner = false;
-    [[maybe_unused]] u32x4 k_new16[G::kSteps], v_new16 = u32x4{0u, 0u, 0u, 0u};
-    if constexpr (STORE) {
+    // A wave without a tile (most, at a short position) goes straight to the merge.  (Asking for some tile all the same, so as
+    // to keep loads out of branches, seven such waves kept their CU's load unit busy for 1.2 us ahead of the eighth's
+    // values: Qwen2.5-1.5B at position 200 of 4096 6.7 -> 5.9 us a launch pair, Qwen2.5-7B at 2000 of 32768 8.0 -> 6.7.)
+    if (tile < n_tiles) {
+        fetch_k(tile);
+        fetch_v(tile);
+        asm volatile("" ::: "memory"); // (as above: ahead of the conversions that follow, not behind them)
+        __builtin_amdgcn_sched_barrier(0);
+        FA_STAMP(1);
+        if constexpr (kProbeCutOff) { // (cut-off build: wait for the tile, keep every load alive, leave)
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            unsigned acc = __float_as_uint(q_share.x) ^ __float_as_uint(q_share.w);
 #pragma unroll
-        for (int kk = 0; kk < G::kSteps; ++kk) k_new16[kk] = u32x4{0u, 0u, 0u, 0u};
-        owner = store && tile_first <= own_tile && (own_tile - tile_first) % tile_step == 0;
-        if (owner) {
-            // (Nothing below may be started ahead of this branch: the compiler would otherwise
-            // convert the new row in every wave.)
-            auto here = [](float x) { // a copy the compiler cannot make anywhere else
-                float y;
-                asm volatile("v_mov_b32 %0, %1" : "=v"(y) : "v"(x));
-                return y;
-            };
-            const float4 k_own = float4{here(k_raw.x), here(k_raw.y), here(k_raw.z), here(k_raw.w)};
-            const float4 v_own[2] = {float4{here(v_raw[0].x), here(v_raw[0].y), here(v_raw[0].z), here(v_raw[0].w)},
-                                     float4{here(v_raw[1].x), here(v_raw[1].y), here(v_raw[1].z), here(v_raw[1].w)}};
-            {
-                // The new K row is rotated (rotate + store) and converted by the one wave
-                // that needs it.  It has waited in four registers a lane; the lanes now hand
-                // each other the pieces they hold of a K row through the wave's LDS row.
-                float* const krow = sh_krow_all[wave];
-                if (lane < D / 4) *reinterpret_cast<float4*>(krow + lane * 4) = k_own;
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            for (int i = 0; i < 2 * G::kSteps; ++i) acc ^= kreg[i].x ^ kreg[i].y ^ kreg[i].z ^ kreg[i].w;
 #pragma unroll
-                for (int kk = 0; kk < G::kSteps / 2; ++kk) { // two k-steps at a time: the pair of a "neox" rotation
-                    float x[2][8];
+            for (int i = 0; i < G::kLoads; ++i) acc ^= vreg[i].x ^ vreg[i].y ^ vreg[i].z ^ vreg[i].w;
+            if (acc == 0x9E3779B9u) part_ml[0] = 1.0f;
+            if (acc != 0x9E3779BAu) return;
+        }
+        // (the query pieces met ahead of the tile requests; the operands are picked up while the first tile is on its way)
+        float qf[G::kSteps][8]; // this lane's 8 elements of every k-step: head_dim indices kk*32 + grp*8 + 0..7
 #pragma unroll
-                    for (int u = 0; u < 2; ++u) {
-                        const float* src = krow + (kk + u * (G::kSteps / 2)) * 32 + grp * 8;
-                        const float4 lo = *reinterpret_cast<const float4*>(src), hi = *reinterpret_cast<const float4*>(src + 4);
-                        x[u][0] = lo.x; x[u][1] = lo.y; x[u][2] = lo.z; x[u][3] = lo.w;
-                        x[u][4] = hi.x; x[u][5] = hi.y; x[u][6] = hi.z; x[u][7] = hi.w;
-                    }
-                    if constexpr (ROPE) rotate2(x[0], x[1], kk);
+        for (int kk = 0; kk < G::kSteps; ++kk) {
+            const float4 x0 = *reinterpret_cast<const float4*>(qs + col * G::kQStride + kk * 32 + grp * 8);
+            const float4 x1 = *reinterpret_cast<const float4*>(qs + col * G::kQStride + kk * 32 + grp * 8 + 4);
+            qf[kk][0] = x0.x; qf[kk][1] = x0.y; qf[kk][2] = x0.z; qf[kk][3] = x0.w;
+            qf[kk][4] = x1.x; qf[kk][5] = x1.y; qf[kk][6] = x1.z; qf[kk][7] = x1.w;
+        }
+        // (rotate + store) the rotation of this lane's 8 elements of every k-step, by the wave's table
+        // x0, x1: this lane's elements of k-steps kk and kk + kSteps/2 (head_dim indices kk*32 + grp*8 + e
+        // and the same + head_dim/2)
+        auto rotate2 = [&](float (&x0)[8], float (&x1)[8], int kk) {
+            if (a.neox) { // n_rot == D (checked by the host): element e pairs with e + D/2
 #pragma unroll
-                    for (int u = 0; u < 2; ++u) {
-                        h8 h;
+                for (int e = 0; e < 8; ++e) {
+                    const int i = kk * 32 + grp * 8 + e;
+                    rope_rotate(x0[e], x1[e], sh_cs[i][0], sh_cs[i][1]);
+                }
+            } else {      // elements 2i and 2i + 1, below n_rot
+                // No branch per pair: el0 differs from lane to lane, and a branch around each pair's table
+                // read makes the wave wait out sixteen LDS round trips one after the other (1.7 us of a
+                // Llama-3-8B launch).  Every lane reads an entry (its own, or the table's last), all reads
+                // go out together, and a pair past n_rot keeps its values by a select.
+                const int last = max(a.n_rot / 2 - 1, 0); // (n_rot = 0: nothing is rotated, entry 0 is read and not used)
+                float2 cs0[4], cs1[4];
 #pragma unroll
-                        for (int e = 0; e < 8; ++e) h[e] = (_Float16)x[u][e];
-                        k_new16[kk + u * (G::kSteps / 2)] = __builtin_bit_cast(u32x4, h);
-                    }
+                for (int e = 0; e < 8; e += 2) {
+                    const int el0 = kk * 32 + grp * 8 + e, el1 = el0 + D / 2;
+                    cs0[e / 2] = *reinterpret_cast<const float2*>(sh_cs[min(el0 / 2, last)]);
+                    cs1[e / 2] = *reinterpret_cast<const float2*>(sh_cs[min(el1 / 2, last)]);
+                }
+#pragma unroll
+                for (int e = 0; e < 8; e += 2) {
+                    const int el0 = kk * 32 + grp * 8 + e, el1 = el0 + D / 2;
+                    float a0 = x0[e], a1 = x0[e + 1], b0 = x1[e], b1 = x1[e + 1];
+                    rope_rotate(a0, a1, cs0[e / 2].x, cs0[e / 2].y);
+                    rope_rotate(b0, b1, cs1[e / 2].x, cs1[e / 2].y);
+                    x0[e] = el0 < a.n_rot ? a0 : x0[e];
+                    x0[e + 1] = el0 < a.n_rot ? a1 : x0[e + 1];
+                    x1[e] = el1 < a.n_rot ? b0 : x1[e];
+                    x1[e + 1] = el1 < a.n_rot ? b1 : x1[e + 1];
                 }
             }
-            h8 vh;
-            vh[0] = (_Float16)v_own[0].x; vh[1] = (_Float16)v_own[0].y; vh[2] = (_Float16)v_own[0].z; vh[3] = (_Float16)v_own[0].w;
-            vh[4] = (_Float16)v_own[1].x; vh[5] = (_Float16)v_own[1].y; vh[6] = (_Float16)v_own[1].z; vh[7] = (_Float16)v_own[1].w;
-            v_new16 = __builtin_bit_cast(u32x4, vh);
-            // The cache gets the row now (one head group's wave writes it): whatever the tile request that is under
-            // way brings back for this row is replaced from the registers above, and no other wave reads it, so the
-            // order of the two does not matter, and stores issued here are long done when the kernel ends.
-            if (hg == 0) {
-                const int row = pos % kTile;
-                const size_t row_off = ((size_t)kvh * n_ctx + pos) * D;
-                if (col == row % 16) {
-#pragma unroll
-                    for (int kk = 0; kk < G::kSteps; ++kk)
-                        *reinterpret_cast<u32x4*>(const_cast<uint16_t*>(kc) + row_off + (kk * 4 + grp) * 8) = k_new16[kk];
+        };
+        if constexpr (ROPE) {
+            // (cos, sin) of pair i at the raw position, as the rotary kernel forms them
+            // A table per wave (head_dim <= 128: a wave's 64 lanes cover the pairs), so that no wave
+            // waits here for the others: the waves of a workgroup get their loads out at very
+            // different times when the whole chip is requesting its first tiles.  Write and reads
+            // are the same wave's, and a wave's LDS operations complete in order.
+            static_assert(D / 2 <= 64, "one lane per pair");
+            const int half = a.n_rot / 2;
+            if (!rot_early && lane < half) {
+                if (!a.rope_angles) {
+                    float freq = rope_freq_of(a.freq, lane);
+                    if (a.freq_factors) freq /= ff_given;
+                    const float ang = (float)pos * freq;
+                    cs_given.x = cosf(ang);
+                    cs_given.y = sinf(ang);
                 }
-                if (lane < G::kChunksPerRow) *reinterpret_cast<u32x4*>(const_cast<uint16_t*>(vc) + row_off + lane * 8) = v_new16;
+                sh_cs[lane][0] = cs_given.x;
+                sh_cs[lane][1] = cs_given.y;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            if (!rot_early) {
+#pragma unroll
+                for (int kk = 0; kk < G::kSteps / 2; ++kk) rotate2(qf[kk], qf[kk + G::kSteps / 2], kk);
             }
         }
-    }
+        // ---- query heads -> B operands, fp16 hi + lo ----
+        h8 qhi[G::kSteps], qlo[G::kSteps];
+#pragma unroll
+        for (int kk = 0; kk < G::kSteps; ++kk) {
+            const float* x = qf[kk];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float xe = x[e] * qmul;
+                qhi[kk][e] = (_Float16)xe;
+                qlo[kk][e] = (_Float16)(xe - (float)qhi[kk][e]);
+            }
+        }
 
-    for (; tile < n_tiles; tile += tile_step) {
-        const bool more = tile + tile_step < n_tiles;
+        __builtin_amdgcn_sched_barrier(0);
+        FA_STAMP(2);
+        const int v_rd = (grp * 4 + (col >> 2)) * G::kRowBV + (col & 3) * 8; // + h*16 rows, + db*32 bytes
+
+        // (store, rotate + store) The new row is made ready here, while the tiles travel, by the one wave whose tiles
+        // include the row's (the last visible tile: the wave's own last): converted -- and the K row rotated -- as the
+        // store kernel and the rotary kernel would, the pieces this lane is to substitute and to write kept in
+        // registers.  At that tile only the substitution and the two cache writes are left.  (Made ready at the tile
+        // itself, as it used to be, the LDS round trips and the rotation sat between the arrival of the launch's last
+        // tile and its products: 0.7 us of a Qwen2.5-1.5B launch pair at 32k.)  The row's loads went out ahead of the
+        // tile requests, so waiting for them waits for no tile.
+        const int own_tile = n_tiles - 1;
+        [[maybe_unused]] bool owner = false;
+        [[maybe_unused]] u32x4 k_new16[G::kSteps], v_new16 = u32x4{0u, 0u, 0u, 0u};
         if constexpr (STORE) {
-            if (owner && tile == own_tile) { // the tile of the new row: into the operand registers
-                const int row = pos % kTile;
-                if (col == row % 16) {
 #pragma unroll
-                    for (int kk = 0; kk < G::kSteps; ++kk)
+            for (int kk = 0; kk < G::kSteps; ++kk) k_new16[kk] = u32x4{0u, 0u, 0u, 0u};
+            int last = tile_first; // this wave's last tile (a few steps at most)
+            while (last + tile_step <= own_tile) last += tile_step;
+            owner = store && last == own_tile;
+            if (owner) {
+                // (Nothing below may be started ahead of this branch: the compiler would otherwise
+                // convert the new row in every wave.)
+                auto here = [](float x) { // a copy the compiler cannot make anywhere else
+                    float y;
+                    asm volatile("v_mov_b32 %0, %1" : "=v"(y) : "v"(x));
+                    return y;
+                };
+                const float4 v_own[2] = {float4{here(v_raw[0].x), here(v_raw[0].y), here(v_raw[0].z), here(v_raw[0].w)},
+                                         float4{here(v_raw[1].x), here(v_raw[1].y), here(v_raw[1].z), here(v_raw[1].w)}};
+                {
+                    // K: lane i (of D/4) holds elements 4 i ..: it rotates those -- a "neox" pair's other half is the lane's
+                    // D/8 away -- and converts them, and the lanes pick the pieces they hold of a K row out of LDS.  (Every lane
+                    // rotating the 32 elements it will hold was 250 instructions, 0.6 us of the launch whose last tile is
+                    // this wave's.)
+                    float x[4] = {here(k_raw.x), here(k_raw.y), here(k_raw.z), here(k_raw.w)};
+                    if constexpr (ROPE) {
+                        const int e0 = (lane % (D / 4)) * 4;
+                        if (a.neox) {
+                            const bool second = e0 >= D / 2;
+                            const int i0 = second ? e0 - D / 2 : e0;
 #pragma unroll
-                        for (int t = 0; t < 2; ++t) // (constant register indices: a computed one sends the array to scratch memory)
-                            if (row / 16 == t) kreg[t * G::kSteps + kk] = k_new16[kk];
+                            for (int e = 0; e < 4; ++e) {
+                                const float other = __shfl_xor(x[e], D / 8);
+                                float lo = second ? other : x[e], hi = second ? x[e] : other;
+                                rope_rotate(lo, hi, sh_cs[i0 + e][0], sh_cs[i0 + e][1]);
+                                x[e] = second ? hi : lo;
+                            }
+                        } else {
+                            const int last_pair = max(a.n_rot / 2 - 1, 0);
+#pragma unroll
+                            for (int e = 0; e < 4; e += 2) {
+                                float lo = x[e], hi = x[e + 1];
+                                const int i = min((e0 + e) / 2, last_pair);
+                                rope_rotate(lo, hi, sh_cs[i][0], sh_cs[i][1]);
+                                x[e] = e0 + e < a.n_rot ? lo : x[e];
+                                x[e + 1] = e0 + e < a.n_rot ? hi : x[e + 1];
+                            }
+                        }
+                    }
+                    _Float16* const krow = sh_krow_all[wave];
+                    h4 h;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) h[e] = (_Float16)x[e];
+                    if (lane < D / 4) *reinterpret_cast<h4*>(krow + lane * 4) = h;
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+                    for (int kk = 0; kk < G::kSteps; ++kk) k_new16[kk] = *reinterpret_cast<const u32x4*>(krow + (kk * 4 + grp) * 8);
                 }
+                h8 vh;
+                vh[0] = (_Float16)v_own[0].x; vh[1] = (_Float16)v_own[0].y; vh[2] = (_Float16)v_own[0].z; vh[3] = (_Float16)v_own[0].w;
+                vh[4] = (_Float16)v_own[1].x; vh[5] = (_Float16)v_own[1].y; vh[6] = (_Float16)v_own[1].z; vh[7] = (_Float16)v_own[1].w;
+                v_new16 = __builtin_bit_cast(u32x4, vh);
+                // The cache gets the row now (one head group's wave writes it): whatever the tile request that is under
+                // way brings back for this row is replaced from the registers above, and no other wave reads it, so the
+                // order of the two does not matter, and stores issued here are long done when the kernel ends.
+                if (hg == 0) {
+                    const int row = pos % kTile;
+                    const size_t row_off = ((size_t)kvh * n_ctx + pos) * D;
+                    if (col == row % 16) {
 #pragma unroll
-                for (int i = 0; i < G::kLoads; ++i)
-                    if ((i * 64 + lane) / G::kChunksPerRow == row) vreg[i] = v_new16;
+                        for (int kk = 0; kk < G::kSteps; ++kk)
+                            *reinterpret_cast<u32x4*>(const_cast<uint16_t*>(kc) + row_off + (kk * 4 + grp) * 8) = k_new16[kk];
+                    }
+                    if (lane < G::kChunksPerRow) *reinterpret_cast<u32x4*>(const_cast<uint16_t*>(vc) + row_off + lane * 8) = v_new16;
+                }
             }
         }
-        // ---- S^T = K Q^T : rows = KV row (sub-tile t, row col), columns = query head ----
-        f4 s[2], s2[2]; // the Q-lo product runs as its own accumulation chain
-#pragma unroll
-        for (int t = 0; t < 2; ++t) s[t] = s2[t] = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kk = 0; kk < G::kSteps; ++kk)
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const h8 ka = __builtin_bit_cast(h8, kreg[t * G::kSteps + kk]);
-                s[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qhi[kk], s[t], 0, 0, 0);
-                s2[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qlo[kk], s2[t], 0, 0, 0);
-            }
-        s[0] += s2[0];
-        s[1] += s2[1];
-        if (more) fetch_k(tile + tile_step); // the operand registers are free again
-        FA_STAMP(3);
 
-        // ---- softmax weights; lane (col, grp) holds rows t*16 + grp*4 + i of its column ----
-        float v[8];
+        for (; tile < n_tiles; tile += tile_step) {
+            const bool more = tile + tile_step < n_tiles;
+            if constexpr (STORE) {
+                if (owner && tile == own_tile) { // the tile of the new row: into the operand registers
+                    const int row = pos % kTile;
+                    if (col == row % 16) {
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+                        for (int kk = 0; kk < G::kSteps; ++kk)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) v[t * 4 + i] = s[t][i];
-        if (tile * kTile + kTile > npos) { // the last tile: rows past the position do not exist
+                            for (int t = 0; t < 2; ++t) // (constant register indices: a computed one sends the array to scratch memory)
+                                if (row / 16 == t) kreg[t * G::kSteps + kk] = k_new16[kk];
+                    }
+#pragma unroll
+                    for (int i = 0; i < G::kLoads; ++i)
+                        if ((i * 64 + lane) / G::kChunksPerRow == row) vreg[i] = v_new16;
+                }
+            }
+            // ---- S^T = K Q^T : rows = KV row (sub-tile t, row col), columns = query head ----
+            f4 s[2], s2[2]; // the Q-lo product runs as its own accumulation chain
+#pragma unroll
+            for (int t = 0; t < 2; ++t) s[t] = s2[t] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int kk = 0; kk < G::kSteps; ++kk)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const h8 ka = __builtin_bit_cast(h8, kreg[t * G::kSteps + kk]);
+                    s[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qhi[kk], s[t], 0, 0, 0);
+                    s2[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qlo[kk], s2[t], 0, 0, 0);
+                }
+            s[0] += s2[0];
+            s[1] += s2[1];
+            if (more) fetch_k(tile + tile_step); // the operand registers are free again
+            FA_STAMP(3);
+
+            // ---- softmax weights; lane (col, grp) holds rows t*16 + grp*4 + i of its column ----
+            float v[8];
 #pragma unroll
             for (int t = 0; t < 2; ++t)
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (tile * kTile + t * 16 + grp * 4 + i >= npos) v[t * 4 + i] = -INFINITY;
-        }
-        float mx = fmaxf(fmaxf(v[0], v[1]), v[2]);
-        mx = fmaxf(fmaxf(mx, v[3]), v[4]);
-        mx = fmaxf(fmaxf(mx, v[5]), v[6]);
-        mx = xor_max(fmaxf(mx, v[7]));
-        // move the reference only when this tile's maximum is far above it (or it is unset)
-        const bool move = (mx - m_ref) * c2 > kLazy || (m_ref == -INFINITY && mx > -INFINITY);
-        if (__builtin_amdgcn_ballot_w64(move) != 0) {
-            const float alpha = move ? fast_exp2((m_ref - mx) * c2) : 1.0f; // unset reference -> 0
-            if (move) m_ref = mx;
-            l_run *= alpha;
+                for (int i = 0; i < 4; ++i) v[t * 4 + i] = s[t][i];
+            if (tile * kTile + kTile > npos) { // the last tile: rows past the position do not exist
 #pragma unroll
-            for (int db = 0; db < G::kDBlk; ++db) o[db] *= alpha;
-        }
-        // exponent = s*c2 - m_ref*c2 + shift; a column that has seen no visible row keeps weight 0
-        const float nb = (m_ref == -INFINITY) ? kPShift : kPShift - m_ref * c2;
-        h8 ph, pl;
+                for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const float pe = fast_exp2(__builtin_fmaf(v[e], c2, nb));
-            l_run += pe;
-            ph[e] = (_Float16)pe;
-            pl[e] = (_Float16)(pe - (float)ph[e]);
-        }
+                    for (int i = 0; i < 4; ++i)
+                        if (tile * kTile + t * 16 + grp * 4 + i >= npos) v[t * 4 + i] = -INFINITY;
+            }
+            float mx = fmaxf(fmaxf(v[0], v[1]), v[2]);
+            mx = fmaxf(fmaxf(mx, v[3]), v[4]);
+            mx = fmaxf(fmaxf(mx, v[5]), v[6]);
+            mx = xor_max(fmaxf(mx, v[7]));
+            // move the reference only when this tile's maximum is far above it (or it is unset)
+            const bool move = (mx - m_ref) * c2 > kLazy || (m_ref == -INFINITY && mx > -INFINITY);
+            if (__builtin_amdgcn_ballot_w64(move) != 0) {
+                const float alpha = move ? fast_exp2((m_ref - mx) * c2) : 1.0f; // unset reference -> 0
+                if (move) m_ref = mx;
+                l_run *= alpha;
+#pragma unroll
+                for (int db = 0; db < G::kDBlk; ++db) o[db] *= alpha;
+            }
+            // exponent = s*c2 - m_ref*c2 + shift; a column that has seen no visible row keeps weight 0
+            const float nb = (m_ref == -INFINITY) ? kPShift : kPShift - m_ref * c2;
+            h8 ph, pl;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float pe = fast_exp2(__builtin_fmaf(v[e], c2, nb));
+                l_run += pe;
+                ph[e] = (_Float16)pe;
+                pl[e] = (_Float16)(pe - (float)ph[e]);
+            }
 
-        // ---- V: registers -> this wave's LDS slice (K was needed first and arrives first) ----
-        const int rows_left = npos - tile * kTile; // rows of this tile below the position (>= 32: all)
+            // ---- V: registers -> this wave's LDS slice (K was needed first and arrives first) ----
+            const int rows_left = npos - tile * kTile; // rows of this tile below the position (>= 32: all)
 #pragma unroll
-        for (int i = 0; i < G::kLoads; ++i) {
-            const int c = i * 64 + lane;
-            // rows at or past the position may hold anything; their weights are zero, and 0 * NaN is not
-            const u32x4 x = (c / G::kChunksPerRow) < rows_left ? vreg[i] : u32x4{0u, 0u, 0u, 0u};
-            *reinterpret_cast<u32x4*>(vs + (c / G::kChunksPerRow) * G::kRowBV + (c % G::kChunksPerRow) * 16) = x;
-        }
-        if (more) fetch_v(tile + tile_step);
-        wave_lds_sync();
+            for (int i = 0; i < G::kLoads; ++i) {
+                const int c = i * 64 + lane;
+                // rows at or past the position may hold anything; their weights are zero, and 0 * NaN is not
+                const u32x4 x = (c / G::kChunksPerRow) < rows_left ? vreg[i] : u32x4{0u, 0u, 0u, 0u};
+                *reinterpret_cast<u32x4*>(vs + (c / G::kChunksPerRow) * G::kRowBV + (c % G::kChunksPerRow) * 16) = x;
+            }
+            if (more) fetch_v(tile + tile_step);
+            wave_lds_sync();
 
-        // ---- O^T += V^T P : rows = head_dim index, columns = query head, k = the tile's 32 KV rows
-        //      in the order (grp, t, i) that matches the layout P already has ----
+            // ---- O^T += V^T P : rows = head_dim index, columns = query head, k = the tile's 32 KV rows
+            //      in the order (grp, t, i) that matches the layout P already has ----
 #pragma unroll
-        for (int db = 0; db < G::kDBlk; ++db) {
-            const h4 v0 = lds_read_tr(vs + v_rd + db * 32);
-            const h4 v1 = lds_read_tr(vs + v_rd + 16 * G::kRowBV + db * 32);
-            const h8 va = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
-            o[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, ph, o[db], 0, 0, 0);
-            o[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pl, o[db], 0, 0, 0);
+            for (int db = 0; db < G::kDBlk; ++db) {
+                const h4 v0 = lds_read_tr(vs + v_rd + db * 32);
+                const h4 v1 = lds_read_tr(vs + v_rd + 16 * G::kRowBV + db * 32);
+                const h8 va = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+                o[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, ph, o[db], 0, 0, 0);
+                o[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pl, o[db], 0, 0, 0);
+            }
+            wave_lds_sync(); // the slice is overwritten at the top of the next iteration
         }
-        wave_lds_sync(); // the slice is overwritten at the top of the next iteration
+    } else { // (marks for the timeline build)
+        FA_STAMP(1);
+        FA_STAMP(2);
     }
 
     FA_STAMP(4);
@@ -570,41 +595,47 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
     __syncthreads();
     FA_STAMP(6);
 
-    for (int idx = threadIdx.x; idx < 16 * (D / 4); idx += kThreads) {
-        const int c = idx / (D / 4);
-        const int d4 = (idx % (D / 4)) * 4;
-        const int h_local = hg * 16 + c;
-        if (h_local >= r) continue;
-        float mw[kWaves], lw[kWaves];
-        float m_all = -INFINITY;
+    // (waves from the wu-th on have had no tile: two cases, so that the sums of a full run are not read under conditions)
+    auto merge = [&](auto waves) {
+        constexpr int W = decltype(waves)::value;
+        for (int idx = threadIdx.x; idx < 16 * (D / 4); idx += kThreads) {
+            const int c = idx / (D / 4);
+            const int d4 = (idx % (D / 4)) * 4;
+            const int h_local = hg * 16 + c;
+            if (h_local >= r) continue;
+            float mw[W], lw[W];
+            float m_all = -INFINITY;
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w) {
-            mw[w] = ml[(w * 16 + c) * 2 + 0];
-            lw[w] = ml[(w * 16 + c) * 2 + 1];
-            m_all = fmaxf(m_all, mw[w]);
-        }
-        float l_all = 0.0f;
-        f4 acc = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int w = 0; w < kWaves; ++w) {
-            const float wgt = fast_exp2(mw[w] - m_all); // a wave that had no tile has m = -inf -> weight 0
-            l_all += lw[w] * wgt;
-            acc += *reinterpret_cast<const f4*>(smem + w * G::kWaveB + ((size_t)c * G::kOStride + d4) * 4) * wgt;
-        }
-        const int head = kvh * r + h_local;
-        if (n_splits > 1) {
-            const size_t pi = (size_t)id * n_head + head;
-            *reinterpret_cast<f4*>(part_o + pi * D + d4) = acc;
-            if (d4 == 0) {
-                const size_t mi = (size_t)head * n_splits + id; // [head][split]: a head's pairs are one run of memory for the combine kernel
-                part_ml[mi * 2 + 0] = m_all;
-                part_ml[mi * 2 + 1] = l_all;
+            for (int w = 0; w < W; ++w) {
+                mw[w] = ml[(w * 16 + c) * 2 + 0];
+                lw[w] = ml[(w * 16 + c) * 2 + 1];
+                m_all = fmaxf(m_all, mw[w]);
             }
-        } else {
-            const float inv = l_all > 0.0f ? 1.0f / l_all : 0.0f;
-            *reinterpret_cast<f4*>(dst + (size_t)head * D + d4) = acc * inv; // (no splits: dst is the output)
+            float l_all = 0.0f;
+            f4 acc = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                const float wgt = fast_exp2(mw[w] - m_all); // a wave that had no tile has m = -inf -> weight 0
+                l_all += lw[w] * wgt;
+                acc += *reinterpret_cast<const f4*>(smem + w * G::kWaveB + ((size_t)c * G::kOStride + d4) * 4) * wgt;
+            }
+            const int head = kvh * r + h_local;
+            if (n_splits > 1) {
+                const size_t pi = (size_t)id * n_head + head;
+                *reinterpret_cast<f4*>(part_o + pi * D + d4) = acc;
+                if (d4 == 0) {
+                    const size_t mi = (size_t)head * n_splits + id; // [head][split]: a head's pairs are one run of memory for the combine kernel
+                    part_ml[mi * 2 + 0] = m_all;
+                    part_ml[mi * 2 + 1] = l_all;
+                }
+            } else {
+                const float inv = l_all > 0.0f ? 1.0f / l_all : 0.0f;
+                *reinterpret_cast<f4*>(dst + (size_t)head * D + d4) = acc * inv; // (no splits: dst is the output)
+            }
         }
-    }
+    };
+    if (wu <= 2) merge(std::integral_constant<int, 2>());
+    else merge(std::integral_constant<int, kWaves>());
     FA_STAMP(7);
 }
 

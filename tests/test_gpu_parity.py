@@ -119,6 +119,20 @@ def test_decode_small(fa, d, r):
     del torch
 
 
+@pytest.mark.parametrize("H,G,d", [(12, 2, 128), (8, 8, 64)])
+def test_decode_where_the_number_of_waves_with_tiles_changes(fa, H, G, d):
+    """The last position at which one, two, three ... waves of a workgroup have a tile, and the first at which another has."""
+    n_ctx, scale = 4096, 1.0 / np.sqrt(d)
+    q, kc, vc = make_case(171 + d, H, G, d, n_ctx, n_ctx, 1, outliers=4)
+    dk, dv = _dev(kc), _dev(vc)
+    rows = np.array([(0, h) for h in range(H)], np.int32)
+    run = 32 * int(fa.lib().orin_fa_decode_splits(H, G, d, n_ctx))
+    for npos in sorted({n for k in (1, 2, 3, 7) for n in (k * run - 1, k * run, k * run + 1) if n <= n_ctx}):
+        want = ref.flash_attention_rows(q, kc, vc, rows, H, G, d, n_ctx, npos - 1, np.float32(scale))
+        got = gpu_decode(fa, q[0], None, None, H, G, d, n_ctx, npos - 1, scale, dk=dk, dv=dv)
+        check(got, want.reshape(got.shape), f"decode d{d} npos{npos}", floor=FLOOR_DECODE)
+
+
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("r", [1, 2, 3, 4, 5, 6, 7, 8, 11])
 def test_prefill_small(fa, d, r):
