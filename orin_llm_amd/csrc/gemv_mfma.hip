@@ -686,14 +686,13 @@ bool launch_rows_as(const GemvArgs& a, int wgs, int shares, int n_in_wg, hipStre
         go(std::integral_constant<int, kRowsOneItem>());
         return true;
     }
-    if constexpr (kWaves == 4) {
-        // (two matrices' tiles are half as large: up to three tiles for two workgroups)
-        const bool few = DUAL ? wgs * 3 >= rows_tiles(a) * 2 : wgs * shares <= g_rows_resident * 3 / 4;
-        if (few && passes <= 2) {
-            if (passes == 1) go(std::integral_constant<int, kRowsOnePass>());
-            else go(std::integral_constant<int, kRowsTwoPasses>());
-            return true;
-        }
+    // (two matrices' tiles are half as large: up to three tiles for two workgroups)
+    // Workgroups of eight waves (q, k, v of Llama-3-8B in Q8_0 9.6 -> 8.9 us): up to half the waves that are resident.
+    const bool few = DUAL ? wgs * 3 >= rows_tiles(a) * 2 : wgs * shares <= g_rows_resident * (kWaves == 4 ? 3 : 2) / 4;
+    if (few && passes <= 2) {
+        if (passes == 1) go(std::integral_constant<int, kRowsOnePass>());
+        else go(std::integral_constant<int, kRowsTwoPasses>());
+        return true;
     }
     go(std::integral_constant<int, kRowsAny>());
     return true;
@@ -713,7 +712,7 @@ bool launch_rows(const GemvArgs& a, int wgs, int shares, bool wide, int nb_wg, h
     if (a.w_up && !rows_base_ok(T, a.w_up)) return false;
     const int n_in_wg = nb_wg * 256;
     if constexpr (T == kQ8_0) { // (272 bytes are a long run already: two blocks only where they make one item of a wave's share)
-        if (wide) return nb_wg <= 16 ? launch_rows_as<T, false, 8, 2>(a, wgs, shares, n_in_wg, stream) : launch_rows_as<T, false, 8, 1>(a, wgs, shares, n_in_wg, stream);
+        if (wide) return nb_wg <= 16 && wgs <= g_rows_resident / 3 ? launch_rows_as<T, false, 8, 2>(a, wgs, shares, n_in_wg, stream) : launch_rows_as<T, false, 8, 1>(a, wgs, shares, n_in_wg, stream);
         if (!a.w_up && nb_wg > 4 && nb_wg <= 8 && wgs == rows_tiles(a)) return launch_rows_as<T, false, 4, 2>(a, wgs, shares, n_in_wg, stream);
         return a.w_up ? launch_rows_as<T, true, 4, 1>(a, wgs, shares, n_in_wg, stream) : launch_rows_as<T, false, 4, 1>(a, wgs, shares, n_in_wg, stream);
     }
@@ -769,7 +768,9 @@ hipError_t launch(const GemvArgs& a, int cu_count, hipStream_t stream) {
                 while (tiles * ks_r * 2 <= cu_count && ks_r * 2 <= kMostRowsShares && nb_row >= ks_r * 4) ks_r *= 2;
             }
         }
-        const bool wide_r = ks_r == 1 && nb_row >= 16 && !a.w_up && wgs == tiles;
+        // Eight waves from 9 blocks a row on, which gives a wave one item up to 16 (Qwen2.5-7B's q, k, v in Q5_K and Q6_K 8.4 ->
+        // 6.4 us); Q8_0's buffers for that leave room for one such workgroup a CU.
+        const bool wide_r = ks_r == 1 && nb_row > (T == kQ8_0 && tiles > cu_count ? 15 : 8) && !a.w_up && wgs == tiles;
         if (launch_rows<T>(a, wgs, ks_r, wide_r, (nb_row + ks_r - 1) / ks_r, stream)) return hipGetLastError();
     }
     const size_t lds = lds_bytes<T>((nb_row + ks - 1) / ks * 256);
@@ -797,10 +798,8 @@ hipError_t allow_lds(const void* kernel) { return hipFuncSetAttribute(kernel, hi
 template <int T, bool DUAL, int kWaves, int CB>
 hipError_t allow_rows() {
     hipError_t e;
-    if constexpr (kWaves == 4) {
-        if ((e = allow_lds(reinterpret_cast<const void*>(&gemv_rows_kernel<T, DUAL, kWaves, CB, kRowsOnePass>))) != hipSuccess) return e;
-        if ((e = allow_lds(reinterpret_cast<const void*>(&gemv_rows_kernel<T, DUAL, kWaves, CB, kRowsTwoPasses>))) != hipSuccess) return e;
-    }
+    if ((e = allow_lds(reinterpret_cast<const void*>(&gemv_rows_kernel<T, DUAL, kWaves, CB, kRowsOnePass>))) != hipSuccess) return e;
+    if ((e = allow_lds(reinterpret_cast<const void*>(&gemv_rows_kernel<T, DUAL, kWaves, CB, kRowsTwoPasses>))) != hipSuccess) return e;
     if ((e = allow_lds(reinterpret_cast<const void*>(&gemv_rows_kernel<T, DUAL, kWaves, CB, kRowsOneItem>))) != hipSuccess) return e;
     return allow_lds(reinterpret_cast<const void*>(&gemv_rows_kernel<T, DUAL, kWaves, CB, kRowsAny>));
 }
@@ -837,7 +836,7 @@ hipError_t gemv_mfma_mixed_launch(GemvArgs a, int cu_count, hipStream_t stream) 
         const int per_cu = rows_wgs_per_cu(a.mfma_wgs_per_cu), nb = a.n_in / 256;
         const int tiles = rows_tiles(a);
         const int wgs = per_cu > 0 ? min(tiles, cu_count * per_cu) : tiles;
-        const bool wide_r = nb >= 16 && wgs == tiles;
+        const bool wide_r = nb > 8 && wgs == tiles; // (as in launch() above)
         RowsHead h;
         if (rows_head(a, wgs, 1, h)) {
             h.shape &= ~0x3ff80u;
