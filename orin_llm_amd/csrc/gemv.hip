@@ -462,7 +462,7 @@ bool gemv_use_mfma() {
 }
 void gemv_set_use_mfma(bool on) { g_use_mfma = on ? 1 : 0; }
 
-// Shares of a row that an accumulating projection may be cut into (0: the launcher chooses 1, 2 or 4 by shape;
+// Shares of a row that an accumulating projection may be cut into (0: the launcher chooses by shape;
 // 1: never cut, which makes `y += W x` a plain sum with a fixed order; orin_gemv_row_shares(), or ORIN_GEMV_KSPLIT in
 // the environment as the initial value).
 static int g_row_shares = -1;
