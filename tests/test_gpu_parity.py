@@ -235,6 +235,18 @@ def test_prefill_row_equals_decode_and_chunk_split(fa):
         check(dec, whole[t], f"prefill row {t} vs decode", tol=1e-3)  # (prefill against decode: the prefill bound)
 
 
+@pytest.mark.parametrize("n_past,batch", [(0, 301), (0, 512), (724, 300), (725, 300)])
+def test_prefill_head_dim_64_on_short_and_longer_walks(fa, n_past, batch):
+    """More than half the CUs' worth of 64-column workgroups: up to 1024 rows of context in 32-column ones, two a CU."""
+    H, G, d, n_ctx = 32, 8, 64, 1100
+    scale = 1.0 / np.sqrt(d)
+    q, kc, vc = make_case(61 + n_past + batch, H, G, d, n_ctx, n_past + batch, batch, outliers=4, poison_tail=True)
+    rows = np.array([(t, h) for t in sorted({0, 1, 7, 8, 9, 31, 32, batch // 2, batch - 2, batch - 1}) for h in (0, 3, 4, 17, 31)], np.int32)
+    want = ref.flash_attention_rows(q, kc, vc, rows, H, G, d, n_ctx, n_past, np.float32(scale))
+    got = gpu_prefill(fa, q, kc, vc, H, G, d, n_ctx, n_past, batch, scale)
+    check(got[rows[:, 0], rows[:, 1]], want, f"prefill d64 P{n_past} B{batch}")
+
+
 def test_decode_ignores_cache_tail_and_position_is_read_on_device(fa):
     import torch
 
