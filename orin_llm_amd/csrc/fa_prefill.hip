@@ -468,8 +468,8 @@ __global__ __launch_bounds__(kPrefillWaves * 64) void fa_prefill_kernel(
     // and beside their trip to memory: left alone, the compiler fetches each where it is first
     // used, one wait behind the other after the first products.
     {
-        const void *p0 = a.out, *p1 = a.part_o, *p2 = a.part_ml;
-        asm volatile("" ::"s"(p0), "s"(p1), "s"(p2), "s"(a.c));
+        const void *p0 = a.out, *p1 = a.part_o;
+        asm volatile("" ::"s"(p0), "s"(p1), "s"(a.c));
     }
     FA_STAMP(10);
     // ---- query block -> LDS (fp16) ----
@@ -958,7 +958,7 @@ __global__ __launch_bounds__(kPrefillWaves * 64) void fa_prefill_kernel(
         if (kv_split_shift > 0) { // this split's normalised share and its log-sum-exp, for the combine kernel
             const size_t prow = (size_t)split * batch * n_head + orow;
             dst = a.part_o + prow * D;
-            if (part == 0) a.part_ml[prow] = l_all > 0.0f ? m_all + __builtin_amdgcn_logf(l_all) : -INFINITY;
+            if (part == 0) a.out[orow * D + split] = l_all > 0.0f ? m_all + __builtin_amdgcn_logf(l_all) : -INFINITY; // (where the combine kernel finds it)
         }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -990,42 +990,33 @@ __global__ __launch_bounds__(kPrefillWaves * 64) void fa_prefill_kernel(
 }
 
 // out = sum over the KV splits of their normalised outputs, weighted by 2^(lse_s - max lse) and
-// divided by the weights' sum.  One thread per 16 bytes of out; rows = batch * n_head.
-template <int D>
-__global__ __launch_bounds__(256) void fa_prefill_combine_kernel(const float* part_o, const float* part_lse, float* out,
-                                                                 int rows, int splits) {
+// divided by the weights' sum.  One thread per 16 bytes of out; rows = batch * n_head.  A trip to memory
+// and little else, so every split's piece is asked for before anything is waited for (four at a time,
+// sixteen splits were four trips one after the other: 8 tokens of Qwen2.5-1.5B at 2600 13.4 -> 11.4 us a launch pair).
+// A row's log-sum-exps sit in its own piece of out, which the threads of one wave read and then write: the workspace holds
+// partial outputs alone.
+template <int D, int S>
+__global__ __launch_bounds__(256) void fa_prefill_combine_kernel(const float* part_o, float* out, int rows) {
     const int idx = blockIdx.x * 256 + threadIdx.x;
     const int row = idx / (D / 4), piece = idx % (D / 4);
     if (row >= rows) return;
-    float lse[4];
-    f4 x[4];
-    // (the loads of four splits at a time go out together; 2 or 4 splits is the common case)
-    float m = -INFINITY, wsum = 0.0f;
+    float lse[S];
+    f4 x[S];
+#pragma unroll
+    for (int u = 0; u < S; ++u) {
+        lse[u] = out[(size_t)row * D + u];
+        x[u] = *reinterpret_cast<const f4*>(part_o + ((size_t)u * rows + row) * D + piece * 4);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    float m = lse[0], wsum = 0.0f;
+#pragma unroll
+    for (int u = 1; u < S; ++u) m = fmaxf(m, lse[u]);
     f4 acc = f4{0.f, 0.f, 0.f, 0.f};
-    for (int s0 = 0; s0 < splits; s0 += 4) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (s0 + u < splits) {
-                lse[u] = part_lse[(size_t)(s0 + u) * rows + row];
-                x[u] = *reinterpret_cast<const f4*>(part_o + ((size_t)(s0 + u) * rows + row) * D + piece * 4);
-            }
-        float m_new = m;
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (s0 + u < splits) m_new = fmaxf(m_new, lse[u]);
-        if (m_new > -INFINITY) { // (else: no split so far held a visible row of this column)
-            const float keep = fast_exp2(m - m_new); // 0 on the first splits that hold one
-            wsum *= keep;
-            acc *= keep;
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (s0 + u < splits) {
-                    const float w = fast_exp2(lse[u] - m_new); // 0 for a split without a visible row
-                    wsum += w;
-                    acc += x[u] * w;
-                }
-            m = m_new;
-        }
+    for (int u = 0; u < S; ++u) {
+        const float w = m > -INFINITY ? fast_exp2(lse[u] - m) : 0.0f; // 0 for a split without a visible row
+        wsum += w;
+        acc += x[u] * w;
     }
     const float inv = wsum > 0.0f ? 1.0f / wsum : 0.0f;
     *reinterpret_cast<f4*>(out + (size_t)row * D + piece * 4) = acc * inv;
@@ -1049,7 +1040,7 @@ hipError_t allow_lds() {
 
 constexpr int kMaxPrefillSplitShift = 4; // up to 16 workgroups share a token tile's KV rows (small chunks on long contexts)
 
-// Rows of context from which cutting a token tile's rows among several workgroups pays for the
+// Rows of context from which cutting a token tile's rows between two workgroups pays for the
 // second launch and the partial results' trip through memory (Qwen2.5-1.5B heads, 512-token
 // chunk: 35.1 -> 33.2 us at 6144 rows, 106 -> 71 us at 16896, 304 -> 121 us at 32768; slower
 // below about 4600 rows).
@@ -1081,14 +1072,20 @@ hipError_t launch(FaArgs a, int cu_count, hipStream_t stream, void* workspace, s
         int shift = 1;
         while (shift < kMaxPrefillSplitShift && (wgs64 << (shift + 1)) <= cu_count) ++shift;
         const size_t rows = (size_t)a.batch * a.n_head;
-        const size_t need = (rows << shift) * (D + 1) * sizeof(float);
-        // (with four or more workgroups per token tile the walk shortens enough to pay from about
-        // 2500 rows: 19.9 -> 17.7 us at 4000 rows for a 256-token chunk)
-        const int min_rows = shift >= 2 ? (kSplitMinRows * 3) / 5 : kSplitMinRows;
-        if (a.n_past + a.batch >= min_rows && workspace && need <= workspace_bytes) {
+        // (as many as the workspace has room for: 128 tokens of Qwen3-0.6B heads at 8000, whose eight splits take more,
+        // ran unsplit in 55.6 us and take 26.3 with four)
+        while (shift > 0 && (rows << shift) * D * sizeof(float) > workspace_bytes) --shift;
+        // Where that pays: the more workgroups per token tile, the shorter the walk and the sooner, and the more partial
+        // results, the later.  The lines lie at or just above where both ways took the same over 8 to 200 tokens at 700 to 4500 rows of five
+        // models' heads (head_dim 64, whose walk costs half a row, breaks even at half as many rows again): 8 tokens of
+        // Qwen2.5-1.5B at 2000 15.2 -> 10.6 us, 45 at 2400 16.8 -> 12.7, 100 of Qwen2.5-7B at 3000 18.6 -> 17.0.
+        const int kb = (int)((rows << shift) * D * sizeof(float) / 1024);
+        int min_rows = shift >= 4 ? 1100 + kb * 11 / 100 : shift == 3 ? 850 + kb * 21 / 100 : 300 + kb * 38 / 100;
+        if (D == 64) min_rows += min_rows / 2;
+        if (shift <= 1) min_rows = kSplitMinRows;
+        if (shift > 0 && a.n_past + a.batch >= min_rows && workspace) {
             a.kv_split_shift = shift;
             a.part_o = static_cast<float*>(workspace);
-            a.part_ml = a.part_o + (rows << shift) * D;
         } else {
             ncb = 1;
             a.tq = 32 / a.heads_per_group;
@@ -1109,8 +1106,13 @@ hipError_t launch(FaArgs a, int cu_count, hipStream_t stream, void* workspace, s
     if (e != hipSuccess || a.kv_split_shift == 0) return e;
     const int rows = a.batch * a.n_head;
     const unsigned blocks = (unsigned)(((size_t)rows * (D / 4) + 255) / 256);
-    hipLaunchKernelGGL(fa_prefill_combine_kernel<D>, dim3(blocks), dim3(256), 0, stream, a.part_o, a.part_ml, a.out, rows,
-                       1 << a.kv_split_shift);
+    switch (a.kv_split_shift) {
+    case 1: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 2>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.out, rows); break;
+    case 2: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 4>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.out, rows); break;
+    case 3: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 8>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.out, rows); break;
+    default: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 16>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.out, rows); break;
+    }
+    static_assert(kMaxPrefillSplitShift == 4, "the cases above");
     return hipGetLastError();
 }
 

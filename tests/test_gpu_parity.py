@@ -247,6 +247,25 @@ def test_prefill_head_dim_64_on_short_and_longer_walks(fa, n_past, batch):
     check(got[rows[:, 0], rows[:, 1]], want, f"prefill d64 P{n_past} B{batch}")
 
 
+@pytest.mark.parametrize("H,G,d,batch,n_past", [(12, 2, 128, 8, 1500), (12, 2, 128, 45, 1700), (12, 2, 128, 100, 2000), (28, 4, 128, 100, 2700),
+                                                (32, 8, 128, 128, 4000), (16, 8, 128, 128, 2500), (32, 8, 64, 16, 2000), (12, 2, 128, 512, 4700)])
+def test_prefill_rows_cut_among_workgroups(fa, H, G, d, batch, n_past):
+    """Two, four, eight and sixteen workgroups a token tile, the partial results filling the workspace at most, the log-sum-exps
+    in the output rows; no row of the output that is not the chunk's is touched."""
+    import torch
+
+    n_ctx, scale = n_past + batch + 7, 1.0 / np.sqrt(d)
+    q, kc, vc = make_case(67 + n_past + batch, H, G, d, n_ctx, n_past + batch, batch, outliers=4, poison_tail=True)
+    rows = np.array([(t, h) for t in sorted({0, 1, 7, batch // 2, batch - 2, batch - 1}) for h in (0, H // 2, H - 1)], np.int32)
+    want = ref.flash_attention_rows(q, kc, vc, rows, H, G, d, n_ctx, n_past, np.float32(scale))
+    out = torch.full((batch + 1, H, d), 12345.0, device="cuda")
+    fa.flash_attention(_dev(q), _dev(kc), _dev(vc), out, H, G, d, n_ctx, n_past, batch, float(scale))
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    assert (got[batch] == 12345.0).all()
+    check(got[rows[:, 0], rows[:, 1]], want, f"prefill r{H // G} d{d} P{n_past} B{batch}")
+
+
 def test_decode_ignores_cache_tail_and_position_is_read_on_device(fa):
     import torch
 
