@@ -242,8 +242,13 @@ int orin_decode_layer(const orin_decode_layer_desc* L) {
         }
     }
     // ---- per-head norms of q and k (reference: src/model_gpu.cu:274-275) ----
-    if (L->q_norm && (rc = orin_rms_norm_rows(L->q, L->q_norm, L->n_head, L->head_dim, L->rms_eps, L->q)) != ORIN_FA_OK) return rc;
-    if (L->k_norm && (rc = orin_rms_norm_rows(L->k, L->k_norm, L->n_kv, L->head_dim, L->rms_eps, L->k)) != ORIN_FA_OK) return rc;
+    if (L->q_norm && L->k_norm) { // both in one launch: a layer 2 us less
+        rc = hip_rc(rms_norm_pair_launch(L->q, L->q_norm, L->n_head, L->q, L->k, L->k_norm, L->n_kv, L->k, L->head_dim, L->rms_eps, lib_stream()));
+        if (rc != ORIN_FA_OK) return rc;
+    } else {
+        if (L->q_norm && (rc = orin_rms_norm_rows(L->q, L->q_norm, L->n_head, L->head_dim, L->rms_eps, L->q)) != ORIN_FA_OK) return rc;
+        if (L->k_norm && (rc = orin_rms_norm_rows(L->k, L->k_norm, L->n_kv, L->head_dim, L->rms_eps, L->k)) != ORIN_FA_OK) return rc;
+    }
     // ---- rotary embedding, cache store, attention (reference: src/model_gpu.cu:277-282) ----
     const bool fused_rope = !L->neox || L->n_rot == 0 || L->n_rot == L->head_dim;
     if (fused_rope) {

@@ -53,6 +53,9 @@ int gemv_row_shares();          // 0: chosen by shape; 1: accumulating projectio
 void gemv_set_row_shares(int n);
 
 hipError_t rms_norm_launch(const float* x, const float* w, int rows, int cols, float eps, float* y, hipStream_t stream);
+// Two matrices of rows of one length, each with its own weights, in one launch.
+hipError_t rms_norm_pair_launch(const float* x0, const float* w0, int rows0, float* y0, const float* x1, const float* w1, int rows1, float* y1,
+                                int cols, float eps, hipStream_t stream);
 hipError_t stage_launch(const float* x, float* stage, int n, hipStream_t stream);
 hipError_t swiglu_launch(float* act, const float* gate, const float* up, int n, hipStream_t stream);
 hipError_t dequant_row_launch(int type, const void* src, float* y, int n, hipStream_t stream);

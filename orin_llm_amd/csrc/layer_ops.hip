@@ -12,15 +12,34 @@ namespace {
 
 // y = x / sqrt(mean(x^2) + eps) * w over each row of cols elements (reference CPU statement:
 // src/model_cpu.cpp:13-18; w is shared by the rows).  One workgroup per row; y may be x: a thread
-// writes only elements it has read itself.
-template <int THREADS>
-__global__ __launch_bounds__(THREADS) void rms_norm_kernel(const float* x, const float* __restrict__ w, int cols,
-                                                            float eps, float* y) {
+// writes only elements it has read itself.  Two matrices of rows in one launch, for the per-head norms of q and k: a
+// launch boundary is most of what either takes.  Rows from rows0 on are the second's.  KEEP > 0: a row of at most KEEP
+// elements a thread stays in registers with its weights asked for beside it, one trip to memory instead of two behind
+// each other (4096 columns: 2.88 -> 2.28 us); masks of elements a thread does not have cost more than the trip (1536
+// columns with KEEP = 8: 2.2 -> 2.5 us), so KEEP follows the row's length.
+template <int THREADS, int KEEP>
+__global__ __launch_bounds__(THREADS) void rms_norm_kernel(const float* x0, const float* w0, const float* x1, const float* w1, int rows0,
+                                                            int cols, float eps, float* y0, float* y1) {
     __shared__ float sh[THREADS / 64];
-    const float* xr = x + (size_t)blockIdx.x * cols;
-    float* yr = y + (size_t)blockIdx.x * cols;
+    const bool one = (int)blockIdx.x < rows0;
+    const size_t off = (size_t)(one ? blockIdx.x : blockIdx.x - rows0) * cols;
+    const float* const xr = (one ? x0 : x1) + off;
+    const float* const w = one ? w0 : w1;
+    float* const yr = (one ? y0 : y1) + off;
+    [[maybe_unused]] float xk[KEEP + 1], wk[KEEP + 1];
     float ss = 0.0f;
-    for (int i = threadIdx.x; i < cols; i += THREADS) ss += xr[i] * xr[i];
+    if constexpr (KEEP > 0) {
+#pragma unroll
+        for (int j = 0; j < KEEP; ++j) {
+            const int i = threadIdx.x + j * THREADS;
+            xk[j] = i < cols ? xr[i] : 0.0f;
+            wk[j] = i < cols ? w[i] : 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < KEEP; ++j) ss += xk[j] * xk[j];
+    } else {
+        for (int i = threadIdx.x; i < cols; i += THREADS) ss += xr[i] * xr[i];
+    }
     ss = wave_sum(ss);
     if constexpr (THREADS > 64) {
         if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = ss;
@@ -30,7 +49,15 @@ __global__ __launch_bounds__(THREADS) void rms_norm_kernel(const float* x, const
         for (int k = 0; k < THREADS / 64; ++k) ss += sh[k];
     }
     const float rinv = 1.0f / sqrtf(ss / (float)cols + eps);
-    for (int i = threadIdx.x; i < cols; i += THREADS) yr[i] = xr[i] * rinv * w[i];
+    if constexpr (KEEP > 0) {
+#pragma unroll
+        for (int j = 0; j < KEEP; ++j) {
+            const int i = threadIdx.x + j * THREADS;
+            if (i < cols) yr[i] = xk[j] * rinv * wk[j];
+        }
+    } else {
+        for (int i = threadIdx.x; i < cols; i += THREADS) yr[i] = xr[i] * rinv * w[i];
+    }
 }
 
 __global__ __launch_bounds__(256) void stage_kernel(const float* __restrict__ x, float* __restrict__ stage, int n) {
@@ -106,13 +133,21 @@ __global__ __launch_bounds__(256) void dequant_row_kernel(int type, const unsign
 
 } // namespace
 
-hipError_t rms_norm_launch(const float* x, const float* w, int rows, int cols, float eps, float* y, hipStream_t stream) {
+hipError_t rms_norm_pair_launch(const float* x0, const float* w0, int rows0, float* y0, const float* x1, const float* w1, int rows1, float* y1,
+                                int cols, float eps, hipStream_t stream) {
     drop_stale_error();
-    if (cols <= 256)
-        hipLaunchKernelGGL((rms_norm_kernel<64>), dim3(rows), dim3(64), 0, stream, x, w, cols, eps, y);
-    else
-        hipLaunchKernelGGL((rms_norm_kernel<1024>), dim3(rows), dim3(1024), 0, stream, x, w, cols, eps, y);
+    const auto go = [&](auto kernel, int threads) {
+        hipLaunchKernelGGL(kernel, dim3(rows0 + rows1), dim3(threads), 0, stream, x0, w0, x1, w1, rows0, cols, eps, y0, y1);
+    };
+    if (cols <= 256) go(rms_norm_kernel<64, 4>, 64);
+    else if (cols <= 2048) go(rms_norm_kernel<1024, 2>, 1024);
+    else if (cols <= 4096) go(rms_norm_kernel<1024, 4>, 1024);
+    else go(rms_norm_kernel<1024, 0>, 1024);
     return hipGetLastError();
+}
+
+hipError_t rms_norm_launch(const float* x, const float* w, int rows, int cols, float eps, float* y, hipStream_t stream) {
+    return rms_norm_pair_launch(x, w, rows, y, x, w, 0, y, cols, eps, stream);
 }
 
 hipError_t stage_launch(const float* x, float* stage, int n, hipStream_t stream) {

@@ -457,6 +457,20 @@ def test_rms_norm_rows_swiglu_and_in_place(ly):
     assert vec_err(act.cpu().numpy()[:1000], ref.swiglu(g, u).astype(np.float64)) < 1e-6
 
 
+@pytest.mark.parametrize("cols", [1, 63, 65, 256, 257, 2048, 2049, 4095, 4096, 4097, 8961])
+def test_rms_norm_where_rows_stop_fitting_the_registers(ly, cols):
+    import torch
+
+    rs = lm.Stream(5100 + cols)
+    x, w = rs.sym(3 * cols, 4.0), (1.0 + rs.sym(cols, 0.3)).astype(np.float32)
+    want = np.concatenate([ref.rms_norm(x[r * cols:(r + 1) * cols], w, 1e-6) for r in range(3)]).astype(np.float64)
+    y = out_buf(3 * cols)
+    ly.rms_norm_rows(_dev(x), _dev(w), 3, cols, 1e-6, y)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy()
+    assert vec_err(got[:3 * cols], want) < 1e-6 and (got[3 * cols:] == 12345.0).all()
+
+
 @pytest.mark.parametrize("wtype", TYPES)
 def test_dequant_row_bit_exact(ly, wtype):
     import torch
