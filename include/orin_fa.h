@@ -57,7 +57,7 @@ void orin_fa_set_stream(void* stream);
  * points the library at a caller-owned block of at least that size (256-byte
  * aligned).  Optional: orin_fa_init already allocates a block of this size.
  * orin_fa_prefill uses the same block when it cuts a long context's KV rows among
- * workgroups (few query columns, 3072 rows or more): launches that use the block must
+ * workgroups (few query columns, from about 1100 rows on): launches that use the block must
  * not overlap, which one stream guarantees.  The block's address is baked into a captured
  * graph like every other pointer argument: set the workspace before capturing, keep the
  * block alive while the graph may be replayed, and capture again after changing it (a second
@@ -69,7 +69,8 @@ int orin_fa_set_workspace(void* dev_ptr, size_t bytes);
  * src/kernels.cu:1974-1981): causal GQA attention for a chunk of `batch` query
  * tokens at cache positions [n_past, n_past + batch).  Token b attends to cache
  * positions [0, n_past + b]; the cache must already hold the chunk's own K/V
- * (call site: src/model_gpu.cu:383-384).  Writes every (token < batch, head, i). */
+ * (call site: src/model_gpu.cu:383-384).  Writes every (token < batch, head, i).
+ * out may be q (in place); any other overlap of the two is not allowed. */
 int orin_fa_prefill(const float* q, const uint16_t* kc, const uint16_t* vc, float* out,
                     int n_head, int n_kv, int head_dim, int n_ctx, int n_past, int batch, float scale);
 

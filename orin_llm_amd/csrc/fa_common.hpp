@@ -74,8 +74,10 @@ struct FaArgs {
     int heads_per_group; // prefill: query heads per head group
     int n_splits;      // decode: KV splits
     int kv_split_shift; // prefill: log2 of the number of KV splits a token tile's rows are shared among (0: none);
-                        // with splits, part_o [split][batch][n_head][D] and part_ml [split][batch][n_head] (log-sum-exp, log2
-                        // units) receive what the combine kernel turns into out
+                        // with splits, part_o [split][batch][n_head][D] and part_ml [batch][n_head][lse_stride], of which the
+                        // first [split] are used (log-sum-exp, log2 units; out itself with lse_stride = D, or workspace), receive
+                        // what the combine kernel turns into out
+    int lse_stride;
     float c;           // |scale| * log2(e), clamped away from zero
     float qsign;       // sign of scale, folded into Q
 };

@@ -468,8 +468,8 @@ __global__ __launch_bounds__(kPrefillWaves * 64) void fa_prefill_kernel(
     // and beside their trip to memory: left alone, the compiler fetches each where it is first
     // used, one wait behind the other after the first products.
     {
-        const void *p0 = a.out, *p1 = a.part_o;
-        asm volatile("" ::"s"(p0), "s"(p1), "s"(a.c));
+        const void *p0 = a.out, *p1 = a.part_o, *p2 = a.part_ml;
+        asm volatile("" ::"s"(p0), "s"(p1), "s"(p2), "s"(a.lse_stride), "s"(a.c));
     }
     FA_STAMP(10);
     // ---- query block -> LDS (fp16) ----
@@ -958,7 +958,7 @@ __global__ __launch_bounds__(kPrefillWaves * 64) void fa_prefill_kernel(
         if (kv_split_shift > 0) { // this split's normalised share and its log-sum-exp, for the combine kernel
             const size_t prow = (size_t)split * batch * n_head + orow;
             dst = a.part_o + prow * D;
-            if (part == 0) a.out[orow * D + split] = l_all > 0.0f ? m_all + __builtin_amdgcn_logf(l_all) : -INFINITY; // (where the combine kernel finds it)
+            if (part == 0) a.part_ml[orow * a.lse_stride + split] = l_all > 0.0f ? m_all + __builtin_amdgcn_logf(l_all) : -INFINITY;
         }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -993,10 +993,11 @@ __global__ __launch_bounds__(kPrefillWaves * 64) void fa_prefill_kernel(
 // divided by the weights' sum.  One thread per 16 bytes of out; rows = batch * n_head.  A trip to memory
 // and little else, so every split's piece is asked for before anything is waited for (four at a time,
 // sixteen splits were four trips one after the other: 8 tokens of Qwen2.5-1.5B at 2600 13.4 -> 11.4 us a launch pair).
-// A row's log-sum-exps sit in its own piece of out, which the threads of one wave read and then write: the workspace holds
-// partial outputs alone.
+// A row's log-sum-exps (lse_of, lse_stride floats from one row's to the next's) sit in its own piece of out, which the threads of
+// one wave read and then write, so that the workspace holds partial outputs alone; they are in the workspace where out is
+// the queries' memory (launch() below), and out is then written here and nowhere before.
 template <int D, int S>
-__global__ __launch_bounds__(256) void fa_prefill_combine_kernel(const float* part_o, float* out, int rows) {
+__global__ __launch_bounds__(256) void fa_prefill_combine_kernel(const float* part_o, const float* lse_of, int lse_stride, float* out, int rows) {
     const int idx = blockIdx.x * 256 + threadIdx.x;
     const int row = idx / (D / 4), piece = idx % (D / 4);
     if (row >= rows) return;
@@ -1004,7 +1005,7 @@ __global__ __launch_bounds__(256) void fa_prefill_combine_kernel(const float* pa
     f4 x[S];
 #pragma unroll
     for (int u = 0; u < S; ++u) {
-        lse[u] = out[(size_t)row * D + u];
+        lse[u] = lse_of[(size_t)row * lse_stride + u];
         x[u] = *reinterpret_cast<const f4*>(part_o + ((size_t)u * rows + row) * D + piece * 4);
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -1072,9 +1073,14 @@ hipError_t launch(FaArgs a, int cu_count, hipStream_t stream, void* workspace, s
         int shift = 1;
         while (shift < kMaxPrefillSplitShift && (wgs64 << (shift + 1)) <= cu_count) ++shift;
         const size_t rows = (size_t)a.batch * a.n_head;
+        // A split that is done writes its log-sum-exps while others of its token tile may still have their queries to read, so
+        // they go into out only where out shares no byte with q (in place is allowed); else behind the partial outputs.
+        const uintptr_t q0 = reinterpret_cast<uintptr_t>(a.q), out0 = reinterpret_cast<uintptr_t>(a.out), bytes = rows * D * sizeof(float);
+        const bool in_place = q0 < out0 + bytes && out0 < q0 + bytes;
+        const size_t row_floats = in_place ? D + 1 : D; // of workspace, per row and split
         // (as many as the workspace has room for: 128 tokens of Qwen3-0.6B heads at 8000, whose eight splits take more,
         // ran unsplit in 55.6 us and take 26.3 with four)
-        while (shift > 0 && (rows << shift) * D * sizeof(float) > workspace_bytes) --shift;
+        while (shift > 0 && (rows << shift) * row_floats * sizeof(float) > workspace_bytes) --shift;
         // Where that pays: the more workgroups per token tile, the shorter the walk and the sooner, and the more partial
         // results, the later.  The lines lie at or just above where both ways took the same over 8 to 200 tokens at 700 to 4500 rows of five
         // models' heads (head_dim 64, whose walk costs half a row, breaks even at half as many rows again): 8 tokens of
@@ -1086,6 +1092,8 @@ hipError_t launch(FaArgs a, int cu_count, hipStream_t stream, void* workspace, s
         if (shift > 0 && a.n_past + a.batch >= min_rows && workspace) {
             a.kv_split_shift = shift;
             a.part_o = static_cast<float*>(workspace);
+            a.part_ml = in_place ? a.part_o + (rows << shift) * D : a.out;
+            a.lse_stride = in_place ? 1 << shift : D;
         } else {
             ncb = 1;
             a.tq = 32 / a.heads_per_group;
@@ -1107,10 +1115,10 @@ hipError_t launch(FaArgs a, int cu_count, hipStream_t stream, void* workspace, s
     const int rows = a.batch * a.n_head;
     const unsigned blocks = (unsigned)(((size_t)rows * (D / 4) + 255) / 256);
     switch (a.kv_split_shift) {
-    case 1: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 2>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.out, rows); break;
-    case 2: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 4>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.out, rows); break;
-    case 3: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 8>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.out, rows); break;
-    default: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 16>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.out, rows); break;
+    case 1: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 2>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.part_ml, a.lse_stride, a.out, rows); break;
+    case 2: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 4>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.part_ml, a.lse_stride, a.out, rows); break;
+    case 3: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 8>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.part_ml, a.lse_stride, a.out, rows); break;
+    default: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 16>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.part_ml, a.lse_stride, a.out, rows); break;
     }
     static_assert(kMaxPrefillSplitShift == 4, "the cases above");
     return hipGetLastError();

@@ -392,6 +392,38 @@ def test_cfg2_full_stack_28_layers(fa):
     print(f"cfg2 28 layers x 2 chunks: worst err_row {worst:.3e}", flush=True)
 
 
+@pytest.mark.parametrize("H,G,d,n_ctx,n_past,batch", [
+    (12, 2, 128, 4096, 2600, 8),     # sixteen splits
+    (16, 8, 128, 8192, 5000, 100),   # eight
+    (32, 8, 128, 8192, 5000, 100),   # four
+    (12, 2, 128, 8192, 5632, 512),   # two
+    (32, 8, 64, 4096, 2400, 40),     # eight, head_dim 64
+    (32, 8, 128, 8192, 8000, 128),   # partial outputs that fill the workspace to the byte: fewer splits in place
+    (12, 2, 128, 4096, 100, 45),     # none
+])
+def test_prefill_in_place(fa, H, G, d, n_ctx, n_past, batch):
+    """out = q: a split's log-sum-exps must not land in query rows that another split of the tile has still to read."""
+    import torch
+
+    scale = float(1.0 / np.sqrt(d))
+    q, kc, vc = make_case(700 + n_past, H, G, d, n_ctx, n_past + batch, batch, outliers=4, poison_tail=True)
+    want = gpu_prefill(fa, q, kc, vc, H, G, d, n_ctx, n_past, batch, scale)
+    dk, dv, src = _dev(kc), _dev(vc), _dev(q)
+    x = torch.empty_like(src)
+    same = batch * H * d * 4 * 4 != fa.workspace_bytes()
+    for _ in range(5):
+        x.copy_(src)
+        fa.flash_attention(x, dk, dv, x, H, G, d, n_ctx, n_past, batch, scale)
+        torch.cuda.synchronize()
+        got = x.cpu().numpy()
+        if same:
+            assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+        else: # (another number of splits than out of place: against the oracle, as every other shape is)
+            rows = _sample_rows(np.random.default_rng(7), batch, H, H // G)
+            exact = ref.flash_attention_rows(q, kc, vc, rows, H, G, d, n_ctx, n_past, np.float32(scale))
+            check(got[rows[:, 0], rows[:, 1]], exact, "in place, other splits")
+
+
 # ---------------------------------------------------------------- error behaviour
 
 def test_rejects_bad_arguments(fa):
