@@ -39,9 +39,12 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_f16_kernel(const F16Args a) 
     const int n_in = a.g.n_in;
     const unsigned row_bytes = (unsigned)n_in * 2u;
 
-    unsigned off[RUNS]; // of this lane's 16 bytes of each run; past the row's end: its last 16 bytes, against an activation of zero
+    unsigned off[RUNS]; // of this lane's 16 bytes of each run; past the row's end: its last 16 bytes, whose products are discarded
 #pragma unroll
     for (int j = 0; j < RUNS; ++j) off[j] = min((unsigned)((j * kWaves + wave) * kRun + lane * 8) * 2u, row_bytes - 16u);
+
+    // (the launcher's RUNS is the smallest that covers the row: only a wave's last run can reach past its end)
+    const bool last_live = ((RUNS - 1) * kWaves + wave) * kRun + lane * 8 < n_in;
 
     const int b01 = a.batches[0], b012 = b01 + a.batches[1], total = b012 + a.batches[2];
     auto seg_of = [&](int b, int& row) {
@@ -81,7 +84,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_f16_kernel(const F16Args a) 
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int j = 0; j < RUNS; ++j) {
-            const bool live = ((j * kWaves + wave) * kRun + lane * 8) < n_in;
+            const bool live = j < RUNS - 1 || last_live;
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const float v = live ? x[j][i] : 0.0f;
@@ -101,12 +104,14 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_f16_kernel(const F16Args a) 
         for (int m = 0; m < M; ++m)
 #pragma unroll
             for (int i = 0; i < RB; ++i) {
-                float acc = 0.0f;
+                float acc = 0.0f, whole = 0.0f;
 #pragma unroll
-                for (int j = 0; j < RUNS; ++j)
+                for (int j = 0; j < RUNS; ++j) {
+                    whole = acc;
 #pragma unroll
                     for (int k = 0; k < 8; ++k) acc = __builtin_fmaf((float)r[m][i][j][k], x[j][k], acc);
-                acc = wave_sum(acc);
+                }
+                acc = wave_sum(last_live ? acc : whole); // (a select, not a factor of zero: the row's last weights may be infinite)
                 if (lane == 0) sh_part[set][wave][m * RB + i] = acc;
             }
         lds_meet();

@@ -436,6 +436,31 @@ def test_f16_rows_in_runs(ly, n_in):
         assert vec_err(got[:n], want) < TOL_OP, what
 
 
+@pytest.mark.parametrize("n_in", [32, 512, 1536, 2080, 3584, 16416])
+def test_f16_an_infinite_weight_anywhere_in_a_row(ly, n_in):
+    """Lanes past a row's end fetch its last sixteen bytes: an infinity there must reach the sum once, as itself."""
+    import torch
+
+    spots = sorted({0, n_in // 2, *range(n_in - 8, n_in)})
+    rs = lm.Stream(9100 + n_in)
+    w = np.array(lm.make_tensor(rs, lm.F16, n_in, len(spots))[1]).view(np.uint16).reshape(len(spots), n_in)
+    for r, at in enumerate(spots):
+        w[r, at] = 0x7C00 if r % 2 else 0xFC00
+    x = (1.5 + rs.sym(n_in, 1.0)).astype(np.float32)
+    nw = (1.5 + rs.sym(n_in, 1.0)).astype(np.float32)
+    raw = np.ascontiguousarray(w).reshape(-1).view(np.uint8)
+    want = np.array([np.inf if r % 2 else -np.inf for r in range(len(spots))], np.float32)
+    assert np.array_equal(ref.gemv(lm.F16, raw, x, n_in, len(spots)), want)
+    y, yn, ya = out_buf(len(spots)), out_buf(len(spots)), _dev(np.zeros(len(spots), np.float32))
+    dw, dx = dev_bytes(raw), _dev(x)
+    ly.gemv(lm.F16, dw, dx, y, n_in, len(spots))
+    ly.gemv_multi(lm.F16, [dw], None, [yn], [len(spots)], dx, _dev(nw), 1e-5, n_in)
+    ly.gemv_multi(lm.F16, [dw], None, [ya], [len(spots)], dx, None, 0.0, n_in, True)
+    torch.cuda.synchronize()
+    for got in (y, yn, ya):
+        assert np.array_equal(got.cpu().numpy()[:len(spots)], want)
+
+
 def test_rms_norm_rows_swiglu_and_in_place(ly):
     import torch
 
