@@ -61,14 +61,18 @@ int decode_splits(int n_head, int n_kv, int head_dim, int n_ctx) {
     const int n_hgroups = (r + 15) / 16;
     const int cus = g_state.cu_count > 0 ? g_state.cu_count : 256;
     int s = cus / (n_kv * n_hgroups); // one 8-wave workgroup per CU
-    // A cache too short for eight tiles a split on every CU gets splits of two, up to 64 of them: more CUs then share its
+    // A cache of at most eight tiles, one a wave, stays with one workgroup, which writes the output itself: the combine launch
+    // costs more than other CUs take off it (Qwen2.5-1.5B, one split against two to four, us: 5.2 and 6.7 at 95 of 96
+    // rows, 5.4 and 6.9 at 127 of 128, 4.7 and 6.8 at 20 of 256; at 255 of 256 7.4 and 7.0).
+    // A longer cache still too short for eight tiles a split on every CU gets splits of two, up to 64 of them: more CUs then share its
     // bytes (a CU's load unit takes 64 a clock), and that many partial results cost the combine kernel no more.  Qwen2.5-1.5B at
     // 4095 of 4096 rows 10.2 -> 7.5 us a launch pair, at 200 7.0 as before; 128 splits of an 8192-row cache would be
     // 0.6 us faster at its end and 0.15 slower below a thousand rows.
     const size_t per_split = decode_bytes_per_split(n_head, head_dim);
     const int by_ctx = (n_ctx + kDecodeWaves * kTile - 1) / (kDecodeWaves * kTile);
     const int by_pairs = min((n_ctx + 2 * kTile - 1) / (2 * kTile), min(64, (int)(kStaticScratchBytes / per_split)));
-    if (s > max(by_ctx, by_pairs)) s = max(by_ctx, by_pairs);
+    const int most = by_ctx == 1 ? 1 : max(by_ctx, by_pairs);
+    if (s > most) s = most;
     if (s > kMaxSplits) s = kMaxSplits;
     const size_t ws = g_state.ws ? g_state.ws_bytes : kWorkspaceBytes;
     if ((size_t)s * per_split > ws) s = (int)(ws / per_split);

@@ -119,6 +119,23 @@ def test_decode_small(fa, d, r):
     del torch
 
 
+@pytest.mark.parametrize("H,G,d", [(12, 2, 128), (32, 8, 64), (20, 1, 128)])
+@pytest.mark.parametrize("n_ctx,splits", [(1, 1), (33, 1), (256, 1), (257, 5), (2048, 32), (4096, 64), (4097, 64), (32768, 128)])
+def test_decode_number_of_splits(fa, H, G, d, n_ctx, splits):
+    """One split while a workgroup's waves have a tile each, then splits of two tiles up to 64, then of eight; fewer where the
+    KV heads and head groups fill the chip."""
+    splits = min(splits, 256 // (G * ((H // G + 15) // 16)))
+    assert fa.decode_splits(H, G, d, n_ctx) == splits
+    scale = 1.0 / np.sqrt(d)
+    q, kc, vc = make_case(211 + n_ctx, H, G, d, n_ctx, n_ctx, 1, outliers=4)
+    dk, dv = _dev(kc), _dev(vc)
+    rows = np.array([(0, h) for h in range(H)], np.int32)
+    for pos in sorted({0, n_ctx // 2, n_ctx - 1}):
+        want = ref.flash_attention_rows(q, kc, vc, rows, H, G, d, n_ctx, pos, np.float32(scale))
+        got = gpu_decode(fa, q[0], kc, vc, H, G, d, n_ctx, pos, scale, dk=dk, dv=dv)
+        check(got, want.reshape(got.shape), f"decode d{d} n_ctx{n_ctx} pos{pos}", floor=FLOOR_DECODE)
+
+
 @pytest.mark.parametrize("H,G,d", [(12, 2, 128), (8, 8, 64)])
 def test_decode_where_the_number_of_waves_with_tiles_changes(fa, H, G, d):
     """The last position at which one, two, three ... waves of a workgroup have a tile, and the first at which another has."""
