@@ -462,7 +462,7 @@ bool gemv_use_mfma() {
 }
 void gemv_set_use_mfma(bool on) { g_use_mfma = on ? 1 : 0; }
 
-// Shares of a row that an accumulating projection may be cut into (0: the launcher chooses by shape;
+// Shares of a row that an accumulating projection is cut into (0: the launcher chooses by shape, 1 to kMaxRowShares;
 // 1: never cut, which makes `y += W x` a plain sum with a fixed order; orin_gemv_row_shares(), or ORIN_GEMV_KSPLIT in
 // the environment as the initial value).
 static int g_row_shares = -1;
@@ -470,11 +470,11 @@ int gemv_row_shares() {
     if (g_row_shares < 0) {
         const char* e = getenv("ORIN_GEMV_KSPLIT");
         const int n = e ? atoi(e) : 0;
-        g_row_shares = n >= 0 && n <= 4 ? n : 0;
+        g_row_shares = n >= 0 && n <= kMaxRowShares ? n : 0;
     }
     return g_row_shares;
 }
-void gemv_set_row_shares(int n) { g_row_shares = n >= 0 && n <= 4 ? n : 0; }
+void gemv_set_row_shares(int n) { g_row_shares = n >= 0 && n <= kMaxRowShares ? n : 0; }
 
 size_t weight_row_bytes(int type, int n) {
     switch (type) {

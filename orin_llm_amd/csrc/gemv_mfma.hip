@@ -268,7 +268,7 @@ struct RowsHead {
 };
 constexpr unsigned kMostRowsWgs = 8190, kMostRowsTurns = 62; // what these words have room for
 constexpr int kMostRowsOneTurn = 16383; // (workgroups with one tile each of one matrix)
-constexpr int kMostRowsShares = 16;
+static_assert(kMaxRowShares <= 16, "share_extra: four bits of RowsHead::shape");
 constexpr unsigned kNoMatrix = 8191; // as the first workgroup of a matrix that is not there
 __device__ __forceinline__ int rows_seg(const RowsHead& h, int wg) {
     const unsigned first1 = h.turns1 >> 19, first2 = h.turns2 >> 19;
@@ -640,7 +640,7 @@ bool rows_head(const GemvArgs& a, int wgs, int shares, RowsHead& h) {
     }
     h = RowsHead{w[0], a.w_up ? a.w_up : w[1], w[2], a.x, a.norm_w, turns[0], turns[1], turns[2],
                  (unsigned)(nb - 1) | (unsigned)(nb / shares - 1) << 7 | (unsigned)(nb % shares) << 14 | first << 18};
-    return (first <= kMostRowsWgs || (a.n_seg == 1 && first == tiles[0] && first <= (unsigned)kMostRowsOneTurn)) && shares <= kMostRowsShares && shares <= nb && nb <= 128;
+    return (first <= kMostRowsWgs || (a.n_seg == 1 && first == tiles[0] && first <= (unsigned)kMostRowsOneTurn)) && shares <= kMaxRowShares && shares <= nb && nb <= 128;
 }
 #define ROWS_HEAD_OF(h) (h).w0, (h).w1, (h).w2, (h).x, (h).norm_w, (h).turns0, (h).turns1, (h).turns2, (h).shape
 
@@ -764,8 +764,8 @@ hipError_t launch(const GemvArgs& a, int cu_count, hipStream_t stream) {
         if (a.k_split_override <= 0) {
             ks_r = 1;
             if (a.accumulate && !a.w_up && !a.norm_w && tiles <= cu_count) {
-                ks_r = min((nb_row + 7) / 8, kMostRowsShares);
-                while (tiles * ks_r * 2 <= cu_count && ks_r * 2 <= kMostRowsShares && nb_row >= ks_r * 4) ks_r *= 2;
+                ks_r = min((nb_row + 7) / 8, kMaxRowShares);
+                while (tiles * ks_r * 2 <= cu_count && ks_r * 2 <= kMaxRowShares && nb_row >= ks_r * 4) ks_r *= 2;
             }
         }
         // Eight waves from 9 blocks a row on, which gives a wave one item up to 16 (Qwen2.5-7B's q, k, v in Q5_K and Q6_K 8.4 ->

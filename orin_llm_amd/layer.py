@@ -72,7 +72,7 @@ def use_matrix_cores(on):
 
 
 def gemv_row_shares(shares):
-    """Shares an accumulating projection may cut a row into: 0 = chosen by shape (default), 1 = never cut (every
+    """Shares an accumulating projection may cut a row into: 0 = chosen by shape (default), 2 to 16 = forced, 1 = never cut (every
     result bit for bit reproducible)."""
     _lib().orin_gemv_row_shares(int(shares))
 

@@ -212,6 +212,31 @@ def test_accumulating_projection_is_bit_stable_with_one_share(ly, wtype, n_in, n
 
 
 @pytest.mark.parametrize("wtype", [lm.Q4_K, lm.Q6_K, lm.Q8_0])
+@pytest.mark.parametrize("n_in,n_out", [(1536, 48), (4096, 37), (14336, 32), (18944, 64)])
+def test_every_number_of_shares_can_be_forced(ly, wtype, n_in, n_out):
+    """What the launcher chooses by shape, up to 16 shares, is reached by name too, and a share that is a block longer than its
+    neighbour sums as it should; more shares than a row has blocks are cut to those."""
+    import torch
+
+    rs = lm.Stream(7100 + wtype + n_in)
+    t = lm.make_tensor(rs, wtype, n_in, n_out)
+    x, y0 = rs.sym(n_in, 1.0), rs.sym(n_out, 2.0)
+    want = (y0 + ref.gemv(wtype, t[1], x, n_in, n_out)).astype(np.float64)
+    w, dx = dev_bytes(t[1]), _dev(x)
+    try:
+        for shares in (0, 1, 2, 3, 7, 10, 15, 16):
+            ly.gemv_row_shares(shares)
+            y = _dev(np.concatenate([y0, np.full(4, 12345.0, np.float32)]))
+            ly.gemv_multi(wtype, [w], None, [y], [n_out], dx, None, 0.0, n_in, True)
+            torch.cuda.synchronize()
+            got = y.cpu().numpy()
+            assert (got[n_out:] == 12345.0).all()
+            assert vec_err(got[:n_out], want) < TOL_OP, shares
+    finally:
+        ly.gemv_row_shares(0)
+
+
+@pytest.mark.parametrize("wtype", [lm.Q4_K, lm.Q6_K, lm.Q8_0])
 @pytest.mark.parametrize("bad", [float("nan"), float("inf"), float("-inf")])
 def test_a_non_finite_activation_is_not_laundered(ly, wtype, bad):
     """An infinity or a NaN in the activation makes every row's sum non-finite on the matrix cores as on the vector
