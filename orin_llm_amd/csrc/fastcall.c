@@ -1,6 +1,7 @@
 /* The calls a prefill layer makes eagerly (kernels.py), without ctypes in between: a chunk's depth and size are arguments
- * by value, so these launches cannot be kept in a graph, and on small chunks the host is what bounds them.  A call of 12 to
- * 15 arguments costs 1.4 us through ctypes before the library is entered and 0.5 us here; the launch itself is 3 us.
+ * by value, so these launches cannot be kept in a graph, and on small chunks the host is what bounds them.  A call of 11
+ * arguments, four of them tensors, that the library refuses at once takes 1.0 us through ctypes and 0.3 here (0.03 of it for giving
+ * up the interpreter lock); with its launch a call is 4 us.
  *
  * Pointer arguments are None, integers or objects with data_ptr(); every function returns the library's code.  Linked
  * against liborin_fa.so beside it, so that it shares that library's state with every other caller. */
@@ -54,13 +55,24 @@ static int take(PyObject* const* args, Py_ssize_t n, const char* kinds, void** p
     return 1;
 }
 
+/* The library's code for a call made without the interpreter lock: a launch that waits for a full queue, or the first one,
+ * which loads the kernels, must not stop the program's other threads (nor did it through ctypes). */
+#define unlocked(call) \
+    PyLong_FromLong(__extension__({ \
+        int rc_; \
+        Py_BEGIN_ALLOW_THREADS \
+        rc_ = (call); \
+        Py_END_ALLOW_THREADS \
+        rc_; \
+    }))
+
 static PyObject* prefill(PyObject* self, PyObject* const* args, Py_ssize_t n) {
     void* p[4];
     int i[6];
     float f[1];
     (void)self;
     if (!take(args, n, "ppppiiiiiif", p, i, f)) return NULL;
-    return PyLong_FromLong(orin_fa_prefill(p[0], p[1], p[2], p[3], i[0], i[1], i[2], i[3], i[4], i[5], f[0]));
+    return unlocked(orin_fa_prefill(p[0], p[1], p[2], p[3], i[0], i[1], i[2], i[3], i[4], i[5], f[0]));
 }
 
 static PyObject* rope_store_batch(PyObject* self, PyObject* const* args, Py_ssize_t n) {
@@ -69,7 +81,7 @@ static PyObject* rope_store_batch(PyObject* self, PyObject* const* args, Py_ssiz
     float f[1];
     (void)self;
     if (!take(args, n, "pppppiiiiiiifpi", p, i, f)) return NULL;
-    return PyLong_FromLong(orin_fa_rope_store_batch(p[0], p[1], p[2], p[3], p[4], i[0], i[1], i[2], i[3], i[4], i[5], i[6], f[0], p[5], i[7]));
+    return unlocked(orin_fa_rope_store_batch(p[0], p[1], p[2], p[3], p[4], i[0], i[1], i[2], i[3], i[4], i[5], i[6], f[0], p[5], i[7]));
 }
 
 static PyObject* rope_batch(PyObject* self, PyObject* const* args, Py_ssize_t n) {
@@ -78,7 +90,7 @@ static PyObject* rope_batch(PyObject* self, PyObject* const* args, Py_ssize_t n)
     float f[1];
     (void)self;
     if (!take(args, n, "piiifiipi", p, i, f)) return NULL;
-    return PyLong_FromLong(orin_fa_rope_batch(p[0], i[0], i[1], i[2], f[0], i[3], i[4], p[1], i[5]));
+    return unlocked(orin_fa_rope_batch(p[0], i[0], i[1], i[2], f[0], i[3], i[4], p[1], i[5]));
 }
 
 static PyObject* kv_store_batch(PyObject* self, PyObject* const* args, Py_ssize_t n) {
@@ -86,7 +98,7 @@ static PyObject* kv_store_batch(PyObject* self, PyObject* const* args, Py_ssize_
     int i[5];
     (void)self;
     if (!take(args, n, "ppppiiiii", p, i, NULL)) return NULL;
-    return PyLong_FromLong(orin_fa_kv_store_batch(p[0], p[1], p[2], p[3], i[0], i[1], i[2], i[3], i[4]));
+    return unlocked(orin_fa_kv_store_batch(p[0], p[1], p[2], p[3], i[0], i[1], i[2], i[3], i[4]));
 }
 
 static PyMethodDef methods[] = {

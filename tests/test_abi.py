@@ -2,7 +2,9 @@
 import ctypes
 import os
 import re
+import shutil
 import subprocess
+import sys
 
 import pytest
 
@@ -249,3 +251,40 @@ def test_eager_calls_take_what_the_wrappers_document():
         k.flash_attention(1, 1, 1, 1, 12, 2, 128, 4096, 0, "45", 0.1)
     with pytest.raises(AttributeError):
         k.kv_store_batch("cache", 1, 1, 1, 2, 128, 4096, 0, 45)
+
+
+def test_eager_calls_let_other_threads_run(tmp_path):
+    """The extension module gives up the interpreter lock while the library works: another thread counts on while a call
+    waits (a stand-in library that sleeps; no GPU)."""
+    import sysconfig
+
+    include = sysconfig.get_paths()["include"]
+    if not os.path.exists(os.path.join(include, "Python.h")) or not shutil.which("gcc"):
+        pytest.skip("no C compiler or no Python headers")
+    names = ("orin_fa_prefill", "orin_fa_rope_store_batch", "orin_fa_rope_batch", "orin_fa_kv_store_batch")
+    (tmp_path / "stub.c").write_text("#include <unistd.h>\n" + "".join(f"int {n}() {{ usleep(300000); return {i + 1}; }}\n" for i, n in enumerate(names)))
+    subprocess.run(["gcc", "-shared", "-fPIC", str(tmp_path / "stub.c"), "-o", str(tmp_path / "libstub.so")], check=True)
+    subprocess.run(["gcc", "-O2", "-Wall", "-Werror", "-shared", "-fPIC", "-I" + include, os.path.join(ROOT, "orin_llm_amd", "csrc", "fastcall.c"), "-L" + str(tmp_path),
+                    "-l:libstub.so", "-Wl,-rpath,$ORIGIN", "-o", str(tmp_path / "_fastcall.so")], check=True)
+    (tmp_path / "run.py").write_text("""
+import threading, time
+import _fastcall as m
+ticks, stop = 0, False
+def count():
+    global ticks
+    while not stop:
+        ticks += 1
+        time.sleep(0.005)
+t = threading.Thread(target=count)
+t.start()
+for want, call in enumerate((lambda: m.prefill(1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1.0), lambda: m.rope_store_batch(1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1.0, None, 1),
+                             lambda: m.rope_batch(1, 1, 1, 1, 1.0, 1, 1, None, 1), lambda: m.kv_store_batch(1, 1, 1, 1, 1, 1, 1, 1, 1))):
+    before = ticks
+    assert call() == want + 1
+    print(ticks - before)
+stop = True
+t.join()
+""")
+    out = subprocess.run([sys.executable, "run.py"], cwd=tmp_path, capture_output=True, text=True, timeout=60)
+    assert out.returncode == 0, out.stderr
+    assert all(int(n) >= 5 for n in out.stdout.split()) and len(out.stdout.split()) == 4, out.stdout  # (60 of them fit a call)
