@@ -1,7 +1,8 @@
 """Builds liborin_fa.so (HIP kernels + C ABI + llm::cuda shim) for gfx950, in-tree, with the extension module that calls it
-from Python (_fastcall.so), and beside it the two
+from Python (_fastcall, where there is a C compiler and the Python headers: the C ABI needs neither), and beside it the two
 measurement-aid libraries that bench.py and one GPU test load (liborin_fa_stamps.so, liborin_fa_bench.so)."""
 import os
+import shutil
 import subprocess
 import sysconfig
 from concurrent.futures import ThreadPoolExecutor
@@ -15,8 +16,8 @@ STAMPED = ("fa_prefill.hip", "fa_decode.hip", "gemv_mfma.hip", "fa_api.hip")
 # Read-only stand-ins and a do-nothing kernel (csrc/bench_aids.hip), a library of their own: the product exports none of them.
 BENCH_LIB = os.path.join(HERE, "liborin_fa_bench.so")
 BENCH_SOURCE = os.path.join(HERE, "csrc", "bench_aids.hip")
-# The eager calls of kernels.py as a CPython extension on top of LIB (csrc/fastcall.c).
-FASTCALL = os.path.join(HERE, "_fastcall.so")
+# The eager calls of kernels.py as a CPython extension on top of LIB (csrc/fastcall.c), for the interpreter that builds it.
+FASTCALL = os.path.join(HERE, "_fastcall" + sysconfig.get_config_var("EXT_SUFFIX"))
 FASTCALL_SOURCE = os.path.join(HERE, "csrc", "fastcall.c")
 # The cut-off builds: the decode split kernel with parts taken out (-DORIN_FA_DECODE_PROBE=flags, see fa_decode.hip;
 # results wrong by design), one library per flag set, for bench.py's cut-off workloads.  Measurement aids, built
@@ -63,8 +64,18 @@ def check_toolchain():
 def _run(cmd):
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
-        raise RuntimeError("hipcc failed:\n" + " ".join(cmd) + "\n" + res.stdout + res.stderr)
+        raise RuntimeError("compiler failed:\n" + " ".join(cmd) + "\n" + res.stdout + res.stderr)
     return " ".join(cmd)
+
+
+def fastcall_command(lib=LIB, out=FASTCALL):
+    """The command that builds the extension module, or None where it cannot be built (kernels.py then calls through ctypes)."""
+    include = sysconfig.get_paths()["include"]
+    cc = next((c for c in map(shutil.which, ("gcc", "cc", "clang", os.path.join(os.path.dirname(HIPCC), "amdclang"))) if c), None)
+    if not cc or not os.path.exists(os.path.join(include, "Python.h")):
+        return None
+    return [cc, "-O2", "-Wall", "-shared", "-fPIC", "-I" + include, FASTCALL_SOURCE, "-L" + os.path.dirname(lib), "-l:" + os.path.basename(lib),
+            "-Wl,-rpath,$ORIGIN", "-o", out]
 
 
 def build(verbose=False, probes=False):
@@ -91,8 +102,14 @@ def build(verbose=False, probes=False):
     lines.append(_run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC"] + [stamped.get(s, o) for s, o in zip(SOURCES, objs)]
                       + ["-o", STAMPS_LIB]))
     lines.append(_run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", bench_obj, "-o", BENCH_LIB]))
-    lines.append(_run(["gcc", "-O2", "-Wall", "-shared", "-fPIC", "-I" + sysconfig.get_paths()["include"], FASTCALL_SOURCE,
-                       "-L" + HERE, "-l:" + os.path.basename(LIB), "-Wl,-rpath,$ORIGIN", "-o", FASTCALL]))
+    for old in {FASTCALL, os.path.join(HERE, "_fastcall.so")}: # (never one of an earlier build beside a newer library)
+        if os.path.exists(old):
+            os.remove(old)
+    fastcall = fastcall_command()
+    if fastcall:
+        lines.append(_run(fastcall))
+    else:
+        print("no C compiler or no Python headers: the eager calls go through ctypes (0.7 us more each)")
     for f, o in probes.items():
         lines.append(_run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC"] + [o if s == dec else x for s, x in zip(SOURCES, objs)]
                           + ["-o", PROBE_LIB.format(f)]))

@@ -5,7 +5,9 @@ the reference's print-and-abort (src/common.h:14-22).  There is no fallback: a m
 library is an ImportError.
 """
 import ctypes
+import importlib
 import os
+import types
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "liborin_fa.so")
@@ -83,17 +85,26 @@ def lib():
     return _lib
 
 
+def _through_ctypes():
+    L = lib()
+
+    def taking(fn, pointers):
+        return lambda *a: fn(*[_ptr(v) if i in pointers else v for i, v in enumerate(a)])
+
+    return types.SimpleNamespace(prefill=taking(L.orin_fa_prefill, (0, 1, 2, 3)), rope_store_batch=taking(L.orin_fa_rope_store_batch, (0, 1, 2, 3, 4, 13)),
+                                 rope_batch=taking(L.orin_fa_rope_batch, (0, 7)), kv_store_batch=taking(L.orin_fa_kv_store_batch, (0, 1, 2, 3)))
+
+
 def _calls():
-    """The eager calls as an extension module (csrc/fastcall.c): what ctypes spends on a call's arguments is a quarter of
-    a small launch."""
+    """The eager calls as an extension module (csrc/fastcall.c): what ctypes spends on a call's arguments is a fifth of
+    a small launch.  Through ctypes where the module was not built for this interpreter."""
     global _fastcall
     if _fastcall is None:
         lib()  # (says what is missing, if it is)
         try:
-            from . import _fastcall as m
-        except ImportError as e:
-            raise ImportError(f"{os.path.join(_HERE, '_fastcall.so')} is missing or does not load ({e}): build it with __graft_entry__.build()") from e
-        _fastcall = m
+            _fastcall = importlib.import_module("._fastcall", __package__)
+        except ModuleNotFoundError: # (one that is there and does not load raises)
+            _fastcall = _through_ctypes()
     return _fastcall
 
 

@@ -2,7 +2,6 @@
 import ctypes
 import os
 import re
-import shutil
 import subprocess
 import sys
 
@@ -225,10 +224,16 @@ int main(int argc, char**) {
     assert r.returncode == 0, r.stderr
 
 
-def test_eager_calls_take_what_the_wrappers_document():
-    """The extension module behind the eager calls: integers, None and objects with data_ptr() as pointers, keywords, and
-    errors that are not swallowed (the library itself refuses every call here: it has not been initialised)."""
+@pytest.mark.parametrize("binding", ["module", "ctypes"])
+def test_eager_calls_take_what_the_wrappers_document(binding, monkeypatch):
+    """The extension module behind the eager calls, and what stands in where it cannot be built: integers, None and objects
+    with data_ptr() as pointers, keywords, and errors that are not swallowed (the library itself refuses every call here:
+    it has not been initialised)."""
     from orin_llm_amd import kernels as k
+
+    monkeypatch.setattr(k, "_fastcall", k._through_ctypes() if binding == "ctypes" else None)
+    if binding == "module" and not hasattr(k._calls(), "__file__"):
+        pytest.skip("the extension module is not built for this interpreter")
 
     class Tensor:
         def data_ptr(self):
@@ -247,25 +252,39 @@ def test_eager_calls_take_what_the_wrappers_document():
         assert e.value.code == -4
     with pytest.raises(ValueError):
         k.flash_attention(Broken(), 1, 1, 1, 12, 2, 128, 4096, 0, 45, 0.1)
-    with pytest.raises(TypeError):
+    with pytest.raises(ctypes.ArgumentError if binding == "ctypes" else TypeError):
         k.flash_attention(1, 1, 1, 1, 12, 2, 128, 4096, 0, "45", 0.1)
     with pytest.raises(AttributeError):
         k.kv_store_batch("cache", 1, 1, 1, 2, 128, 4096, 0, 45)
 
 
+def test_the_extension_module_is_built_for_one_interpreter_or_not_at_all(monkeypatch):
+    """Its file carries the interpreter's tag; without a C compiler or the Python headers nothing is asked of either."""
+    import sysconfig
+
+    from orin_llm_amd import build as fa_build
+
+    assert fa_build.FASTCALL.endswith(sysconfig.get_config_var("EXT_SUFFIX"))
+    with monkeypatch.context() as m:
+        m.setattr(fa_build.shutil, "which", lambda name: None)
+        assert fa_build.fastcall_command() is None
+    with monkeypatch.context() as m:
+        m.setattr(fa_build.sysconfig, "get_paths", lambda: {"include": "/nonexistent"})
+        assert fa_build.fastcall_command() is None
+
+
 def test_eager_calls_let_other_threads_run(tmp_path):
     """The extension module gives up the interpreter lock while the library works: another thread counts on while a call
     waits (a stand-in library that sleeps; no GPU)."""
-    import sysconfig
+    from orin_llm_amd import build as fa_build
 
-    include = sysconfig.get_paths()["include"]
-    if not os.path.exists(os.path.join(include, "Python.h")) or not shutil.which("gcc"):
+    command = fa_build.fastcall_command(str(tmp_path / "libstub.so"), str(tmp_path / "_fastcall.so"))
+    if not command:
         pytest.skip("no C compiler or no Python headers")
     names = ("orin_fa_prefill", "orin_fa_rope_store_batch", "orin_fa_rope_batch", "orin_fa_kv_store_batch")
     (tmp_path / "stub.c").write_text("#include <unistd.h>\n" + "".join(f"int {n}() {{ usleep(300000); return {i + 1}; }}\n" for i, n in enumerate(names)))
-    subprocess.run(["gcc", "-shared", "-fPIC", str(tmp_path / "stub.c"), "-o", str(tmp_path / "libstub.so")], check=True)
-    subprocess.run(["gcc", "-O2", "-Wall", "-Werror", "-shared", "-fPIC", "-I" + include, os.path.join(ROOT, "orin_llm_amd", "csrc", "fastcall.c"), "-L" + str(tmp_path),
-                    "-l:libstub.so", "-Wl,-rpath,$ORIGIN", "-o", str(tmp_path / "_fastcall.so")], check=True)
+    subprocess.run([command[0], "-shared", "-fPIC", str(tmp_path / "stub.c"), "-o", str(tmp_path / "libstub.so")], check=True)
+    subprocess.run(command + ["-Werror"], check=True)
     (tmp_path / "run.py").write_text("""
 import threading, time
 import _fastcall as m
