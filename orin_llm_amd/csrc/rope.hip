@@ -114,7 +114,7 @@ struct RopeArgs {
 template <bool NEOX, int U>
 __global__ __launch_bounds__(kRopeThreads) void rope_pieces_kernel(const RopeArgs a) {
 #pragma clang fp contract(off)
-    __shared__ float2 sh_cs[kRopeThreads];
+    __shared__ __attribute__((aligned(16))) float2 sh_cs[kRopeThreads]; // (read two pairs at a time)
     const int tid = threadIdx.x, token0 = (int)blockIdx.x * a.block_tokens, head0 = (int)blockIdx.y << a.block_heads_log2;
     const int o1 = NEOX ? a.half : 4;
     float4 lo[U], hi[U];
