@@ -714,6 +714,33 @@ def test_workgroups_and_shares_of_rows_in_runs(ly, types, n_in, heights):
         assert e < TOL_OP, what
 
 
+@pytest.mark.parametrize("wtype", [lm.Q4_K, lm.Q6_K, lm.Q8_0])
+@pytest.mark.parametrize("blocks", [8, 9, 15, 16, 17])
+def test_rows_where_the_number_of_waves_changes(ly, wtype, blocks):
+    """Eight waves a workgroup from nine blocks of 256 elements a row on (in Q8_0 from sixteen where there are more tiles than
+    CUs), one item a wave up to sixteen, while a workgroup has one tile: either side of each of these lines, in one matrix and,
+    beside one of another type, in a launch of two types."""
+    import torch
+
+    n_in, rs = 256 * blocks, lm.Stream(7970 + blocks + wtype)
+    other = lm.Q5_K
+    x, nw, eps = rs.sym(n_in, 1.0), (1.0 + rs.sym(n_in, 0.3)).astype(np.float32), 1e-5
+    xn, dx, dnw = ref.rms_norm(x, nw, eps), _dev(x), _dev(nw)
+    big, small = lm.make_tensor(rs, wtype, n_in, 16 * 769), lm.make_tensor(rs, other, n_in, 16)
+    want, want_small = (ref.gemv(t, m[1], xn, n_in, n).astype(np.float64) for t, m, n in ((wtype, big, 16 * 769), (other, small, 16)))
+    w, ws = dev_bytes(big[1]), dev_bytes(small[1])
+    for tiles in (1, 256, 257, 768, 769):
+        n_out = 16 * tiles
+        y, z, zs = out_buf(n_out), out_buf(n_out), out_buf(16)
+        ly.gemv_multi(wtype, [w], None, [y], [n_out], dx, dnw, eps, n_in)
+        ly.gemv_multi_types([wtype, other], [w, ws], None, [z, zs], [n_out, 16], dx, dnw, eps, n_in)
+        torch.cuda.synchronize()
+        for got, exact in ((y, want[:n_out]), (z, want[:n_out]), (zs, want_small)):
+            g = got.cpu().numpy()
+            assert (g[len(exact):] == 12345.0).all()
+            assert vec_err(g[:len(exact)], exact) < TOL_OP, (tiles, len(exact))
+
+
 @pytest.mark.parametrize("n_in", [256, 1792])
 def test_more_row_tiles_than_a_launch_counts_workgroups_for(ly, n_in):
     """A vocabulary's worth of rows: 8200 tiles, one workgroup each or several tiles a workgroup."""
