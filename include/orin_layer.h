@@ -92,7 +92,8 @@ void orin_gemv_use_matrix_cores(int on);
  * chooses 1 to 16 by shape (up to 8 blocks of 256 elements a share: 7 for rows of 14336 elements, 10 for 18944),
  * which is fastest and leaves the order of a row's adds open (see orin_gemv_q8_add);
  * 1 = never cut, every result bit for bit reproducible, at up to 0.4 us more per output projection and 1 to
- * 4.5 us more per down projection; 2 to 16 = forced (tuning; no more than a row has blocks); anything else = 0.  Takes effect with the next launch; graphs captured earlier keep the launches they recorded.
+ * 4.5 us more per down projection; 2 to 16 = forced (tuning; no more than a row has blocks); anything else = 0.
+ * Takes effect with the next launch; graphs captured earlier keep the launches they recorded.
  * ORIN_GEMV_KSPLIT in the environment sets the initial value. */
 void orin_gemv_row_shares(int shares);
 
@@ -106,7 +107,7 @@ int orin_gemv_multi(int type, int n_mat, const void* const* W, const float* cons
                     const int* n_out, const float* x, const float* norm_w, float eps, int n_in, int accumulate);
 
 /* The same with a type per matrix (a file that keeps attn_v in Q6_K beside Q4_K projections): one launch
- * where every type is Q4_K or Q6_K, one launch per matrix otherwise. */
+ * where every type is a block type and n_in a multiple of 256, one launch per matrix otherwise. */
 int orin_gemv_multi_types(const int* types, int n_mat, const void* const* W, const float* const* bias, float* const* y,
                           const int* n_out, const float* x, const float* norm_w, float eps, int n_in);
 

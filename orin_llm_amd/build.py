@@ -80,7 +80,7 @@ def fastcall_command(lib=LIB, out=FASTCALL):
 
 def build(verbose=False, probes=False):
     """Compiles every source (in parallel) and links the shared library and its timeline build.  Always recompiles.
-    probes=True also builds the eleven cut-off libraries (measurement aids whose results are wrong by design)."""
+    probes=True also builds the thirteen cut-off libraries (measurement aids whose results are wrong by design)."""
     check_toolchain()
     os.makedirs(OBJ_DIR, exist_ok=True)
     objs = [os.path.join(OBJ_DIR, os.path.basename(s) + ".o") for s in SOURCES]

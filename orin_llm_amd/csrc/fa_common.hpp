@@ -31,8 +31,9 @@ constexpr int kMaxSplits = 256;                 // decode KV splits per KV head,
 constexpr size_t kWorkspaceBytes = 8u << 20;    // split-KV partial results
 
 // The rotary frequencies theta^(-2 i / n_rot), as kernels take them: where -2 i / n_rot is exact in fp32 (n_rot a power of
-// two: every model shape) by the doubles theta^(-2 2^k / n_rot), a frequency being the product over the bits k of i -- within
-// a few of a double's ulps of the power, so the same float, for 20 instructions instead of 300.  Else by theta itself.
+// two: every model shape) by the doubles theta^(-2 2^k / n_rot), a frequency being the product over the bits k of i, for
+// 20 instructions instead of 300.  Squaring carries the first double's rounding along: up to 54 of a double's ulps from the power at
+// n_rot 128, 221 at 512 (a float's ulp is 2^29 of them), over 209 bases from 1.5 to 1e8 never another float (106799 compared).  Else by theta itself.
 struct RopeFreq {
     double step[8];
     float theta;

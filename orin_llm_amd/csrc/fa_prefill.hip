@@ -992,7 +992,7 @@ __global__ __launch_bounds__(kPrefillWaves * 64) void fa_prefill_kernel(
 // out = sum over the KV splits of their normalised outputs, weighted by 2^(lse_s - max lse) and
 // divided by the weights' sum.  One thread per 16 bytes of out; rows = batch * n_head.  A trip to memory
 // and little else, so every split's piece is asked for before anything is waited for (four at a time,
-// sixteen splits were four trips one after the other: 8 tokens of Qwen2.5-1.5B at 2600 13.4 -> 11.4 us a launch pair).
+// sixteen splits were four trips one after the other: 8 tokens of Qwen2.5-1.5B at 2600 13.0 -> 10.6 us a launch pair).
 // A row's log-sum-exps (lse_of, lse_stride floats from one row's to the next's) sit in its own piece of out, which the threads of
 // one wave read and then write, so that the workspace holds partial outputs alone; they are in the workspace where out is
 // the queries' memory (launch() below), and out is then written here and nowhere before.

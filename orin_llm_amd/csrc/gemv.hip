@@ -509,7 +509,7 @@ hipError_t gemv_launch(int type, GemvArgs a, int cu_count, hipStream_t stream) {
     }
 }
 
-// Matrices of different types over one activation: one launch when every one of them is Q4_K or Q6_K and the
+// Matrices of different types over one activation: one launch when every one of them is of a block type and the
 // matrix-core kernel takes the shape; hipErrorNotSupported otherwise (the caller then launches them one by one).
 hipError_t gemv_mixed_launch(GemvArgs a, int cu_count, hipStream_t stream) {
     drop_stale_error();

@@ -711,7 +711,10 @@ bool launch_rows(const GemvArgs& a, int wgs, int shares, bool wide, int nb_wg, h
         if (a.seg[i].n_out % 16 != 0 || !rows_base_ok(T, a.seg[i].w)) return false;
     if (a.w_up && !rows_base_ok(T, a.w_up)) return false;
     const int n_in_wg = nb_wg * 256;
-    if constexpr (T == kQ8_0) { // (272 bytes are a long run already: two blocks only where they make one item of a wave's share)
+    // Q8_0: 272 bytes are a long run already, so two blocks only where they make one item of a wave's share, and with eight waves,
+    // whose buffers then leave room for one workgroup a CU, only up to a workgroup a CU (two blocks against one: 4096 x 4096 5.7 and
+    // 6.05 us, 4096 x 1024 4.7 and 5.2; 4096 x 6144, 384 workgroups, 9.3 and 8.4).
+    if constexpr (T == kQ8_0) {
         if (wide) return nb_wg <= 16 && wgs <= g_rows_resident / 3 ? launch_rows_as<T, false, 8, 2>(a, wgs, shares, n_in_wg, stream) : launch_rows_as<T, false, 8, 1>(a, wgs, shares, n_in_wg, stream);
         if (!a.w_up && nb_wg > 4 && nb_wg <= 8 && wgs == rows_tiles(a)) return launch_rows_as<T, false, 4, 2>(a, wgs, shares, n_in_wg, stream);
         return a.w_up ? launch_rows_as<T, true, 4, 1>(a, wgs, shares, n_in_wg, stream) : launch_rows_as<T, false, 4, 1>(a, wgs, shares, n_in_wg, stream);
@@ -769,7 +772,9 @@ hipError_t launch(const GemvArgs& a, int cu_count, hipStream_t stream) {
             }
         }
         // Eight waves from 9 blocks a row on, which gives a wave one item up to 16 (Qwen2.5-7B's q, k, v in Q5_K and Q6_K 8.4 ->
-        // 6.4 us); Q8_0's buffers for that leave room for one such workgroup a CU.
+        // 6.4 us); of Q8_0, up to 15 blocks only where there is a workgroup a CU at most.  (Between one and two a CU eight waves, one
+        // block an item, measure faster as well, 3072 x 6144 8.45 -> 7.45 us, 2560 x 6144 7.1 -> 6.6; beyond, 3 % slower to 8 %
+        // faster.  The line could lie at two.)
         const bool wide_r = ks_r == 1 && nb_row > (T == kQ8_0 && tiles > cu_count ? 15 : 8) && !a.w_up && wgs == tiles;
         if (launch_rows<T>(a, wgs, ks_r, wide_r, (nb_row + ks_r - 1) / ks_r, stream)) return hipGetLastError();
     }

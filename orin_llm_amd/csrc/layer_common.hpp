@@ -39,12 +39,12 @@ struct GemvArgs {
 size_t weight_row_bytes(int type, int n); // 0: unknown type or n not a whole number of blocks
 int weight_align(int type);               // alignment the kernels need of a matrix's base address
 hipError_t gemv_launch(int type, GemvArgs args, int cu_count, hipStream_t stream);
-// Q4_K and Q6_K on the matrix cores (gemv_mfma.hip): whether type and shape fit, the launch, and the once-only
+// The block types (Q4_K, Q5_K, Q6_K, Q8_0) on the matrix cores (gemv_mfma.hip): whether type and shape fit, the launch, and the once-only
 // permission for large LDS blocks.
 bool gemv_mfma_ok(int type, const GemvArgs& args);
 hipError_t gemv_mfma_launch(int type, const GemvArgs& args, int cu_count, hipStream_t stream);
 hipError_t gemv_mfma_allow_lds();
-// Up to three matrices, each Q4_K or Q6_K (GemvSeg::type), in one launch on the matrix cores.
+// Up to three matrices, each of a block type of its own (GemvSeg::type), in one launch on the matrix cores.
 hipError_t gemv_mixed_launch(GemvArgs args, int cu_count, hipStream_t stream);
 hipError_t gemv_mfma_mixed_launch(GemvArgs args, int cu_count, hipStream_t stream);
 hipError_t gemv_f16_launch(const GemvArgs& args, int cu_count, hipStream_t stream); // F16 (gemv_f16.hip)
