@@ -35,6 +35,8 @@
 // hit conflict-free.  Each wave walks its tiles from the diagonal backwards, so the only tile
 // that can need the causal mask is handled in the prologue and the steady state is mask-free.
 //
+// A chunk near the start of its context takes a second kernel (fa_prefill_short_kernel).
+//
 // Few query columns on a long context (a model with few heads, or a short chunk): the launcher
 // lets 2 to 16 workgroups share a token tile's KV rows (runs of four tiles go to the splits in
 // turn); each writes its normalised output and log-sum-exp to the workspace and
@@ -231,6 +233,13 @@ __device__ __forceinline__ void lds_copy_1k(i32x4 desc, unsigned lds_base, int o
                  :
                  : "v"(off), "s"(desc), "s"(soff), "n"(IMM), "s"(lds_base)
                  : "memory", "m0");
+}
+
+// A 16-byte streaming store, spelled out: as a builtin the hint is lost when the compiler merges it with a plain store on
+// another branch.  The wait states are the block's own: the compiler, which cannot see the store, may write its data registers
+// in the very next instruction, and the last words of the old data are read a cycle or two after the issue.
+__device__ __forceinline__ void store_stream(float* p, f4 v) {
+    asm volatile("global_store_dwordx4 %0, %1, off nt\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
 }
 
 // The vector instructions of stage B for one 32x32 score block (16 scores per lane), in issue
@@ -981,12 +990,299 @@ __global__ __launch_bounds__(kPrefillWaves * 64) void fa_prefill_kernel(
                 for (int j = 0; j < kHalfJ; ++j) *reinterpret_cast<f4*>(dst + ((h * kHalfJ + j) * kParts + part) * 4) = acc[j];
             } else {
 #pragma unroll
-                for (int j = 0; j < kHalfJ; ++j) // (spelled out: as a builtin the hint is lost when the compiler merges the two branches)
-                    asm volatile("global_store_dwordx4 %0, %1, off nt" ::"v"(dst + ((h * kHalfJ + j) * kParts + part) * 4), "v"(acc[j]) : "memory");
+                for (int j = 0; j < kHalfJ; ++j) store_stream(dst + ((h * kHalfJ + j) * kParts + part) * 4, acc[j]);
             }
         }
     }
     FA_STAMP(8);
+}
+
+// ---------------------------------------------------------------------------------------------
+// Short walks: a chunk near the start of its context, whose workgroups see a few tiles of KV rows.  The kernel above is built for its steady state: a wave asks for two tiles of K ahead, multiplies a
+// second tile while it scans the first, and leaves through its pipeline's drain, 4 us for a chunk whose waves have a tile each
+// (stage marks of 45 tokens of Qwen2.5-1.5B at depth 0).  Here eight waves -- two a SIMD, each the cover for the other's waits --
+// take a tile of 32 rows each, 256 rows a workgroup and turn, with nothing between a tile's arrival and its use: one buffer for K and
+// one for V a wave, the next tile's K asked for when this one's products are through with the buffer, its V likewise.
+// 32 query columns a workgroup, packed as above; the same layouts in LDS, the same (m, l, O) hand-over, over the waves that had a
+// tile.  Softmax with the tiles' true maxima, row sums in fp32.  Bound by its chain -- queries there 1.25 us after the first wave's entry,
+// scores 2.1, weights 2.3, outputs 2.7, handed over 3.1, stored 3.5 -- and, from five tiles on, by the 64 bytes a clock at which a
+// CU takes them in.  Qwen2.5-1.5B heads at depth 0, us a launch: 16 tokens 5.15 -> 4.2, 45 5.3 -> 4.35, 100 5.75 -> 4.8, 200 6.3 -> 6.2;
+// Llama-3.2-1B's: 45 tokens 4.4 -> 3.8.
+// ---------------------------------------------------------------------------------------------
+constexpr int kShortWaves = 8;
+template <int D>
+struct SGeom {
+    using G = PGeom<D, 1>;
+    static constexpr int kWaveB = 2 * G::kTileB; // K, V; the merge buffer takes their place (32 columns x D floats: the same size)
+    static_assert(kWaveB >= G::kMergeB, "merge buffer");
+    static constexpr int kMlOff = kShortWaves * kWaveB;
+    static constexpr int kQOff = kMlOff + kShortWaves * 32 * 2 * 4;
+    static constexpr int kLdsB = kQOff + 32 * G::kQStride;
+};
+
+template <int D>
+__global__ __launch_bounds__(kShortWaves * 64, D == 64 ? 4 : 2) void fa_prefill_short_kernel(
+    const float* q_in, const uint16_t* kc, const uint16_t* vc, const int n_ctx, // (as above: what the first requests need)
+    const int n_past, const int batch, const int n_head, const int r_heads, const int n_ttiles, const unsigned packed,
+    const float qsign, const FaArgs a) {
+    using G = PGeom<D, 1>;
+    using SG = SGeom<D>;
+    constexpr int kWaves = kShortWaves, kC = G::kCopies, kVar = G::kCopyVariants;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int heads_per_group = packed & 15, tq = (packed >> 8) & 255;
+    const int tq_magic = packed >> 16;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c32 = lane & 31, hh = lane >> 5;
+    const int kvh = __builtin_amdgcn_readfirstlane(blockIdx.x);
+    const int hg = __builtin_amdgcn_readfirstlane(blockIdx.y);
+    const int t0 = (n_ttiles - 1 - __builtin_amdgcn_readfirstlane(blockIdx.z)) * tq; // longest rows first
+    const int head_lo = hg * heads_per_group;
+    const int tok_hi = (t0 + tq < batch) ? t0 + tq : batch;
+    const int kv_end = n_past + tok_hi;
+    const int full_end = n_past + t0 + 1;
+    const int n_tiles = (kv_end + kTile - 1) / kTile;
+    const int n_mine = n_tiles > wave ? ((n_tiles - 1 - wave) >> 3) + 1 : 0; // wave w takes tiles w, w + 8, ...
+    static_assert(kWaves == 8, "tile distance as a shift");
+    const int n_act = min(n_tiles, kWaves); // waves with a tile: one at least
+    auto col_valid = [&](int c, int& tok, int& hl) { // (as above)
+        const int hq = (c * tq_magic) >> 16;
+        tok = t0 + c - hq * tq;
+        hl = head_lo + hq;
+        return hq < heads_per_group && hl < r_heads && tok < batch;
+    };
+    unsigned char* const ws = smem + wave * SG::kWaveB;
+    const unsigned ws_addr = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)ws);
+
+    // ---- requests: queries (the wave's four columns), its first tile's K and V ----
+    constexpr int kColsPerLoad = 256 / D, kQLoads = 32 / kWaves / kColsPerLoad;
+    static_assert(kQLoads >= 1, "queries of a wave");
+    u32x4 qraw[kQLoads];
+    float qmul[kQLoads];
+    int qcol[kQLoads];
+    {
+        const i32x4 qdesc = make_desc(q_in, (unsigned)batch * n_head * D * 4);
+        static_for<0, kQLoads>([&](auto jc) {
+            constexpr int j = decltype(jc)::value;
+            const int c = (wave * kQLoads + j) * kColsPerLoad + lane / (D / 4);
+            int tok, hl;
+            const bool valid = col_valid(c, tok, hl);
+            qcol[j] = c;
+            qmul[j] = valid ? qsign : 0.0f;
+            const int q_off = valid ? ((tok * n_head + kvh * r_heads + hl) * D + (lane % (D / 4)) * 4) * 4 : 0;
+            reg_load16<0>(qraw[j], qdesc, q_off, 0);
+        });
+    }
+    const i32x4 kdesc = make_desc(kc + (size_t)kvh * n_ctx * D, (unsigned)kv_end * D * 2);
+    const i32x4 vdesc = make_desc(vc + (size_t)kvh * n_ctx * D, (unsigned)kv_end * D * 2);
+    int g_off[kVar];
+    {
+        const int r_in = lane / G::kChunks, pc = lane % G::kChunks;
+#pragma unroll
+        for (int v = 0; v < kVar; ++v) g_off[v] = r_in * G::kRowB + ((pc ^ G::swz(v * G::kRowsPerCopy + r_in)) & (G::kChunks - 1)) * 16;
+    }
+    auto copy_tile = [&](const i32x4& desc, unsigned lds_dst, int tile) { // (range-checked: rows at or past kv_end are not fetched)
+        const int base = tile * G::kTileB;
+        lds_copy_4k(desc, lds_dst, base + g_off[0], base + g_off[1 % kVar], base + g_off[2 % kVar], base + g_off[3 % kVar], 0);
+        if (G::kCopies > 4)
+            lds_copy_4k(desc, lds_dst + 4096, base + 4096 + g_off[0], base + 4096 + g_off[1 % kVar], base + 4096 + g_off[2 % kVar],
+                        base + 4096 + g_off[3 % kVar], 0);
+    };
+    const unsigned k_addr = ws_addr, v_addr = ws_addr + G::kTileB;
+    // A tile that ends past the visible rows: those rows of V are not fetched, and a stale bit pattern must not meet a zero
+    // weight (0 * NaN is not 0): cleared first.  (The buffer is the wave's own.)
+    auto copy_v = [&](int tile) {
+        if (tile * kTile + kTile > kv_end) {
+#pragma unroll
+            for (int i = 0; i < kC; ++i) *reinterpret_cast<u32x4*>(ws + G::kTileB + i * 1024 + lane * 16) = u32x4{0u, 0u, 0u, 0u};
+            __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0)
+        }
+        copy_tile(vdesc, v_addr, tile);
+    };
+    if (n_mine > 0) {
+        copy_tile(kdesc, k_addr, wave);
+        copy_v(wave);
+    }
+    {   // (the arguments that did not arrive in registers, beside the loads)
+        const void* p0 = a.out;
+        asm volatile("" ::"s"(p0), "s"(a.c));
+    }
+    const unsigned char* kp[G::kSteps];
+#pragma unroll
+    for (int ks = 0; ks < G::kSteps; ++ks) kp[ks] = ws + c32 * G::kRowB + (((ks * 2 + hh) ^ G::swz(c32)) * 16);
+    const unsigned char* vp[2][G::kDBlk];
+    {
+        const int i16 = lane & 15, g2 = (lane >> 4) & 1;
+        const int r0 = 4 * hh + (i16 >> 2);
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int db = 0; db < G::kDBlk; ++db)
+                vp[u][db] = ws + G::kTileB + (r0 + 8 * u) * G::kRowB + (((db * 4 + g2 * 2 + ((i16 & 3) >> 1)) ^ G::swz(r0 + 8 * u)) * 16) + (i16 & 1) * 8;
+    }
+    auto wait_copies = [&](auto newer) { // (loads and copies retire in order)
+        constexpr int n = decltype(newer)::value;
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(0x0F70 | (n & 15) | ((n >> 4) << 14));
+        wave_lds_sync();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // ---- query block -> LDS (fp16), and back as operands ----
+    if (n_mine > 0) wait_copies(IntC<2 * kC>{});
+    else wait_copies(IntC<0>{});
+    static_for<0, kQLoads>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        asm volatile("" : "+v"(qraw[j])); // (not read ahead of the wait)
+        h4 hv;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) hv[e] = (_Float16)(__uint_as_float(qraw[j][e]) * qmul[j]);
+        *reinterpret_cast<h4*>(smem + SG::kQOff + qcol[j] * G::kQStride + (lane % (D / 4)) * 8) = hv;
+    });
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); // (LDS only: the copies travel on)
+
+    float* const ml = reinterpret_cast<float*>(smem + SG::kMlOff);
+    if (n_mine > 0) {
+        h8 q[G::kSteps];
+#pragma unroll
+        for (int ks = 0; ks < G::kSteps; ++ks) q[ks] = *reinterpret_cast<const h8*>(smem + SG::kQOff + c32 * G::kQStride + (ks * 16 + hh * 8) * 2);
+        int tok, hl;
+        const int limit = col_valid(c32, tok, hl) ? n_past + tok + 1 : 0x7fffffff;
+        f16v o[G::kDBlk];
+#pragma unroll
+        for (int db = 0; db < G::kDBlk; ++db)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[db][r] = 0.0f;
+        float m = -INFINITY, nb = 0.0f, l = 0.0f;
+        int tile = wave;
+        for (int left = n_mine - 1;; --left) {
+            const int next = tile + kWaves;
+            wait_copies(IntC<kC>{}); // K(tile); V(tile) may be in flight
+            h8 ka[G::kSteps];
+#pragma unroll
+            for (int ks = 0; ks < G::kSteps; ++ks) ka[ks] = *reinterpret_cast<const h8*>(kp[ks]);
+            f16v s, s2; // (two chains of products: one waits for its own last result)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = s2[r] = 0.0f;
+#pragma unroll
+            for (int ks = 0; ks < G::kSteps; ks += 2) {
+                s = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[ks], q[ks], s, 0, 0, 0);
+                s2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[ks + 1], q[ks + 1], s2, 0, 0, 0);
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] += s2[r];
+            if (left > 0) {
+                __builtin_amdgcn_sched_barrier(0);
+                __builtin_amdgcn_s_waitcnt(0xC07F); // K's reads have returned
+                copy_tile(kdesc, k_addr, next);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (tile * kTile + kTile > full_end) { // rows some column may not see
+                const int row0 = tile * kTile + 4 * hh;
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    if (row0 + 8 * (r / 4) + (r % 4) >= limit) s[r] = -INFINITY;
+            }
+            float mx[4] = {s[0], s[1], s[2], s[3]};
+#pragma unroll
+            for (int r = 4; r < 16; ++r) mx[r % 4] = fmaxf(mx[r % 4], s[r]);
+            const float m_new = fmaxf(m, pair_max(fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3]))));
+            const float nb_new = kPShift - (m_new == -INFINITY ? 0.0f : m_new) * a.c;
+            if (left + 1 < n_mine && __builtin_amdgcn_ballot_w64(m_new > m) != 0) { // (not the first tile, whose O is zero)
+                const float alpha = m == -INFINITY ? 0.0f : fast_exp2(nb_new - nb);
+                l *= alpha;
+#pragma unroll
+                for (int db = 0; db < G::kDBlk; ++db)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
+            }
+            m = m_new;
+            nb = nb_new;
+            h8 p[2];
+            float sump[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                p[r / 8][r % 8] = (_Float16)fast_exp2(__builtin_fmaf(s[r], a.c, nb));
+                sump[r % 4] += (float)p[r / 8][r % 8];
+            }
+            l += (sump[0] + sump[1]) + (sump[2] + sump[3]);
+            if (left > 0) wait_copies(IntC<kC>{}); // V(tile); the next K may be in flight
+            else wait_copies(IntC<0>{});
+#pragma unroll
+            for (int kh = 0; kh < 2; ++kh)
+#pragma unroll
+                for (int db = 0; db < G::kDBlk; ++db) {
+                    const h4 v0 = lds_read_tr(vp[0][db] + kh * 16 * G::kRowB), v1 = lds_read_tr(vp[1][db] + kh * 16 * G::kRowB);
+                    o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7), p[kh], o[db], 0, 0, 0);
+                }
+            if (left == 0) break;
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_waitcnt(0xC07F); // V's reads have returned
+            copy_v(next);
+            __builtin_amdgcn_sched_barrier(0);
+            tile = next;
+        }
+        // ---- hand-over (as above: m in log2 units, weight 0 for a column without a visible row) ----
+        const float l_tot = pair_sum(l);
+        if (hh == 0) {
+            ml[(wave * 32 + c32) * 2 + 0] = l_tot > 0.0f ? -nb : -INFINITY;
+            ml[(wave * 32 + c32) * 2 + 1] = l_tot;
+        }
+        __builtin_amdgcn_s_waitcnt(0xC07F); // (V's reads, before the merge buffer takes its place)
+#pragma unroll
+        for (int db = 0; db < G::kDBlk; ++db)
+#pragma unroll
+            for (int qd = 0; qd < 4; ++qd)
+                *reinterpret_cast<f4*>(ws + (db * 4 + qd) * 1024 + G::o_chunk(c32, hh, qd) * 16) =
+                    f4{o[db][4 * qd], o[db][4 * qd + 1], o[db][4 * qd + 2], o[db][4 * qd + 3]};
+    }
+    __syncthreads();
+    // ---- merge and store: sixteen threads a column, 16-byte pieces.  Sixteen neighbouring threads read eight pieces of each
+    // of two columns: sixteen different chunk columns of the banks (PGeom::o_chunk). ----
+    const int cm = (threadIdx.x >> 5) * 2 + ((threadIdx.x >> 3) & 1), part = (threadIdx.x & 7) + 8 * ((threadIdx.x >> 4) & 1);
+    int tok, hl;
+    if (!col_valid(cm, tok, hl)) return;
+    constexpr int kPieces = D / 64; // of a thread
+    f4 acc[kPieces];
+#pragma unroll
+    for (int j = 0; j < kPieces; ++j) acc[j] = f4{0.f, 0.f, 0.f, 0.f};
+    float m_all = -INFINITY, l_all = 0.0f;
+    auto merge = [&](auto countc) { // of the first waves, those without a tile at weight zero and unread
+        constexpr int kN = decltype(countc)::value;
+        float mw[kN], lw[kN];
+        f4 x[kN][kPieces];
+#pragma unroll
+        for (int w = 0; w < kN; ++w) {
+            const int wr = w < n_act ? w : 0;
+            mw[w] = ml[(wr * 32 + cm) * 2 + 0];
+            lw[w] = ml[(wr * 32 + cm) * 2 + 1];
+#pragma unroll
+            for (int j = 0; j < kPieces; ++j) x[w][j] = *reinterpret_cast<const f4*>(smem + wr * SG::kWaveB + G::o_byte(cm, j * 16 + part));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int w = 0; w < kN; ++w) {
+            if (w >= n_act) mw[w] = -INFINITY;
+            m_all = fmaxf(m_all, mw[w]);
+        }
+#pragma unroll
+        for (int w = 0; w < kN; ++w) {
+            const float wgt = m_all > -INFINITY ? fast_exp2(mw[w] - m_all) : 0.0f;
+            l_all += lw[w] * wgt;
+#pragma unroll
+            for (int j = 0; j < kPieces; ++j) acc[j] += x[w][j] * wgt;
+        }
+    };
+    if (n_act == 1) merge(IntC<1>{});
+    else if (n_act == 2) merge(IntC<2>{});
+    else if (n_act > 4) merge(IntC<8>{});
+    else if (n_act > 2) merge(IntC<4>{});
+    const float inv = l_all > 0.0f ? 1.0f / l_all : 0.0f;
+    const size_t orow = (size_t)tok * n_head + kvh * r_heads + hl;
+    f4 v[kPieces];
+#pragma unroll
+    for (int j = 0; j < kPieces; ++j) v[j] = acc[j] * inv;
+#pragma unroll
+    for (int j = 0; j < kPieces; ++j) store_stream(a.out + orow * D + (j * 16 + part) * 4, v[j]);
 }
 
 // out = sum over the KV splits of their normalised outputs, weighted by 2^(lse_s - max lse) and
@@ -1032,6 +1328,20 @@ hipError_t launch_kernel(const FaArgs& a, dim3 grid, hipStream_t stream) {
     return hipGetLastError();
 }
 
+template <int D>
+hipError_t launch_short(const FaArgs& a, dim3 grid, hipStream_t stream) {
+    const unsigned packed = (unsigned)a.heads_per_group | (unsigned)a.tq << 8 | (unsigned)a.tq_magic << 16;
+    hipLaunchKernelGGL((fa_prefill_short_kernel<D>), grid, dim3(kShortWaves * 64), SGeom<D>::kLdsB, stream, a.q, a.kc, a.vc, a.n_ctx, a.n_past,
+                       a.batch, a.n_head, a.r, a.n_ttiles, packed, a.qsign, a);
+    return hipGetLastError();
+}
+
+template <int D>
+hipError_t allow_lds_short() {
+    const auto kernel = fa_prefill_short_kernel<D>;
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, SGeom<D>::kLdsB);
+}
+
 template <int D, int NCB>
 hipError_t allow_lds() {
     const auto kernel = fa_prefill_kernel<D, NCB>;
@@ -1041,14 +1351,34 @@ hipError_t allow_lds() {
 
 constexpr int kMaxPrefillSplitShift = 4; // up to 16 workgroups share a token tile's KV rows (small chunks on long contexts)
 
-// Rows of context from which cutting a token tile's rows between two workgroups pays for the
-// second launch and the partial results' trip through memory (Qwen2.5-1.5B heads, 512-token
-// chunk: 35.1 -> 33.2 us at 6144 rows, 106 -> 71 us at 16896, 304 -> 121 us at 32768; slower
-// below about 4600 rows).
-#ifndef ORIN_FA_SPLIT_MIN_ROWS
-#define ORIN_FA_SPLIT_MIN_ROWS 5120
-#endif
-constexpr int kSplitMinRows = ORIN_FA_SPLIT_MIN_ROWS;
+// What a launch takes, in us, to choose by: fitted to 9000 measurements (five models' heads, 12 chunk sizes of 4 to 512 tokens,
+// 13 depths of 0 to 32000, every form below that fits the chip; within 10 % of most of them, and over those shapes the form it
+// picks is 0.3 % slower than the fastest measured, 23 % at most).  `rows`: KV rows the last token sees; a step is 128 of them, a tile for
+// each of four waves; wgs: workgroups of the launch, KV splits included.
+//   32 columns   5.3 us and 0.5 a step (bound by the 64 bytes a clock of the CU's vector memory path); more where so few
+//                workgroups walk that each waits for its own trips to memory, and on walks that leave the L2
+//   64 columns   6.9 and 0.7, 0.85 where the whole chip multiplies (clock, L2)
+//   short walk   4.0 and 0.8 (no tile asked for ahead of the last one's use)
+//   KV splits    2.2 for the second launch and 0.65 for every MB of partial results
+// head_dim 64 has half the bytes a row and two workgroups a CU.
+template <int D>
+float prefill_estimate(int cols, bool short_walk, int shift, long long wgs, int rows, double partial_bytes, int cus) {
+    float base = 6.9f, step = wgs * 3 < (long long)cus * 2 ? 0.7f : 0.85f;
+    if (cols == 32) {
+        base = 5.3f;
+        step = (wgs * 6 >= cus ? 0.5f : 0.56f) * (1.0f + fminf(fmaxf((float)(rows - 4000) / 8000.0f, 0.0f), 0.4f));
+    }
+    if (short_walk) base = 4.0f, step = 0.8f;
+    long long turns = (wgs + cus - 1) / cus;
+    if (D == 64) {
+        base -= short_walk ? 0.6f : cols == 32 ? 1.1f : 1.5f;
+        step *= 0.75f;
+        if (wgs > cus) step *= cols == 32 ? 2.0f : 1.4f;
+        turns = (turns + 1) / 2;
+    }
+    const float t = (float)turns * (base + step * (float)rows / (float)(128 << shift));
+    return shift > 0 ? t + 2.2f + 0.65e-6f * (float)partial_bytes : t;
+}
 
 template <int D>
 hipError_t launch(FaArgs a, int cu_count, hipStream_t stream, void* workspace, size_t workspace_bytes) {
@@ -1058,67 +1388,57 @@ hipError_t launch(FaArgs a, int cu_count, hipStream_t stream, void* workspace, s
     const int r = a.r;
     a.heads_per_group = r < 8 ? r : 8;
     a.n_hgroups = (r + a.heads_per_group - 1) / a.heads_per_group;
-    int ncb = 2;
-    a.tq = 64 / a.heads_per_group;
-    // A workgroup occupies a whole CU and the kernel lasts as long as its longest workgroup, so
-    // a grid that would leave half the CUs idle is cut finer: 32 columns per workgroup.
-    // On a long context the better cut is along the KV rows: the workgroup keeps its 64 columns
-    // (a step's K and V tiles then serve twice the columns: in the 32-column shape the step is
-    // bound by what the CU's vector memory path delivers, 64 bytes a clock, not by the matrix
-    // pipe) and 2, 4, 8 or 16 workgroups share a token tile's rows; a second, small kernel merges
-    // their results.  Needs room for the partial results in the workspace.
-    a.kv_split_shift = 0;
-    const int wgs64 = a.n_kv * a.n_hgroups * ((a.batch + a.tq - 1) / a.tq);
-    if (2 * wgs64 <= cu_count) {
-        int shift = 1;
-        while (shift < kMaxPrefillSplitShift && (wgs64 << (shift + 1)) <= cu_count) ++shift;
-        const size_t rows = (size_t)a.batch * a.n_head;
-        // A split that is done writes its log-sum-exps while others of its token tile may still have their queries to read, so
-        // they go into out only where out shares no byte with q (in place is allowed); else behind the partial outputs.
-        const uintptr_t q0 = reinterpret_cast<uintptr_t>(a.q), out0 = reinterpret_cast<uintptr_t>(a.out), bytes = rows * D * sizeof(float);
-        const bool in_place = q0 < out0 + bytes && out0 < q0 + bytes;
-        const size_t row_floats = in_place ? D + 1 : D; // of workspace, per row and split
-        // (as many as the workspace has room for: 128 tokens of Qwen3-0.6B heads at 8000, whose eight splits take more,
-        // ran unsplit in 55.6 us and take 26.3 with four)
-        while (shift > 0 && (rows << shift) * row_floats * sizeof(float) > workspace_bytes) --shift;
-        // Where that pays: the more workgroups per token tile, the shorter the walk and the sooner, and the more partial
-        // results, the later.  The lines lie at or just above where both ways took the same over 8 to 200 tokens at 700 to 4500 rows of five
-        // models' heads (head_dim 64, whose walk costs half a row, breaks even at half as many rows again): 8 tokens of
-        // Qwen2.5-1.5B at 2000 15.2 -> 10.6 us, 45 at 2400 16.8 -> 12.7, 100 of Qwen2.5-7B at 3000 18.6 -> 17.0.
-        const int kb = (int)((rows << shift) * D * sizeof(float) / 1024);
-        int min_rows = shift >= 4 ? 1100 + kb * 11 / 100 : shift == 3 ? 850 + kb * 21 / 100 : 300 + kb * 38 / 100;
-        if (D == 64) min_rows += min_rows / 2;
-        if (shift <= 1) min_rows = kSplitMinRows;
-        if (shift > 0 && a.n_past + a.batch >= min_rows && workspace) {
-            a.kv_split_shift = shift;
-            a.part_o = static_cast<float*>(workspace);
-            a.part_ml = in_place ? a.part_o + (rows << shift) * D : a.out;
-            a.lse_stride = in_place ? 1 << shift : D;
-        } else {
-            ncb = 1;
-            a.tq = 32 / a.heads_per_group;
-        }
+    // Four forms (prefill_estimate() above), the one that is expected to be done first:
+    //   64 columns a workgroup, which occupies a whole CU (head_dim 64: half of one), so that every tile it fetches serves
+    //   twice the columns;
+    //   32 columns, where the coarser grid would leave CUs idle;
+    //   either with 2, 4, 8 or 16 workgroups sharing a token tile's KV rows, whose partial results a second, small kernel merges:
+    //   few query columns on a long context.  Never more workgroups than the chip holds at once, and only as many as the
+    //   workspace has room for;
+    //   the kernel for short walks, where few tiles are visible.
+    // (45 tokens of Qwen2.5-1.5B at 1501 12.1 -> 9.3 us with eight splits of 32 columns, at 0 5.3 -> 4.3 by the short kernel; 260 tokens of
+    // Qwen2.5-7B at 1501, whose 260 workgroups of 32 columns are one turn and four workgroups, 22.9 -> 15.9; 260 of Llama-3.2-1B at
+    // 32000 177 -> 114, two half walks a CU.)
+    const size_t rows = (size_t)a.batch * a.n_head;
+    // A split that is done writes its log-sum-exps while others of its token tile may still have their queries to read, so
+    // they go into out only where out shares no byte with q (in place is allowed); else behind the partial outputs.
+    const uintptr_t q0 = reinterpret_cast<uintptr_t>(a.q), out0 = reinterpret_cast<uintptr_t>(a.out), bytes = rows * D * sizeof(float);
+    const bool in_place = q0 < out0 + bytes && out0 < q0 + bytes;
+    const size_t row_floats = in_place ? D + 1 : D; // of workspace, per row and split
+    const int resident = D == 64 ? 2 * cu_count : cu_count;
+    int cols = 64, shift = 0;
+    bool short_walk = false;
+    float least = INFINITY;
+    auto consider = [&](int c, int sh, bool sw) {
+        const long long wgs = ((long long)a.n_kv * a.n_hgroups * ((a.batch + c / a.heads_per_group - 1) / (c / a.heads_per_group))) << sh;
+        if (sh > 0 && (wgs > resident || !workspace || (rows << sh) * row_floats * sizeof(float) > workspace_bytes)) return;
+        const float t = prefill_estimate<D>(c, sw, sh, wgs, a.n_past + a.batch, (double)(rows << sh) * D * sizeof(float), cu_count);
+        if (t < least) least = t, cols = c, shift = sh, short_walk = sw;
+    };
+    for (int sh = 0; sh <= kMaxPrefillSplitShift; ++sh) {
+        consider(64, sh, false);
+        consider(32, sh, false);
     }
-    // head_dim 64: two 32-column workgroups fit a CU's LDS, and on a short walk, which is mostly prologue and merge, one covers
-    // the other's waits (Llama-3.2-1B heads at depth 0: 301 tokens 7.3 -> 6.6 us, 512 8.3 -> 7.6; at 1500 rows even, beyond
-    // slower, where the copies of the tiles bound both).
-    if (D == 64 && ncb == 2 && a.kv_split_shift == 0 && a.n_past + a.batch <= 1024 && wgs64 <= cu_count) {
-        ncb = 1;
-        a.tq = 32 / a.heads_per_group;
+    consider(32, 0, true);
+    a.tq = cols / a.heads_per_group;
+    a.kv_split_shift = shift;
+    if (shift > 0) {
+        a.part_o = static_cast<float*>(workspace);
+        a.part_ml = in_place ? a.part_o + (rows << shift) * D : a.out;
+        a.lse_stride = in_place ? 1 << shift : D;
     }
     a.n_ttiles = (a.batch + a.tq - 1) / a.tq;
     a.tq_magic = 65536 / a.tq + 1;
     if ((a.n_hgroups << a.kv_split_shift) > 65535 || a.n_ttiles > 65535) return hipErrorInvalidValue;
     const dim3 grid(a.n_kv, a.n_hgroups << a.kv_split_shift, a.n_ttiles);
-    const hipError_t e = ncb == 2 ? launch_kernel<D, 2>(a, grid, stream) : launch_kernel<D, 1>(a, grid, stream);
+    const hipError_t e = short_walk ? launch_short<D>(a, grid, stream) : cols == 64 ? launch_kernel<D, 2>(a, grid, stream) : launch_kernel<D, 1>(a, grid, stream);
     if (e != hipSuccess || a.kv_split_shift == 0) return e;
-    const int rows = a.batch * a.n_head;
-    const unsigned blocks = (unsigned)(((size_t)rows * (D / 4) + 255) / 256);
+    const unsigned blocks = (unsigned)((rows * (D / 4) + 255) / 256);
     switch (a.kv_split_shift) {
-    case 1: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 2>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.part_ml, a.lse_stride, a.out, rows); break;
-    case 2: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 4>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.part_ml, a.lse_stride, a.out, rows); break;
-    case 3: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 8>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.part_ml, a.lse_stride, a.out, rows); break;
-    default: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 16>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.part_ml, a.lse_stride, a.out, rows); break;
+    case 1: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 2>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.part_ml, a.lse_stride, a.out, (int)rows); break;
+    case 2: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 4>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.part_ml, a.lse_stride, a.out, (int)rows); break;
+    case 3: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 8>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.part_ml, a.lse_stride, a.out, (int)rows); break;
+    default: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 16>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.part_ml, a.lse_stride, a.out, (int)rows); break;
     }
     static_assert(kMaxPrefillSplitShift == 4, "the cases above");
     return hipGetLastError();
@@ -1139,7 +1459,9 @@ hipError_t prefill_allow_lds() {
     if ((e = allow_lds<128, 1>()) != hipSuccess) return e;
     if ((e = allow_lds<128, 2>()) != hipSuccess) return e;
     if ((e = allow_lds<64, 1>()) != hipSuccess) return e;
-    return allow_lds<64, 2>();
+    if ((e = allow_lds<64, 2>()) != hipSuccess) return e;
+    if ((e = allow_lds_short<128>()) != hipSuccess) return e;
+    return allow_lds_short<64>();
 }
 
 hipError_t prefill_stamps(long long* host, size_t n) {

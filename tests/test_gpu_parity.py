@@ -219,6 +219,22 @@ def test_prefill_kv_splits(fa, H, G, d, n_past, batch, scale):
     check(got[rows[:, 0], rows[:, 1]], want, f"prefill kv splits H{H} G{G} d{d} P{n_past} B{batch}")
 
 
+@pytest.mark.parametrize("n_past,batch", [
+    (0, 1), (0, 31), (0, 33), (24, 40), (31, 1), (90, 45), (255, 1),  # a tile a wave, up to the eight of a workgroup
+    (249, 8), (240, 45), (270, 11),                                   # a second turn of one wave and of several
+    (1100, 20), (1501, 45), (2500, 4),                                # few columns, many rows: 32 columns, the rows shared
+])
+@pytest.mark.parametrize("H,G,d,scale", [(12, 2, 128, 0.0883883), (32, 8, 64, -0.3), (5, 1, 64, 0.125), (20, 1, 128, 1.0)])
+def test_prefill_short_chunks(fa, H, G, d, scale, n_past, batch):
+    """Chunks of few tokens at the edges of the forms they take: the kernel for short walks, and 32 columns with shared rows."""
+    n_ctx = n_past + batch + 3
+    q, kc, vc = make_case(300 + H + n_past, H, G, d, n_ctx, n_past + batch, batch, outliers=2, poison_tail=True)
+    rows = np.array([(t, h) for t in range(batch) for h in range(H)], np.int32)
+    want = ref.flash_attention_rows(q, kc, vc, rows, H, G, d, n_ctx, n_past, np.float32(scale))
+    got = gpu_prefill(fa, q, kc, vc, H, G, d, n_ctx, n_past, batch, scale)
+    check(got.reshape(-1, d), want.reshape(-1, d), f"short chunk H{H} G{G} d{d} P{n_past} B{batch}")
+
+
 @pytest.mark.parametrize("scale", [1.0, 0.35, -0.0883883])
 @pytest.mark.parametrize("H,G,batch", [(4, 2, 96), (32, 8, 600)])
 def test_prefill_moving_reference(fa, scale, H, G, batch):
