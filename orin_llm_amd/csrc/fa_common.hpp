@@ -84,10 +84,29 @@ struct FaArgs {
 };
 
 // hipGetLastError() returns, and clears, the last error of any HIP call this host thread has made, the host
-// application's own included.  Every launcher below starts by dropping what is pending, so that the code it
+// application's own included.  A launcher that asks for it starts by dropping what is pending, so that the code it
 // returns after its launch is the launch's own and an unrelated stale error is not blamed on (and, through the
 // llm::cuda shim, does not abort) an operator that worked.
 inline void drop_stale_error() { (void)hipGetLastError(); }
+
+// What the launches of a prefill layer cost the host, since they are eager (depth and chunk size are arguments by value): us a launch, beside
+// torch's HIP runtime, 3.86 with eleven arguments, three of them pointers, and 248 bytes of struct behind them; 3.2 with seven and 40
+// bytes (an argument is 0.06, a byte of them, which the host writes to device memory, 0.004); 3.0 with the pointers as integers (the
+// runtime looks up the allocation behind each pointer); 2.85 by hipLaunchKernel, without the launch configuration that the triple brackets push and
+// pop.  45 tokens of Qwen2.5-1.5B, rotation with store and attention: 7.7 -> 7.05 us of host time a layer.  And its return value is the launch's own, so nobody has to ask for, or clear, the thread's last error.
+template <class... P>
+hipError_t launch_lean(void (*kernel)(P...), dim3 grid, unsigned threads, size_t lds, hipStream_t stream, P... args) {
+    void* pointers[] = {&args...};
+    const hipError_t e = hipLaunchKernel(reinterpret_cast<const void*>(kernel), grid, dim3(threads), pointers, lds, stream);
+    if (e != hipSuccess) (void)hipGetLastError(); // (reported by the return value: not left for somebody else to find)
+    return e;
+}
+inline uint64_t arg_pair(unsigned lo, unsigned hi) { return (uint64_t)lo | (uint64_t)hi << 32; }
+inline uint64_t arg_ptr(const void* p) { return reinterpret_cast<uintptr_t>(p); }
+template <class T>
+__device__ __forceinline__ T* ptr_arg(uint64_t bits) { // (said to be device memory: the accesses are global ones, not generic)
+    return (T*)(__attribute__((address_space(1))) T*)bits;
+}
 
 // Launchers (defined next to their kernels).  All return hipError_t of the launch.
 hipError_t prefill_launch(const FaArgs& args, int head_dim, int cu_count, hipStream_t stream, void* workspace,

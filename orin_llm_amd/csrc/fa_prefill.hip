@@ -43,6 +43,8 @@
 // fa_prefill_combine_kernel merges them into `out`.
 #include "fa_common.hpp"
 
+#include <string.h>
+
 // Stage marks: wall-clock stamps in the timeline build, nothing otherwise (fa_common.hpp).
 #ifdef ORIN_FA_STAMPS
 namespace orin_fa {
@@ -275,15 +277,29 @@ constexpr ItemTable make_items() {
 constexpr ItemTable kItemsOfBlock = make_items();
 constexpr int kItemsPerBlock = 48;
 
+// The arguments of a launch.  What the prologue's loads need comes first, as scalars: the leading fourteen words are
+// handed to a wave in registers when it starts (kernel-argument preload), so the query block and the first tiles are requested at
+// once, not behind a trip to memory for their addresses.  Few and small, pointers as integers: launch_lean().
+struct PrefillTail { // what the epilogue needs
+    float *out, *part_o, *part_ml;
+    int lse_stride;
+    float c;
+};
+#define PREFILL_ARGS                                                                                                              \
+    const uint64_t q_bits, const uint64_t k_bits, const uint64_t v_bits, const uint64_t ctx_past, const uint64_t batch_heads,    \
+        const uint64_t r_tiles, const uint64_t packed_sign, const PrefillTail a
+// packed: heads_per_group | kv_split_shift << 4 | tq << 8 | tq_magic << 16
+#define PREFILL_UNPACK                                                                                                            \
+    const float* const q_in = ptr_arg<const float>(q_bits);                                                                       \
+    const uint16_t *const kc = ptr_arg<const uint16_t>(k_bits), *const vc = ptr_arg<const uint16_t>(v_bits);                       \
+    const int n_ctx = (int)(unsigned)ctx_past, n_past = (int)(ctx_past >> 32), batch = (int)(unsigned)batch_heads,                 \
+              n_head = (int)(batch_heads >> 32), r_heads = (int)(unsigned)r_tiles, n_ttiles = (int)(r_tiles >> 32);                \
+    const unsigned packed = (unsigned)packed_sign;                                                                                \
+    const float qsign = __uint_as_float((unsigned)(packed_sign >> 32))
+
 template <int D, int NCB>
-__global__ __launch_bounds__(kPrefillWaves * 64) void fa_prefill_kernel(
-    // What the prologue's loads need comes first, as scalars: the leading kernel arguments are
-    // handed to a wave in registers when it starts (kernel-argument preload), so the query block
-    // and the first tiles are requested at once, not behind a trip to memory for their addresses.
-    // packed: heads_per_group | kv_split_shift << 4 | tq << 8 | tq_magic << 16.
-    const float* q_in, const uint16_t* kc, const uint16_t* vc, const int n_ctx,
-    const int n_past, const int batch, const int n_head, const int r_heads, const int n_ttiles, const unsigned packed,
-    const float qsign, const FaArgs a) {
+__global__ __launch_bounds__(kPrefillWaves * 64) void fa_prefill_kernel(PREFILL_ARGS) {
+    PREFILL_UNPACK;
     using G = PGeom<D, NCB>;
     constexpr int kWaves = kPrefillWaves;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -1021,10 +1037,8 @@ struct SGeom {
 };
 
 template <int D>
-__global__ __launch_bounds__(kShortWaves * 64, D == 64 ? 4 : 2) void fa_prefill_short_kernel(
-    const float* q_in, const uint16_t* kc, const uint16_t* vc, const int n_ctx, // (as above: what the first requests need)
-    const int n_past, const int batch, const int n_head, const int r_heads, const int n_ttiles, const unsigned packed,
-    const float qsign, const FaArgs a) {
+__global__ __launch_bounds__(kShortWaves * 64, D == 64 ? 4 : 2) void fa_prefill_short_kernel(PREFILL_ARGS) {
+    PREFILL_UNPACK;
     using G = PGeom<D, 1>;
     using SG = SGeom<D>;
     constexpr int kWaves = kShortWaves, kC = G::kCopies, kVar = G::kCopyVariants;
@@ -1293,7 +1307,10 @@ __global__ __launch_bounds__(kShortWaves * 64, D == 64 ? 4 : 2) void fa_prefill_
 // one wave read and then write, so that the workspace holds partial outputs alone; they are in the workspace where out is
 // the queries' memory (launch() below), and out is then written here and nowhere before.
 template <int D, int S>
-__global__ __launch_bounds__(256) void fa_prefill_combine_kernel(const float* part_o, const float* lse_of, int lse_stride, float* out, int rows) {
+__global__ __launch_bounds__(256) void fa_prefill_combine_kernel(const uint64_t part_bits, const uint64_t lse_bits, const uint64_t out_bits, const uint64_t stride_rows) {
+    const float *const part_o = ptr_arg<const float>(part_bits), *const lse_of = ptr_arg<const float>(lse_bits);
+    float* const out = ptr_arg<float>(out_bits);
+    const int lse_stride = (int)(unsigned)stride_rows, rows = (int)(stride_rows >> 32);
     const int idx = blockIdx.x * 256 + threadIdx.x;
     const int row = idx / (D / 4), piece = idx % (D / 4);
     if (row >= rows) return;
@@ -1319,21 +1336,20 @@ __global__ __launch_bounds__(256) void fa_prefill_combine_kernel(const float* pa
     *reinterpret_cast<f4*>(out + (size_t)row * D + piece * 4) = acc * inv;
 }
 
-template <int D, int NCB>
-hipError_t launch_kernel(const FaArgs& a, dim3 grid, hipStream_t stream) {
-    constexpr int lds = PGeom<D, NCB>::kLdsB;
-    const unsigned packed = (unsigned)a.heads_per_group | (unsigned)a.kv_split_shift << 4 | (unsigned)a.tq << 8 | (unsigned)a.tq_magic << 16;
-    hipLaunchKernelGGL((fa_prefill_kernel<D, NCB>), grid, dim3(kPrefillWaves * 64), lds, stream, a.q, a.kc, a.vc, a.n_ctx, a.n_past,
-                       a.batch, a.n_head, a.r, a.n_ttiles, packed, a.qsign, a);
-    return hipGetLastError();
-}
-
+// cols: 64 or 32 query columns a workgroup, 0: the kernel for short walks
 template <int D>
-hipError_t launch_short(const FaArgs& a, dim3 grid, hipStream_t stream) {
-    const unsigned packed = (unsigned)a.heads_per_group | (unsigned)a.tq << 8 | (unsigned)a.tq_magic << 16;
-    hipLaunchKernelGGL((fa_prefill_short_kernel<D>), grid, dim3(kShortWaves * 64), SGeom<D>::kLdsB, stream, a.q, a.kc, a.vc, a.n_ctx, a.n_past,
-                       a.batch, a.n_head, a.r, a.n_ttiles, packed, a.qsign, a);
-    return hipGetLastError();
+hipError_t launch_kernel(const FaArgs& a, int cols, dim3 grid, hipStream_t stream) {
+    const unsigned packed = (unsigned)a.heads_per_group | (unsigned)a.kv_split_shift << 4 | (unsigned)a.tq << 8 | (unsigned)a.tq_magic << 16;
+    unsigned sign;
+    memcpy(&sign, &a.qsign, sizeof(sign));
+    auto go = [&](auto kernel, int waves, size_t lds) {
+        return launch_lean(kernel, grid, waves * 64, lds, stream, arg_ptr(a.q), arg_ptr(a.kc), arg_ptr(a.vc), arg_pair(a.n_ctx, a.n_past),
+                           arg_pair(a.batch, a.n_head), arg_pair(a.r, a.n_ttiles), arg_pair(packed, sign),
+                           PrefillTail{a.out, a.part_o, a.part_ml, a.lse_stride, a.c});
+    };
+    if (cols == 64) return go(fa_prefill_kernel<D, 2>, kPrefillWaves, PGeom<D, 2>::kLdsB);
+    if (cols == 32) return go(fa_prefill_kernel<D, 1>, kPrefillWaves, PGeom<D, 1>::kLdsB);
+    return go(fa_prefill_short_kernel<D>, kShortWaves, SGeom<D>::kLdsB);
 }
 
 template <int D>
@@ -1431,24 +1447,25 @@ hipError_t launch(FaArgs a, int cu_count, hipStream_t stream, void* workspace, s
     a.tq_magic = 65536 / a.tq + 1;
     if ((a.n_hgroups << a.kv_split_shift) > 65535 || a.n_ttiles > 65535) return hipErrorInvalidValue;
     const dim3 grid(a.n_kv, a.n_hgroups << a.kv_split_shift, a.n_ttiles);
-    const hipError_t e = short_walk ? launch_short<D>(a, grid, stream) : cols == 64 ? launch_kernel<D, 2>(a, grid, stream) : launch_kernel<D, 1>(a, grid, stream);
+    const hipError_t e = launch_kernel<D>(a, short_walk ? 0 : cols, grid, stream);
     if (e != hipSuccess || a.kv_split_shift == 0) return e;
     const unsigned blocks = (unsigned)((rows * (D / 4) + 255) / 256);
+    auto combine = [&](auto kernel) {
+        return launch_lean(kernel, dim3(blocks), 256, 0, stream, arg_ptr(a.part_o), arg_ptr(a.part_ml), arg_ptr(a.out), arg_pair(a.lse_stride, (unsigned)rows));
+    };
     switch (a.kv_split_shift) {
-    case 1: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 2>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.part_ml, a.lse_stride, a.out, (int)rows); break;
-    case 2: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 4>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.part_ml, a.lse_stride, a.out, (int)rows); break;
-    case 3: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 8>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.part_ml, a.lse_stride, a.out, (int)rows); break;
-    default: hipLaunchKernelGGL((fa_prefill_combine_kernel<D, 16>), dim3(blocks), dim3(256), 0, stream, a.part_o, a.part_ml, a.lse_stride, a.out, (int)rows); break;
+    case 1: return combine(fa_prefill_combine_kernel<D, 2>);
+    case 2: return combine(fa_prefill_combine_kernel<D, 4>);
+    case 3: return combine(fa_prefill_combine_kernel<D, 8>);
+    default: return combine(fa_prefill_combine_kernel<D, 16>);
     }
     static_assert(kMaxPrefillSplitShift == 4, "the cases above");
-    return hipGetLastError();
 }
 
 } // namespace
 
 hipError_t prefill_launch(const FaArgs& a, int head_dim, int cu_count, hipStream_t stream, void* workspace,
                           size_t workspace_bytes) {
-    drop_stale_error();
     return head_dim == 128 ? launch<128>(a, cu_count, stream, workspace, workspace_bytes)
                            : launch<64>(a, cu_count, stream, workspace, workspace_bytes);
 }

@@ -27,23 +27,30 @@ namespace {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 
-// VEC = 8: head_dim is a multiple of 8 (16-byte cache pieces); VEC = 1: any head_dim.
+// VEC = 8: head_dim is a multiple of 8 (16-byte cache pieces); VEC = 1: any head_dim.  A launch has fewer than 2^31 threads, so
+// that its divisions are 32-bit ones (64-bit: some 500 instructions ahead of the first load); its arguments are few (launch_lean())
+// and in registers when a wave starts (kernel-argument preload).  Bound by the launch: 301 tokens of Llama-3.2-1B 2.25 -> 2.2 us.
+//   shape   heads | head_dim << 32        rows   n_ctx | pos_base << 32        pos_or_batch   the position's address, or the tokens
 template <int VEC, bool IND>
-__global__ __launch_bounds__(256) void kv_store_kernel(uint16_t* kc, uint16_t* vc, const float* k, const float* v,
-                                                       int heads, int head_dim, int n_ctx, int pos_base, int batch,
-                                                       const int* d_pos) {
-    const int per_row = head_dim / VEC;                       // threads per (token, head) row
-    const long long rows = (long long)batch * heads;
-    const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
-    const bool is_v = idx >= rows * per_row;                  // second half of the grid stores V
-    const long long j = is_v ? idx - rows * per_row : idx;
-    if (j >= rows * per_row) return;
-    const long long row = j / per_row;                        // = token * heads + head
-    const int piece = (int)(j % per_row);
-    const int head = (int)(row % heads);
-    const int pos = IND ? *d_pos : pos_base + (int)(row / heads);
+__global__ __launch_bounds__(256) void kv_store_kernel(const uint64_t kc_bits, const uint64_t vc_bits, const uint64_t k_bits, const uint64_t v_bits,
+                                                       const uint64_t shape, const uint64_t rows, const uint64_t pos_or_batch) {
+    uint16_t *const kc = ptr_arg<uint16_t>(kc_bits), *const vc = ptr_arg<uint16_t>(vc_bits);
+    const float *const k = ptr_arg<const float>(k_bits), *const v = ptr_arg<const float>(v_bits);
+    const int* const d_pos = ptr_arg<const int>(IND ? pos_or_batch : 0);
+    const unsigned batch = IND ? 1u : (unsigned)pos_or_batch;
+    const unsigned heads = (unsigned)shape, head_dim = (unsigned)(shape >> 32);
+    const int n_ctx = (int)(unsigned)rows, pos_base = (int)(rows >> 32);
+    const unsigned per_row = head_dim / VEC;                  // threads per (token, head) row
+    const unsigned half = batch * heads * per_row;
+    const unsigned idx = blockIdx.x * 256 + threadIdx.x;
+    const bool is_v = idx >= half;                            // second half of the grid stores V
+    const unsigned j = is_v ? idx - half : idx;
+    if (j >= half) return;
+    const unsigned row = j / per_row, piece = j - row * per_row; // row = token * heads + head
+    const unsigned token = row / heads, head = row - token * heads;
+    const int pos = IND ? *d_pos : pos_base + (int)token;
     if (pos < 0 || pos >= n_ctx) return;                      // (the reference would write out of bounds)
-    const float* src = (is_v ? v : k) + row * head_dim + piece * VEC;
+    const float* src = (is_v ? v : k) + (size_t)row * head_dim + piece * VEC;
     uint16_t* dst = (is_v ? vc : kc) + ((size_t)head * n_ctx + pos) * head_dim + piece * VEC;
     if constexpr (VEC == 8) {
         const float4 x0 = *reinterpret_cast<const float4*>(src);
@@ -96,21 +103,23 @@ __global__ __launch_bounds__(256) void kv_shift_kernel(uint16_t* kc, uint16_t* v
 
 hipError_t kv_store_launch(uint16_t* kc, uint16_t* vc, const float* k, const float* v, int heads, int head_dim,
                            int n_ctx, int pos_base, int batch, const int* d_pos, hipStream_t stream) {
-    drop_stale_error();
     const bool vec = head_dim % 8 == 0 &&
                      ((reinterpret_cast<uintptr_t>(kc) | reinterpret_cast<uintptr_t>(vc) |
                        reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v)) & 15u) == 0;
-    const long long threads = 2ll * batch * heads * (head_dim / (vec ? 8 : 1));
-    const unsigned grid = (unsigned)((threads + 255) / 256);
-    if (grid == 0) return hipSuccess;
-    if (vec) {
-        if (d_pos) hipLaunchKernelGGL((kv_store_kernel<8, true>), dim3(grid), dim3(256), 0, stream, kc, vc, k, v, heads, head_dim, n_ctx, 0, 1, d_pos);
-        else hipLaunchKernelGGL((kv_store_kernel<8, false>), dim3(grid), dim3(256), 0, stream, kc, vc, k, v, heads, head_dim, n_ctx, pos_base, batch, nullptr);
-    } else {
-        if (d_pos) hipLaunchKernelGGL((kv_store_kernel<1, true>), dim3(grid), dim3(256), 0, stream, kc, vc, k, v, heads, head_dim, n_ctx, 0, 1, d_pos);
-        else hipLaunchKernelGGL((kv_store_kernel<1, false>), dim3(grid), dim3(256), 0, stream, kc, vc, k, v, heads, head_dim, n_ctx, pos_base, batch, nullptr);
+    const long long per_token = 2ll * heads * (head_dim / (vec ? 8 : 1)); // threads
+    if (per_token > 0x7fffff00ll) return hipErrorInvalidValue;
+    const int most = (int)(0x7fffff00ll / per_token); // tokens of a launch
+    for (int t = 0; t < batch; t += most) { // (batch = 1 with a position on the device)
+        const int n = batch - t < most ? batch - t : most;
+        auto go = [&](auto kernel) {
+            return launch_lean(kernel, dim3((unsigned)((per_token * n + 255) / 256)), 256, 0, stream, arg_ptr(kc), arg_ptr(vc), arg_ptr(k + (size_t)t * heads * head_dim),
+                               arg_ptr(v + (size_t)t * heads * head_dim), arg_pair(heads, head_dim), arg_pair(n_ctx, pos_base + t), d_pos ? arg_ptr(d_pos) : (uint64_t)n);
+        };
+        const hipError_t e = vec ? (d_pos ? go(kv_store_kernel<8, true>) : go(kv_store_kernel<8, false>))
+                                 : (d_pos ? go(kv_store_kernel<1, true>) : go(kv_store_kernel<1, false>));
+        if (e != hipSuccess) return e;
     }
-    return hipGetLastError();
+    return hipSuccess;
 }
 
 hipError_t kv_shift_launch(uint16_t* kc, uint16_t* vc, int n_layer, int n_kv, int head_dim, int n_ctx, int n_keep,

@@ -99,48 +99,70 @@ __global__ __launch_bounds__(256) void rope_kernel(float* x, int tokens, int hea
 // 4.1 -> 3.9; 512 tokens of Llama-3-8B (25 MB) stay at the memory's 7.5 us.
 constexpr int kRopeThreads = 256;
 
-struct RopeArgs {
-    float *q, *k;
-    const float* v;
+// What the first loads need comes first, as scalars that are in a wave's registers when it starts (kernel-argument preload); the
+// rest in as few bytes as will do (launch_lean()).
+//   counts   tokens | heads of Q, K and V together << 32
+//   heads    heads of Q << 0 | of K << 32
+//   shape    pairs of a head, 10 bits | pieces of a head, 7 | tokens of a block, 10 | log2 of its heads, 5 | head_dim << 32
+//   magic    x / pieces = x * magic >> 16, x < 1024 | the same for pairs, x < 256, << 32
+struct RopeRest {
     uint16_t *kc, *vc;
     const int* d_pos;
     const float* freq_factors;
-    RopeFreq freq;
-    int tokens, n_past, n_ctx, head_dim, n_q, n_k, n_heads; // n_heads = n_q + n_k + V heads
-    int half, quads, block_tokens, block_heads_log2;
-    unsigned half_magic, quads_magic; // x / half = x * magic >> 16, x < 256 (quads: x < 1024)
+    double step; // theta^(-2 / n_rot), 0: no power of two (RopeFreq)
+    float theta;
+    int n_past, n_ctx;
 };
 
+// rope_freq() of the plan whose first double is `step`: the same squares, taken here.
+__device__ __forceinline__ float rope_freq_of_step(int i, int n_rot, const RopeRest& a) {
+    RopeFreq f;
+    f.theta = a.theta;
+    f.n_rot = n_rot;
+    f.by_steps = a.step != 0.0;
+    double s = a.step;
+#pragma unroll
+    for (int k = 0; k < 8; ++k, s *= s) f.step[k] = s;
+    return rope_freq(i, f, a.freq_factors);
+}
+
 template <bool NEOX, int U>
-__global__ __launch_bounds__(kRopeThreads) void rope_pieces_kernel(const RopeArgs a) {
+__global__ __launch_bounds__(kRopeThreads) void rope_pieces_kernel(const uint64_t q_bits, const uint64_t k_bits, const uint64_t v_bits, const uint64_t counts,
+                                                                   const uint64_t heads, const uint64_t shape, const uint64_t magic, const RopeRest a) {
 #pragma clang fp contract(off)
+    float *const q = ptr_arg<float>(q_bits), *const k = ptr_arg<float>(k_bits);
+    const float* const v = ptr_arg<const float>(v_bits);
     __shared__ __attribute__((aligned(16))) float2 sh_cs[kRopeThreads]; // (read two pairs at a time)
-    const int tid = threadIdx.x, token0 = (int)blockIdx.x * a.block_tokens, head0 = (int)blockIdx.y << a.block_heads_log2;
-    const int o1 = NEOX ? a.half : 4;
+    const int tokens = (int)(unsigned)counts, n_heads = (int)(counts >> 32), n_q = (int)(unsigned)heads, n_k = (int)(heads >> 32);
+    const int half = (int)(shape & 1023u), quads = (int)((shape >> 10) & 127u), block_tokens = (int)((shape >> 17) & 1023u);
+    const int block_heads_log2 = (int)((shape >> 27) & 31u), head_dim = (int)(shape >> 32);
+    const unsigned quads_magic = (unsigned)magic, half_magic = (unsigned)(magic >> 32);
+    const int tid = threadIdx.x, token0 = (int)blockIdx.x * block_tokens, head0 = (int)blockIdx.y << block_heads_log2;
+    const int o1 = NEOX ? half : 4;
     float4 lo[U], hi[U];
     int token[U], head[U], quad[U];
     bool live[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-        const int s = tid + kRopeThreads * u, rest = (int)((unsigned)s * a.quads_magic >> 16);
-        quad[u] = s - rest * a.quads;
-        head[u] = head0 + (rest & ((1 << a.block_heads_log2) - 1));
-        const int t = rest >> a.block_heads_log2;
+        const int s = tid + kRopeThreads * u, rest = (int)((unsigned)s * quads_magic >> 16);
+        quad[u] = s - rest * quads;
+        head[u] = head0 + (rest & ((1 << block_heads_log2) - 1));
+        const int t = rest >> block_heads_log2;
         token[u] = token0 + t;
-        live[u] = t < a.block_tokens && token[u] < a.tokens && head[u] < a.n_heads;
+        live[u] = t < block_tokens && token[u] < tokens && head[u] < n_heads;
         if (live[u]) {
-            const bool is_q = head[u] < a.n_q, is_k = head[u] < a.n_q + a.n_k;
-            const float* const row = is_q ? a.q + ((size_t)token[u] * a.n_q + head[u]) * a.head_dim
-                                          : (is_k ? a.k : a.v) + ((size_t)token[u] * a.n_k + (head[u] - a.n_q - (is_k ? 0 : a.n_k))) * a.head_dim;
+            const bool is_q = head[u] < n_q, is_k = head[u] < n_q + n_k;
+            const float* const row = is_q ? q + ((size_t)token[u] * n_q + head[u]) * head_dim
+                                          : (is_k ? k : v) + ((size_t)token[u] * n_k + (head[u] - n_q - (is_k ? 0 : n_k))) * head_dim;
             const float* const p = row + quad[u] * (NEOX ? 4 : 8);
             lo[u] = *reinterpret_cast<const float4*>(p);
             hi[u] = *reinterpret_cast<const float4*>(p + o1);
         }
     }
     {
-        const int t = (int)((unsigned)tid * a.half_magic >> 16), i = tid - t * a.half;
-        if (t < a.block_tokens) {
-            const float ang = (float)(a.d_pos ? *a.d_pos : a.n_past + token0 + t) * rope_freq(i, a.freq, a.freq_factors);
+        const int t = (int)((unsigned)tid * half_magic >> 16), i = tid - t * half;
+        if (t < block_tokens) {
+            const float ang = (float)(a.d_pos ? *a.d_pos : a.n_past + token0 + t) * rope_freq_of_step(i, 2 * half, a);
             sh_cs[tid] = float2{cosf(ang), sinf(ang)};
         }
     }
@@ -148,9 +170,9 @@ __global__ __launch_bounds__(kRopeThreads) void rope_pieces_kernel(const RopeArg
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         if (!live[u]) continue;
-        const bool is_q = head[u] < a.n_q, is_k = !is_q && head[u] < a.n_q + a.n_k;
+        const bool is_q = head[u] < n_q, is_k = !is_q && head[u] < n_q + n_k;
         if (is_q || is_k) {
-            const float4* const cs = reinterpret_cast<const float4*>(sh_cs + (token[u] - token0) * a.half + 4 * quad[u]);
+            const float4* const cs = reinterpret_cast<const float4*>(sh_cs + (token[u] - token0) * half + 4 * quad[u]);
             const float4 c01 = cs[0], c23 = cs[1];
             float4 &x = lo[u], &y = hi[u];
             if (NEOX) {
@@ -164,14 +186,14 @@ __global__ __launch_bounds__(kRopeThreads) void rope_pieces_kernel(const RopeArg
                 rope_rotate(y.x, y.y, c23.x, c23.y);
                 rope_rotate(y.z, y.w, c23.z, c23.w);
             }
-            float* const row = is_q ? a.q + ((size_t)token[u] * a.n_q + head[u]) * a.head_dim : a.k + ((size_t)token[u] * a.n_k + (head[u] - a.n_q)) * a.head_dim;
+            float* const row = is_q ? q + ((size_t)token[u] * n_q + head[u]) * head_dim : k + ((size_t)token[u] * n_k + (head[u] - n_q)) * head_dim;
             float* const p = row + quad[u] * (NEOX ? 4 : 8);
             store_stream(p, x);
             store_stream(p + o1, y);
         }
         if (!is_q && a.kc) {
-            const int h = head[u] - a.n_q - (is_k ? 0 : a.n_k);
-            uint16_t* const p = (is_k ? a.kc : a.vc) + ((size_t)h * a.n_ctx + a.n_past + token[u]) * a.head_dim + quad[u] * (NEOX ? 4 : 8);
+            const int h = head[u] - n_q - (is_k ? 0 : n_k);
+            uint16_t* const p = (is_k ? a.kc : a.vc) + ((size_t)h * a.n_ctx + a.n_past + token[u]) * head_dim + quad[u] * (NEOX ? 4 : 8);
             half4_t l, m;
             l[0] = (_Float16)lo[u].x; l[1] = (_Float16)lo[u].y; l[2] = (_Float16)lo[u].z; l[3] = (_Float16)lo[u].w;
             m[0] = (_Float16)hi[u].x; m[1] = (_Float16)hi[u].y; m[2] = (_Float16)hi[u].z; m[3] = (_Float16)hi[u].w;
@@ -182,34 +204,32 @@ __global__ __launch_bounds__(kRopeThreads) void rope_pieces_kernel(const RopeArg
 }
 
 // n_k, n_v: heads behind the n_q ones that go to the cache (0: the rotation alone).
-hipError_t pieces_launch(RopeArgs a, int n_rot, float theta, int n_v, bool neox, hipStream_t stream) {
-    a.freq = rope_freq_plan(n_rot, theta);
-    a.half = n_rot / 2;
-    a.quads = n_rot / 8;
-    a.n_heads = a.n_q + a.n_k + n_v;
-    a.half_magic = 65536u / a.half + 1;
-    a.quads_magic = 65536u / a.quads + 1;
-    a.block_tokens = kRopeThreads / a.half;
-    if (a.block_tokens > a.tokens) a.block_tokens = a.tokens;
+hipError_t pieces_launch(float* q, float* k, const float* v, RopeRest a, int tokens, int head_dim, int n_rot, float theta, int n_q, int n_k, int n_v,
+                         bool neox, hipStream_t stream) {
+    const RopeFreq f = rope_freq_plan(n_rot, theta);
+    a.step = f.by_steps ? f.step[0] : 0.0;
+    a.theta = theta;
+    const int half = n_rot / 2, quads = n_rot / 8, n_heads = n_q + n_k + n_v;
+    int block_tokens = kRopeThreads / half;
+    if (block_tokens > tokens) block_tokens = tokens;
     // Heads of a block: as many as give every thread a piece, more where that would be over four blocks a CU (the angles
     // are formed once per block).
-    const int groups = (a.tokens + a.block_tokens - 1) / a.block_tokens, slots = a.block_tokens * a.quads;
+    const int groups = (tokens + block_tokens - 1) / block_tokens, slots = block_tokens * quads;
     int u = 1, log2 = 0;
-    auto fill = [&](int pieces) { log2 = 0; while ((slots << (log2 + 1)) <= pieces && (1 << log2) < a.n_heads) ++log2; };
+    auto fill = [&](int pieces) { log2 = 0; while ((slots << (log2 + 1)) <= pieces && (1 << log2) < n_heads) ++log2; };
     for (;; u *= 2) {
         fill(kRopeThreads * u);
-        if (u == 4 || groups * ((a.n_heads + (1 << log2) - 1) >> log2) <= 1024) break;
+        if (u == 4 || groups * ((n_heads + (1 << log2) - 1) >> log2) <= 1024) break;
     }
-    a.block_heads_log2 = log2;
-    const dim3 grid(groups, (a.n_heads + (1 << log2) - 1) >> log2);
-#define ORIN_ROPE_PIECES(U) \
-    if (neox) hipLaunchKernelGGL((rope_pieces_kernel<true, U>), grid, dim3(kRopeThreads), 0, stream, a); \
-    else hipLaunchKernelGGL((rope_pieces_kernel<false, U>), grid, dim3(kRopeThreads), 0, stream, a)
-    if (u == 1) { ORIN_ROPE_PIECES(1); }
-    else if (u == 2) { ORIN_ROPE_PIECES(2); }
-    else { ORIN_ROPE_PIECES(4); }
-#undef ORIN_ROPE_PIECES
-    return hipGetLastError();
+    const dim3 grid(groups, (n_heads + (1 << log2) - 1) >> log2);
+    const uint64_t shape = arg_pair((unsigned)half | (unsigned)quads << 10 | (unsigned)block_tokens << 17 | (unsigned)log2 << 27, head_dim);
+    auto go = [&](auto kernel) {
+        return launch_lean(kernel, grid, kRopeThreads, 0, stream, arg_ptr(q), arg_ptr(k), arg_ptr(v), arg_pair(tokens, n_heads), arg_pair(n_q, n_k), shape,
+                           arg_pair(65536u / quads + 1, 65536u / half + 1), RopeRest(a));
+    };
+    if (u == 1) return neox ? go(rope_pieces_kernel<true, 1>) : go(rope_pieces_kernel<false, 1>);
+    if (u == 2) return neox ? go(rope_pieces_kernel<true, 2>) : go(rope_pieces_kernel<false, 2>);
+    return neox ? go(rope_pieces_kernel<true, 4>) : go(rope_pieces_kernel<false, 4>);
 }
 
 // (cos, sin) of every pair at the position *d_pos: what each thread of rope_kernel forms for
@@ -245,27 +265,24 @@ bool rope_store_fused_ok(const float* q, const float* k, const float* v, const u
 hipError_t rope_store_launch(float* q, float* k, const float* v, uint16_t* kc, uint16_t* vc, int tokens, int n_head,
                              int n_kv, int head_dim, int n_ctx, int n_past, float theta, const float* freq_factors,
                              bool neox, hipStream_t stream) {
-    drop_stale_error();
     if (tokens == 0) return hipSuccess;
-    RopeArgs a{};
-    a.q = q; a.k = k; a.v = v; a.kc = kc; a.vc = vc; a.freq_factors = freq_factors;
-    a.tokens = tokens; a.n_past = n_past; a.n_ctx = n_ctx; a.head_dim = head_dim; a.n_q = n_head; a.n_k = n_kv;
-    return pieces_launch(a, head_dim, theta, n_kv, neox, stream);
+    RopeRest a{};
+    a.kc = kc; a.vc = vc; a.freq_factors = freq_factors; a.n_past = n_past; a.n_ctx = n_ctx;
+    return pieces_launch(q, k, v, a, tokens, head_dim, head_dim, theta, n_head, n_kv, n_kv, neox, stream);
 }
 
 hipError_t rope_launch(float* x, int rows, int head_dim, int n_rot, float theta, int n_past, int heads,
                        const int* d_pos, const float* freq_factors, bool neox, hipStream_t stream) {
-    drop_stale_error();
     // batch form: rows = tokens * heads; single-token form: every row belongs to the one token
     const int tokens = d_pos ? 1 : rows / heads;
     const int heads_per_token = d_pos ? rows : heads;
     if (tokens == 0 || heads_per_token == 0) return hipSuccess;
     if (n_rot % 8 == 0 && n_rot / 2 <= 256 && head_dim % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0) {
-        RopeArgs a{};
-        a.q = x; a.d_pos = d_pos; a.freq_factors = freq_factors;
-        a.tokens = tokens; a.n_past = n_past; a.head_dim = head_dim; a.n_q = heads_per_token;
-        return pieces_launch(a, n_rot, theta, 0, neox, stream);
+        RopeRest a{};
+        a.d_pos = d_pos; a.freq_factors = freq_factors; a.n_past = n_past;
+        return pieces_launch(x, nullptr, nullptr, a, tokens, head_dim, n_rot, theta, heads_per_token, 0, 0, neox, stream);
     }
+    drop_stale_error();
     const int n_hgroups = (heads_per_token + kHeadsPerThread - 1) / kHeadsPerThread;
     const long long threads = (long long)tokens * n_hgroups * (n_rot / 2);
     const unsigned grid = (unsigned)((threads + 255) / 256);
