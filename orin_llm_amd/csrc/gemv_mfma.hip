@@ -304,8 +304,8 @@ __device__ __forceinline__ void gemv_rows_body(const RowsHead h, const GemvArgs&
     const int seg_wg = (int)blockIdx.x - (int)(turns >> 19), grid_x = (int)min(next >> 19, h.shape >> 18) - (int)(turns >> 19); // among the matrix's workgroups
     const int nb_row = (int)(h.shape & 0x7fu) + 1, share_blocks = (int)((h.shape >> 7) & 0x7fu) + 1, share_extra = (int)((h.shape >> 14) & 15u);
     const int n_mine = (int)(turns & 63u) + (seg_wg < (int)((turns >> 6) & 0x1fffu) ? 1 : 0); // tiles of this workgroup, one at least
-    const int b0 = (int)blockIdx.z * share_blocks + min((int)blockIdx.z, share_extra);
-    const int nb = share_blocks + ((int)blockIdx.z < share_extra ? 1 : 0);
+    const int b0 = (int)blockIdx.z * share_blocks + min((int)blockIdx.z, share_extra) * G::kUnit;
+    const int nb = share_blocks + ((int)blockIdx.z < share_extra ? G::kUnit : 0);
     const int n_in = nb << 8;
     const unsigned row_bytes = (unsigned)nb_row * F::kBlockBytes;
     float* const red = reinterpret_cast<float*>(smem + L::red_off(n_in));
@@ -336,7 +336,10 @@ __device__ __forceinline__ void gemv_rows_body(const RowsHead h, const GemvArgs&
             const unsigned r = DUAL ? row & 7u : row; // (of its matrix)
             // (slots past the sixteenth row: cut to the item's last piece by the request -- or some row's first of two matrices --
             // and to the buffer's spare piece here)
-            if constexpr (F::kBlockBytes == 16 * P) {
+            if constexpr (F::kRun) {
+                const unsigned piece = s - __umul24(row, G::kRowPieces);
+                goff[i] = __umul24(r, row_bytes) + (piece + 1 == (unsigned)G::kRowPieces ? (unsigned)F::kLastPiece : 16u * piece);
+            } else if constexpr (F::kBlockBytes == 16 * P) {
                 if constexpr (DUAL) goff[i] = __umul24(r, row_bytes) + 16u * (s - __umul24(row, G::kRowPieces));
                 else goff[i] = __umul24(row, row_bytes - 16u * G::kRowPieces) + 16u * s;
             } else {
@@ -357,7 +360,9 @@ __device__ __forceinline__ void gemv_rows_body(const RowsHead h, const GemvArgs&
     auto request = [&](u32x4 (&r)[NL], bool real = true) {
         // pieces past the chunk's end in rows above the last are the row's next blocks or the next row's first (fetched,
         // never used); in the last row they are cut to the last piece
-        unsigned limit = (kTileOut - 1u) * row_bytes + (unsigned)((min(CB, nb - rq_c * CB) - 1) * F::kBlockBytes + F::piece_off(P - 1));
+        unsigned limit = (kTileOut - 1u) * row_bytes;
+        if constexpr (F::kRun) limit += (unsigned)F::kLastPiece;
+        else limit += (unsigned)((min(CB, nb - rq_c * CB) - 1) * F::kBlockBytes + F::piece_off(P - 1));
         if (!real) limit = 0; // (one address for all: the same count of loads on every path)
         const unsigned char *const first = w_first + rq_off, *const second = w_second + rq_off;
 #pragma unroll
@@ -366,8 +371,10 @@ __device__ __forceinline__ void gemv_rows_body(const RowsHead h, const GemvArgs&
             constexpr int kFirst = DUAL ? 8 * G::kRowPieces : 64 * NL;
             const unsigned char* const base = 64 * i + 63 < kFirst ? first : 64 * i >= kFirst ? second : 64 * i + lane < kFirst ? first : second;
             // whole runs, read once: streaming loads
-            if constexpr (F::kAligned) r[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(base + min(goff[i], limit)));
-            else r[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_a2*>(base + min(goff[i], limit)));
+            const unsigned char* const p = base + min(goff[i], limit);
+            if constexpr (F::kAlign == 16) r[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+            else if constexpr (F::kAlign == 4) r[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_a4*>(p));
+            else r[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_a2*>(p));
         }
     };
     auto advance = [&] { // to the next item
@@ -552,10 +559,15 @@ __device__ __forceinline__ void gemv_rows_body(const RowsHead h, const GemvArgs&
         ++n_consumed;
         const int cb = min(CB, nb - cs_c * CB);
         // (unrolled over CB with a test per block, not a loop over cb: every LDS offset is a constant of its instruction)
-        float v = F::from_lds(transit + c.n * R * 16, c, addr, cs_c * CB);
-#pragma unroll
-        for (int j = 1; j < CB; ++j)
-            if (j < cb) v += F::from_lds(transit + (c.n * R + j * P) * 16, c, addr, cs_c * CB + j);
+        auto block = [&](auto jc) {
+            constexpr int j = decltype(jc)::value;
+            if constexpr (F::kRun) return F::template from_run<j>(transit + c.n * R * 16, c, addr, cs_c * CB + j);
+            else return F::from_lds(transit + (c.n * R + j * P) * 16, c, addr, cs_c * CB + j);
+        };
+        float v = block(IntC<0>{});
+        static_assert(CB <= 2, "blocks of an item");
+        if constexpr (CB == 2)
+            if (F::kRun || cb == 2) v += block(IntC<1>{});
         rowacc += v;
         cs_c += kWaves;
         if (cs_c >= n_chunks) {
@@ -612,21 +624,25 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_mfma_mixed_kernel(const Gemv
 
 // The same for the kernel that reads rows in long runs (no Q8_0 there: a file of that format has no other beside it).
 // (nothing is cut into shares here: RowsHead::shape's bits for those carry the types, two bits each)
-constexpr unsigned rows_type_code(int type) { return type == kQ4_K ? 0u : type == kQ5_K ? 1u : 2u; }
+constexpr unsigned rows_type_code(int type) { return type == kQ4_K ? 0u : type == kQ5_K ? 1u : type == kQ6_K ? 2u : 3u; }
 template <int kWaves, int CB, int kMode>
 __global__ __launch_bounds__(kWaves * 64) void gemv_rows_mixed_kernel(ROWS_HEAD_ARGS, const GemvArgs a) {
     const RowsHead h{w0, w1, w2, x, norm_w, turns0, turns1, turns2, (shape & ~0x3ff80u) | (shape & 0x7fu) << 7};
     switch ((shape >> (7 + 2 * rows_seg(h, (int)blockIdx.x))) & 3u) {
     case rows_type_code(kQ4_K): gemv_rows_body<kQ4_K, false, kWaves, CB, kMode>(h, a); break;
     case rows_type_code(kQ5_K): gemv_rows_body<kQ5_K, false, kWaves, CB, kMode>(h, a); break;
-    default: gemv_rows_body<kQ6_K, false, kWaves, CB, kMode>(h, a); break;
+    case rows_type_code(kQ6_K): gemv_rows_body<kQ6_K, false, kWaves, CB, kMode>(h, a); break;
+    default:
+        if constexpr (CB == 2) gemv_rows_body<kQ6_KRun, false, kWaves, CB, kMode>(h, a);
+        break;
     }
 }
 
 // The leading arguments of a launch of `wgs` workgroups for every share of a row (as many as the matrices have tiles, or
-// fewer, which then divide over the matrices as the tiles do), and whether they hold it.
-bool rows_head(const GemvArgs& a, int wgs, int shares, RowsHead& h) {
-    const int nb = a.n_in / 256;
+// fewer, which then divide over the matrices as the tiles do), and whether they hold it.  A row is cut into shares of whole units.
+bool rows_head(const GemvArgs& a, int wgs, int shares, int unit, RowsHead& h) {
+    const int nb = a.n_in / 256, units = nb / unit;
+    if (shares > units) return false;
     const void* w[3] = {};
     unsigned tiles[3] = {}, turns[3] = {kNoMatrix << 19, kNoMatrix << 19, kNoMatrix << 19}, total = 0, first = 0;
     for (int i = 0; i < a.n_seg; ++i) total += tiles[i] = (unsigned)a.seg[i].n_out / (a.w_up ? 8 : 16);
@@ -639,8 +655,8 @@ bool rows_head(const GemvArgs& a, int wgs, int shares, RowsHead& h) {
         first += mine;
     }
     h = RowsHead{w[0], a.w_up ? a.w_up : w[1], w[2], a.x, a.norm_w, turns[0], turns[1], turns[2],
-                 (unsigned)(nb - 1) | (unsigned)(nb / shares - 1) << 7 | (unsigned)(nb % shares) << 14 | first << 18};
-    return (first <= kMostRowsWgs || (a.n_seg == 1 && first == tiles[0] && first <= (unsigned)kMostRowsOneTurn)) && shares <= kMaxRowShares && shares <= nb && nb <= 128;
+                 (unsigned)(nb - 1) | (unsigned)(units / shares * unit - 1) << 7 | (unsigned)(units % shares) << 14 | first << 18};
+    return (first <= kMostRowsWgs || (a.n_seg == 1 && first == tiles[0] && first <= (unsigned)kMostRowsOneTurn)) && shares <= kMaxRowShares && nb <= 128;
 }
 #define ROWS_HEAD_OF(h) (h).w0, (h).w1, (h).w2, (h).x, (h).norm_w, (h).turns0, (h).turns1, (h).turns2, (h).shape
 
@@ -672,11 +688,13 @@ int rows_tiles(const GemvArgs& a) {
 int g_rows_resident = 768; // workgroups of four waves the chip holds at once (three a CU; set by the launcher)
 
 template <int T, bool DUAL, int kWaves, int CB>
-bool launch_rows_as(const GemvArgs& a, int wgs, int shares, int n_in_wg, hipStream_t stream) {
+bool launch_rows_as(const GemvArgs& a, int wgs, int shares, hipStream_t stream) {
+    constexpr int kUnit = RowsGeom<T, CB>::kUnit;
+    const int n_in_wg = (a.n_in / 256 / kUnit + shares - 1) / shares * kUnit * 256;
     const size_t lds = RowsGeom<T, CB>::lds_bytes(n_in_wg, kWaves);
     if (lds > kMfmaLdsMax) return false;
     RowsHead h;
-    if (!rows_head(a, wgs, shares, h)) return false;
+    if (!rows_head(a, wgs, shares, kUnit, h)) return false;
     const dim3 grid(h.shape >> 18, 1, shares);
     const int per_wave = ((n_in_wg / 256 + CB - 1) / CB + kWaves - 1) / kWaves, passes = CB == 2 ? per_wave : (per_wave + 1) / 2; // of a tile, at most
     auto go = [&](auto mode) {
@@ -704,30 +722,43 @@ bool launch_rows_as(const GemvArgs& a, int wgs, int shares, int n_in_wg, hipStre
 // q, k, v 8.4 -> 6.5, output projection 6.5 -> 4.5, logits 63.4 -> 45.8 us (279 MB, 6.1 TB/s).
 bool rows_base_ok(int type, const void* w) { return type != kQ8_0 || (reinterpret_cast<uintptr_t>(w) & 15u) == 0; }
 
+// Q6_K in runs of two blocks (kQ6_KRun): rows of an even number of blocks, at least two a share, in matrices that start on a word.
+bool rows_run_base_ok(const void* w) { return (reinterpret_cast<uintptr_t>(w) & 3u) == 0; }
+bool rows_runs_ok(const GemvArgs& a, int shares) {
+    const int nb = a.n_in / 256;
+    bool ok = nb % 2 == 0 && nb / 2 >= shares && (!a.w_up || rows_run_base_ok(a.w_up));
+    for (int i = 0; i < a.n_seg; ++i) ok = ok && rows_run_base_ok(a.seg[i].w);
+    return ok;
+}
+
 template <int T>
 bool launch_rows(const GemvArgs& a, int wgs, int shares, bool wide, int nb_wg, hipStream_t stream) {
     if (!rows_enabled()) return false;
     for (int i = 0; i < a.n_seg; ++i)
         if (a.seg[i].n_out % 16 != 0 || !rows_base_ok(T, a.seg[i].w)) return false;
     if (a.w_up && !rows_base_ok(T, a.w_up)) return false;
-    const int n_in_wg = nb_wg * 256;
     // Q8_0: 272 bytes are a long run already, so two blocks only where they make one item of a wave's share, and with eight waves,
     // whose buffers then leave room for one workgroup a CU, only up to a workgroup a CU (two blocks against one: 4096 x 4096 5.7 and
     // 6.05 us, 4096 x 1024 4.7 and 5.2; 4096 x 6144, 384 workgroups, 9.3 and 8.4).
     if constexpr (T == kQ8_0) {
-        if (wide) return nb_wg <= 16 && wgs <= g_rows_resident / 3 ? launch_rows_as<T, false, 8, 2>(a, wgs, shares, n_in_wg, stream) : launch_rows_as<T, false, 8, 1>(a, wgs, shares, n_in_wg, stream);
-        if (!a.w_up && nb_wg > 4 && nb_wg <= 8 && wgs == rows_tiles(a)) return launch_rows_as<T, false, 4, 2>(a, wgs, shares, n_in_wg, stream);
-        return a.w_up ? launch_rows_as<T, true, 4, 1>(a, wgs, shares, n_in_wg, stream) : launch_rows_as<T, false, 4, 1>(a, wgs, shares, n_in_wg, stream);
+        if (wide) return nb_wg <= 16 && wgs <= g_rows_resident / 3 ? launch_rows_as<T, false, 8, 2>(a, wgs, shares, stream) : launch_rows_as<T, false, 8, 1>(a, wgs, shares, stream);
+        if (!a.w_up && nb_wg > 4 && nb_wg <= 8 && wgs == rows_tiles(a)) return launch_rows_as<T, false, 4, 2>(a, wgs, shares, stream);
+        return a.w_up ? launch_rows_as<T, true, 4, 1>(a, wgs, shares, stream) : launch_rows_as<T, false, 4, 1>(a, wgs, shares, stream);
     }
     else { // (the other branch returned)
-    if (wide) return launch_rows_as<T, false, 8, 2>(a, wgs, shares, n_in_wg, stream); // (sixteen blocks at least; never two matrices)
     // runs of 288 (352) bytes read within a few percent of longer ones, and the wave's last item, which nothing
     // overlaps, is half as long as with four blocks
     const int cb = min(kRowsMaxCb, (nb_wg + 3) / 4);
-    if (a.w_up) {
-        return cb == 1 ? launch_rows_as<T, true, 4, 1>(a, wgs, shares, n_in_wg, stream) : launch_rows_as<T, true, 4, 2>(a, wgs, shares, n_in_wg, stream);
+    if constexpr (T == kQ6_K) {
+        if (rows_runs_ok(a, shares) && (wide || cb == 2))
+            return wide ? launch_rows_as<kQ6_KRun, false, 8, 2>(a, wgs, shares, stream)
+                        : a.w_up ? launch_rows_as<kQ6_KRun, true, 4, 2>(a, wgs, shares, stream) : launch_rows_as<kQ6_KRun, false, 4, 2>(a, wgs, shares, stream);
     }
-    return cb == 1 ? launch_rows_as<T, false, 4, 1>(a, wgs, shares, n_in_wg, stream) : launch_rows_as<T, false, 4, 2>(a, wgs, shares, n_in_wg, stream);
+    if (wide) return launch_rows_as<T, false, 8, 2>(a, wgs, shares, stream); // (sixteen blocks at least; never two matrices)
+    if (a.w_up) {
+        return cb == 1 ? launch_rows_as<T, true, 4, 1>(a, wgs, shares, stream) : launch_rows_as<T, true, 4, 2>(a, wgs, shares, stream);
+    }
+    return cb == 1 ? launch_rows_as<T, false, 4, 1>(a, wgs, shares, stream) : launch_rows_as<T, false, 4, 2>(a, wgs, shares, stream);
     }
 }
 
@@ -815,6 +846,13 @@ hipError_t allow_mixed() {
     return e != hipSuccess ? e : allow_lds(reinterpret_cast<const void*>(&gemv_rows_mixed_kernel<kWaves, CB, kRowsAny>));
 }
 
+hipError_t allow_rows_runs() {
+    hipError_t e;
+    if ((e = allow_rows<kQ6_KRun, false, 8, 2>()) != hipSuccess) return e;
+    if ((e = allow_rows<kQ6_KRun, false, 4, 2>()) != hipSuccess) return e;
+    return allow_rows<kQ6_KRun, true, 4, 2>();
+}
+
 template <int T>
 hipError_t allow_rows_all() {
     hipError_t e;
@@ -843,9 +881,13 @@ hipError_t gemv_mfma_mixed_launch(GemvArgs a, int cu_count, hipStream_t stream) 
         const int wgs = per_cu > 0 ? min(tiles, cu_count * per_cu) : tiles;
         const bool wide_r = nb > 8 && wgs == tiles; // (as in launch() above)
         RowsHead h;
-        if (rows_head(a, wgs, 1, h)) {
+        if (rows_head(a, wgs, 1, 1, h)) {
             h.shape &= ~0x3ff80u;
-            for (int i = 0; i < a.n_seg; ++i) h.shape |= rows_type_code(a.seg[i].type) << (7 + 2 * i);
+            const bool two = wide_r || nb > 4; // blocks an item
+            for (int i = 0; i < a.n_seg; ++i) {
+                const bool runs = a.seg[i].type == kQ6_K && two && nb % 2 == 0 && rows_run_base_ok(a.seg[i].w);
+                h.shape |= rows_type_code(runs ? kQ6_KRun : a.seg[i].type) << (7 + 2 * i);
+            }
             auto go = [&](auto waves, auto blocks) {
                 constexpr int W = decltype(waves)::value, CB = decltype(blocks)::value;
                 // (the largest of the types' layouts: Q6_K's digits in groups of 16, Q5_K's 11 pieces a block are within Q6_K's 14)
@@ -859,7 +901,7 @@ hipError_t gemv_mfma_mixed_launch(GemvArgs a, int cu_count, hipStream_t stream) 
             using One = std::integral_constant<int, 1>;
             using Two = std::integral_constant<int, 2>;
             const bool done = wide_r ? go(std::integral_constant<int, 8>(), Two())
-                                     : (nb <= 4 ? go(std::integral_constant<int, 4>(), One()) : go(std::integral_constant<int, 4>(), Two()));
+                                     : (!two ? go(std::integral_constant<int, 4>(), One()) : go(std::integral_constant<int, 4>(), Two()));
             if (done) return hipGetLastError();
         }
     }
@@ -902,6 +944,7 @@ hipError_t gemv_mfma_allow_lds() {
     if ((e = allow_rows_all<kQ4_K>()) != hipSuccess) return e;
     if ((e = allow_rows_all<kQ5_K>()) != hipSuccess) return e;
     if ((e = allow_rows_all<kQ6_K>()) != hipSuccess) return e;
+    if ((e = allow_rows_runs()) != hipSuccess) return e;
     if ((e = allow_rows<kQ8_0, false, 8, 1>()) != hipSuccess) return e;
     if ((e = allow_rows<kQ8_0, false, 8, 2>()) != hipSuccess) return e;
     if ((e = allow_rows<kQ8_0, false, 4, 2>()) != hipSuccess) return e;
