@@ -356,7 +356,7 @@ int orin_fa_rope_store_batch(float* q, float* k, const float* v, uint16_t* kc, u
     if (n_rot < 0 || n_rot > head_dim || (n_rot & 1)) return ORIN_FA_E_INVALID;
     if ((long long)n_past + batch > n_ctx) return ORIN_FA_E_INVALID;
     if (batch == 0) return ORIN_FA_OK;
-    if (rope_store_fused_ok(q, k, v, kc, vc, head_dim, n_rot))
+    if (rope_store_fused_ok(q, k, v, kc, vc, n_head + 2LL * n_kv, head_dim, n_rot))
         return hip_code(rope_store_launch(q, k, v, kc, vc, batch, n_head, n_kv, head_dim, n_ctx, n_past, theta,
                                           freq_factors, neox != 0, g_state.stream));
     // any other shape: the three launches this call stands for

@@ -58,8 +58,11 @@ __global__ __launch_bounds__(256) void kv_store_kernel(const uint64_t kc_bits, c
         half8 h;
         h[0] = (_Float16)x0.x; h[1] = (_Float16)x0.y; h[2] = (_Float16)x0.z; h[3] = (_Float16)x0.w;
         h[4] = (_Float16)x1.x; h[5] = (_Float16)x1.y; h[6] = (_Float16)x1.z; h[7] = (_Float16)x1.w;
-        // (streaming store: the row is read next by another kernel, from other compute units)
-        __builtin_nontemporal_store(h, reinterpret_cast<half8*>(dst));
+        // (An ordinary store: the attention of the same chunk reads these rows next, once per query tile and head group, and
+        // finds them in the last-level cache.  With streaming stores, this launch and the attention behind it: 45 tokens of
+        // Llama-3-8B 6.5 us for 6.3, 512 of Qwen2.5-1.5B at the start of a sequence 10.6 for 9.8, at 4096 27.0 for 26.6;
+        // 301 of Llama-3.2-1B at 1501 14.3 for 14.5.)
+        *reinterpret_cast<half8*>(dst) = h;
     } else {
         const _Float16 h = (_Float16)src[0];
         dst[0] = __builtin_bit_cast(uint16_t, h);

@@ -96,15 +96,24 @@ __global__ __launch_bounds__(256) void rope_kernel(float* x, int tokens, int hea
 // pieces), no power (a product of doubles the host prepares; 300 instructions) and 32-bit index arithmetic by
 // multiplication (64-bit divisions: 500).  Measured, per launch: 45 tokens
 // of Qwen2.5-1.5B (Q, K and V rows) 4.3 -> 3.0 us, a single token's Q rows 4.0 -> 2.9 us, 301 tokens of Llama-3.2-1B's Q rows
-// 4.1 -> 3.9; 512 tokens of Llama-3-8B (25 MB) stay at the memory's 7.5 us.
+// 4.1 -> 3.9; 512 tokens of Llama-3-8B (25 MB) stay at the memory's 7.7 us.  Two or four pieces per thread, which form an
+// angle once for more heads, were no faster at any size (512 tokens of Qwen2.5-7B 4.5 with one, 4.9 with two; 4096 tokens
+// 31.2, 31.9, 32.6 with one, two, four).
+//
+// The cache rows go out as ordinary stores, Q and K as streaming ones: the attention of the same chunk reads the new rows
+// once per query tile and head group, and finds them in the last-level cache where a streaming store had sent them past it.
+// This launch and the attention behind it, 512 tokens at the start of a sequence, streaming -> ordinary: Qwen2.5-1.5B 11.6
+// -> 10.5 us, Qwen3-0.6B 13.1 -> 12.0, Llama-3-8B 17.7 -> 17.2; 512 tokens at 4096, where they are an eighth of the rows
+// read, 27.0 -> 26.7, 31.5 -> 31.2, 46.4 -> 46.5.
 constexpr int kRopeThreads = 256;
+constexpr int kRopePieceHeads = 65535 * (kRopeThreads / 64); // heads of a token a grid can hold: a block takes four or more
 
 // What the first loads need comes first, as scalars that are in a wave's registers when it starts (kernel-argument preload); the
 // rest in as few bytes as will do (launch_lean()).
 //   counts   tokens | heads of Q, K and V together << 32
 //   heads    heads of Q << 0 | of K << 32
 //   shape    pairs of a head, 10 bits | pieces of a head, 7 | tokens of a block, 10 | log2 of its heads, 5 | head_dim << 32
-//   magic    x / pieces = x * magic >> 16, x < 1024 | the same for pairs, x < 256, << 32
+//   magic    x / pieces = x * magic >> 16, x < 256 | the same for pairs, x < 256, << 32
 struct RopeRest {
     uint16_t *kc, *vc;
     const int* d_pos;
@@ -126,7 +135,7 @@ __device__ __forceinline__ float rope_freq_of_step(int i, int n_rot, const RopeR
     return rope_freq(i, f, a.freq_factors);
 }
 
-template <bool NEOX, int U>
+template <bool NEOX>
 __global__ __launch_bounds__(kRopeThreads) void rope_pieces_kernel(const uint64_t q_bits, const uint64_t k_bits, const uint64_t v_bits, const uint64_t counts,
                                                                    const uint64_t heads, const uint64_t shape, const uint64_t magic, const RopeRest a) {
 #pragma clang fp contract(off)
@@ -139,25 +148,17 @@ __global__ __launch_bounds__(kRopeThreads) void rope_pieces_kernel(const uint64_
     const unsigned quads_magic = (unsigned)magic, half_magic = (unsigned)(magic >> 32);
     const int tid = threadIdx.x, token0 = (int)blockIdx.x * block_tokens, head0 = (int)blockIdx.y << block_heads_log2;
     const int o1 = NEOX ? half : 4;
-    float4 lo[U], hi[U];
-    int token[U], head[U], quad[U];
-    bool live[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        const int s = tid + kRopeThreads * u, rest = (int)((unsigned)s * quads_magic >> 16);
-        quad[u] = s - rest * quads;
-        head[u] = head0 + (rest & ((1 << block_heads_log2) - 1));
-        const int t = rest >> block_heads_log2;
-        token[u] = token0 + t;
-        live[u] = t < block_tokens && token[u] < tokens && head[u] < n_heads;
-        if (live[u]) {
-            const bool is_q = head[u] < n_q, is_k = head[u] < n_q + n_k;
-            const float* const row = is_q ? q + ((size_t)token[u] * n_q + head[u]) * head_dim
-                                          : (is_k ? k : v) + ((size_t)token[u] * n_k + (head[u] - n_q - (is_k ? 0 : n_k))) * head_dim;
-            const float* const p = row + quad[u] * (NEOX ? 4 : 8);
-            lo[u] = *reinterpret_cast<const float4*>(p);
-            hi[u] = *reinterpret_cast<const float4*>(p + o1);
-        }
+    float4 lo, hi;
+    const int rest = (int)((unsigned)tid * quads_magic >> 16), quad = tid - rest * quads;
+    const int head = head0 + (rest & ((1 << block_heads_log2) - 1)), block_token = rest >> block_heads_log2, token = token0 + block_token;
+    const bool live = block_token < block_tokens && token < tokens && head < n_heads;
+    const bool is_q = head < n_q, is_k = !is_q && head < n_q + n_k;
+    if (live) {
+        const float* const row = is_q ? q + ((size_t)token * n_q + head) * head_dim
+                                      : (is_k ? k : v) + ((size_t)token * n_k + (head - n_q - (is_k ? 0 : n_k))) * head_dim;
+        const float* const p = row + quad * (NEOX ? 4 : 8);
+        lo = *reinterpret_cast<const float4*>(p);
+        hi = *reinterpret_cast<const float4*>(p + o1);
     }
     {
         const int t = (int)((unsigned)tid * half_magic >> 16), i = tid - t * half;
@@ -167,39 +168,34 @@ __global__ __launch_bounds__(kRopeThreads) void rope_pieces_kernel(const uint64_
         }
     }
     __syncthreads();
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        if (!live[u]) continue;
-        const bool is_q = head[u] < n_q, is_k = !is_q && head[u] < n_q + n_k;
-        if (is_q || is_k) {
-            const float4* const cs = reinterpret_cast<const float4*>(sh_cs + (token[u] - token0) * half + 4 * quad[u]);
-            const float4 c01 = cs[0], c23 = cs[1];
-            float4 &x = lo[u], &y = hi[u];
-            if (NEOX) {
-                rope_rotate(x.x, y.x, c01.x, c01.y);
-                rope_rotate(x.y, y.y, c01.z, c01.w);
-                rope_rotate(x.z, y.z, c23.x, c23.y);
-                rope_rotate(x.w, y.w, c23.z, c23.w);
-            } else {
-                rope_rotate(x.x, x.y, c01.x, c01.y);
-                rope_rotate(x.z, x.w, c01.z, c01.w);
-                rope_rotate(y.x, y.y, c23.x, c23.y);
-                rope_rotate(y.z, y.w, c23.z, c23.w);
-            }
-            float* const row = is_q ? q + ((size_t)token[u] * n_q + head[u]) * head_dim : k + ((size_t)token[u] * n_k + (head[u] - n_q)) * head_dim;
-            float* const p = row + quad[u] * (NEOX ? 4 : 8);
-            store_stream(p, x);
-            store_stream(p + o1, y);
+    if (!live) return;
+    if (is_q || is_k) {
+        const float4* const cs = reinterpret_cast<const float4*>(sh_cs + block_token * half + 4 * quad);
+        const float4 c01 = cs[0], c23 = cs[1];
+        if (NEOX) {
+            rope_rotate(lo.x, hi.x, c01.x, c01.y);
+            rope_rotate(lo.y, hi.y, c01.z, c01.w);
+            rope_rotate(lo.z, hi.z, c23.x, c23.y);
+            rope_rotate(lo.w, hi.w, c23.z, c23.w);
+        } else {
+            rope_rotate(lo.x, lo.y, c01.x, c01.y);
+            rope_rotate(lo.z, lo.w, c01.z, c01.w);
+            rope_rotate(hi.x, hi.y, c23.x, c23.y);
+            rope_rotate(hi.z, hi.w, c23.z, c23.w);
         }
-        if (!is_q && a.kc) {
-            const int h = head[u] - n_q - (is_k ? 0 : n_k);
-            uint16_t* const p = (is_k ? a.kc : a.vc) + ((size_t)h * a.n_ctx + a.n_past + token[u]) * head_dim + quad[u] * (NEOX ? 4 : 8);
-            half4_t l, m;
-            l[0] = (_Float16)lo[u].x; l[1] = (_Float16)lo[u].y; l[2] = (_Float16)lo[u].z; l[3] = (_Float16)lo[u].w;
-            m[0] = (_Float16)hi[u].x; m[1] = (_Float16)hi[u].y; m[2] = (_Float16)hi[u].z; m[3] = (_Float16)hi[u].w;
-            __builtin_nontemporal_store(l, reinterpret_cast<half4_t*>(p));
-            __builtin_nontemporal_store(m, reinterpret_cast<half4_t*>(p + o1));
-        }
+        float* const row = is_q ? q + ((size_t)token * n_q + head) * head_dim : k + ((size_t)token * n_k + (head - n_q)) * head_dim;
+        float* const p = row + quad * (NEOX ? 4 : 8);
+        store_stream(p, lo);
+        store_stream(p + o1, hi);
+    }
+    if (!is_q && a.kc) {
+        const int h = head - n_q - (is_k ? 0 : n_k);
+        uint16_t* const p = (is_k ? a.kc : a.vc) + ((size_t)h * a.n_ctx + a.n_past + token) * head_dim + quad * (NEOX ? 4 : 8);
+        half4_t l, m;
+        l[0] = (_Float16)lo.x; l[1] = (_Float16)lo.y; l[2] = (_Float16)lo.z; l[3] = (_Float16)lo.w;
+        m[0] = (_Float16)hi.x; m[1] = (_Float16)hi.y; m[2] = (_Float16)hi.z; m[3] = (_Float16)hi.w;
+        *reinterpret_cast<half4_t*>(p) = l;
+        *reinterpret_cast<half4_t*>(p + o1) = m;
     }
 }
 
@@ -212,24 +208,17 @@ hipError_t pieces_launch(float* q, float* k, const float* v, RopeRest a, int tok
     const int half = n_rot / 2, quads = n_rot / 8, n_heads = n_q + n_k + n_v;
     int block_tokens = kRopeThreads / half;
     if (block_tokens > tokens) block_tokens = tokens;
-    // Heads of a block: as many as give every thread a piece, more where that would be over four blocks a CU (the angles
-    // are formed once per block).
+    // Heads of a block: as many as give every thread a piece.
     const int groups = (tokens + block_tokens - 1) / block_tokens, slots = block_tokens * quads;
-    int u = 1, log2 = 0;
-    auto fill = [&](int pieces) { log2 = 0; while ((slots << (log2 + 1)) <= pieces && (1 << log2) < n_heads) ++log2; };
-    for (;; u *= 2) {
-        fill(kRopeThreads * u);
-        if (u == 4 || groups * ((n_heads + (1 << log2) - 1) >> log2) <= 1024) break;
-    }
+    int log2 = 0;
+    while ((slots << (log2 + 1)) <= kRopeThreads && (1 << log2) < n_heads) ++log2;
     const dim3 grid(groups, (n_heads + (1 << log2) - 1) >> log2);
     const uint64_t shape = arg_pair((unsigned)half | (unsigned)quads << 10 | (unsigned)block_tokens << 17 | (unsigned)log2 << 27, head_dim);
     auto go = [&](auto kernel) {
         return launch_lean(kernel, grid, kRopeThreads, 0, stream, arg_ptr(q), arg_ptr(k), arg_ptr(v), arg_pair(tokens, n_heads), arg_pair(n_q, n_k), shape,
                            arg_pair(65536u / quads + 1, 65536u / half + 1), RopeRest(a));
     };
-    if (u == 1) return neox ? go(rope_pieces_kernel<true, 1>) : go(rope_pieces_kernel<false, 1>);
-    if (u == 2) return neox ? go(rope_pieces_kernel<true, 2>) : go(rope_pieces_kernel<false, 2>);
-    return neox ? go(rope_pieces_kernel<true, 4>) : go(rope_pieces_kernel<false, 4>);
+    return neox ? go(rope_pieces_kernel<true>) : go(rope_pieces_kernel<false>);
 }
 
 // (cos, sin) of every pair at the position *d_pos: what each thread of rope_kernel forms for
@@ -256,10 +245,10 @@ hipError_t rope_angles_launch(float* angles, int n_rot, float theta, const int* 
 }
 
 bool rope_store_fused_ok(const float* q, const float* k, const float* v, const uint16_t* kc, const uint16_t* vc,
-                         int head_dim, int n_rot) {
+                         long long heads, int head_dim, int n_rot) {
     const uintptr_t bits = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v) |
                            reinterpret_cast<uintptr_t>(kc) | reinterpret_cast<uintptr_t>(vc);
-    return n_rot == head_dim && head_dim % 8 == 0 && head_dim / 2 <= 256 && (bits & 15u) == 0;
+    return n_rot == head_dim && head_dim % 8 == 0 && head_dim / 2 <= 256 && heads <= kRopePieceHeads && (bits & 15u) == 0;
 }
 
 hipError_t rope_store_launch(float* q, float* k, const float* v, uint16_t* kc, uint16_t* vc, int tokens, int n_head,
@@ -277,7 +266,7 @@ hipError_t rope_launch(float* x, int rows, int head_dim, int n_rot, float theta,
     const int tokens = d_pos ? 1 : rows / heads;
     const int heads_per_token = d_pos ? rows : heads;
     if (tokens == 0 || heads_per_token == 0) return hipSuccess;
-    if (n_rot % 8 == 0 && n_rot / 2 <= 256 && head_dim % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0) {
+    if (n_rot % 8 == 0 && n_rot / 2 <= 256 && head_dim % 4 == 0 && heads_per_token <= kRopePieceHeads && (reinterpret_cast<uintptr_t>(x) & 15u) == 0) {
         RopeRest a{};
         a.d_pos = d_pos; a.freq_factors = freq_factors; a.n_past = n_past;
         return pieces_launch(x, nullptr, nullptr, a, tokens, head_dim, n_rot, theta, heads_per_token, 0, 0, neox, stream);
