@@ -741,6 +741,62 @@ def test_rows_where_the_number_of_waves_changes(ly, wtype, blocks):
             assert vec_err(g[:len(exact)], exact) < TOL_OP, (tiles, len(exact))
 
 
+@pytest.mark.parametrize("n_in", [512, 1536, 2304, 2560, 4608, 7680, 18944])
+@pytest.mark.parametrize("offset", [0, 2, 4])
+def test_q6_k_rows_in_runs_of_two_blocks(ly, n_in, offset):
+    """Rows of an even number of blocks are read two blocks at a time where the matrix starts on a word: one pair a wave, several
+    over all waves, shares cut between pairs (of 18 blocks, of 30 in 15 and in more shares than pairs, of 74 in 10), the pair of
+    gate and up, beside a matrix of another type; and what is left to single blocks, an odd number and a matrix 2 bytes on."""
+    import torch
+
+    ly.use_matrix_cores(True)
+    n_out, rs = 48, lm.Stream(7990 + n_in)
+    a, b, other = lm.make_tensor(rs, lm.Q6_K, n_in, n_out), lm.make_tensor(rs, lm.Q6_K, n_in, n_out), lm.make_tensor(rs, lm.Q4_K, n_in, 16)
+    x, y0 = rs.sym(n_in, 1.0), rs.sym(n_out, 1.0)
+    prod = [ref.gemv(t, m[1], x, n_in, n).astype(np.float64) for t, m, n in ((lm.Q6_K, a, n_out), (lm.Q6_K, b, n_out), (lm.Q4_K, other, 16))]
+    wa, wb, wo, dx = dev_bytes(a[1], offset), dev_bytes(b[1], offset), dev_bytes(other[1]), _dev(x)
+    y, yg, ym, yo = (out_buf(n) for n in (n_out, n_out, n_out, 16))
+    ly.gemv(lm.Q6_K, wa, dx, y, n_in, n_out)
+    ly.quantize_activation(dx, n_in)
+    ly.gemv_fused_gate_up_swiglu(lm.Q6_K, wa, wb, yg, n_in, n_out)
+    ly.gemv_multi_types([lm.Q4_K, lm.Q6_K], [wo, wb], None, [yo, ym], [16, n_out], dx, None, 0.0, n_in)
+    cases = [("one", y, prod[0]), ("gate/up", yg, ref.swiglu(prod[0].astype(np.float32), prod[1].astype(np.float32))), ("mixed", ym, prod[1]), ("beside", yo, prod[2])]
+    try:
+        for shares in (1, 2, 3, 10, 15, 16):
+            ly.gemv_row_shares(shares)
+            z = _dev(np.concatenate([y0, np.full(4, 12345.0, np.float32)]))
+            ly.gemv_multi(lm.Q6_K, [wa], None, [z], [n_out], dx, None, 0.0, n_in, True)
+            cases.append((f"{shares} shares", z, y0 + prod[0]))
+    finally:
+        ly.gemv_row_shares(0)
+    torch.cuda.synchronize()
+    for what, got, want in cases:
+        g = got.cpu().numpy()
+        assert (g[len(want):] == 12345.0).all(), what
+        assert vec_err(g[:len(want)], np.asarray(want, np.float64)) < TOL_OP, what
+
+
+@pytest.mark.parametrize("n_in", [3328, 3584, 4096])
+def test_q8_0_matrices_of_many_turns(ly, n_in):
+    """From eight row tiles a workgroup on (at three workgroups on each of 256 CUs), rows of fourteen blocks of 256 elements and
+    more go two blocks at a time: either side of both lines, and a last turn that few workgroups have."""
+    import torch
+
+    base_rows, rs = 512, lm.Stream(8020 + n_in)
+    t, x = lm.make_tensor(rs, lm.Q8_0, n_in, base_rows), rs.sym(n_in, 1.0)
+    line = 16 * 8 * 3 * 256
+    pick = np.arange(line + 16 * 5, dtype=np.int64) * 197 % 509   # (neighbours, and rows a tile or a turn apart, differ)
+    w = torch.from_numpy(t[1].reshape(base_rows, -1)).cuda()[torch.from_numpy(pick).cuda()].reshape(-1)
+    want = ref.gemv(lm.Q8_0, t[1], x, n_in, base_rows).astype(np.float64)[pick]
+    for n_out in (line - 16, line, len(pick)):
+        y = out_buf(n_out)
+        ly.gemv(lm.Q8_0, w, _dev(x), y, n_in, n_out)
+        torch.cuda.synchronize()
+        got = y.cpu().numpy()
+        assert (got[n_out:] == 12345.0).all()
+        assert vec_err(got[:n_out], want[:n_out]) < TOL_OP, n_out
+
+
 @pytest.mark.parametrize("n_in", [256, 1792])
 def test_more_row_tiles_than_a_launch_counts_workgroups_for(ly, n_in):
     """A vocabulary's worth of rows: 8200 tiles, one workgroup each or several tiles a workgroup."""

@@ -127,6 +127,20 @@ def test_rope_batch_at_the_edges_of_its_blocks(fa, head_dim, n_rot, heads, token
     _check(guard[:-1].cpu().numpy(), want, x, n_rot, f"rope blocks neox={neox} {head_dim} {n_rot} {heads} {tokens}")
 
 
+# the most heads a grid of the kernel in pieces holds (four a block with 512 rotated elements), and one more; every row the same
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads", [4 * 65535, 4 * 65535 + 1])
+def test_rope_batch_of_more_heads_than_a_grid_holds(fa, heads):
+    import torch
+    row = np.random.default_rng(5).standard_normal((1, 512)).astype(np.float32)
+    want = ref.rope_batch(row, 512, 512, 1.0e6, 1234, 1, None, True)
+    x = torch.from_numpy(row).cuda().expand(heads, 512).contiguous()
+    fa.rope_neox_batch(x, heads, 512, 512, 1.0e6, 1234, heads, None)
+    torch.cuda.synchronize()
+    assert (x == x[:1]).all()
+    _check(x[:1].cpu().numpy(), want, row, 512, f"rope heads {heads}")
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("neox", [True, False])
 def test_rope_ind_reads_the_position_on_the_device_and_replays(fa, neox):
