@@ -807,10 +807,10 @@ hipError_t launch(const GemvArgs& a, int cu_count, hipStream_t stream) {
             }
         }
         // Eight waves from 9 blocks a row on, which gives a wave one item up to 16 (Qwen2.5-7B's q, k, v in Q5_K and Q6_K 8.4 ->
-        // 6.4 us); of Q8_0, up to 15 blocks only where there is a workgroup a CU at most.  (Between one and two a CU eight waves, one
-        // block an item, measure faster as well, 3072 x 6144 8.45 -> 7.45 us, 2560 x 6144 7.1 -> 6.6; beyond, 3 % slower to 8 %
-        // faster.  The line could lie at two.)
-        const bool wide_r = ks_r == 1 && nb_row > (T == kQ8_0 && tiles > cu_count ? 15 : 8) && !a.w_up && wgs == tiles;
+        // 6.4 us); of Q8_0, up to 15 blocks only where there are three workgroups on two CUs at most: 288 of them 6.85 -> 6.36
+        // us with 9 blocks, 8.25 -> 7.46 with 12, 8.26 -> 8.06 with 14, 384 of them 7.0 -> 6.65, 8.5 -> 7.8, 9.04 -> 9.0; with 448
+        // 7.2 -> 7.1, 9.45 -> 9.1, but 9.6 -> 9.8.
+        const bool wide_r = ks_r == 1 && nb_row > (T == kQ8_0 && 2 * tiles > 3 * cu_count ? 15 : 8) && !a.w_up && wgs == tiles;
         if (launch_rows<T>(a, wgs, ks_r, wide_r, (nb_row + ks_r - 1) / ks_r, stream)) return hipGetLastError();
     }
     const size_t lds = lds_bytes<T>((nb_row + ks - 1) / ks * 256);

@@ -717,8 +717,8 @@ def test_workgroups_and_shares_of_rows_in_runs(ly, types, n_in, heights):
 @pytest.mark.parametrize("wtype", [lm.Q4_K, lm.Q6_K, lm.Q8_0])
 @pytest.mark.parametrize("blocks", [8, 9, 15, 16, 17])
 def test_rows_where_the_number_of_waves_changes(ly, wtype, blocks):
-    """Eight waves a workgroup from nine blocks of 256 elements a row on (in Q8_0 from sixteen where there are more tiles than
-    CUs), one item a wave up to sixteen, while a workgroup has one tile: either side of each of these lines, in one matrix and,
+    """Eight waves a workgroup from nine blocks of 256 elements a row on (in Q8_0 from sixteen where there are more than
+    three tiles on two CUs), one item a wave up to sixteen, while a workgroup has one tile: either side of each of these lines, in one matrix and,
     beside one of another type, in a launch of two types."""
     import torch
 
@@ -789,6 +789,23 @@ def test_q8_0_matrices_of_many_turns(ly, n_in):
     w = torch.from_numpy(t[1].reshape(base_rows, -1)).cuda()[torch.from_numpy(pick).cuda()].reshape(-1)
     want = ref.gemv(lm.Q8_0, t[1], x, n_in, base_rows).astype(np.float64)[pick]
     for n_out in (line - 16, line, len(pick)):
+        y = out_buf(n_out)
+        ly.gemv(lm.Q8_0, w, _dev(x), y, n_in, n_out)
+        torch.cuda.synchronize()
+        got = y.cpu().numpy()
+        assert (got[n_out:] == 12345.0).all()
+        assert vec_err(got[:n_out], want[:n_out]) < TOL_OP, n_out
+
+
+@pytest.mark.parametrize("blocks", [9, 12, 15])
+def test_q8_0_rows_either_side_of_three_workgroups_on_two_cus(ly, blocks):
+    """Eight waves up to 384 tiles on 256 CUs, four beyond, for rows of 9 to 15 blocks of 256 elements."""
+    import torch
+
+    n_in, most, rs = 256 * blocks, 16 * 385, lm.Stream(8060 + blocks)
+    t, x = lm.make_tensor(rs, lm.Q8_0, n_in, most), rs.sym(n_in, 1.0)
+    want, w = ref.gemv(lm.Q8_0, t[1], x, n_in, most).astype(np.float64), dev_bytes(t[1])
+    for n_out in (16 * 288, 16 * 384, most):
         y = out_buf(n_out)
         ly.gemv(lm.Q8_0, w, _dev(x), y, n_in, n_out)
         torch.cuda.synchronize()
