@@ -9,7 +9,7 @@
 namespace orin_fa {
 namespace {
 
-constexpr int kMaxWaves = 8; // waves per workgroup: 4, or 8 where a matrix has few 16-row tiles and long rows
+constexpr int kMaxWaves = 8; // waves per workgroup: 4; 8 where a matrix has few 16-row tiles and long rows; 2 or 3 where many and short ones
 constexpr float kDigitRange = 8388608.0f - 65536.0f; // largest |integer| the three signed digits hold
 
 struct XPair {

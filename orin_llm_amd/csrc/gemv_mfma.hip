@@ -731,12 +731,45 @@ bool rows_runs_ok(const GemvArgs& a, int shares) {
     return ok;
 }
 
+// Workgroups of as many waves as a row has items of two blocks, two or three, where every workgroup has one tile: 0 for the four
+// (or eight) waves of the other launches.  Four waves take a row of 4 blocks a block at a time, in runs half as long (and in
+// Q6_K from any 2-byte boundary), and of a row of 5 or 6 blocks leave the fourth wave its place and nothing to do: with many
+// workgroups a CU longer runs and more tiles in flight win, with few a wave's shorter chain does.  Four waves -> two or three,
+// us a launch, 1024 elements a row: 151936 rows in Q6_K 30.9 -> 26.0, in Q4_K 21.7 -> 19.6, in Q5_K 24.3 -> 23.3, in Q8_0 31.0 ->
+// 29.3; 16384 rows (four workgroups a CU) 5.9 -> 5.5, 5.0 -> 4.5, 5.25 -> 5.0, 6.1 -> 6.1; 12288 rows 4.9 -> 4.9, 4.3 -> 4.25, 4.4 ->
+// 4.7, 5.1 -> 5.2.  1536 elements a row: 151936 rows in Q6_K 38.6 -> 36.6, in Q5_K 32.9 -> 31.6, in Q8_0 47.2 -> 42.3, in Q4_K 27.0
+// -> 27.1 (not taken); 16384 rows 6.95 -> 6.93, 6.1 -> 6.3, 8.1 -> 7.8; two matrices of 8960 rows 8.1 -> 7.6, 6.7 -> 6.8, 9.05 ->
+// 8.9.  In Q8_0, whose items of one block these would otherwise be, three waves are at least as fast at every size (64 tiles
+// of two matrices 3.9 -> 3.7).
+template <int T>
+int rows_small_waves(const GemvArgs& a, int wgs, int shares, int nb) {
+    const int tiles = rows_tiles(a), cus = g_rows_resident / 3;
+    if (shares != 1 || wgs != tiles || nb < 4 || nb > 6 || (T == kQ6_K && !rows_runs_ok(a, 1))) return 0;
+    if (nb == 4) return tiles >= 4 * cus ? 2 : 0;
+    if (T == kQ8_0) return 3;
+    return T != kQ4_K && tiles >= (T == kQ6_K && a.w_up ? 4 : 6) * cus ? 3 : 0;
+}
+
+template <int T, bool DUAL, int kWaves>
+bool launch_rows_one_item(const GemvArgs& a, int wgs, hipStream_t stream) {
+    const size_t lds = RowsGeom<T, 2>::lds_bytes(a.n_in, kWaves);
+    RowsHead h;
+    if (lds > 64u * 1024u || !rows_head(a, wgs, 1, RowsGeom<T, 2>::kUnit, h)) return false;
+    hipLaunchKernelGGL((gemv_rows_kernel<T, DUAL, kWaves, 2, kRowsOneItem>), dim3(h.shape >> 18), dim3(kWaves * 64), lds, stream, ROWS_HEAD_OF(h), a);
+    return true;
+}
+
 template <int T>
 bool launch_rows(const GemvArgs& a, int wgs, int shares, bool wide, int nb_wg, hipStream_t stream) {
     if (!rows_enabled()) return false;
     for (int i = 0; i < a.n_seg; ++i)
         if (a.seg[i].n_out % 16 != 0 || !rows_base_ok(T, a.seg[i].w)) return false;
     if (a.w_up && !rows_base_ok(T, a.w_up)) return false;
+    if (const int waves = wide ? 0 : rows_small_waves<T>(a, wgs, shares, nb_wg)) {
+        constexpr int R = T == kQ6_K ? (int)kQ6_KRun : T;
+        if (waves == 2 ? (a.w_up ? launch_rows_one_item<R, true, 2>(a, wgs, stream) : launch_rows_one_item<R, false, 2>(a, wgs, stream))
+                       : (a.w_up ? launch_rows_one_item<R, true, 3>(a, wgs, stream) : launch_rows_one_item<R, false, 3>(a, wgs, stream))) return true;
+    }
     // Q8_0: 272 bytes are a long run already, so two blocks only where they make one item of a wave's share, and with eight waves,
     // whose buffers then leave room for one workgroup a CU, only up to a workgroup a CU (two blocks against one: 4096 x 4096 5.7 and
     // 6.05 us, 4096 x 1024 4.7 and 5.2; 4096 x 6144, 384 workgroups, 9.3 and 8.4).
@@ -789,10 +822,10 @@ hipError_t launch(const GemvArgs& a, int cu_count, hipStream_t stream) {
         const int tiles = rows_tiles(a);
         // One item a wave where a row is short enough: as many workgroups as there are tiles, for the chip to hand out, and
         // no second turn.  Of two matrices up to 8 blocks (Qwen2.5-1.5B's gate/up in Q4_K 6.5 -> 6.1 us; 16 blocks in workgroups
-        // of eight waves: Llama-3-8B's 15.0 -> 17.4), in Q8_0 up to 4 (its items of two blocks: 9.9 -> 10.2 us); of one
+        // of eight waves: Llama-3-8B's 15.0 -> 17.4), in Q8_0 up to 6 (rows_small_waves(); 8 blocks: Llama-3.2-1B's 9.9 -> 10.2 us); of one
         // matrix up to 6, which would leave a fourth of the waves of long-lived workgroups without a chunk
         // (Qwen2.5-1.5B's logits in Q6_K 38.4 -> 35.7 us; 8 blocks: Llama-3.2-1B's in Q5_K 32.6 -> 34.4).
-        const bool one_item = nb_row <= (!a.w_up ? 6 : T == kQ8_0 ? 4 : 8) && tiles <= kMostRowsOneTurn;
+        const bool one_item = nb_row <= (!a.w_up || T == kQ8_0 ? 6 : 8) && tiles <= kMostRowsOneTurn;
         const int wgs = one_item || per_cu <= 0 ? tiles : min(tiles, cu_count * per_cu);
         // Shares of a row of a matrix that is accumulated into: up to 8 blocks, so that every wave has one item.  Digits
         // are each share's own, so more shares make no more of them, and the chip evens out what workgroups of two long

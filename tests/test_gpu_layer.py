@@ -814,6 +814,37 @@ def test_q8_0_rows_either_side_of_three_workgroups_on_two_cus(ly, blocks):
         assert vec_err(got[:n_out], want[:n_out]) < TOL_OP, n_out
 
 
+@pytest.mark.parametrize("wtype", [lm.Q4_K, lm.Q5_K, lm.Q6_K, lm.Q8_0])
+@pytest.mark.parametrize("blocks", [4, 5, 6])
+def test_rows_of_four_to_six_blocks_in_workgroups_of_two_and_three_waves(ly, wtype, blocks):
+    """One item of two blocks a wave, either side of four and of six tiles on each of 256 CUs, in one matrix and in a pair, with the
+    norm and without; in Q6_K from a word boundary and 2 bytes on (which stays with four waves)."""
+    import torch
+
+    n_in, base_rows, most, rs = 256 * blocks, 512, 1537, lm.Stream(8090 + blocks + wtype)
+    a, b = lm.make_tensor(rs, wtype, n_in, base_rows), lm.make_tensor(rs, wtype, n_in, base_rows)
+    x, nw, eps = rs.sym(n_in, 1.0), (1.0 + rs.sym(n_in, 0.3)).astype(np.float32), 1e-5
+    xn, dx, dnw = ref.rms_norm(x, nw, eps), _dev(x), _dev(nw)
+    pick = np.arange(16 * most, dtype=np.int64) * 197 % 509   # (neighbours, and rows a tile apart, differ)
+
+    def rows(raw, offset):
+        return dev_bytes(np.ascontiguousarray(raw.reshape(base_rows, -1)[pick]).reshape(-1), offset)
+
+    plain = ref.gemv(wtype, a[1], x, n_in, base_rows).astype(np.float64)[pick]
+    act = ref.swiglu(ref.gemv(wtype, a[1], xn, n_in, base_rows), ref.gemv(wtype, b[1], xn, n_in, base_rows)).astype(np.float64)[pick]
+    for offset in (0, 2) if wtype == lm.Q6_K else (0,):
+        wa, wb = rows(a[1], offset), rows(b[1], offset)
+        for tiles in (3, 1023, 1024, 1535, 1536, most):
+            n_out, n_pair = 16 * tiles, 8 * tiles
+            y, yp = out_buf(n_out), out_buf(n_pair)
+            ly.gemv(wtype, wa, dx, y, n_in, n_out)
+            ly.gemv_norm_gate_up_swiglu(wtype, wa, wb, dx, dnw, eps, yp, n_in, n_pair)
+            torch.cuda.synchronize()
+            for got, want in ((y.cpu().numpy(), plain[:n_out]), (yp.cpu().numpy(), act[:n_pair])):
+                assert (got[len(want):] == 12345.0).all()
+                assert vec_err(got[:len(want)], want) < TOL_OP, (tiles, offset, len(want))
+
+
 @pytest.mark.parametrize("n_in", [256, 1792])
 def test_more_row_tiles_than_a_launch_counts_workgroups_for(ly, n_in):
     """A vocabulary's worth of rows: 8200 tiles, one workgroup each or several tiles a workgroup."""
