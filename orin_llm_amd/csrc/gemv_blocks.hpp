@@ -170,7 +170,16 @@ struct MFK45 {
         // pairs g (first half of the block) and 4 + g (second half) of the twelve packed bytes
         const float sc[2] = {(float)(b0 & 63u), (float)((b2 & 0x0fu) | ((b0 >> 6) << 4))};
         const float mn[2] = {(float)(b1 & 63u), (float)((b2 >> 4) | ((b1 >> 6) << 4))};
-        return math(dd, sc, mn, q1, q2, fifth, c, ad, b);
+        return math(dd, sc, mn, q1, q2, fifth, [&](int h) { return digits(c, ad, b, h); });
+    }
+    // What half a block's product takes from the activation: A operands and sub-block pairs.
+    struct Digits {
+        i32x4 lo, hi;
+        XPair xp;
+    };
+    static __device__ __forceinline__ Digits digits(const LaneCtx& c, const Addr& ad, int b, int h) {
+        return Digits{*reinterpret_cast<const i32x4*>(c.smem + operand_at(ad.lo_base, ad.lo_step, 256 * b + 128 * h)),
+                      *reinterpret_cast<const i32x4*>(c.smem + operand_at(ad.hi_base, ad.hi_step, 256 * b + 128 * h)), c.pairs[8 * b + 4 * h + c.g]};
     }
     // A block laid out in LDS piece after piece (the kernel that reads rows in long runs): piece k is the block's
     // bytes 16 k ...
@@ -178,30 +187,37 @@ struct MFK45 {
     static constexpr bool kRun = false;
     static constexpr int kAlign = 16;
     static __host__ __device__ constexpr int piece_off(int k) { return 16 * k; }
-    static __device__ __forceinline__ float from_lds(const unsigned char* blk, const LaneCtx& c, const Addr& ad, int b) {
-        const u32x4 hdr = *reinterpret_cast<const u32x4*>(blk);
-        const u32x4 q1 = *reinterpret_cast<const u32x4*>(blk + kQs + 16 * c.g);
-        const u32x4 q2 = *reinterpret_cast<const u32x4*>(blk + kQs + 64 + 16 * c.g);
-        u32x4 fifth = {0u, 0u, 0u, 0u};
-        if constexpr (FIVE) fifth = *reinterpret_cast<const u32x4*>(blk + 16 + 16 * (c.g & 1)) >> (unsigned)(2 * (c.g >> 1));
+    struct Words {
+        u32x4 hdr, q1, q2, fifth;
+    };
+    static __device__ __forceinline__ Words words(const unsigned char* blk, const LaneCtx& c) {
+        Words w{*reinterpret_cast<const u32x4*>(blk), *reinterpret_cast<const u32x4*>(blk + kQs + 16 * c.g),
+                *reinterpret_cast<const u32x4*>(blk + kQs + 64 + 16 * c.g), u32x4{0u, 0u, 0u, 0u}};
+        if constexpr (FIVE) w.fifth = *reinterpret_cast<const u32x4*>(blk + 16 + 16 * (c.g & 1));
+        return w;
+    }
+    // `of_half`(h): the digits of half h
+    template <typename X>
+    static __device__ __forceinline__ float product(const Words& w, const X& of_half, const LaneCtx& c) {
         // the six-bit pairs straight out of the three words (bit fields at 8 g: no byte is put together first)
         const unsigned s8 = 8 * c.g;
-        const float sc[2] = {(float)__builtin_amdgcn_ubfe(hdr.y, s8, 6), (float)(__builtin_amdgcn_ubfe(hdr.w, s8, 4) | ((hdr.y >> (s8 + 2)) & 0x30u))};
-        const float mn[2] = {(float)__builtin_amdgcn_ubfe(hdr.z, s8, 6), (float)(__builtin_amdgcn_ubfe(hdr.w, s8 + 4, 4) | ((hdr.z >> (s8 + 2)) & 0x30u))};
-        return math(hdr.x, sc, mn, q1, q2, fifth, c, ad, b);
+        const float sc[2] = {(float)__builtin_amdgcn_ubfe(w.hdr.y, s8, 6), (float)(__builtin_amdgcn_ubfe(w.hdr.w, s8, 4) | ((w.hdr.y >> (s8 + 2)) & 0x30u))};
+        const float mn[2] = {(float)__builtin_amdgcn_ubfe(w.hdr.z, s8, 6), (float)(__builtin_amdgcn_ubfe(w.hdr.w, s8 + 4, 4) | ((w.hdr.z >> (s8 + 2)) & 0x30u))};
+        return math(w.hdr.x, sc, mn, w.q1, w.q2, FIVE ? w.fifth >> (unsigned)(2 * (c.g >> 1)) : w.fifth, of_half);
     }
+    template <typename X>
+    static __device__ __forceinline__ float from_lds(const unsigned char* blk, const X& of_half, const LaneCtx& c) { return product(words(blk, c), of_half, c); }
     // In lane (n, g): dd = the block's two fp16 scales, sc / mn = the six-bit scales and minima of sub-blocks g (first
     // half of the block) and 4 + g (second half), q1 / q2 = piece g of each half of the nibbles, fifth = the fifth
     // bits of this lane's elements shifted down to bit 0 (Q5_K).
+    template <typename X>
     static __device__ __forceinline__ float math(unsigned dd, const float (&sc)[2], const float (&mn)[2], const u32x4& q1, const u32x4& q2,
-                                                 const u32x4& fifth, const LaneCtx& c, const Addr& ad, int b) {
+                                                 const u32x4& fifth, const X& of_half) {
         const float d = half_of(dd & 0xffffu), dmin = half_of(dd >> 16);
         float scaled[2], offset[2]; // sum of sc * q * x and of mn * x over a sub-block pair; the block's two scales come last
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const i32x4 alo = *reinterpret_cast<const i32x4*>(c.smem + operand_at(ad.lo_base, ad.lo_step, 256 * b + 128 * h));
-            const i32x4 ahi = *reinterpret_cast<const i32x4*>(c.smem + operand_at(ad.hi_base, ad.hi_step, 256 * b + 128 * h));
-            const XPair xp = c.pairs[8 * b + 4 * h + c.g];
+            const Digits x = of_half(h);
             const u32x4 qs = h ? q2 : q1;
             i32x4 lo, hi;
 #pragma unroll
@@ -217,10 +233,10 @@ struct MFK45 {
                 hi[i] = (int)u;
             }
             i32x4 acc = {0, 0, 0, 0};
-            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(alo, lo, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(ahi, hi, acc, 0, 0, 0);
-            scaled[h] = sc[h] * (digits_sum(acc) * xp.scale);
-            offset[h] = mn[h] * xp.sum;
+            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x.lo, lo, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x.hi, hi, acc, 0, 0, 0);
+            scaled[h] = sc[h] * (digits_sum(acc) * x.xp.scale);
+            offset[h] = mn[h] * x.xp.sum;
         }
         return d * (scaled[0] + scaled[1]) - dmin * (offset[0] + offset[1]);
     }
@@ -290,30 +306,55 @@ struct MF<kQ8_0> {
     static constexpr bool kRun = false;
     static constexpr int kAlign = 16;
     static __host__ __device__ constexpr int piece_off(int k) { return 16 * k; }
-    static __device__ __forceinline__ float from_lds(const unsigned char* blk, const LaneCtx& c, const Addr& ad, int b) {
+    struct Digits {
+        i32x4 a[2]; // of the runs
+        XPair xp;
+    };
+    static __device__ __forceinline__ Digits digits(const LaneCtx& c, const Addr& ad, int b, int h) {
+        return Digits{{*reinterpret_cast<const i32x4*>(c.smem + operand_at(ad.lo_base, ad.lo_step, 256 * b + 128 * h)),
+                       *reinterpret_cast<const i32x4*>(c.smem + operand_at(ad.hi_base, ad.hi_step, 256 * b + 128 * h))}, c.pairs[8 * b + 4 * h + c.g]};
+    }
+    struct HalfWords {
+        unsigned v[2][5]; // of the runs
+        uint16_t d;
+    };
+    struct Words {
+        HalfWords half[2];
+    };
+    static __device__ __forceinline__ HalfWords half_words(const unsigned char* blk, const LaneCtx& c, int h) {
+        const unsigned char* const mine = blk + 34 * (c.g >> 1) + 2 + 16 * (c.g & 1) - (c.g < 2 ? 2u : 0u); // (word aligned)
+        HalfWords w;
+        w.d = *reinterpret_cast<const uint16_t*>(blk + 34 * (4 * h + c.g));
+#pragma unroll
+        for (int run = 0; run < 2; ++run)
+#pragma unroll
+            for (int i = 0; i < 5; ++i) w.v[run][i] = reinterpret_cast<const unsigned*>(mine + 34 * (4 * h + 2 * run))[i];
+        return w;
+    }
+    static __device__ __forceinline__ Words words(const unsigned char* blk, const LaneCtx& c) { return Words{{half_words(blk, c, 0), half_words(blk, c, 1)}}; }
+    static __device__ __forceinline__ float half_product(const HalfWords& words, const Digits& x, const LaneCtx& c) {
         const unsigned shift = c.g < 2 ? 2u : 0u;
-        const unsigned char* const mine = blk + 34 * (c.g >> 1) + 2 + 16 * (c.g & 1) - shift; // (word aligned)
+        i32x4 w[2], acc = {0, 0, 0, 0};
+#pragma unroll
+        for (int run = 0; run < 2; ++run) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) w[run][i] = (int)__builtin_amdgcn_alignbyte(words.v[run][i + 1], words.v[run][i], shift);
+            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x.a[run], w[run], acc, 0, 0, 0);
+        }
+        return half_of(words.d) * (digits_sum(acc) * x.xp.scale);
+    }
+    // `of_half`(h): the digits of half h
+    template <typename X>
+    static __device__ __forceinline__ float product(const Words& w, const X& of_half, const LaneCtx& c) {
+        return half_product(w.half[0], of_half(0), c) + half_product(w.half[1], of_half(1), c);
+    }
+    template <typename X>
+    static __device__ __forceinline__ float from_lds(const unsigned char* blk, const X& of_half, const LaneCtx& c) {
         float out[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const i32x4 a0 = *reinterpret_cast<const i32x4*>(c.smem + operand_at(ad.lo_base, ad.lo_step, 256 * b + 128 * h));
-            const i32x4 a1 = *reinterpret_cast<const i32x4*>(c.smem + operand_at(ad.hi_base, ad.hi_step, 256 * b + 128 * h));
-            const XPair xp = c.pairs[8 * b + 4 * h + c.g];
-            const float d = half_of(*reinterpret_cast<const uint16_t*>(blk + 34 * (4 * h + c.g)));
-            i32x4 w[2];
-#pragma unroll
-            for (int run = 0; run < 2; ++run) {
-                const unsigned* const p = reinterpret_cast<const unsigned*>(mine + 34 * (4 * h + 2 * run));
-                unsigned v[5];
-#pragma unroll
-                for (int i = 0; i < 5; ++i) v[i] = p[i];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) w[run][i] = (int)__builtin_amdgcn_alignbyte(v[i + 1], v[i], shift);
-            }
-            i32x4 acc = {0, 0, 0, 0};
-            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, w[0], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, w[1], acc, 0, 0, 0);
-            out[h] = d * (digits_sum(acc) * xp.scale);
+            const Digits x = of_half(h);
+            out[h] = half_product(half_words(blk, c, h), x, c);
         }
         return out[0] + out[1];
     }
@@ -368,7 +409,7 @@ struct MF<kQ6_K> {
             }
         }
         const int sc[4] = {(int)(ss << 24) >> 24, (int)(ss << 16) >> 24, (int)(ss << 8) >> 24, (int)ss >> 24};
-        return math(sc, dd, ql, qh, c, ad, b);
+        return math(sc, dd, ql, qh, c, [&](int h) { return digits(c, ad, b, h); });
     }
     // A block laid out in LDS piece after piece (the kernel that reads rows in long runs): pieces 0 ... 12 are the
     // block's bytes 16 k ..., piece 13 its last 16 bytes (194 ... 209: the fp16 scale in its last two), so that no
@@ -377,30 +418,46 @@ struct MF<kQ6_K> {
     static constexpr bool kRun = false;
     static constexpr int kAlign = 2;
     static __host__ __device__ constexpr int piece_off(int k) { return k < 13 ? 16 * k : 194; }
-    static __device__ __forceinline__ float from_lds(const unsigned char* blk, const LaneCtx& c, const Addr& ad, int b) {
-        int sc[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) sc[k] = reinterpret_cast<const signed char*>(blk)[192 + 4 * k + c.g];
-        const unsigned dd = *reinterpret_cast<const unsigned*>(blk + 13 * 16 + 12) >> 16;
+    struct Words {
         u32x4 ql[2], qh[2];
+        int sc[4];
+        unsigned d;
+    };
+    static __device__ __forceinline__ Words words(const unsigned char* blk, const LaneCtx& c) {
+        Words w;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            ql[h] = *reinterpret_cast<const u32x4*>(blk + 64 * h + 16 * c.g);
-            qh[h] = *reinterpret_cast<const u32x4*>(blk + 128 + 32 * h + 16 * (c.g & 1));
+            w.ql[h] = *reinterpret_cast<const u32x4*>(blk + 64 * h + 16 * c.g);
+            w.qh[h] = *reinterpret_cast<const u32x4*>(blk + 128 + 32 * h + 16 * (c.g & 1));
         }
-        return math(sc, dd, ql, qh, c, ad, b);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) w.sc[k] = reinterpret_cast<const signed char*>(blk)[192 + 4 * k + c.g];
+        w.d = *reinterpret_cast<const unsigned*>(blk + 13 * 16 + 12) >> 16;
+        return w;
     }
+    struct Digits {
+        i32x4 lo, hi;
+        XPair xlo, xhi;
+    };
+    static __device__ __forceinline__ Digits digits(const LaneCtx& c, const Addr& ad, int b, int h) {
+        return Digits{*reinterpret_cast<const i32x4*>(c.smem + operand_at(ad.base, ad.step, 256 * b + 128 * h)),
+                      *reinterpret_cast<const i32x4*>(c.smem + operand_at(ad.base, ad.step, 256 * b + 128 * h + 64)),
+                      c.pairs[16 * b + 8 * h + c.g], c.pairs[16 * b + 8 * h + 4 + c.g]};
+    }
+    template <typename X>
+    static __device__ __forceinline__ float product(const Words& w, const X& of_half, const LaneCtx& c) { return math(w.sc, w.d, w.ql, w.qh, c, of_half); }
+    template <typename X>
+    static __device__ __forceinline__ float from_lds(const unsigned char* blk, const X& of_half, const LaneCtx& c) { return product(words(blk, c), of_half, c); }
     // In lane (n, g): sc = the scales g, 4 + g, 8 + g and 12 + g, dd = the block's fp16 scale, ql / qh = piece g of each half's low nibbles and the piece of high bit pairs that covers it.
+    template <typename X>
     static __device__ __forceinline__ float math(const int (&sc)[4], unsigned dd, const u32x4 (&ql)[2], const u32x4 (&qh)[2], const LaneCtx& c,
-                                                 const Addr& ad, int b) {
+                                                 const X& of_half) {
         const float d = half_of(dd & 0xffffu);
         const int s1 = 2 * (c.g >> 1);
         float out[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const i32x4 alo = *reinterpret_cast<const i32x4*>(c.smem + operand_at(ad.base, ad.step, 256 * b + 128 * h));
-            const i32x4 ahi = *reinterpret_cast<const i32x4*>(c.smem + operand_at(ad.base, ad.step, 256 * b + 128 * h + 64));
-            const XPair xlo = c.pairs[16 * b + 8 * h + c.g], xhi = c.pairs[16 * b + 8 * h + 4 + c.g];
+            const Digits x = of_half(h);
             i32x4 lo, hi;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -411,10 +468,10 @@ struct MF<kQ6_K> {
                 hi[i] = (int)low_nibbles_of(l >> 4, u);
             }
             const i32x4 zero = {0, 0, 0, 0};
-            const i32x4 acc_lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(alo, lo, zero, 0, 0, 0);
-            const i32x4 acc_hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(ahi, hi, zero, 0, 0, 0);
+            const i32x4 acc_lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(x.lo, lo, zero, 0, 0, 0);
+            const i32x4 acc_hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(x.hi, hi, zero, 0, 0, 0);
             const float sc_lo = (float)sc[2 * h], sc_hi = (float)sc[2 * h + 1];
-            out[h] = sc_lo * (digits_sum(acc_lo) * xlo.scale - 32.0f * xlo.sum) + sc_hi * (digits_sum(acc_hi) * xhi.scale - 32.0f * xhi.sum);
+            out[h] = sc_lo * (digits_sum(acc_lo) * x.xlo.scale - 32.0f * x.xlo.sum) + sc_hi * (digits_sum(acc_hi) * x.xhi.scale - 32.0f * x.xhi.sum);
         }
         return d * (out[0] + out[1]);
     }
@@ -434,7 +491,7 @@ struct MF<kQ6_KRun> : MF<kQ6_K> {
     static constexpr bool kRun = true;
     static constexpr int kAlign = 4, kRunBytes = 2 * kBlockBytes, kRunPieces = (kRunBytes + 15) / 16, kLastPiece = kRunBytes - 16;
     template <int J>
-    static __device__ __forceinline__ float from_run(const unsigned char* row, const LaneCtx& c, const Addr& ad, int b) {
+    static __device__ __forceinline__ Words run_words(const unsigned char* row, const LaneCtx& c) {
         constexpr int kShift = J * kBlockBytes % 16, kFloor = J * kBlockBytes - kShift;
         auto piece = [&](int off) {
             const u32x4 v = *reinterpret_cast<const u32x4*>(row + kFloor + off);
@@ -446,12 +503,11 @@ struct MF<kQ6_KRun> : MF<kQ6_K> {
                              __builtin_amdgcn_alignbyte(v[3], v[2], kShift), __builtin_amdgcn_alignbyte(behind, v[3], kShift)};
             }
         };
-        u32x4 ql[2], qh[2];
-        int sc[4];
+        Words w;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            ql[h] = piece(64 * h + 16 * c.g);
-            qh[h] = piece(128 + 32 * h + 16 * (c.g & 1));
+            w.ql[h] = piece(64 * h + 16 * c.g);
+            w.qh[h] = piece(128 + 32 * h + 16 * (c.g & 1));
         }
         // (what lies behind the run's last whole piece is in the last one, further on by as much as that overlaps)
         constexpr int kWhole = kRunBytes / 16 * 16, kOn = kWhole - kLastPiece;
@@ -459,10 +515,10 @@ struct MF<kQ6_KRun> : MF<kQ6_K> {
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             static_assert(kBlockBytes + 192 + 4 * 2 + 3 < kWhole && kBlockBytes + 192 + 4 * 3 + 1 < kWhole && kBlockBytes + 192 + 4 * 3 + 2 >= kWhole, "scales 14 and 15 of block 1");
-            sc[k] = reinterpret_cast<const signed char*>(row)[J * kBlockBytes + 192 + 4 * k + c.g + (k == 3 ? lane_on : 0)];
+            w.sc[k] = reinterpret_cast<const signed char*>(row)[J * kBlockBytes + 192 + 4 * k + c.g + (k == 3 ? lane_on : 0)];
         }
-        const unsigned dd = *reinterpret_cast<const uint16_t*>(row + J * kBlockBytes + 208 + (J == 1 ? kOn : 0));
-        return math(sc, dd, ql, qh, c, ad, b);
+        w.d = *reinterpret_cast<const uint16_t*>(row + J * kBlockBytes + 208 + (J == 1 ? kOn : 0));
+        return w;
     }
 };
 
