@@ -284,7 +284,13 @@ __device__ __forceinline__ int rows_seg(const RowsHead& h, int wg) {
 //                   two: one that fills the chip with work runs longer this way (Llama-3-8B's gate/up by 1 us), its second
 //                   round of requests getting in the way of the first.
 //   kRowsAny        anything: the digits come behind the wave's first two items.
-enum : int { kRowsAny = 0, kRowsOnePass = 1, kRowsTwoPasses = 2, kRowsOneItem = 3 };
+//   kRowsOneItemNorm  one item, with a norm, and at most one workgroup of up to four waves a CU: the norm's factor (two divisions and a
+//                   root, about 60 instructions, in the wave that finishes the rows) is made behind a barrier of its own while
+//                   the weights are on their way.  In the other modes it stands between the first tile's last product and its
+//                   store, once a workgroup.  128 workgroups of 6 blocks in Q4_K 3.11 -> 3.04 us, in Q6_K 3.56 -> 3.44, in Q8_0 3.68 -> 3.52,
+//                   256 of them 3.26 -> 3.18, 3.79 -> 3.67, 3.95 -> 3.81; but 384 3.93 -> 4.00, 4.56 -> 4.66, 4.93 -> 5.09, and with eight
+//                   waves 224 workgroups 4.2 -> 4.35: there the vector ALU has other waves' work to do meanwhile.
+enum : int { kRowsAny = 0, kRowsOnePass = 1, kRowsTwoPasses = 2, kRowsOneItem = 3, kRowsOneItemNorm = 4 };
 
 template <int T, bool DUAL, int kWaves, int CB, int kMode>
 __device__ __forceinline__ void gemv_rows_body(const RowsHead h, const GemvArgs& a) {
@@ -314,10 +320,11 @@ __device__ __forceinline__ void gemv_rows_body(const RowsHead h, const GemvArgs&
     const int n_chunks = (int)((unsigned)(nb + CB - 1) / CB);
     const int my_chunks = (int)((unsigned)(n_chunks + kWaves - 1 - wave) / kWaves);
     const int total = n_mine * my_chunks;
-    const bool has_norm = h.norm_w != nullptr;
+    const bool has_norm = kMode == kRowsOneItemNorm || h.norm_w != nullptr;
     float* const wave_ss = red + 2 * kMaxWaves * 2 * 16;
     if (kMode != kRowsAny && total == 0) { // (fewer chunks than waves: this wave only leaves its zeros and keeps the barriers' count)
         if (lane == 0) wave_ss[wave] = 0.0f;
+        if (kMode == kRowsOneItemNorm) lds_barrier();
         for (int t = 0; t < n_mine; ++t) {
             if (lane < 16) red[(t & 1) * (kMaxWaves * 2 * 16) + wave * 16 + lane] = 0.0f;
             lds_barrier();
@@ -354,7 +361,7 @@ __device__ __forceinline__ void gemv_rows_body(const RowsHead h, const GemvArgs&
     int rq_tile = seg_wg, rq_c = wave;
     size_t rq_off = (size_t)((unsigned)seg_wg * (unsigned)kTileOut) * row_bytes + (size_t)((unsigned)(b0 + wave * CB) * (unsigned)F::kBlockBytes);
     const size_t next_tile = (size_t)((unsigned)grid_x * (unsigned)kTileOut) * row_bytes - (size_t)((unsigned)(my_chunks * (kWaves * CB)) * (unsigned)F::kBlockBytes);
-    constexpr int kRing = kMode == kRowsOneItem ? 1 : 2; // items on their way or in use
+    constexpr int kRing = kMode == kRowsOneItem || kMode == kRowsOneItemNorm ? 1 : 2; // items on their way or in use
     u32x4 buf[kRing][NL];
     float bias_v[kRing];
     auto request = [&](u32x4 (&r)[NL], bool real = true) {
@@ -508,13 +515,23 @@ __device__ __forceinline__ void gemv_rows_body(const RowsHead h, const GemvArgs&
             }
         }
     }
+    float rinv = 0.0f;
+    auto norm_factor = [&] {
+        float ss = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) ss += wave_ss[w];
+        rinv = 1.0f / sqrtf(ss / (float)n_in + norm_eps);
+    };
     if (has_norm) {
         ss = wave_sum(ss);
         if (lane == 0) wave_ss[wave] = ss;
+        if constexpr (kMode == kRowsOneItemNorm) {
+            lds_barrier();
+            if (wave == 0) norm_factor();
+        }
     }
     ROWS_STAMP(2);
     [[maybe_unused]] int n_consumed = 0;
-    const float norm_n = (float)n_in;
     int set = 0;
     auto tile_end = [&](int tile, float rowacc, float bias) {
         float* const mine = red + set * (kMaxWaves * 2 * 16);
@@ -527,10 +544,8 @@ __device__ __forceinline__ void gemv_rows_body(const RowsHead h, const GemvArgs&
 #pragma unroll
             for (int w = 0; w < kWaves; ++w) y += mine[w * 16 + threadIdx.x];
             if (has_norm) { // (every wave has left its sum of squares before its first barrier here)
-                float ss = 0.0f;
-#pragma unroll
-                for (int w = 0; w < kWaves; ++w) ss += wave_ss[w];
-                y *= 1.0f / sqrtf(ss / norm_n + norm_eps);
+                if (kMode != kRowsOneItemNorm && tile == seg_wg) norm_factor();
+                y *= rinv;
             }
             if constexpr (DUAL) { // SiLU(gate) * up: rows 0-7 and 8-15
                 const float up = dpp_row_ror8(y);
@@ -567,7 +582,7 @@ __device__ __forceinline__ void gemv_rows_body(const RowsHead h, const GemvArgs&
         const int cb = min(CB, nb - cs_c * CB);
         float v;
         // (unrolled over CB with a test per block, not a loop over cb: every LDS offset is a constant of its instruction)
-        if constexpr (kMode == kRowsOneItem && kWaves < 8) {
+        if constexpr (kRing == 1 && kWaves < 8) {
             // What the products take from the activation is fetched while the weights are on their way, and all of an item's
             // weights are asked of LDS at once: one trip to LDS between their arrival and the products, not one for every
             // few operands.  Per launch, before -> now: Qwen2.5-1.5B's q, k, v (v in Q6_K) 3.62 -> 3.50 us, gate/up in Q4_K 5.95 -> 5.87,
@@ -720,6 +735,8 @@ int rows_tiles(const GemvArgs& a) {
 
 int g_rows_resident = 768; // workgroups of four waves the chip holds at once (three a CU; set by the launcher)
 
+bool rows_norm_first(const GemvArgs& a, int wgs) { return a.norm_w && wgs * 3 <= g_rows_resident; } // (kRowsOneItemNorm)
+
 template <int T, bool DUAL, int kWaves, int CB>
 bool launch_rows_as(const GemvArgs& a, int wgs, int shares, hipStream_t stream) {
     constexpr int kUnit = RowsGeom<T, CB>::kUnit;
@@ -734,6 +751,12 @@ bool launch_rows_as(const GemvArgs& a, int wgs, int shares, hipStream_t stream) 
         hipLaunchKernelGGL((gemv_rows_kernel<T, DUAL, kWaves, CB, decltype(mode)::value>), grid, dim3(kWaves * 64), lds, stream, ROWS_HEAD_OF(h), a);
     };
     if (per_wave == 1 && wgs == rows_tiles(a)) {
+        if constexpr (kWaves == 4) {
+            if (rows_norm_first(a, wgs)) {
+                go(std::integral_constant<int, kRowsOneItemNorm>());
+                return true;
+            }
+        }
         go(std::integral_constant<int, kRowsOneItem>());
         return true;
     }
@@ -788,7 +811,16 @@ bool launch_rows_one_item(const GemvArgs& a, int wgs, hipStream_t stream) {
     const size_t lds = RowsGeom<T, 2>::lds_bytes(a.n_in, kWaves);
     RowsHead h;
     if (lds > 64u * 1024u || !rows_head(a, wgs, 1, RowsGeom<T, 2>::kUnit, h)) return false;
-    hipLaunchKernelGGL((gemv_rows_kernel<T, DUAL, kWaves, 2, kRowsOneItem>), dim3(h.shape >> 18), dim3(kWaves * 64), lds, stream, ROWS_HEAD_OF(h), a);
+    auto go = [&](auto mode) {
+        hipLaunchKernelGGL((gemv_rows_kernel<T, DUAL, kWaves, 2, decltype(mode)::value>), dim3(h.shape >> 18), dim3(kWaves * 64), lds, stream, ROWS_HEAD_OF(h), a);
+    };
+    if constexpr (T == kQ8_0 && kWaves == 3) { // (the others here are launches of several workgroups a CU)
+        if (rows_norm_first(a, wgs)) {
+            go(std::integral_constant<int, kRowsOneItemNorm>());
+            return true;
+        }
+    }
+    go(std::integral_constant<int, kRowsOneItem>());
     return true;
 }
 
@@ -907,12 +939,16 @@ hipError_t allow_rows() {
     if ((e = allow_lds(reinterpret_cast<const void*>(&gemv_rows_kernel<T, DUAL, kWaves, CB, kRowsOnePass>))) != hipSuccess) return e;
     if ((e = allow_lds(reinterpret_cast<const void*>(&gemv_rows_kernel<T, DUAL, kWaves, CB, kRowsTwoPasses>))) != hipSuccess) return e;
     if ((e = allow_lds(reinterpret_cast<const void*>(&gemv_rows_kernel<T, DUAL, kWaves, CB, kRowsOneItem>))) != hipSuccess) return e;
+    if constexpr (kWaves == 4)
+        if ((e = allow_lds(reinterpret_cast<const void*>(&gemv_rows_kernel<T, DUAL, kWaves, CB, kRowsOneItemNorm>))) != hipSuccess) return e;
     return allow_lds(reinterpret_cast<const void*>(&gemv_rows_kernel<T, DUAL, kWaves, CB, kRowsAny>));
 }
 
 template <int kWaves, int CB>
 hipError_t allow_mixed() {
-    const hipError_t e = allow_lds(reinterpret_cast<const void*>(&gemv_rows_mixed_kernel<kWaves, CB, kRowsOneItem>));
+    hipError_t e = allow_lds(reinterpret_cast<const void*>(&gemv_rows_mixed_kernel<kWaves, CB, kRowsOneItem>));
+    if constexpr (kWaves == 4)
+        if (e == hipSuccess) e = allow_lds(reinterpret_cast<const void*>(&gemv_rows_mixed_kernel<kWaves, CB, kRowsOneItemNorm>));
     return e != hipSuccess ? e : allow_lds(reinterpret_cast<const void*>(&gemv_rows_mixed_kernel<kWaves, CB, kRowsAny>));
 }
 
@@ -964,6 +1000,12 @@ hipError_t gemv_mfma_mixed_launch(GemvArgs a, int cu_count, hipStream_t stream) 
                 const size_t lds = RowsGeom<kQ6_K, CB>::lds_bytes(a.n_in, W);
                 if (lds > kMfmaLdsMax) return false;
                 const dim3 gr(h.shape >> 18), block(W * 64);
+                if constexpr (W == 4) {
+                    if (nb <= W * CB && wgs == tiles && rows_norm_first(a, wgs)) {
+                        hipLaunchKernelGGL((gemv_rows_mixed_kernel<W, CB, kRowsOneItemNorm>), gr, block, lds, stream, ROWS_HEAD_OF(h), a);
+                        return true;
+                    }
+                }
                 if (nb <= W * CB && wgs == tiles) hipLaunchKernelGGL((gemv_rows_mixed_kernel<W, CB, kRowsOneItem>), gr, block, lds, stream, ROWS_HEAD_OF(h), a);
                 else hipLaunchKernelGGL((gemv_rows_mixed_kernel<W, CB, kRowsAny>), gr, block, lds, stream, ROWS_HEAD_OF(h), a);
                 return true;
