@@ -92,12 +92,12 @@ __device__ __forceinline__ unsigned from_lane(int src_lane4, unsigned v) {
 __device__ __forceinline__ float digits_sum(const i32x4& acc) {
     return (float)(acc[0] * 256 + acc[1]) * 256.0f + (float)acc[2];
 }
-// Every byte's low nibble from a, its high nibble from b, in one instruction (spelled out, since the compiler, which
-// knows which bits of b can be set, narrows the mask and then needs an AND and an AND-OR).
+// Every byte's low nibble from a, its high nibble from b, in one instruction (as a three-input operation: of AND and OR the
+// compiler, which knows which bits of b can be set, narrows the mask and then needs two).  Not as inline assembly: what
+// it writes goes straight into a matrix instruction, which needs two instructions between (the compiler's business, and it does
+// not see into assembly).
 __device__ __forceinline__ unsigned low_nibbles_of(unsigned a, unsigned b) {
-    unsigned r;
-    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(r) : "v"(0x0f0f0f0fu), "v"(a), "v"(b));
-    return r;
+    return __builtin_amdgcn_bitop3_b32(0x0f0f0f0fu, a, b, 0xca); // first ? second : third
 }
 // LDS byte offset of a lane's A operand: base + x for a lane that holds digits (step 1), base (the zero bytes) for
 // one whose rows are zero (step 0); x is the same in every lane.  One 24-bit multiply-add.
