@@ -308,17 +308,21 @@ __device__ __forceinline__ void gemv_rows_body(const RowsHead h, const GemvArgs&
     if (seg == 1) w_mine = h.w1, turns = h.turns1, next = h.turns2;
     if (seg == 2) w_mine = h.w2, turns = h.turns2, next = ~0u;
     const int seg_wg = (int)blockIdx.x - (int)(turns >> 19), grid_x = (int)min(next >> 19, h.shape >> 18) - (int)(turns >> 19); // among the matrix's workgroups
-    const int nb_row = (int)(h.shape & 0x7fu) + 1, share_blocks = (int)((h.shape >> 7) & 0x7fu) + 1, share_extra = (int)((h.shape >> 14) & 15u);
-    const int n_mine = (int)(turns & 63u) + (seg_wg < (int)((turns >> 6) & 0x1fffu) ? 1 : 0); // tiles of this workgroup, one at least
-    const int b0 = (int)blockIdx.z * share_blocks + min((int)blockIdx.z, share_extra) * G::kUnit;
-    const int nb = share_blocks + ((int)blockIdx.z < share_extra ? G::kUnit : 0);
+    // (what a mode says of the launch is a constant here: the way to the first request is scalar instructions, 2 ns each)
+    constexpr bool kOneItem = kMode == kRowsOneItem || kMode == kRowsOneItemNorm, kWholeRows = DUAL || kMode == kRowsOneItemNorm;
+    constexpr bool kStraight = kOneItem && kWaves < 8;
+    const int nb_row = (int)(h.shape & 0x7fu) + 1, share_blocks = kWholeRows ? nb_row : (int)((h.shape >> 7) & 0x7fu) + 1;
+    const int share_extra = kWholeRows ? 0 : (int)((h.shape >> 14) & 15u), share = kWholeRows ? 0 : (int)blockIdx.z;
+    const int n_mine = kStraight ? 1 : (int)(turns & 63u) + (seg_wg < (int)((turns >> 6) & 0x1fffu) ? 1 : 0); // tiles of this workgroup, one at least
+    const int b0 = share * share_blocks + min(share, share_extra) * G::kUnit;
+    const int nb = share_blocks + (share < share_extra ? G::kUnit : 0);
     const int n_in = nb << 8;
     const unsigned row_bytes = (unsigned)nb_row * F::kBlockBytes;
     float* const red = reinterpret_cast<float*>(smem + L::red_off(n_in));
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); // (scalar: what follows from it stays in scalar registers)
     unsigned char* const transit = smem + L::red_off(n_in) + kRowsRedBytes + wave * G::kWaveBytes;
     const int n_chunks = (int)((unsigned)(nb + CB - 1) / CB);
-    const int my_chunks = (int)((unsigned)(n_chunks + kWaves - 1 - wave) / kWaves);
+    const int my_chunks = kStraight ? (wave < n_chunks ? 1 : 0) : (int)((unsigned)(n_chunks + kWaves - 1 - wave) / kWaves);
     const int total = n_mine * my_chunks;
     const bool has_norm = kMode == kRowsOneItemNorm || h.norm_w != nullptr;
     float* const wave_ss = red + 2 * kMaxWaves * 2 * 16;
@@ -361,7 +365,7 @@ __device__ __forceinline__ void gemv_rows_body(const RowsHead h, const GemvArgs&
     int rq_tile = seg_wg, rq_c = wave;
     size_t rq_off = (size_t)((unsigned)seg_wg * (unsigned)kTileOut) * row_bytes + (size_t)((unsigned)(b0 + wave * CB) * (unsigned)F::kBlockBytes);
     const size_t next_tile = (size_t)((unsigned)grid_x * (unsigned)kTileOut) * row_bytes - (size_t)((unsigned)(my_chunks * (kWaves * CB)) * (unsigned)F::kBlockBytes);
-    constexpr int kRing = kMode == kRowsOneItem || kMode == kRowsOneItemNorm ? 1 : 2; // items on their way or in use
+    constexpr int kRing = kOneItem ? 1 : 2; // items on their way or in use
     u32x4 buf[kRing][NL];
     float bias_v[kRing];
     auto request = [&](u32x4 (&r)[NL], bool real = true) {
@@ -550,7 +554,7 @@ __device__ __forceinline__ void gemv_rows_body(const RowsHead h, const GemvArgs&
             if constexpr (DUAL) { // SiLU(gate) * up: rows 0-7 and 8-15
                 const float up = dpp_row_ror8(y);
                 y = y / (1.0f + expf(-y)) * up;
-            } else if (seg_bias && blockIdx.z == 0) {
+            } else if (seg_bias && share == 0) {
                 y += bias;
             }
             const int r = tile * kTileOut + (int)threadIdx.x;
@@ -582,7 +586,7 @@ __device__ __forceinline__ void gemv_rows_body(const RowsHead h, const GemvArgs&
         const int cb = min(CB, nb - cs_c * CB);
         float v;
         // (unrolled over CB with a test per block, not a loop over cb: every LDS offset is a constant of its instruction)
-        if constexpr (kRing == 1 && kWaves < 8) {
+        if constexpr (kStraight) {
             // What the products take from the activation is fetched while the weights are on their way, and all of an item's
             // weights are asked of LDS at once: one trip to LDS between their arrival and the products, not one for every
             // few operands.  Per launch, before -> now: Qwen2.5-1.5B's q, k, v (v in Q6_K) 3.62 -> 3.50 us, gate/up in Q4_K 5.95 -> 5.87,
@@ -618,7 +622,7 @@ __device__ __forceinline__ void gemv_rows_body(const RowsHead h, const GemvArgs&
         }
         rowacc += v;
         cs_c += kWaves;
-        if (cs_c >= n_chunks) {
+        if (kStraight || cs_c >= n_chunks) {
             tile_end(cs_tile, rowacc, bias);
             cs_c = wave;
             cs_tile += grid_x;
