@@ -308,9 +308,10 @@ __device__ __forceinline__ void gemv_rows_body(const RowsHead h, const GemvArgs&
     if (seg == 1) w_mine = h.w1, turns = h.turns1, next = h.turns2;
     if (seg == 2) w_mine = h.w2, turns = h.turns2, next = ~0u;
     const int seg_wg = (int)blockIdx.x - (int)(turns >> 19), grid_x = (int)min(next >> 19, h.shape >> 18) - (int)(turns >> 19); // among the matrix's workgroups
-    // (what a mode says of the launch is a constant here: the way to the first request is scalar instructions, 2 ns each)
+    // (what a mode says of the launch is a constant here: the way to the first request is scalar instructions, 2 ns each.  Of eight waves
+    // only for Q6_K in runs, 14 blocks a row, 224 tiles 5.13 -> 4.88 us; Q4_K was slower for it, 4.2 -> 4.4.)
     constexpr bool kOneItem = kMode == kRowsOneItem || kMode == kRowsOneItemNorm, kWholeRows = DUAL || kMode == kRowsOneItemNorm;
-    constexpr bool kStraight = kOneItem && kWaves < 8;
+    constexpr bool kAhead = kOneItem && kWaves < 8, kStraight = kOneItem && (kWaves < 8 || F::kRun);
     const int nb_row = (int)(h.shape & 0x7fu) + 1, share_blocks = kWholeRows ? nb_row : (int)((h.shape >> 7) & 0x7fu) + 1;
     const int share_extra = kWholeRows ? 0 : (int)((h.shape >> 14) & 15u), share = kWholeRows ? 0 : (int)blockIdx.z;
     const int n_mine = kStraight ? 1 : (int)(turns & 63u) + (seg_wg < (int)((turns >> 6) & 0x1fffu) ? 1 : 0); // tiles of this workgroup, one at least
@@ -586,7 +587,7 @@ __device__ __forceinline__ void gemv_rows_body(const RowsHead h, const GemvArgs&
         const int cb = min(CB, nb - cs_c * CB);
         float v;
         // (unrolled over CB with a test per block, not a loop over cb: every LDS offset is a constant of its instruction)
-        if constexpr (kStraight) {
+        if constexpr (kAhead) {
             // What the products take from the activation is fetched while the weights are on their way, and all of an item's
             // weights are asked of LDS at once: one trip to LDS between their arrival and the products, not one for every
             // few operands.  Per launch, before -> now: Qwen2.5-1.5B's q, k, v (v in Q6_K) 3.62 -> 3.50 us, gate/up in Q4_K 5.95 -> 5.87,
