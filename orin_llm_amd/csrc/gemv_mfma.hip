@@ -849,7 +849,14 @@ bool launch_rows(const GemvArgs& a, int wgs, int shares, bool wide, int nb_wg, h
         // One matrix in many turns: two-block items, where a run of one block begins and ends inside a line that the next wave's fetches again
         // (logits of Llama-3-8B 92.7 -> 87.8 us, 6.4 TB/s, of Qwen2.5-7B 99.6 -> 93.2).  With fewer turns the longer last item costs more (even
         // at five, 4 % slower at four, 7 at three, 28 at one and a third), and so does a wave without an item (8 blocks a row: 47.5 -> 52.4).
-        if (!a.w_up && nb_wg >= 14 && rows_tiles(a) >= 8 * wgs) return launch_rows_as<T, false, 4, 2>(a, wgs, shares, stream);
+        // From 19 blocks on two workgroups fit a CU instead of three, and it is faster still (152064 rows, one block -> two: of 20 blocks
+        // 141 -> 133, 32 214 -> 197, 72 484 -> 445); up to where the buffers and the digits fit LDS, where one-block items take over (80
+        // blocks 517 us; the kernel that does not read in runs 731).  Items that four waves share within 30 %, so not nine of them: 18 blocks
+        // 107 -> 117 us with 128256 rows, 127 -> 134 with 152064 (but 215 -> 200 with 256000); 17 blocks the same or 2 % faster.
+        if (!a.w_up && nb_wg >= 14 && rows_tiles(a) >= 8 * wgs) {
+            const int items = (nb_wg + 1) / 2, most = (items + 3) / 4; // of a tile, of a wave
+            if (most * 40 <= items * 13 && RowsGeom<T, 2>::lds_bytes(nb_wg * 256, 4) <= kMfmaLdsMax) return launch_rows_as<T, false, 4, 2>(a, wgs, shares, stream);
+        }
         return a.w_up ? launch_rows_as<T, true, 4, 1>(a, wgs, shares, stream) : launch_rows_as<T, false, 4, 1>(a, wgs, shares, stream);
     }
     else { // (the other branch returned)
