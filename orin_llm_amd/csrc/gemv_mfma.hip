@@ -851,12 +851,13 @@ bool launch_rows(const GemvArgs& a, int wgs, int shares, bool wide, int nb_wg, h
         // at five, 4 % slower at four, 7 at three, 28 at one and a third), and so does a wave without an item (8 blocks a row: 47.5 -> 52.4).
         // From 19 blocks on two workgroups fit a CU instead of three, and it is faster still (152064 rows, one block -> two: of 20 blocks
         // 141 -> 133, 32 214 -> 197, 72 484 -> 445); up to where the buffers and the digits fit LDS, where one-block items take over (80
-        // blocks 517 us; the kernel that does not read in runs 731).  Items that four waves share within 30 %, so not nine of them: 18 blocks
-        // 107 -> 117 us with 128256 rows, 127 -> 134 with 152064 (but 215 -> 200 with 256000); 17 blocks the same or 2 % faster.
-        if (!a.w_up && nb_wg >= 14 && rows_tiles(a) >= 8 * wgs) {
-            const int items = (nb_wg + 1) / 2, most = (items + 3) / 4; // of a tile, of a wave
-            if (most * 40 <= items * 13 && RowsGeom<T, 2>::lds_bytes(nb_wg * 256, 4) <= kMfmaLdsMax) return launch_rows_as<T, false, 4, 2>(a, wgs, shares, stream);
-        }
+        // blocks 517 us; the kernel that does not read in runs 731).  18 blocks, nine items for four waves, lose where some workgroups
+        // have a turn more than others and there are few turns (of 768 workgroups, 8 1/2 turns 87.4 -> 96.7 us, 10 1/2 108 -> 116, 12 1/2
+        // 129 -> 133; but 10 whole ones 103 -> 97, 14 1/2 150 -> 142, 21 208 -> 198); 17 blocks, whose ninth item is half as long, do not.
+        const int turns = rows_tiles(a) / wgs;
+        const bool uneven = nb_wg == 18 && turns < 13 && rows_tiles(a) % wgs != 0;
+        if (!a.w_up && nb_wg >= 14 && turns >= 8 && !uneven && RowsGeom<T, 2>::lds_bytes(nb_wg * 256, 4) <= kMfmaLdsMax)
+            return launch_rows_as<T, false, 4, 2>(a, wgs, shares, stream);
         return a.w_up ? launch_rows_as<T, true, 4, 1>(a, wgs, shares, stream) : launch_rows_as<T, false, 4, 1>(a, wgs, shares, stream);
     }
     else { // (the other branch returned)

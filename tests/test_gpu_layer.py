@@ -779,8 +779,8 @@ def test_q6_k_rows_in_runs_of_two_blocks(ly, n_in, offset):
 @pytest.mark.parametrize("n_in", [3328, 3584, 4096] + [256 * b for b in (18, 19, 72, 73)])
 def test_q8_0_matrices_of_many_turns(ly, n_in):
     """From eight row tiles a workgroup on (at three workgroups on each of 256 CUs), rows of fourteen blocks of 256 elements and
-    more go two blocks at a time, where they divide over four waves and their buffers fit: either side of the lines, and a last
-    turn that few workgroups have."""
+    more go two blocks at a time, up to 72 whose buffers fit, of 18 in whole turns: either side of the lines, and a last turn that
+    few workgroups have."""
     import torch
 
     base_rows, rs = 512, lm.Stream(8020 + n_in)
