@@ -200,7 +200,9 @@ def _decode_layer_calls(o, ka, hp, L, bufs, kc, vc, d_pos, n_ctx):
     rope_ind(k, nkv, hd, hp["n_rot"], hp["rope_theta"], d_pos, hp.get("freq_factors_dev"))
     ka.kv_store_ind(kc, vc, k, v, nkv, hd, n_ctx, d_pos)
     ka.flash_attention_decode_ind(q, kc, vc, attn, nh, nkv, hd, n_ctx, d_pos, scale)
-    quantize_activation(attn, ne)  # (as the reference: n_embd elements staged, the product reads the first n_head * head_dim)
+    # (the reference stages n_embd elements, of which the product reads the first n_head * head_dim; where those are more, as with
+    # heads wider than the model, it multiplies by whatever an earlier call left behind them: here they are staged)
+    quantize_activation(attn, max(ne, nh * hd))
     gemv_q8_add(L["wo"][0], L["wo"][1], x, nh * hd, ne)
     rms_norm(x, L["ffn_norm"], ne, eps, xn2)
     quantize_activation(xn2, ne)

@@ -1,7 +1,8 @@
 """orin_decode_layer at the benchmark's model shapes, against the CPU oracle's operators in the reference's order
 (src/model_gpu.cu:251-293): one Llama-3-8B-shaped layer at cache length 8192, one Qwen2.5-1.5B-shaped and one
-Qwen2.5-7B-shaped layer (with q/k/v biases; seven query heads per KV head in the latter) at 32768, and one
-Llama-3.2-1B-shaped layer (head_dim 64, rotary frequencies divided by per-pair factors) at 8192, weights in the mix
+Qwen2.5-7B-shaped layer (with q/k/v biases; seven query heads per KV head in the latter) at 32768, one
+Llama-3.2-1B-shaped layer (head_dim 64, rotary frequencies divided by per-pair factors) at 8192, and one
+Qwen3-0.6B-shaped layer (heads wider than the model, per-head norms) at 3000 of 4096, weights in the mix
 of a Q4_K_M file (Q4_K; attn_v and ffn_down Q6_K).  These are the shapes
 at which the layer's launches take the forms the small whole-model fixtures never reach: q, k, v of two types in one
 launch with eight waves a workgroup, accumulating projections whose rows are shared among workgroups, the kernel for
@@ -35,6 +36,9 @@ MODELS = {
                    eps=1.0e-6),
     "llama1b": dict(n_embd=2048, n_head=32, n_kv=8, head_dim=64, n_ff=8192, n_ctx=8192, L=8192, bias=False, neox=0, theta=5.0e5,
                     eps=1.0e-5, freq_factors=True),
+    # (heads wider than the model: rows of wo are twice n_embd; per-head norms of q and k)
+    "qwen3": dict(n_embd=1024, n_head=16, n_kv=8, head_dim=128, n_ff=3072, n_ctx=4096, L=3000, bias=False, neox=1, theta=1.0e6,
+                  eps=1.0e-6, qk_norm=True),
 }
 TYPES = dict(wq=lm.Q4_K, wk=lm.Q4_K, wv=lm.Q6_K, wo=lm.Q4_K, ffn_gate=lm.Q4_K, ffn_up=lm.Q4_K, ffn_down=lm.Q6_K)
 
@@ -49,6 +53,8 @@ def make_layer(name):
     L["ffn_norm"] = (1.0 + rs.sym(ne, 0.2)).astype(np.float32)
     if c["bias"]:
         L["bq"], L["bk"], L["bv"] = rs.sym(nq, 0.3), rs.sym(nkv, 0.3), rs.sym(nkv, 0.3)
+    if c.get("qk_norm"):
+        L["q_norm"], L["k_norm"] = ((1.0 + rs.sym(c["head_dim"], 0.2)).astype(np.float32) for _ in range(2))
     if c.get("freq_factors"):   # (the long-context scaling of the Llama-3 family: low frequencies slowed down)
         L["freq_factors"] = np.linspace(1.0, 8.0, c["head_dim"] // 2).astype(np.float32)
     x0 = rs.sym(ne, 1.0)
@@ -66,6 +72,9 @@ def oracle_layer(c, L, dims, x0, kc, vc):
     q, k, v = mv("wq", xn), mv("wk", xn), mv("wv", xn)
     if c["bias"]:
         q, k, v = q + L["bq"], k + L["bk"], v + L["bv"]
+    if c.get("qk_norm"):
+        q = np.stack([ref.rms_norm(row, L["q_norm"], c["eps"]) for row in q.reshape(H, d)])
+        k = np.stack([ref.rms_norm(row, L["k_norm"], c["eps"]) for row in k.reshape(G, d)])
     q = ref.rope_batch(q.reshape(H, d), d, d, c["theta"], pos, H, L.get("freq_factors"), bool(c["neox"]))
     k = ref.rope_batch(k.reshape(G, d), d, d, c["theta"], pos, G, L.get("freq_factors"), bool(c["neox"]))
     kc, vc = kc.copy(), vc.copy()
