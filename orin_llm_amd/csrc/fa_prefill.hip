@@ -1374,7 +1374,9 @@ constexpr int kMaxPrefillSplitShift = 4; // up to 16 workgroups share a token ti
 //   32 columns   5.3 us and 0.5 a step (bound by the 64 bytes a clock of the CU's vector memory path); more where so few
 //                workgroups walk that each waits for its own trips to memory, and on walks that leave the L2
 //   64 columns   6.9 and 0.7, 0.85 where the whole chip multiplies (clock, L2)
-//   short walk   4.0 and 0.8 (no tile asked for ahead of the last one's use)
+//   short walk   4.0 and 0.8; 0.25 more a step behind the second (nothing is asked for ahead of the last tile's use: measured to 1300
+//                rows, behind 256 of them it keeps up with the 32 columns while the caches have the rows, and does not where
+//                they come from memory: 100 tokens of Qwen2.5-1.5B at 420 6.9 us for 7.2, but 8.7 for 7.7)
 //   KV splits    2.2 for the second launch and 0.65 for every MB of partial results
 // head_dim 64 has half the bytes a row and two workgroups a CU.
 template <int D>
@@ -1384,7 +1386,11 @@ float prefill_estimate(int cols, bool short_walk, int shift, long long wgs, int 
         base = 5.3f;
         step = (wgs * 6 >= cus ? 0.5f : 0.56f) * (1.0f + fminf(fmaxf((float)(rows - 4000) / 8000.0f, 0.0f), 0.4f));
     }
-    if (short_walk) base = 4.0f, step = 0.8f;
+    if (short_walk) {
+        base = 4.0f, step = 0.8f;
+        // (not half of a head of 64, whose tiles are half as long on their way)
+        if (D == 128 && wgs * 10 >= cus) base += 0.25f * fmaxf((float)rows / 128.0f - 2.0f, 0.0f);
+    }
     long long turns = (wgs + cus - 1) / cus;
     if (D == 64) {
         base -= short_walk ? 0.6f : cols == 32 ? 1.1f : 1.5f;

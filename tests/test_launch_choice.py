@@ -21,3 +21,43 @@ def test_q8_0_matrices_of_many_turns(blocks, item, n_out):
     it.  Of 18 blocks two-block items where the turns are whole (98304 rows on 256 CUs) or many (256000)."""
     want = item or (2 if n_out in (98304, 256000) else 1)
     assert rows_form(recorder().calls("orin_gemv", Q8_0, ptr(1), ptr(2), ptr(3), blocks * 256, n_out)) == (4, want)
+
+
+HEADS = {  # query heads, KV heads, head size
+    "qwen1.5b": (12, 2, 128), "qwen7b": (28, 4, 128), "llama8b": (32, 8, 128), "llama1b": (32, 8, 64), "qwen3": (16, 8, 128),
+}
+
+
+def prefill_form(model, past, tokens):
+    """"short", or the query columns of a workgroup, with the number of KV splits where there are any: "64x4"."""
+    h, g, d = HEADS[model]
+    attend, *combine = recorder().calls("orin_fa_prefill", ptr(1), ptr(2), ptr(3), ptr(4), h, g, d, 32768 + 512, past, tokens, float(d ** -0.5))
+    splits = attend.grid[1]  # (one group of heads at these ratios)
+    assert (splits > 1) == bool(combine)
+    if attend.kernel == "fa_prefill_short_kernel":
+        return "short"
+    cols = 32 * int(attend.params[1])
+    return f"{cols}x{splits}" if splits > 1 else f"{cols}"
+
+
+# us a launch of the forms that come near the fastest, as measured on an MI355X: every layer with rows of its own, replayed from a
+# graph; a pair: that, and the same behind a write of 600 MB that empties the caches, as the layer's matrices do between two launches.
+SHORT_WALKS = [
+    ("qwen1.5b", 0, 45, {"short": (3.7, 4.2), "32": (4.9, 5.2)}),
+    ("llama1b", 0, 45, {"short": (3.1, 3.8), "32": (4.0, 4.5)}),
+    ("qwen1.5b", 0, 200, {"short": (5.7, 6.5), "32": (6.1, 6.6)}),
+    ("qwen1.5b", 140, 100, {"short": (5.9, 6.7), "32": (6.2, 6.6)}),
+    ("qwen1.5b", 550, 4, {"short": (7.1, 9.0), "32": (7.4, 9.2), "32x4": (8.0, 8.4)}),
+    ("qwen1.5b", 0, 512, {"short": (7.3, 9.2), "32": (7.3, 8.3)}),
+    ("qwen1.5b", 420, 100, {"short": (7.2, 8.7), "32": (7.2, 7.7)}),
+    ("qwen1.5b", 550, 70, {"short": (7.5, 9.1), "32": (7.5, 8.1)}),
+    ("qwen3", 550, 70, {"short": (7.5, 9.8), "32": (7.5, 9.0)}),
+    ("qwen3", 200, 301, {"short": (7.4, 9.7), "32": (7.3, 8.6)}),
+    ("llama8b", 420, 100, {"short": (7.3, 9.5), "32": (7.3, 8.4)}),
+]
+
+
+@pytest.mark.parametrize("model, past, tokens, us", SHORT_WALKS)
+def test_short_walks_only_where_they_were_measured_faster(model, past, tokens, us):
+    taken = sum(us[prefill_form(model, past, tokens)])
+    assert taken <= 1.02 * min(map(sum, us.values()))
