@@ -1376,29 +1376,34 @@ constexpr int kMaxPrefillSplitShift = 4; // up to 16 workgroups share a token ti
 //   64 columns   6.9 and 0.7, 0.85 where the whole chip multiplies (clock, L2)
 //   short walk   4.0 and 0.8; 0.25 more a step behind the second (nothing is asked for ahead of the last tile's use: measured to 1300
 //                rows, behind 256 of them it keeps up with the 32 columns while the caches have the rows, and does not where
-//                they come from memory: 100 tokens of Qwen2.5-1.5B at 420 6.9 us for 7.2, but 8.7 for 7.7)
+//                they come from memory: 100 tokens of Qwen2.5-1.5B at 420 7.2 us both, but 8.7 for 7.7)
 //   KV splits    2.2 for the second launch and 0.65 for every MB of partial results
 // head_dim 64 has half the bytes a row and two workgroups a CU.
 template <int D>
-float prefill_estimate(int cols, bool short_walk, int shift, long long wgs, int rows, double partial_bytes, int cus) {
+float prefill_estimate(int cols, bool short_walk, int shift, long long wgs, int past, int batch, double partial_bytes, int cus) {
+    const int rows = past + batch;
     float base = 6.9f, step = wgs * 3 < (long long)cus * 2 ? 0.7f : 0.85f;
     if (cols == 32) {
         base = 5.3f;
         step = (wgs * 6 >= cus ? 0.5f : 0.56f) * (1.0f + fminf(fmaxf((float)(rows - 4000) / 8000.0f, 0.0f), 0.4f));
     }
-    if (short_walk) {
-        base = 4.0f, step = 0.8f;
-        // (not half of a head of 64, whose tiles are half as long on their way)
-        if (D == 128 && wgs * 10 >= cus) base += 0.25f * fmaxf((float)rows / 128.0f - 2.0f, 0.0f);
-    }
-    long long turns = (wgs + cus - 1) / cus;
+    if (short_walk) base = 4.0f, step = 0.8f;
     if (D == 64) {
         base -= short_walk ? 0.6f : cols == 32 ? 1.1f : 1.5f;
         step *= 0.75f;
         if (wgs > cus) step *= cols == 32 ? 2.0f : 1.4f;
-        turns = (turns + 1) / 2;
     }
-    const float t = (float)turns * (base + step * (float)rows / (float)(128 << shift));
+    const float row = step / (float)(128 << shift);
+    float t = base + row * (float)rows;
+    // (not half of a head of 64, whose tiles are half as long on their way)
+    if (D == 128 && short_walk && wgs * 10 >= cus) t += 0.25f * fmaxf((float)rows / 128.0f - 2.0f, 0.0f);
+    // More workgroups than the chip holds.  Those left over are the shortest walks, the first tokens' (longest first), and start where the
+    // shortest of the others end: a turn more where what is visible to all is long, little where the chunk starts a sequence and few
+    // are left over (260 tokens of Llama-3-8B there, 264 short walks of 32 columns: 6.8 us, 301 of them 7.7, 360 9.5; walks of 64
+    // columns 8.3, 8.5, 9.0).  The factors are fitted.
+    const long long resident = D == 64 ? 2ll * cus : cus;
+    if (wgs > 2 * resident) t *= (float)((wgs + resident - 1) / resident);
+    else if (wgs > resident) t = fmaxf(t, 2.0f * base - 0.45f + row * (2.0f * (float)past + 3.2f * (float)batch * (float)(wgs - resident) / (float)wgs));
     return shift > 0 ? t + 2.2f + 0.65e-6f * (float)partial_bytes : t;
 }
 
@@ -1434,7 +1439,7 @@ hipError_t launch(FaArgs a, int cu_count, hipStream_t stream, void* workspace, s
     auto consider = [&](int c, int sh, bool sw) {
         const long long wgs = ((long long)a.n_kv * a.n_hgroups * ((a.batch + c / a.heads_per_group - 1) / (c / a.heads_per_group))) << sh;
         if (sh > 0 && (wgs > resident || !workspace || (rows << sh) * row_floats * sizeof(float) > workspace_bytes)) return;
-        const float t = prefill_estimate<D>(c, sw, sh, wgs, a.n_past + a.batch, (double)(rows << sh) * D * sizeof(float), cu_count);
+        const float t = prefill_estimate<D>(c, sw, sh, wgs, a.n_past, a.batch, (double)(rows << sh) * D * sizeof(float), cu_count);
         if (t < least) least = t, cols = c, shift = sh, short_walk = sw;
     };
     for (int sh = 0; sh <= kMaxPrefillSplitShift; ++sh) {

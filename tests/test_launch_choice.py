@@ -61,3 +61,20 @@ SHORT_WALKS = [
 def test_short_walks_only_where_they_were_measured_faster(model, past, tokens, us):
     taken = sum(us[prefill_form(model, past, tokens)])
     assert taken <= 1.02 * min(map(sum, us.values()))
+
+
+# (as above: a turn of the chip and a few workgroups)
+PARTIAL_TURNS = [
+    ("llama8b", 0, 260, {"short": (6.8, 8.3), "64": (8.3, 9.7), "32": (9.2, 10.6)}),
+    ("qwen7b", 0, 280, {"short": (7.1, 8.3), "64": (8.4, 9.7), "32": (9.2, 10.8)}),
+    ("qwen7b", 30, 260, {"short": (7.5, 9.0), "64": (8.4, 9.6), "32": (9.6, 11.2)}),
+    ("llama8b", 0, 301, {"short": (7.7, 9.5), "64": (8.5, 10.1), "32": (10.0, 11.5)}),
+    ("llama8b", 0, 360, {"short": (9.5, 11.6), "64": (9.0, 10.7), "32": (10.9, 12.5)}),
+    ("qwen7b", 0, 420, {"short": (10.7, 12.7), "64": (9.4, 11.1), "32": (11.2, 13.1)}),
+]
+
+
+@pytest.mark.parametrize("model, past, tokens, us", PARTIAL_TURNS)
+def test_a_partial_turn_costs_what_its_short_walks_take(model, past, tokens, us):
+    taken = sum(us[prefill_form(model, past, tokens)])
+    assert taken <= 1.02 * min(map(sum, us.values()))
