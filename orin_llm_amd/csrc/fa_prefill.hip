@@ -1378,11 +1378,14 @@ constexpr int kMaxPrefillSplitShift = 4; // up to 16 workgroups share a token ti
 //                rows, behind 256 of them it keeps up with the 32 columns while the caches have the rows, and does not where
 //                they come from memory: 100 tokens of Qwen2.5-1.5B at 420 7.2 us both, but 8.7 for 7.7)
 //   KV splits    2.2 for the second launch and 0.65 for every MB of partial results
-// head_dim 64 has half the bytes a row and two workgroups a CU.
+// head_dim 64 has half the bytes a row and two workgroups a CU, of which 64 columns slow down from 1500 rows on, and 32 columns less than
+// by half there where few CUs have both.
 template <int D>
 float prefill_estimate(int cols, bool short_walk, int shift, long long wgs, int past, int batch, double partial_bytes, int cus) {
     const int rows = past + batch;
-    float base = 6.9f, step = wgs * 3 < (long long)cus * 2 ? 0.7f : 0.85f;
+    auto upto1 = [](float x) { return fminf(fmaxf(x, 0.0f), 1.0f); };
+    const bool full = wgs * 3 >= (long long)cus * 2;
+    float base = 6.9f, step = full ? 0.85f : 0.7f;
     if (cols == 32) {
         base = 5.3f;
         step = (wgs * 6 >= cus ? 0.5f : 0.56f) * (1.0f + fminf(fmaxf((float)(rows - 4000) / 8000.0f, 0.0f), 0.4f));
@@ -1390,8 +1393,9 @@ float prefill_estimate(int cols, bool short_walk, int shift, long long wgs, int 
     if (short_walk) base = 4.0f, step = 0.8f;
     if (D == 64) {
         base -= short_walk ? 0.6f : cols == 32 ? 1.1f : 1.5f;
+        if (cols == 64) step = (full ? 0.78f : 0.7f) * (1.0f + (full ? 0.15f : 0.25f) * upto1((float)(rows - 1500) / 3000.0f));
         step *= 0.75f;
-        if (wgs > cus) step *= cols == 32 ? 2.0f : 1.4f;
+        if (wgs > cus) step *= cols == 64 ? 1.45f : 2.0f * (1.0f - 0.3f * upto1((float)(rows - 2000) / 3000.0f) * upto1(2.0f - (float)wgs / (float)cus));
     }
     const float row = step / (float)(128 << shift);
     float t = base + row * (float)rows;

@@ -78,3 +78,24 @@ PARTIAL_TURNS = [
 def test_a_partial_turn_costs_what_its_short_walks_take(model, past, tokens, us):
     taken = sum(us[prefill_form(model, past, tokens)])
     assert taken <= 1.02 * min(map(sum, us.values()))
+
+
+# (us a launch, caches as they are between replays)
+HEADS_OF_64 = [
+    ("llama1b", 1501, 301, {"32": 11.9, "64": 11.9}),
+    ("llama1b", 3584, 280, {"32": 20.7, "64x2": 22.5, "64": 24.0}),
+    ("llama1b", 4500, 260, {"32": 24.5, "64": 29.3}),
+    ("llama1b", 4500, 301, {"32": 25.0, "64x2": 26.0, "64": 29.1}),
+    ("llama1b", 5500, 260, {"64x2": 28.2, "32": 28.4, "64": 34.3}),
+    ("llama1b", 8000, 280, {"64x2": 36.2, "64": 48.1}),
+    ("llama1b", 8000, 330, {"64x2": 38.7, "64": 48.1}),
+    ("llama1b", 900, 420, {"64": 10.1, "32": 10.7}),
+    ("llama1b", 420, 512, {"64": 9.1, "32": 10.5}),  # (32 columns: 9.1 to 12.0 from run to run)
+    ("llama1b", 4500, 512, {"64": 31.1, "32": 32.2, "64x2": 32.9}),
+    ("llama1b", 3584, 512, {"64": 25.9, "32": 27.4}),
+]
+
+
+@pytest.mark.parametrize("model, past, tokens, us", HEADS_OF_64)
+def test_forms_of_head_dim_64_at_depth(model, past, tokens, us):
+    assert us[prefill_form(model, past, tokens)] <= 1.1 * min(us.values())
