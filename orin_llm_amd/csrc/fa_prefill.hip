@@ -1367,12 +1367,16 @@ hipError_t allow_lds() {
 
 constexpr int kMaxPrefillSplitShift = 4; // up to 16 workgroups share a token tile's KV rows (small chunks on long contexts)
 
-// What a launch takes, in us, to choose by: fitted to 9000 measurements (five models' heads, 12 chunk sizes of 4 to 512 tokens,
-// 13 depths of 0 to 32000, every form below that fits the chip; within 10 % of most of them, and over those shapes the form it
-// picks is 0.3 % slower than the fastest measured, 23 % at most).  `rows`: KV rows the last token sees; a step is 128 of them, a tile for
-// each of four waves; wgs: workgroups of the launch, KV splits included.
+// What a launch takes, in us, to choose by: fitted to 30000 measurements (the heads of five models, one query head per KV head, and
+// seven of 64; 26 chunk sizes of 4 to 512 tokens, 23 depths of 0 to 32000, every form below that fits the chip; up to 1200 rows also with
+// empty caches) and checked on 19000 at other sizes.  Of 2384 of those with warm caches the form it picks is 0.3 % slower than the fastest,
+// more than 10 % slower at four (490 tokens of Llama-3.2-1B at 420 11.6 for 9.4: 32 columns on a full chip take 9 to 13 us there from run to run);
+// of 956 with empty caches 0.8 %, nine, most of them few tokens at 800 rows, where splits gain more than with warm ones.
+// `rows`: KV rows the last token sees; a step is 128 of them, a tile for each of four waves; wgs: workgroups of the launch, KV splits included.
 //   32 columns   5.3 us and 0.5 a step (bound by the 64 bytes a clock of the CU's vector memory path); more where so few
-//                workgroups walk that each waits for its own trips to memory, and on walks that leave the L2
+//                workgroups walk that each waits for its own trips to memory, and on walks that leave the L2, most on a full chip whose
+//                XCDs each stream a whole KV head (24 tokens of Qwen3-0.6B at 32000 with 16 splits: 35.3, 64 columns 32.9;
+//                32 of Llama-3-8B at 16000 30.1 and 24.0; of Qwen2.5-1.5B, a quarter of a head an XCD, at 32000 22.3 and 25.6)
 //   64 columns   6.9 and 0.7, 0.85 where the whole chip multiplies (clock, L2)
 //   short walk   4.0 and 0.8; 0.25 more a step behind the second (nothing is asked for ahead of the last tile's use: measured to 1300
 //                rows, behind 256 of them it keeps up with the 32 columns while the caches have the rows, and does not where
@@ -1381,14 +1385,18 @@ constexpr int kMaxPrefillSplitShift = 4; // up to 16 workgroups share a token ti
 // head_dim 64 has half the bytes a row and two workgroups a CU, of which 64 columns slow down from 1500 rows on, and 32 columns less than
 // by half there where few CUs have both.
 template <int D>
-float prefill_estimate(int cols, bool short_walk, int shift, long long wgs, int past, int batch, double partial_bytes, int cus) {
+float prefill_estimate(int cols, bool short_walk, int shift, long long wgs, int n_kv, int past, int batch, double partial_bytes, int cus) {
     const int rows = past + batch;
     auto upto1 = [](float x) { return fminf(fmaxf(x, 0.0f), 1.0f); };
     const bool full = wgs * 3 >= (long long)cus * 2;
     float base = 6.9f, step = full ? 0.85f : 0.7f;
     if (cols == 32) {
         base = 5.3f;
-        step = (wgs * 6 >= cus ? 0.5f : 0.56f) * (1.0f + fminf(fmaxf((float)(rows - 4000) / 8000.0f, 0.0f), 0.4f));
+        // rows of one KV head that an XCD's L2 would have to hold: workgroups go to the eight in turn, KV heads first, then splits
+        const float l2_rows = (float)rows * (n_kv >= 8 ? (float)n_kv / 8.0f : 1.0f / (float)min(1 << shift, 8 / n_kv));
+        float depth = fminf(upto1(((float)rows * fmaxf((float)n_kv / 8.0f, 1.0f) - 4000.0f) / 8000.0f), 0.4f);
+        if (D == 128 && full) depth += 0.3f * upto1((l2_rows - 8000.0f) / 24000.0f);
+        step = (wgs * 6 >= cus ? 0.5f : 0.56f) * (1.0f + depth);
     }
     if (short_walk) base = 4.0f, step = 0.8f;
     if (D == 64) {
@@ -1443,7 +1451,7 @@ hipError_t launch(FaArgs a, int cu_count, hipStream_t stream, void* workspace, s
     auto consider = [&](int c, int sh, bool sw) {
         const long long wgs = ((long long)a.n_kv * a.n_hgroups * ((a.batch + c / a.heads_per_group - 1) / (c / a.heads_per_group))) << sh;
         if (sh > 0 && (wgs > resident || !workspace || (rows << sh) * row_floats * sizeof(float) > workspace_bytes)) return;
-        const float t = prefill_estimate<D>(c, sw, sh, wgs, a.n_past, a.batch, (double)(rows << sh) * D * sizeof(float), cu_count);
+        const float t = prefill_estimate<D>(c, sw, sh, wgs, a.n_kv, a.n_past, a.batch, (double)(rows << sh) * D * sizeof(float), cu_count);
         if (t < least) least = t, cols = c, shift = sh, short_walk = sw;
     };
     for (int sh = 0; sh <= kMaxPrefillSplitShift; ++sh) {

@@ -99,3 +99,18 @@ HEADS_OF_64 = [
 @pytest.mark.parametrize("model, past, tokens, us", HEADS_OF_64)
 def test_forms_of_head_dim_64_at_depth(model, past, tokens, us):
     assert us[prefill_form(model, past, tokens)] <= 1.1 * min(us.values())
+
+
+FEW_TOKENS_DEEP = [
+    ("qwen3", 32000, 24, {"64x16": 32.9, "32x16": 35.3}),
+    ("llama8b", 32000, 11, {"64x16": 32.8, "32x16": 35.3}),
+    ("llama8b", 16000, 32, {"64x16": 24.0, "64x8": 28.0, "32x8": 30.1}),
+    ("qwen7b", 32000, 16, {"64x16": 28.2, "32x16": 30.1, "32x8": 37.4}),
+    ("qwen1.5b", 32000, 32, {"32x16": 22.3, "64x16": 25.6, "32x8": 33.1}),
+    ("llama1b", 32000, 32, {"64x16": 22.5, "32x8": 30.8, "32x16": 31.8}),
+]
+
+
+@pytest.mark.parametrize("model, past, tokens, us", FEW_TOKENS_DEEP)
+def test_few_tokens_deep_in_a_context(model, past, tokens, us):
+    assert us[prefill_form(model, past, tokens)] <= 1.07 * min(us.values())
