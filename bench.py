@@ -98,6 +98,7 @@ WORKLOADS = {
     "llama8b-prefill512-d4096-timeline": ("llama8b", "timeline", 8192, ("prefill", 4096, 512)),
     "qwen1.5b-prefill512-d3584-timeline": ("qwen1.5b", "timeline", 4096, ("prefill", 3584, 512)),
     "qwen1.5b-prefill512-d0-timeline": ("qwen1.5b", "timeline", 4096, ("prefill", 0, 512)),
+    "qwen1.5b-prefill45-d0-timeline": ("qwen1.5b", "timeline", 4096, ("prefill", 0, 45)),   # (the kernel for short walks)
     # not part of the path: the decode split kernel with parts taken out (cut-off builds of the library, results
     # wrong by design), timed like the decode workloads: what the combine launch, the products and the merge,
     # the trip for the position, the query and the operand-order K loads each cost on top of a plain read

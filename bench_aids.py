@@ -70,6 +70,8 @@ PREFILL_STAGES = [(0, "entry"), (9, "queries and first K tile requested"), (11, 
                   (13, "first V tile requested"), (10, "second K tile requested"),
                   (1, "queries in registers"), (2, "first two score tiles"), (3, "first weights"), (4, "main loop done"),
                   (5, "last products done, accumulators in LDS"), (7, "barrier passed"), (8, "output stored")]
+SHORT_STAGES = [(0, "entry"), (1, "queries in LDS"), (2, "scores of the last tile"), (3, "its weights"), (4, "its products"),
+                (5, "accumulators in LDS"), (6, "barrier passed"), (7, "output stored")]
 GEMV_STAGES = [(0, "entry"), (1, "first two items of weights requested"), (2, "digits of the wave's part of the activation done"),
                (3, "item 0 in LDS"), (4, "item 1 in LDS"), (5, "item 2 in LDS"), (6, "item 3 in LDS"), (7, "item 4 in LDS"),
                (10, "item 7 in LDS"), (13, "tile's sums out"), (14, "exit")]
@@ -99,8 +101,8 @@ def run_timeline(torch, kernels, name, steps, warmup, with_cpu):
     layers = [make_layer(torch, 900 + i, H, G, d, n_ctx, min(n_filled, n_ctx), batch, sh["outliers"]) for i in range(n_layers)]
     outs = [torch.empty((batch, H, d), dtype=torch.float32, device="cuda") for _ in range(n_layers)]
     dpos = torch.tensor([a - 1], dtype=torch.int32, device="cuda")
-    waves = 4 if what == "prefill" else 8
-    stages = PREFILL_STAGES if what == "prefill" else DECODE_STAGES
+    # (table, waves a workgroup, marks); a prefill chunk takes one of two kernels
+    tables = [(0, 4, PREFILL_STAGES), (3, 8, SHORT_STAGES)] if what == "prefill" else [(1, 8, DECODE_STAGES)]
 
     def launch(i):
         q, k, v = layers[i]
@@ -112,16 +114,25 @@ def run_timeline(torch, kernels, name, steps, warmup, with_cpu):
         assert rc == 0, rc
 
     rows = []
-    host = np.zeros(1024 * waves * 16, np.int64)
+    host = np.zeros(1024 * 8 * 16, np.int64)
+
+    def marks(which, waves):
+        rc = L.orin_fa_bench_stamps(which, host.ctypes.data, 1024 * waves * 16)
+        assert rc == 0, rc
+        return host[:1024 * waves * 16].reshape(1024, waves, 16)
+
+    for which, waves, _ in tables:        # (whatever earlier launches left)
+        marks(which, waves)
+    launch(0)
+    torch.cuda.synchronize()
+    which, waves, stages = next(t for t in tables if marks(t[0], t[1]).any())
     for rep in range(1 + max(1, min(steps, 5))):
         for i in range(n_layers - rep % 3):  # (the last launch of a pass is a different layer from pass to pass)
             launch(i)
         torch.cuda.synchronize()
-        rc = L.orin_fa_bench_stamps(0 if what == "prefill" else 1, host.ctypes.data, host.size)
-        assert rc == 0, rc
         # (the library hands the table over and clears it, so a mark that a wave did not pass reads zero: workgroups
         # beyond the launch's grid, decode workgroups the position leaves without a tile, prefill waves without one)
-        t = host.reshape(1024, waves, 16)[:, :, [slot for slot, _ in stages]].astype(np.float64) * 0.01  # 100 MHz -> us
+        t = marks(which, waves)[:, :, [slot for slot, _ in stages]].astype(np.float64) * 0.01  # 100 MHz -> us
         passed = t > 0
         passed &= passed[:, :, -1:]       # waves that went all the way
         t0 = t[:, :, 0][passed[:, :, 0]].min()
@@ -134,7 +145,7 @@ def run_timeline(torch, kernels, name, steps, warmup, with_cpu):
     span = float(med[-1][2])
     if what == "prefill":
         work, peak, unit, bound = prefill_flops(H, d, a, batch), PEAK_FLOPS, "TFLOP/s", "mfma"
-        kern = "fa_prefill_kernel (timeline build)"
+        kern = ("fa_prefill_kernel" if which == 0 else "fa_prefill_short_kernel") + " (timeline build)"
     else:
         work, peak, unit, bound = decode_bytes(H, G, d, a), PEAK_BYTES, "GB/s", "hbm"
         kern = "fa_decode_split_kernel (timeline build; the combine kernel follows it)"

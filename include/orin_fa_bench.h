@@ -51,11 +51,12 @@ size_t orin_fa_bench_handoff_stream_bytes(void);
  * back.  Asynchronous. */
 int orin_fa_bench_tiny_launch(const unsigned* src, unsigned* sink, void* stream);
 
-/* liborin_fa_stamps.so only (in the timeline build lane 0 of every wave of the prefill kernel, of the decode split
+/* liborin_fa_stamps.so only (in the timeline build lane 0 of every wave of the two prefill kernels, of the decode split
  * kernel and of the matrix-vector kernel that reads rows in long runs stores the 100 MHz wall clock at the end of
  * each stage).  Copies the table of the kernel's last launch to host memory: which = 0 prefill, n <= 1024
  * workgroups x 4 waves x 16 slots; which = 1 decode split kernel, n <= 1024 x 8 x 16; which = 2 matrix-vector
- * kernel, n <= 1024 x 4 x 16 (waves 0-3 of a workgroup); entry [workgroup][wave][slot], workgroups numbered
+ * kernel, n <= 1024 x 4 x 16 (waves 0-3 of a workgroup); which = 3 the prefill kernel for short walks, n <= 1024 x 8 x 16
+ * (a chunk takes one of the two: the other's table stays empty); entry [workgroup][wave][slot], workgroups numbered
  * x + gridDim.x * (y + gridDim.y * z); a mark a wave did not pass reads 0.  Clears the table afterwards.
  * Synchronous.  Return codes as in orin_fa.h. */
 int orin_fa_bench_stamps(int which, long long* host, size_t n);

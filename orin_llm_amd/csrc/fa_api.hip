@@ -375,8 +375,8 @@ int orin_fa_rope_store_batch(float* q, float* k, const float* v, uint16_t* kc, u
 // Timeline build only (include/orin_fa_bench.h): the stage-mark tables of the kernels' last launches.
 int orin_fa_bench_stamps(int which, long long* host, size_t n) {
     if (!g_state.ready) return ORIN_FA_E_NOT_INIT;
-    if (!host || n == 0 || which < 0 || which > 2) return ORIN_FA_E_INVALID;
-    return hip_code(which == 0 ? prefill_stamps(host, n) : which == 1 ? decode_stamps(host, n) : gemv_stamps(host, n));
+    if (!host || n == 0 || which < 0 || which > 3) return ORIN_FA_E_INVALID;
+    return hip_code(which == 0 ? prefill_stamps(host, n) : which == 1 ? decode_stamps(host, n) : which == 2 ? gemv_stamps(host, n) : prefill_short_stamps(host, n));
 }
 #endif
 

@@ -151,9 +151,10 @@ constexpr int kStampWgs = 1024, kStampSlots = 16;
     } while (0)
 #endif
 // Copies a kernel's table to the host (which: 0 prefill, 4 waves a workgroup; 1 decode split, 8 waves; 2 the
-// matrix-vector kernel, 4 waves);
+// matrix-vector kernel, 4 waves; 3 prefill of short walks, 8 waves);
 // hipErrorNotSupported in the ordinary library.
 hipError_t prefill_stamps(long long* host, size_t n);
+hipError_t prefill_short_stamps(long long* host, size_t n);
 hipError_t decode_stamps(long long* host, size_t n);
 hipError_t gemv_stamps(long long* host, size_t n); // the matrix-vector kernel that reads rows in long runs: waves 0-3 of a workgroup
 

@@ -49,10 +49,13 @@
 #ifdef ORIN_FA_STAMPS
 namespace orin_fa {
 __device__ long long g_prefill_stamps[kStampWgs * kPrefillWaves * kStampSlots];
+__device__ long long g_short_stamps[kStampWgs * 8 * kStampSlots]; // the kernel for short walks, eight waves
 }
 #define FA_STAMP(i) ORIN_FA_STAMP_STORE(orin_fa::g_prefill_stamps, orin_fa::kPrefillWaves, i)
+#define SHORT_STAMP(i) ORIN_FA_STAMP_STORE(orin_fa::g_short_stamps, 8, i)
 #else
 #define FA_STAMP(i)
+#define SHORT_STAMP(i)
 #endif
 
 // Cut-off builds (-DORIN_FA_PREFILL_PROBE=flags, liborin_fa_pprobe_<flags>.so; measurement aids whose RESULTS
@@ -1015,13 +1018,13 @@ __global__ __launch_bounds__(kPrefillWaves * 64) void fa_prefill_kernel(PREFILL_
 
 // ---------------------------------------------------------------------------------------------
 // Short walks: a chunk near the start of its context, whose workgroups see a few tiles of KV rows.  The kernel above is built for its steady state: a wave asks for two tiles of K ahead, multiplies a
-// second tile while it scans the first, and leaves through its pipeline's drain, 4 us for a chunk whose waves have a tile each
-// (stage marks of 45 tokens of Qwen2.5-1.5B at depth 0).  Here eight waves -- two a SIMD, each the cover for the other's waits --
+// second tile while it scans the first, and leaves through its pipeline's drain: 4 us where the waves have a tile each.  Here eight waves -- two a SIMD, each the cover for the other's waits --
 // take a tile of 32 rows each, 256 rows a workgroup and turn, with nothing between a tile's arrival and its use: one buffer for K and
 // one for V a wave, the next tile's K asked for when this one's products are through with the buffer, its V likewise.
 // 32 query columns a workgroup, packed as above; the same layouts in LDS, the same (m, l, O) hand-over, over the waves that had a
-// tile.  Softmax with the tiles' true maxima, row sums in fp32.  Bound by its chain -- queries there 1.25 us after the first wave's entry,
-// scores 2.1, weights 2.3, outputs 2.7, handed over 3.1, stored 3.5 -- and, from five tiles on, by the 64 bytes a clock at which a
+// tile.  Softmax with the tiles' true maxima, row sums in fp32.  Bound by its chain -- 45 tokens of Qwen2.5-1.5B at depth 0, cold: queries
+// there 0.9 us after the first wave's entry, scores 1.4, weights 1.6, outputs 2.0, all handed over 2.5, stored 2.9 (medians of the stage
+// marks, their stores included) -- and, from five tiles on, by the 64 bytes a clock at which a
 // CU takes them in.  Qwen2.5-1.5B heads at depth 0, us a launch: 16 tokens 5.15 -> 4.2, 45 5.3 -> 4.35, 100 5.75 -> 4.8, 200 6.3 -> 6.2;
 // Llama-3.2-1B's: 45 tokens 4.4 -> 3.8.
 // ---------------------------------------------------------------------------------------------
@@ -1043,6 +1046,7 @@ __global__ __launch_bounds__(kShortWaves * 64, D == 64 ? 4 : 2) void fa_prefill_
     using SG = SGeom<D>;
     constexpr int kWaves = kShortWaves, kC = G::kCopies, kVar = G::kCopyVariants;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    SHORT_STAMP(0);
     const int heads_per_group = packed & 15, tq = (packed >> 8) & 255;
     const int tq_magic = packed >> 16;
     const int lane = threadIdx.x & 63;
@@ -1153,6 +1157,7 @@ __global__ __launch_bounds__(kShortWaves * 64, D == 64 ? 4 : 2) void fa_prefill_
         *reinterpret_cast<h4*>(smem + SG::kQOff + qcol[j] * G::kQStride + (lane % (D / 4)) * 8) = hv;
     });
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); // (LDS only: the copies travel on)
+    SHORT_STAMP(1);
 
     float* const ml = reinterpret_cast<float*>(smem + SG::kMlOff);
     if (n_mine > 0) {
@@ -1184,6 +1189,7 @@ __global__ __launch_bounds__(kShortWaves * 64, D == 64 ? 4 : 2) void fa_prefill_
             }
 #pragma unroll
             for (int r = 0; r < 16; ++r) s[r] += s2[r];
+            SHORT_STAMP(2);
             if (left > 0) {
                 __builtin_amdgcn_sched_barrier(0);
                 __builtin_amdgcn_s_waitcnt(0xC07F); // K's reads have returned
@@ -1219,6 +1225,7 @@ __global__ __launch_bounds__(kShortWaves * 64, D == 64 ? 4 : 2) void fa_prefill_
                 sump[r % 4] += (float)p[r / 8][r % 8];
             }
             l += (sump[0] + sump[1]) + (sump[2] + sump[3]);
+            SHORT_STAMP(3);
             if (left > 0) wait_copies(IntC<kC>{}); // V(tile); the next K may be in flight
             else wait_copies(IntC<0>{});
 #pragma unroll
@@ -1228,6 +1235,7 @@ __global__ __launch_bounds__(kShortWaves * 64, D == 64 ? 4 : 2) void fa_prefill_
                     const h4 v0 = lds_read_tr(vp[0][db] + kh * 16 * G::kRowB), v1 = lds_read_tr(vp[1][db] + kh * 16 * G::kRowB);
                     o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7), p[kh], o[db], 0, 0, 0);
                 }
+            SHORT_STAMP(4);
             if (left == 0) break;
             __builtin_amdgcn_sched_barrier(0);
             __builtin_amdgcn_s_waitcnt(0xC07F); // V's reads have returned
@@ -1249,7 +1257,9 @@ __global__ __launch_bounds__(kShortWaves * 64, D == 64 ? 4 : 2) void fa_prefill_
                 *reinterpret_cast<f4*>(ws + (db * 4 + qd) * 1024 + G::o_chunk(c32, hh, qd) * 16) =
                     f4{o[db][4 * qd], o[db][4 * qd + 1], o[db][4 * qd + 2], o[db][4 * qd + 3]};
     }
+    SHORT_STAMP(5);
     __syncthreads();
+    SHORT_STAMP(6);
     // ---- merge and store: sixteen threads a column, 16-byte pieces.  Sixteen neighbouring threads read eight pieces of each
     // of two columns: sixteen different chunk columns of the banks (PGeom::o_chunk). ----
     const int cm = (threadIdx.x >> 5) * 2 + ((threadIdx.x >> 3) & 1), part = (threadIdx.x & 7) + 8 * ((threadIdx.x >> 4) & 1);
@@ -1297,6 +1307,7 @@ __global__ __launch_bounds__(kShortWaves * 64, D == 64 ? 4 : 2) void fa_prefill_
     for (int j = 0; j < kPieces; ++j) v[j] = acc[j] * inv;
 #pragma unroll
     for (int j = 0; j < kPieces; ++j) store_stream(a.out + orow * D + (j * 16 + part) * 4, v[j]);
+    SHORT_STAMP(7);
 }
 
 // out = sum over the KV splits of their normalised outputs, weighted by 2^(lse_s - max lse) and
@@ -1504,18 +1515,23 @@ hipError_t prefill_allow_lds() {
     return allow_lds_short<64>();
 }
 
-hipError_t prefill_stamps(long long* host, size_t n) {
 #ifdef ORIN_FA_STAMPS
-    if (n > (size_t)kStampWgs * kPrefillWaves * kStampSlots) return hipErrorInvalidValue;
-    hipError_t e = hipMemcpyFromSymbol(host, HIP_SYMBOL(g_prefill_stamps), n * sizeof(long long)); // (synchronises with the device)
+namespace {
+template <size_t N>
+hipError_t read_stamps(const long long (&table)[N], long long* host, size_t n) {
+    if (n > N) return hipErrorInvalidValue;
+    hipError_t e = hipMemcpyFromSymbol(host, table, n * sizeof(long long)); // (synchronises with the device)
     void* dev = nullptr;
-    if (e == hipSuccess) e = hipGetSymbolAddress(&dev, HIP_SYMBOL(g_prefill_stamps));
-    if (e == hipSuccess) e = hipMemset(dev, 0, sizeof(g_prefill_stamps)); // the next launch starts from an empty table
+    if (e == hipSuccess) e = hipGetSymbolAddress(&dev, table);
+    if (e == hipSuccess) e = hipMemset(dev, 0, sizeof(table)); // the next launch starts from an empty table
     return e;
-#else
-    (void)host; (void)n;
-    return hipErrorNotSupported;
-#endif
 }
+} // namespace
+hipError_t prefill_stamps(long long* host, size_t n) { return read_stamps(g_prefill_stamps, host, n); }
+hipError_t prefill_short_stamps(long long* host, size_t n) { return read_stamps(g_short_stamps, host, n); }
+#else
+hipError_t prefill_stamps(long long*, size_t) { return hipErrorNotSupported; }
+hipError_t prefill_short_stamps(long long*, size_t) { return hipErrorNotSupported; }
+#endif
 
 } // namespace orin_fa

@@ -50,6 +50,25 @@ def test_timeline_build_gives_the_same_results_and_ordered_marks():
     assert (np.diff(marks, axis=1) >= 0).all(), "a wave's marks are out of order"
     assert (marks[:, -1] - marks[:, 0]).max() < 100 * 1000  # below a millisecond at 100 MHz
 
+    # prefill of a short walk: the other kernel, and a table of its own
+    n_short = 45
+    qs = dq[:n_short].contiguous()
+    a = torch.empty((n_short, H, d), dtype=torch.float32, device="cuda")
+    b = torch.empty_like(a)
+    kernels.flash_attention(qs, dk, dv, a, H, G, d, n_ctx, 0, n_short, float(scale))
+    short = np.zeros(1024 * 8 * 16, np.int64)
+    assert L.orin_fa_bench_stamps(3, short.ctypes.data, short.size) == 0
+    assert L.orin_fa_prefill(qs.data_ptr(), dk.data_ptr(), dv.data_ptr(), b.data_ptr(), H, G, d, n_ctx, 0, n_short, scale) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(a, b)
+    assert L.orin_fa_bench_stamps(0, host.ctypes.data, host.size) == 0 and not host.any()
+    assert L.orin_fa_bench_stamps(3, short.ctypes.data, short.size) == 0
+    st = short.reshape(1024, 8, 16)
+    full = (st[:, :, :8] > 0).all(axis=2)          # (waves with a tile; the others skip the marks of its products)
+    assert full[:18].any(axis=1).all() and not st[18:].any()   # two KV heads, nine token tiles
+    assert (np.diff(st[full][:, :8], axis=1) >= 0).all(), "a wave's marks are out of order"
+    assert (st[:18, :, [0, 1, 5, 6]] > 0).all()
+
     # decode
     pos = torch.tensor([n_past + batch - 1], dtype=torch.int32, device="cuda")
     oa = torch.empty((H, d), dtype=torch.float32, device="cuda")
