@@ -195,14 +195,16 @@ def test_prefill_wide_blocks(fa, d, r):
 
 
 @pytest.mark.parametrize("H,G,d,n_past,batch,scale", [
-    (12, 2, 128, 4608, 512, 0.0883883),   # Qwen2.5-1.5B heads: two workgroups share a token tile's rows
-    (12, 2, 128, 7680, 512, 0.0883883),
-    (2, 1, 128, 4100, 1100, 0.0883883),   # four workgroups per token tile
+    (12, 2, 128, 4608, 512, 0.0883883),   # Qwen2.5-1.5B heads, where splits do not pay yet: 32 columns
+    (12, 2, 128, 7680, 512, 0.0883883),   # two workgroups of 64 columns share a token tile's rows
+    (2, 1, 128, 4100, 1100, 0.0883883),   # four
     (1, 1, 64, 0, 5200, 0.125),           # from an empty cache: early token tiles leave splits without a row
-    (8, 1, 64, 4900, 300, -0.3),          # a ragged end, negative scale (the rescaling path on most tiles)
-    (3, 1, 128, 5200, 1, 0.0883883),      # one token: sixteen workgroups share its rows
-    (12, 2, 128, 9000, 45, 0.0883883),    # a short last chunk of a long prompt: sixteen workgroups per token tile
-    (12, 2, 128, 3100, 200, 0.0883883),   # four workgroups per token tile, from 3072 rows
+    (8, 1, 64, 4900, 300, -0.3),          # a ragged end, negative scale (the rescaling path on most tiles); four of 32 columns
+    (3, 1, 128, 5200, 1, 0.0883883),      # one token: sixteen workgroups of 32 columns share its rows
+    (12, 2, 128, 9000, 45, 0.0883883),    # a short last chunk of a long prompt: sixteen of 64 columns
+    (12, 2, 128, 3100, 200, 0.0883883),   # two of 32 columns
+    (12, 2, 128, 8000, 100, 0.0883883),   # eight of 64 columns
+    (32, 8, 64, 9000, 70, 0.125),         # ... at head_dim 64
 ])
 def test_prefill_kv_splits(fa, H, G, d, n_past, batch, scale):
     """Few query columns on a long context: the launcher cuts a token tile's KV rows among 2 to
@@ -426,13 +428,16 @@ def test_cfg2_full_stack_28_layers(fa):
 
 
 @pytest.mark.parametrize("H,G,d,n_ctx,n_past,batch", [
-    (12, 2, 128, 4096, 2600, 8),     # sixteen splits
-    (16, 8, 128, 8192, 5000, 100),   # eight
-    (32, 8, 128, 8192, 5000, 100),   # four
-    (12, 2, 128, 8192, 5632, 512),   # two
-    (32, 8, 64, 4096, 2400, 40),     # eight, head_dim 64
-    (32, 8, 128, 8192, 8000, 128),   # partial outputs that fill the workspace to the byte: fewer splits in place
-    (12, 2, 128, 4096, 100, 45),     # none
+    (12, 2, 128, 4096, 2600, 8),     # sixteen splits of 32 columns
+    (16, 8, 128, 8192, 5000, 100),   # four
+    (32, 8, 128, 8192, 5000, 100),   # two
+    (12, 2, 128, 8192, 5632, 512),   # two of 64 columns
+    (32, 8, 64, 4096, 2400, 40),     # four of 32, head_dim 64
+    (32, 8, 128, 8192, 8000, 128),   # four of 64, partial outputs that fill the workspace to the byte: two of 32 columns in place
+    (12, 2, 128, 4096, 100, 45),     # none: the kernel for short walks
+    (12, 2, 128, 4096, 550, 4),      # ... with a second and a third tile a wave
+    (32, 8, 64, 4096, 20, 70),       # ... at head_dim 64
+    (12, 2, 128, 16384, 8000, 100),  # eight splits of 64 columns
 ])
 def test_prefill_in_place(fa, H, G, d, n_ctx, n_past, batch):
     """out = q: a split's log-sum-exps must not land in query rows that another split of the tile has still to read."""
@@ -455,6 +460,43 @@ def test_prefill_in_place(fa, H, G, d, n_ctx, n_past, batch):
             rows = _sample_rows(np.random.default_rng(7), batch, H, H // G)
             exact = ref.flash_attention_rows(q, kc, vc, rows, H, G, d, n_ctx, n_past, np.float32(scale))
             check(got[rows[:, 0], rows[:, 1]], exact, "in place, other splits")
+
+
+@pytest.mark.parametrize("H,G,d,n_past,batch", [
+    (12, 2, 128, 0, 45), (12, 2, 128, 100, 45), (32, 8, 64, 20, 70), (12, 2, 128, 550, 4), (32, 8, 64, 300, 4),
+])
+def test_short_walks_keep_infinities_and_nans_where_they_belong(fa, H, G, d, n_past, batch):
+    """In a query, an infinity or a NaN stays in its own row of the output; in a K row that every token sees it leaves a token the
+    non-finite values the oracle has for it; in a V row, its channel.  The other KV heads' outputs do not change in a bit."""
+    n_ctx, scale, r = n_past + batch + 3, 1.0 / np.sqrt(d), H // G
+    q, kc, vc = make_case(810 + n_past, H, G, d, n_ctx, n_past + batch, batch, outliers=2, poison_tail=True)
+    clean = gpu_prefill(fa, q, kc, vc, H, G, d, n_ctx, n_past, batch, scale)
+    row, head = n_past // 2, G - 1     # (row 0 of an empty cache: the one every token sees)
+    others = np.arange(H) // r != head
+    for bits in (0x7C00, 0xFC00, 0x7E00):
+        value = np.array(bits, np.uint16).view(np.float16).astype(np.float32)
+        q2 = q.copy()
+        q2[batch // 2, head * r, 5] = value
+        got = gpu_prefill(fa, q2, kc, vc, H, G, d, n_ctx, n_past, batch, scale)
+        assert not np.isfinite(got[batch // 2, head * r]).any()
+        got[batch // 2, head * r] = clean[batch // 2, head * r]
+        assert np.array_equal(got, clean)
+        for what, cache in (("K", kc), ("V", vc)):
+            kept = cache[head, row, 5]
+            cache[head, row, 5] = bits
+            got = gpu_prefill(fa, q, kc, vc, H, G, d, n_ctx, n_past, batch, scale)
+            want = ref.flash_attention_rows(q, kc, vc, np.array([(t, h) for t in range(batch) for h in range(H)], np.int32), H, G, d, n_ctx, n_past,
+                                            np.float32(scale)).reshape(batch, H, d)
+            cache[head, row, 5] = kept
+            assert np.array_equal(got[:, others], clean[:, others]), what
+            fine = np.isfinite(want)
+            if n_past == 0:   # (token 0 sees that row alone: where its one score is minus infinity, 0 / 0 in the oracle, every form gives zeros)
+                fine[0] |= (got[0] == 0.0).all(axis=1, keepdims=True)
+                want[0][(got[0] == 0.0).all(axis=1)] = 0.0
+            assert np.array_equal(np.isfinite(got), fine), (what, hex(bits))
+            assert not fine[:, ~others].all()
+            whole = fine.all(axis=2)
+            check(got[whole], want[whole], f"{what} {hex(bits)} H{H} d{d} P{n_past} B{batch}")
 
 
 # ---------------------------------------------------------------- error behaviour

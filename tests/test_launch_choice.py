@@ -28,16 +28,19 @@ HEADS = {  # query heads, KV heads, head size
 }
 
 
-def prefill_form(model, past, tokens):
+def form_of(h, g, d, past, tokens, in_place=False):
     """"short", or the query columns of a workgroup, with the number of KV splits where there are any: "64x4"."""
-    h, g, d = HEADS[model]
-    attend, *combine = recorder().calls("orin_fa_prefill", ptr(1), ptr(2), ptr(3), ptr(4), h, g, d, 32768 + 512, past, tokens, float(d ** -0.5))
-    splits = attend.grid[1]  # (one group of heads at these ratios)
+    attend, *combine = recorder().calls("orin_fa_prefill", ptr(1), ptr(2), ptr(3), ptr(1 if in_place else 4), h, g, d, 32768 + 512, past, tokens, float(d ** -0.5))
+    splits = attend.grid[1] // -(-h // g // 8)  # (heads of a group in eights)
     assert (splits > 1) == bool(combine)
     if attend.kernel == "fa_prefill_short_kernel":
         return "short"
     cols = 32 * int(attend.params[1])
     return f"{cols}x{splits}" if splits > 1 else f"{cols}"
+
+
+def prefill_form(model, past, tokens):
+    return form_of(*HEADS[model], past, tokens)
 
 
 # us a launch of the forms that come near the fastest, as measured on an MI355X: every layer with rows of its own, replayed from a
@@ -114,3 +117,50 @@ FEW_TOKENS_DEEP = [
 @pytest.mark.parametrize("model, past, tokens, us", FEW_TOKENS_DEEP)
 def test_few_tokens_deep_in_a_context(model, past, tokens, us):
     assert us[prefill_form(model, past, tokens)] <= 1.07 * min(us.values())
+
+
+def parameters(test):
+    """Every combination of a test's parametrisations, as dictionaries."""
+    out = [{}]
+    for mark in test.pytestmark:
+        if mark.name == "parametrize":
+            names = [n.strip() for n in mark.args[0].split(",")]
+            out = [{**o, **dict(zip(names, v))} for o in out for v in mark.args[1]]
+    return out
+
+
+def test_the_parity_tests_reach_every_form():
+    """The forms of the shapes that test_gpu_parity.py takes on the GPU: each at head_dim 128, in place too; the same comments there."""
+    import test_gpu_parity as t
+
+    def forms(test, d, in_place=False):
+        return {form_of(p["H"], p["G"], p["d"], p["n_past"], p["batch"], in_place) for p in parameters(test) if p["d"] == d}
+
+    splits, shorts = forms(t.test_prefill_kv_splits, 128), forms(t.test_prefill_short_chunks, 128)
+    assert splits | shorts >= {"short", "32"} | {f"{c}x{s}" for c in (32, 64) for s in (2, 4, 8, 16)}
+    assert forms(t.test_prefill_short_chunks, 64) | forms(t.test_prefill_kv_splits, 64) >= {"short", "32x4", "32x16", "64x4", "64x8"}
+    assert forms(t.test_prefill_in_place, 128, True) >= {"short", "32x2", "32x4", "32x16", "64x2", "64x8"}
+    assert forms(t.test_prefill_in_place, 64, True) >= {"short", "32x4"}
+    for p in parameters(t.test_short_walks_keep_infinities_and_nans_where_they_belong):
+        assert form_of(p["H"], p["G"], p["d"], p["n_past"], p["batch"]) == "short", p
+
+
+@pytest.mark.parametrize("heads, head_dim, tokens, start, aligned", [(64, 128, 3000001, 7, True), (8, 128, 8388607, 0, True), (3, 100, 8000000, 5, True),
+                                                                     (64, 128, 400000, 1, False), (8, 64, 1000, 3, True)])
+def test_cache_rows_in_slices_below_two_to_the_31_threads(heads, head_dim, tokens, start, aligned):
+    """A launch counts its threads in 32 bits: a longer store goes out as several, one behind the other, that together move every row once."""
+    off = 0 if aligned else 2
+    launches = recorder().calls("orin_fa_kv_store_batch", ptr(1) + off, ptr(2), ptr(3), ptr(4), heads, head_dim, start + tokens, start, tokens, keep_args=7)
+    vec = 8 if aligned and head_dim % 8 == 0 else 1
+    done = 0
+    for one in launches:
+        assert one.kernel == "kv_store_kernel" and one.params == [str(vec), "false"]
+        kc, vc, k, v, shape, rows, n = one.args
+        threads = one.grid[0] * one.block
+        needed = 2 * n * heads * (head_dim // vec)
+        assert needed <= threads < needed + one.block and threads < 1 << 31
+        assert (kc, vc) == (ptr(1) + off, ptr(2)) and shape == heads | head_dim << 32 and rows == (start + tokens) | (start + done) << 32
+        assert (k, v) == (ptr(3) + 4 * done * heads * head_dim, ptr(4) + 4 * done * heads * head_dim)
+        done += n
+    assert done == tokens
+    assert len(launches) == -(-tokens // (0x7fffff00 // (2 * heads * (head_dim // vec))))
