@@ -659,7 +659,7 @@ def run_rope(torch, kernels, name, steps, warmup, with_cpu):
                             bytes_per_step=nbytes * layers),
                 roofline=dict(bound="hbm", achieved=nbytes / (us * 1e-6) / 1e9, peak=PEAK_BYTES / 1e9, unit="GB/s",
                               frac=nbytes / (us * 1e-6) / PEAK_BYTES, traffic=None,
-                              kernel="rope4_kernel<false, false>, Q rows then K rows", launch_us=us,
+                              kernel="rope_pieces_kernel<false>, Q rows then K rows", launch_us=us,
                               bytes_per_launch=nbytes, note="launch_us and bytes cover the two launches of a layer"),
                 parity=dict(max_rel_to_tensor_max=err, rows="layer 0, all rows, vs CPU oracle"), **forms)
 

@@ -91,8 +91,8 @@ void orin_gemv_use_matrix_cores(int on);
  * the output and down projections of orin_decode_layer) may cut a row into: 0 (default) = the launcher
  * chooses 1 to 16 by shape (up to 8 blocks of 256 elements a share: 7 for rows of 14336 elements, 10 for 18944),
  * which is fastest and leaves the order of a row's adds open (see orin_gemv_q8_add);
- * 1 = never cut, every result bit for bit reproducible, at up to 0.4 us more per output projection and 1 to
- * 4.5 us more per down projection; 2 to 16 = forced (tuning; no more than a row has blocks); anything else = 0.
+ * 1 = never cut, every result bit for bit reproducible, at up to 0.3 us more per output projection and 1 to
+ * 7 us more per down projection; 2 to 16 = forced (tuning; no more than a row has blocks); anything else = 0.
  * Takes effect with the next launch; graphs captured earlier keep the launches they recorded.
  * ORIN_GEMV_KSPLIT in the environment sets the initial value. */
 void orin_gemv_row_shares(int shares);

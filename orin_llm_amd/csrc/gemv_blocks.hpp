@@ -480,9 +480,9 @@ struct MF<kQ6_K> {
 // Q6_K read in runs of two blocks that start on a word: 420 bytes are 27 pieces one behind the other, the last of them the run's
 // last sixteen bytes.  A block fetched as pieces of its own starts on a word only every other time, and its last piece overlaps the one
 // before: reads alone (48 MB) 10.25 us against 9.2, and 43.3 against 38.6 over 255 MB, as fast as 16-byte aligned ones.
-// For rows of an even number of blocks, cut (shares, chunks) at even blocks, and a matrix that starts on a word.  Per launch: down
-// projection of Qwen2.5-7B 15.3 -> 13.6 us (55.7 MB, 4.1 TB/s), Llama-3-8B 12.7 -> 11.9, its logits 74.8 -> 72.0 (6.0 TB/s), Llama-3.2-1B's
-// 40.4 -> 38.6, Qwen2.5-7B's gate/up 24.9 -> 23.4.
+// For rows of an even number of blocks, cut (shares, chunks) at even blocks, and a matrix that starts on a word.  Per launch, the same
+// matrix two bytes off a word (block by block) and on one (in runs): down projection of Qwen2.5-7B 15.1 and 12.9 us (55.7 MB, 4.3
+// TB/s), Llama-3-8B 13.0 and 11.7, its logits 80.3 and 71.8 (6.0 TB/s), Llama-3.2-1B's 42.9 and 37.1, Qwen2.5-7B's gate/up 26.6 and 23.8.
 // In LDS the run lies as it does in memory: block 1 starts two bytes into a piece, and a lane's sixteen bytes there are that
 // piece and the word behind it, shifted down (LDS takes 64 clocks for wide reads off their alignment, 9 on it).
 constexpr int kQ6_KRun = 0x100 + kQ6_K;
