@@ -1395,40 +1395,63 @@ constexpr int kMaxPrefillSplitShift = 4; // up to 16 workgroups share a token ti
 //   KV splits    2.2 for the second launch and 0.65 for every MB of partial results
 // head_dim 64 has half the bytes a row and two workgroups a CU, of which 64 columns slow down from 1500 rows on, and 32 columns less than
 // by half there where few CUs have both.
+// (A launch asks for up to eleven forms and the host's time is what bounds a short chunk, so what the chunk alone decides is worked out once,
+// and next to nothing divides on the way: about 100 ns a launch, 190 to 280 as a function of all its arguments.)
 template <int D>
-float prefill_estimate(int cols, bool short_walk, int shift, long long wgs, int n_kv, int past, int batch, double partial_bytes, int cus) {
-    const int rows = past + batch;
-    auto upto1 = [](float x) { return fminf(fmaxf(x, 0.0f), 1.0f); };
-    const bool full = wgs * 3 >= (long long)cus * 2;
-    float base = 6.9f, step = full ? 0.85f : 0.7f;
-    if (cols == 32) {
-        base = 5.3f;
-        // rows of one KV head that an XCD's L2 would have to hold: workgroups go to the eight in turn, KV heads first, then splits
-        const float l2_rows = (float)rows * (n_kv >= 8 ? (float)n_kv / 8.0f : 1.0f / (float)min(1 << shift, 8 / n_kv));
-        float depth = fminf(upto1(((float)rows * fmaxf((float)n_kv / 8.0f, 1.0f) - 4000.0f) / 8000.0f), 0.4f);
-        if (D == 128 && full) depth += 0.3f * upto1((l2_rows - 8000.0f) / 24000.0f);
-        step = (wgs * 6 >= cus ? 0.5f : 0.56f) * (1.0f + depth);
+struct PrefillEstimate {
+    static float upto1(float x) { return x < 0.0f ? 0.0f : x < 1.0f ? x : 1.0f; }
+    int n_kv, cus;
+    float past, batch, rows, deep32, deep64, mid;
+
+    PrefillEstimate(int n_kv_, int past_, int batch_, int cus_) : n_kv(n_kv_), cus(cus_), past((float)past_), batch((float)batch_), rows(past + batch) {
+        deep32 = upto1((rows * (n_kv > 8 ? (float)n_kv * 0.125f : 1.0f) - 4000.0f) * (1.0f / 8000.0f));
+        if (deep32 > 0.4f) deep32 = 0.4f;
+        deep64 = upto1((rows - 1500.0f) * (1.0f / 3000.0f));
+        mid = upto1((rows - 2000.0f) * (1.0f / 3000.0f));
     }
-    if (short_walk) base = 4.0f, step = 0.8f;
-    if (D == 64) {
-        base -= short_walk ? 0.6f : cols == 32 ? 1.1f : 1.5f;
-        if (cols == 64) step = (full ? 0.78f : 0.7f) * (1.0f + (full ? 0.15f : 0.25f) * upto1((float)(rows - 1500) / 3000.0f));
-        step *= 0.75f;
-        if (wgs > cus) step *= cols == 64 ? 1.45f : 2.0f * (1.0f - 0.3f * upto1((float)(rows - 2000) / 3000.0f) * upto1(2.0f - (float)wgs / (float)cus));
+    template <int cols, bool short_walk>
+    float of(int shift, int wgs, float partial_bytes) const {
+        constexpr float kOf128[kMaxPrefillSplitShift + 1] = {1.0f / 128, 1.0f / 256, 1.0f / 512, 1.0f / 1024, 1.0f / 2048};
+        const bool full = wgs * 3 >= cus * 2;
+        float base, step;
+        if (short_walk) {
+            base = 4.0f, step = 0.8f;
+        } else if (cols == 32) {
+            float depth = deep32;
+            if (D == 128 && full && rows > 8000.0f) {
+                // rows of one KV head that an XCD's L2 would have to hold: workgroups go to the eight in turn, KV heads first, then splits
+                const float l2_rows = rows * (n_kv >= 8 ? (float)n_kv * 0.125f : 1.0f / (float)min(1 << shift, 8 / n_kv));
+                depth += 0.3f * upto1((l2_rows - 8000.0f) * (1.0f / 24000.0f));
+            }
+            base = 5.3f, step = (wgs * 6 >= cus ? 0.5f : 0.56f) * (1.0f + depth);
+        } else if (D == 128) {
+            base = 6.9f, step = full ? 0.85f : 0.7f;
+        } else {
+            base = 6.9f, step = full ? 0.78f * (1.0f + 0.15f * deep64) : 0.7f * (1.0f + 0.25f * deep64);
+        }
+        if (D == 64) {
+            base -= short_walk ? 0.6f : cols == 32 ? 1.1f : 1.5f;
+            step *= 0.75f;
+            if (wgs > cus) step *= cols == 64 ? 1.45f : mid > 0.0f && wgs < 2 * cus ? 2.0f * (1.0f - 0.3f * mid * upto1(2.0f - (float)wgs / (float)cus)) : 2.0f;
+        }
+        const float row = step * kOf128[shift];
+        float t = base + row * rows;
+        // (not half of a head of 64, whose tiles are half as long on their way)
+        if (D == 128 && short_walk && wgs * 10 >= cus && rows > 256.0f) t += 0.25f * (rows * (1.0f / 128.0f) - 2.0f);
+        // More workgroups than the chip holds.  Those left over are the shortest walks, the first tokens' (longest first), and start where the
+        // shortest of the others end: a turn more where what is visible to all is long, little where the chunk starts a sequence and few
+        // are left over (260 tokens of Llama-3-8B there, 264 short walks of 32 columns: 6.8 us, 301 of them 7.7, 360 9.5; walks of 64
+        // columns 8.3, 8.5, 9.0).  The factors are fitted.
+        const int resident = D == 64 ? 2 * cus : cus;
+        if (wgs > 2 * resident) {
+            t *= (float)((wgs + resident - 1) / resident);
+        } else if (wgs > resident) {
+            const float two = 2.0f * base - 0.45f + row * (2.0f * past + 3.2f * batch * (float)(wgs - resident) / (float)wgs);
+            if (two > t) t = two;
+        }
+        return shift > 0 ? t + 2.2f + 0.65e-6f * partial_bytes : t;
     }
-    const float row = step / (float)(128 << shift);
-    float t = base + row * (float)rows;
-    // (not half of a head of 64, whose tiles are half as long on their way)
-    if (D == 128 && short_walk && wgs * 10 >= cus) t += 0.25f * fmaxf((float)rows / 128.0f - 2.0f, 0.0f);
-    // More workgroups than the chip holds.  Those left over are the shortest walks, the first tokens' (longest first), and start where the
-    // shortest of the others end: a turn more where what is visible to all is long, little where the chunk starts a sequence and few
-    // are left over (260 tokens of Llama-3-8B there, 264 short walks of 32 columns: 6.8 us, 301 of them 7.7, 360 9.5; walks of 64
-    // columns 8.3, 8.5, 9.0).  The factors are fitted.
-    const long long resident = D == 64 ? 2ll * cus : cus;
-    if (wgs > 2 * resident) t *= (float)((wgs + resident - 1) / resident);
-    else if (wgs > resident) t = fmaxf(t, 2.0f * base - 0.45f + row * (2.0f * (float)past + 3.2f * (float)batch * (float)(wgs - resident) / (float)wgs));
-    return shift > 0 ? t + 2.2f + 0.65e-6f * (float)partial_bytes : t;
-}
+};
 
 template <int D>
 hipError_t launch(FaArgs a, int cu_count, hipStream_t stream, void* workspace, size_t workspace_bytes) {
@@ -1438,7 +1461,7 @@ hipError_t launch(FaArgs a, int cu_count, hipStream_t stream, void* workspace, s
     const int r = a.r;
     a.heads_per_group = r < 8 ? r : 8;
     a.n_hgroups = (r + a.heads_per_group - 1) / a.heads_per_group;
-    // Four forms (prefill_estimate() above), the one that is expected to be done first:
+    // Four forms (PrefillEstimate above), the one that is expected to be done first:
     //   64 columns a workgroup, which occupies a whole CU (head_dim 64: half of one), so that every tile it fetches serves
     //   twice the columns;
     //   32 columns, where the coarser grid would leave CUs idle;
@@ -1459,17 +1482,25 @@ hipError_t launch(FaArgs a, int cu_count, hipStream_t stream, void* workspace, s
     int cols = 64, shift = 0;
     bool short_walk = false;
     float least = INFINITY;
-    auto consider = [&](int c, int sh, bool sw) {
-        const long long wgs = ((long long)a.n_kv * a.n_hgroups * ((a.batch + c / a.heads_per_group - 1) / (c / a.heads_per_group))) << sh;
-        if (sh > 0 && (wgs > resident || !workspace || (rows << sh) * row_floats * sizeof(float) > workspace_bytes)) return;
-        const float t = prefill_estimate<D>(c, sw, sh, wgs, a.n_kv, a.n_past, a.batch, (double)(rows << sh) * D * sizeof(float), cu_count);
-        if (t < least) least = t, cols = c, shift = sh, short_walk = sw;
+    const PrefillEstimate<D> estimate(a.n_kv, a.n_past, a.batch, cu_count);
+    const size_t split_bytes = rows * row_floats * sizeof(float);
+    const float partial_bytes = (float)(rows * D * sizeof(float));
+    auto consider = [&](auto colsc) {
+        constexpr int c = decltype(colsc)::value;
+        const int tq = c / a.heads_per_group;
+        const long long wgs_long = (long long)a.n_kv * a.n_hgroups * ((a.batch + tq - 1) / tq);
+        const int wgs = (int)min(wgs_long, 1ll << 24); // (far more than the chip holds, and room for the products below)
+        auto take = [&](float t, int sh, bool sw) {
+            if (t < least) least = t, cols = c, shift = sh, short_walk = sw;
+        };
+        take(estimate.template of<c, false>(0, wgs, 0.0f), 0, false);
+        if (workspace)
+            for (int sh = 1; sh <= kMaxPrefillSplitShift && wgs <= resident >> sh && split_bytes << sh <= workspace_bytes; ++sh)
+                take(estimate.template of<c, false>(sh, wgs << sh, partial_bytes * (float)(1 << sh)), sh, false);
+        if (c == 32) take(estimate.template of<32, true>(0, wgs, 0.0f), 0, true);
     };
-    for (int sh = 0; sh <= kMaxPrefillSplitShift; ++sh) {
-        consider(64, sh, false);
-        consider(32, sh, false);
-    }
-    consider(32, 0, true);
+    consider(IntC<64>{});
+    consider(IntC<32>{});
     a.tq = cols / a.heads_per_group;
     a.kv_split_shift = shift;
     if (shift > 0) {
