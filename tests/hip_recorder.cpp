@@ -11,7 +11,6 @@
 #include <string>
 #include <vector>
 
-#define __HIP_PLATFORM_AMD__ 1
 #include <hip/hip_runtime_api.h>
 
 namespace {

@@ -68,6 +68,6 @@ def recorder():
     with ThreadPoolExecutor(max_workers=8) as pool:
         list(pool.map(build._run, compile_one))
     lib = os.path.join(where, "liborin_recorded.so")
-    build._run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-Wl,-Bsymbolic,-z,muldefs", "-I/opt/rocm/include", os.path.join(ROOT, "tests", "hip_recorder.cpp")]
+    build._run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-Wl,-Bsymbolic,-z,muldefs", "-I/opt/rocm/include", "-D__HIP_PLATFORM_AMD__=1", os.path.join(ROOT, "tests", "hip_recorder.cpp")]
                + objs + ["-o", lib])
     return Recorder(ctypes.CDLL(lib))
