@@ -27,6 +27,8 @@
 //     written per split; the combine kernel merges the splits that were active.
 #include "fa_common.hpp"
 
+#include <string.h>
+
 #include <type_traits>
 
 // Stage marks: wall-clock stamps in the timeline build, nothing otherwise (fa_common.hpp).
@@ -67,23 +69,46 @@ struct DGeom {
     static constexpr int kMergeB = 16 * kOStride * 4;
     static constexpr int kWaveB = (kTileBV > kMergeB) ? kTileBV : kMergeB;
     static constexpr int kMlOff = kDecodeWaves * kWaveB;       // (m, l) per wave per column follow the wave slices
-    static constexpr int kQOff = kMlOff + kDecodeWaves * 16 * 2 * 4; // the group's query heads, fp32 [16][kQStride]
-    static constexpr int kQStride = D + 4;                     // floats per head (4 of padding: the operand reads of 16 heads miss each other's banks)
-    static constexpr int kLdsB = kQOff + 16 * kQStride * 4;
+    // The group's query heads: two planes of operands, the fp16 values and what rounding to them left off, [16][kQPlaneB / 16]; or
+    // (angles that come late) fp32 [16][kQStride].  Padded so that the operand reads of 16 heads miss each other's banks.
+    static constexpr int kQOff = kMlOff + kDecodeWaves * 16 * 2 * 4;
+    static constexpr int kQRowB = D * 2 + 16, kQPlaneB = 16 * kQRowB;
+    static constexpr int kQStride = D + 4;
+    static constexpr int kLdsB = kQOff + 2 * kQPlaneB;
+    static_assert(2 * kQPlaneB >= 16 * kQStride * 4, "either form");
 };
 
-// MODE 1 (store): the current token's K and V rows arrive as fp32 beside the cache (FaArgs::k_new,
-// v_new).  The wave whose tile holds row *d_pos takes that row from them -- rounded to fp16 exactly
-// as the store kernel rounds -- instead of from the cache, and writes it to the cache on the way:
-// the store kernel's launch is saved and the result is the same bit for bit.
-// MODE 2 (rotate + store): q and k_new arrive before the rotary embedding, and every workgroup
-// rotates them itself (the inputs stay as they are): the first n_rot/2 lanes of every wave put
-// the angles' cosines and sines (computed, or read from the caller's table) into the wave's own
-// LDS table while the first tile is on its way, and the pairs a lane rotates are ones it holds
-// anyway -- "normal" pairs are neighbours, and for "neox" with
-// n_rot = head_dim element e pairs with e + head_dim/2, the same lane's k-step two (one, at
-// head_dim 64) further on.  Same arithmetic as the rotary kernel, so again bit for bit what the
-// separate launches give, four launches in the place of seven.
+typedef float f4_a8 __attribute__((ext_vector_type(4), aligned(8))); // (a table of angles is 8-byte aligned)
+// 16 bytes a lane through a descriptor (base, byte count): zeros, and no access, at kNowhere.
+constexpr int kNowhere = 0x7ffffff8;
+__device__ __forceinline__ f4 load16(const float* base, unsigned bytes, int off) {
+    return __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(make_rsrc(base, bytes), off, 0, 0));
+}
+// What a launch does besides attending (see the kernel).
+enum : int { kPlain = 0, kStore = 1, kRotate = 2, kRotateNeox = 3, kRotateLate = 4 };
+
+// kStore: the current token's K and V rows arrive as fp32 beside the cache (FaArgs::k_new, v_new).  The workgroup whose tiles
+// include row *d_pos takes that row from them -- rounded to fp16 exactly as the store kernel rounds -- instead of from the
+// cache, and writes it to the cache on the way: the store kernel's launch is saved and the result is the same bit for bit.
+// kRotate, kRotateNeox (rotate + store): q and k_new arrive before the rotary embedding, and the workgroups rotate them (the
+// inputs stay as they are) by the caller's table of angles: "normal" pairs are neighbours, "neox" pairs half a head
+// apart.  Same arithmetic as the rotary kernel, so again bit for bit what the separate launches give, two launches
+// in the place of seven.  A rotation that does not span the whole head, or has no table, is kRotateLate's: every
+// wave keeps a table in LDS (a power, a sine and a cosine a pair, which must not sit ahead of the tile requests) and rotates the whole
+// query behind the workgroup's meeting, and the new row is made ready by the wave whose last tile holds it.
+//
+// A launch is a chain -- position and query, tile, products, merge -- in which a wave issues an instruction every 2 ns, so what
+// can be done once is done once, and off the way from a tile's arrival to the result:
+//   * each wave makes operands of the piece of the query it has fetched (rotates it, splits it into the two fp16 parts) ahead of
+//     the tile requests, and the pieces meet in LDS as operands.  (Every wave used to convert, and for "neox" rotate, the whole query.)
+//   * the new row is made ready by a wave without a tile, while the owner's tile travels, or ahead of the meeting where all have one.  (The
+//     owner used to, which took longer than its tile: products 1.1 us after its requests instead of 0.6.)
+//   * a run of one tile (a position short of a tile a split) goes from registers to the result, without the merge through LDS; a
+//     wave's first tile rescales nothing; rows past the position are voided in the last tile only; and the tile with another behind it is code
+//     of its own, so that every wait is for what is used next.
+// Rotate + store + attend, us a launch pair, caches emptied between replays, before -> now: Qwen2.5-1.5B at 200 of 4096 7.6 -> 6.5, at 4095 7.9 ->
+// 7.0, at 32767 of 32768 11.7 -> 11.2; Llama-3-8B at 1000 of 8192 7.75 -> 6.8, at 8191 11.5 -> 11.1; Qwen2.5-7B at 16001 of 32768 12.3 ->
+// 11.2; Llama-3.2-1B at 1777 of 8192 7.1 -> 6.6.  Plain decode 6.2 -> 6.05, 6.75 -> 6.6, 10.7 -> 10.9, 6.7 -> 6.5, 11.3 -> 11.25, 11.25 -> 11.15, 6.3 -> 6.2.
 template <int D, int MODE>
 __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
     // What the first loads need comes first, as scalars: the leading kernel arguments are handed
@@ -93,16 +118,17 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
     // the statements below that hold them in place)
     // Plain decode needs nothing but these 14 words: no trip to the launch's argument block at
     // all, which is slower than the trip for the position (the caches hold that).  So: the grid
-    // is (KV head, head group, split) and says what n_kv and n_hgroups would; n_splits and r share
-    // a word (splits_r = n_splits | r << 16); the scale carries the sign that goes into Q
-    // (c_signed = |scale| log2(e) with the sign of scale; c2 below is its magnitude); dst is where this kernel writes: the
-    // partial outputs (followed by the (m, l) pairs) when there are splits, else `out` itself.
+    // is (KV head, head group, split) and says what n_kv and n_hgroups would; n_splits, r and the sign that goes into Q share
+    // a word (splits_r = n_splits | negative scale << 15 | r << 16); scale_heads = |scale| log2(e) as its bits | n_head << 32, or,
+    // with a table of angles, the table's address (those two then come from the argument block, being needed last); dst is where
+    // this kernel writes: the partial outputs (followed by the (m, l) pairs) when there are splits, else `out` itself.
     const int* d_pos, const float* q, const uint16_t* kc, const uint16_t* vc,
-    const int n_ctx, const unsigned splits_r, const float c_signed, float* dst, const int n_head,
+    const int n_ctx, const unsigned splits_r, const uint64_t scale_heads, float* dst,
     const FaArgs a) { // (a: what the store and rotate variants need besides)
     using G = DGeom<D>;
     constexpr int kWaves = kDecodeWaves;
     constexpr int kThreads = kWaves * 64;
+    constexpr bool STORE = MODE != kPlain, TABLE = MODE == kRotate || MODE == kRotateNeox, NEOX = MODE == kRotateNeox, LATE = MODE == kRotateLate;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     FA_STAMP(0);
 
@@ -111,83 +137,93 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
     const int col = lane & 15; // MFMA column (query head of the group) / row (KV row or head_dim index) of the lane
     const int grp = lane >> 4; // lane-group: 8-wide k slice of an operand, 4-row slice of an accumulator
 
-    const int n_splits = splits_r & 0xffffu, r = splits_r >> 16;
-    const float c2 = __builtin_fabsf(c_signed), qsign = c_signed < 0.0f ? -1.0f : 1.0f;
+    const int n_splits = splits_r & 0x7fffu, r = splits_r >> 16;
+    const float qsign = (splits_r & 0x8000u) != 0 ? -1.0f : 1.0f;
     // Workgroup -> (KV head, head group, split); the KV head varies fastest in dispatch order.
     const int kvh = blockIdx.x, hg = blockIdx.y, id = blockIdx.z;
-    float* const part_o = dst;
-    float* const part_ml = dst + (size_t)n_splits * n_head * D; // [n_head][split][2]
 
     unsigned char* const vs = smem + wave * G::kWaveB;
 
-    const __amdgpu_buffer_rsrc_t krs = make_rsrc(kc + (size_t)kvh * n_ctx * D, (unsigned)n_ctx * D * 2);
-    const __amdgpu_buffer_rsrc_t vrs = make_rsrc(vc + (size_t)kvh * n_ctx * D, (unsigned)n_ctx * D * 2);
+    const uint16_t *const k_head = kc + (size_t)kvh * n_ctx * D, *const v_head = vc + (size_t)kvh * n_ctx * D;
+    const int k_lane = col * D * 2 + grp * 16, v_lane = lane * 16; // where a lane's first pieces lie in a tile
 
     u32x4 kreg[2 * G::kSteps], vreg[G::kLoads];
     auto fetch_k = [&](int tile) {
-        const int soff = tile * kTile * D * 2;
+        const __amdgpu_buffer_rsrc_t krs = make_rsrc(k_head, (unsigned)n_ctx * D * 2);
+        const int at = tile * kTile * D * 2 + (kProbeKWholeLines ? lane * 16 : k_lane);
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
             for (int kk = 0; kk < G::kSteps; ++kk)
-                kreg[t * G::kSteps + kk] = buf_load16<true>(krs, kProbeKWholeLines ? soff + ((t * G::kSteps + kk) * 64 + lane) * 16
-                                                                                    : soff + (t * 16 + col) * D * 2 + (kk * 4 + grp) * 16);
+                kreg[t * G::kSteps + kk] = buf_load16<true>(krs, at + (kProbeKWholeLines ? (t * G::kSteps + kk) * 1024 : t * 16 * D * 2 + kk * 64));
     };
     auto fetch_v = [&](int tile) {
-        const int soff = tile * kTile * D * 2;
+        const __amdgpu_buffer_rsrc_t vrs = make_rsrc(v_head, (unsigned)n_ctx * D * 2);
+        const int at = tile * kTile * D * 2 + v_lane;
 #pragma unroll
-        for (int i = 0; i < G::kLoads; ++i) vreg[i] = buf_load16<true>(vrs, soff + (i * 64 + lane) * 16);
+        for (int i = 0; i < G::kLoads; ++i) vreg[i] = buf_load16<true>(vrs, at + i * 1024);
     };
     // ---- query heads: requested before the first tile, so that they arrive before it (a wave's
     // loads complete in order) and the score product can start while V is still on its way ----
     const int pos = kProbeConstPos ? n_ctx - 1 - (d_pos == nullptr) : *d_pos; // (read here, ahead of the statement below that may write memory: a scalar load)
-    const int hl = hg * 16 + col;
-    const bool valid = hl < r;
     // Columns past the group's heads are padding: their loads carry an offset past the descriptor's
-    // end, which the hardware answers with zeros without going to memory.  (Every wave of every
-    // workgroup reads its group's heads: fetched for all 16 columns that was as many bytes through
-    // the L2 as the K rows.)
-    // The workgroup fetches its group's heads once: wave w asks for one 16-byte piece per lane --
-    // piece (w & 1) of k-step (w >> 1) -- and the pieces meet in LDS further down.  (Every wave
-    // fetching all of them itself was seven more load instructions a wave whose lanes each count
+    // end, which the hardware answers with zeros without going to memory.
+    // The workgroup fetches its group's heads once, a piece of four elements per lane, neighbouring lanes on one head; the pieces
+    // meet in LDS further down.  (Every wave fetching all of them itself was seven more load instructions a wave whose lanes each count
     // as a look-up of their own in the vector cache, a quarter again of the kernel's look-ups, all
     // of them in the queue ahead of the tile requests: 0.4 us per launch.)
-    const __amdgpu_buffer_rsrc_t qrs = make_rsrc(q, 0x7ffffff0u);
-    const int q_off = valid ? ((kvh * r + hl) * D + grp * 8) * 4 : 0x7ffffff8;
-    const float qmul = valid ? qsign : 0.0f;
+    constexpr int kHeadLanes = D / 4;
+    const int my_head = wave * (64 / kHeadLanes) + lane / kHeadLanes, e0 = (lane % kHeadLanes) * 4; // (head_dim 64: the first four waves have all sixteen)
+    [[maybe_unused]] f4 q_share, cs[2];
+    if constexpr (!LATE) {
+        const bool valid = my_head < 16 && hg * 16 + my_head < r;
+        q_share = kProbeNoQuery ? f4{1.0f, 2.0f, (float)lane, 3.0f} : load16(q, 0x7ffffff0u, valid ? ((kvh * r + hg * 16 + my_head) * D + e0) * 4 : kNowhere);
+    }
+    // (table of angles) The piece's (cos, sin): two pairs, or four, of which it holds one half; the new K row's pieces have the same.
+    const float* const angles = ptr_arg<const float>(TABLE ? scale_heads : 0);
+    if constexpr (TABLE) {
+        const int at = (NEOX ? e0 & (D / 2 - 1) : e0 / 2) * 8;
+        cs[0] = load16(angles, D * 4, at);
+        if constexpr (NEOX) cs[1] = load16(angles, D * 4, at + 16);
+    }
+    // (kRotateLate) The same by pieces of operands: wave w asks for piece (w & 1) of k-step (w >> 1) of every head.
+    const int hl = hg * 16 + col;
+    const bool valid = hl < r;
+    const int q_off = valid ? ((kvh * r + hl) * D + grp * 8) * 4 : kNowhere;
     static_assert(kWaves % (2 * G::kSteps) == 0, "a piece per wave (the same piece twice at head_dim 64)");
     const int q_piece = __builtin_amdgcn_readfirstlane(wave) & (2 * G::kSteps - 1);
-    const float4 q_share = kProbeNoQuery ? float4{1.f, 2.f, (float)q_off, (float)lane}
-                                         : __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(qrs, q_off, (q_piece >> 1) * 128 + (q_piece & 1) * 16, 0));
-    constexpr bool STORE = MODE != 0, ROPE = MODE == 2;
-    // (rotate + store) lane i < n_rot/2 of every wave fetches what pair i's angle needs: its
+    const int q_e0 = (q_piece >> 1) * 32 + grp * 8 + (q_piece & 1) * 4; // the piece's first element of its head
+    float4 q_late = float4{0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (LATE)
+        q_late = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(make_rsrc(q, 0x7ffffff0u), q_off, (q_piece >> 1) * 128 + (q_piece & 1) * 16, 0));
+    // (kRotateLate) lane i < n_rot/2 of every wave fetches what pair i's angle needs: its
     // cosine and sine when the caller supplies them, else its frequency factor if there is one.
     // Both loads are made by every lane, from an address that can be read either way (the query,
     // when the array is absent): a load under a branch makes the compiler wait for every load
     // issued so far where the branch ends.
     float2 cs_given = float2{1.0f, 0.0f};
     float ff_given = 1.0f;
-    if constexpr (ROPE) {
+    if constexpr (LATE) {
         const int pi = min(lane, a.n_rot / 2 - 1);
         const float* anp = a.rope_angles ? a.rope_angles + 2 * pi : q;
         const float* ffp = a.freq_factors ? a.freq_factors + pi : q;
         cs_given = *reinterpret_cast<const float2*>(anp);
         ff_given = *ffp;
     }
-    // (store, rotate + store) The new row, in as few loads as will do, by every wave: only the one whose tiles
-    // include the row's uses it (at its last tile), but which wave that is depends on the position, which is
-    // still on its way, and a load issued later, while the CU's tiles stream in, holds its wave up for a few
-    // hundred cycles each (three of them: 0.5 us between the query's arrival and its conversion).  Here they
-    // are small loads ahead of the flood, hits in the cache for all but the first wave to ask.  K: elements
-    // 4*lane .. 4*lane+3 (the lanes hand each other the pieces they hold of a K row through LDS then); V: piece
-    // lane % (D/8), which is what the lane holds of a V row.
-    float4 k_raw = float4{0.f, 0.f, 0.f, 0.f}, v_raw[2] = {k_raw, k_raw};
+    // (store, rotate + store) The new row, in as few loads as will do: which workgroup owns it depends on the position, which
+    // is still on its way, and a load issued later, while the CU's tiles stream in, holds its wave up for a few
+    // hundred cycles each.  For the last wave, which makes the row ready (kRotateLate: for every wave); the others' loads go nowhere (under
+    // a branch, the last wave would wait for the row where it waits for its share of the query).  K: the lane's piece, as of
+    // the query; V: piece lane % (D/8), eight elements.
+    constexpr int kRowWave = kWaves - 1;
+    [[maybe_unused]] f4 k_raw, v_raw[2];
     if constexpr (STORE) {
-        const float* kp4 = a.k_new + (size_t)kvh * D + (lane % (D / 4)) * 4;
-        const float* vp8 = a.v_new + (size_t)kvh * D + (lane % G::kChunksPerRow) * 8;
-        k_raw = *reinterpret_cast<const float4*>(kp4);
-        v_raw[0] = *reinterpret_cast<const float4*>(vp8);
-        v_raw[1] = *reinterpret_cast<const float4*>(vp8 + 4);
+        const float *const kp = a.k_new + (size_t)kvh * D, *const vp = a.v_new + (size_t)kvh * D;
+        const int v_e0 = (lane % G::kChunksPerRow) * 8;
+        const bool mine = LATE || wave == kRowWave;
+        k_raw = load16(kp, D * 4, mine ? e0 * 4 : kNowhere);
+        v_raw[0] = load16(vp, D * 4, mine ? v_e0 * 4 : kNowhere);
+        v_raw[1] = load16(vp, D * 4, mine ? v_e0 * 4 + 16 : kNowhere);
     }
     __builtin_amdgcn_sched_barrier(0); // the small loads first: they return first, and nothing that needs them waits for a tile
 
@@ -202,11 +238,15 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
     // here, in the trip to memory that brings the position: left alone, the compiler fetches
     // each where it is first used, behind the first tile's arrival.  (Fetched behind the tile
     // requests instead, they queue behind the chip's 33 MB of tile traffic: 0.5 us per layer.)
-    if constexpr (MODE != 0) {
+    const float c2 = TABLE ? a.c : __uint_as_float((unsigned)scale_heads);
+    const int n_head = TABLE ? a.n_head : (int)(scale_heads >> 32);
+    if constexpr (MODE != kPlain) {
         const void *p0 = a.k_new, *p1 = a.v_new;
-        asm volatile("" ::"s"(p0), "s"(p1), "s"(a.n_rot), "s"(a.neox), "s"(pos));
+        asm volatile("" ::"s"(p0), "s"(p1), "s"(a.n_rot), "s"(a.neox), "s"(c2), "s"(n_head), "s"(pos));
     }
     __builtin_amdgcn_sched_barrier(0);
+    float* const part_o = dst;
+    float* const part_ml = dst + (size_t)n_splits * n_head * D; // [n_head][split][2]
 
     int p = pos < 0 ? 0 : pos;
     const int npos = (p > n_ctx - 1 ? n_ctx - 1 : p) + 1; // rows [0, npos) are visible
@@ -218,54 +258,15 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
     // (CUs, each with its own 64 B/clk into the vector cache) as there are instead of filling a
     // few workgroups' eight waves.  (Interleaving single tiles among the splits at every length
     // cost 8 % at full length on Qwen2.5-7B: neighbouring 8 KB pieces then alternate between XCDs.)
-    int wu = (n_tiles + n_splits - 1) / n_splits;
-    wu = wu > kWaves ? kWaves : wu;
+    int wu = 0; // = min(ceil(n_tiles / n_splits), 8), by halves: a division is three times as long, and the tile requests wait for it
+    static_assert(kWaves == 8, "three halves");
+#pragma unroll
+    for (int h = 4; h > 0; h >>= 1) wu += n_tiles > (wu + h) * n_splits ? h : 0;
+    ++wu;
     const int tile_first = wave < wu ? id * wu + wave : n_tiles; // (n_tiles: none)
     const int tile_step = wu * n_splits;
     int tile = tile_first;
-    float* const qs = reinterpret_cast<float*>(smem + G::kQOff);
-    __shared__ __attribute__((aligned(16))) float sh_cs_all[ROPE ? kWaves : 1][D / 2][2];
-    __shared__ __attribute__((aligned(16))) _Float16 sh_krow_all[STORE ? kWaves : 1][D];
-    float (*const sh_cs)[2] = sh_cs_all[ROPE ? wave : 0];
-    const bool rot_early = ROPE && !a.neox && a.rope_angles != nullptr; // (the query is rotated piece by piece before it is parked)
-    if (id * wu < n_tiles) {
-        // The query pieces meet in LDS: each wave parks the piece it fetched, then a barrier that
-        // waits for LDS only.  Ahead of the tile requests, where the eight waves are still in
-        // step (the position and the pieces arrive together); behind them the waves are microseconds
-        // apart -- the load unit takes a CU's 128 KB of requests as fast as memory answers them --
-        // and a barrier there holds every wave's products until the last has all its requests out.
-        float4 q_park = q_share;
-        if constexpr (ROPE) {
-            // "Normal" pairs are neighbours, so the piece a wave fetched holds two whole pairs: with the caller's
-            // table of angles at hand the wave rotates just those before it parks the piece, and nobody has to
-            // rotate the whole query behind the barrier (eight waves each used to: sixteen table reads and as
-            // many rotations a lane between the query's arrival and its conversion; 0.4 us of a Llama-3-8B
-            // launch pair).  Without a table the angles are a power, a sine and a cosine away, which must not
-            // sit ahead of the tile requests.  ("neox" pairs sit half a head apart, in another wave's piece:
-            // fetching that piece as well and rotating early was built and gained nothing.)
-            if (rot_early) {
-                if (lane < a.n_rot / 2) {
-                    sh_cs[lane][0] = cs_given.x;
-                    sh_cs[lane][1] = cs_given.y;
-                }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                const int e0 = (q_piece >> 1) * 32 + grp * 8 + (q_piece & 1) * 4, last = max(a.n_rot / 2 - 1, 0);
-                const float2 c0 = *reinterpret_cast<const float2*>(sh_cs[min(e0 / 2, last)]);
-                const float2 c1 = *reinterpret_cast<const float2*>(sh_cs[min(e0 / 2 + 1, last)]);
-                float x0 = q_park.x, x1 = q_park.y, y0 = q_park.z, y1 = q_park.w;
-                rope_rotate(x0, x1, c0.x, c0.y);
-                rope_rotate(y0, y1, c1.x, c1.y);
-                q_park.x = e0 < a.n_rot ? x0 : q_park.x;
-                q_park.y = e0 < a.n_rot ? x1 : q_park.y;
-                q_park.z = e0 + 2 < a.n_rot ? y0 : q_park.z;
-                q_park.w = e0 + 2 < a.n_rot ? y1 : q_park.w;
-            }
-        }
-        *reinterpret_cast<float4*>(qs + col * G::kQStride + (q_piece >> 1) * 32 + grp * 8 + (q_piece & 1) * 4) = q_park;
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    }
+    const int own_tile = n_tiles - 1; // the new row's
     if (id * wu >= n_tiles) {
         // Inactive split: it leaves "no row seen" for its heads, so that the combine kernel can tell
         // without reading the position itself (one more trip to memory on its short critical path);
@@ -277,6 +278,129 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
         }
         return;
     }
+    float* const qs = reinterpret_cast<float*>(smem + G::kQOff);
+    __shared__ __attribute__((aligned(16))) float sh_cs_all[LATE ? kWaves : 1][D / 2][2];
+    __shared__ __attribute__((aligned(16))) _Float16 sh_krow_all[LATE ? kWaves : 1][D];
+    __shared__ __attribute__((aligned(16))) _Float16 sh_vrow[STORE && !LATE ? D : 8];
+    __shared__ int sh_row_there;
+    // (said to be LDS: a generic pointer's accesses count as memory's too, and every wait behind one is for everything)
+    [[maybe_unused]] auto* const row_there = (__attribute__((address_space(3))) volatile int*)&sh_row_there;
+    float (*const sh_cs)[2] = sh_cs_all[LATE ? wave : 0];
+    const bool rot_early = LATE && !a.neox && a.rope_angles != nullptr; // (the query is rotated piece by piece before it is parked)
+    // The query pieces meet in LDS: each wave parks the piece it fetched, then a barrier that
+    // waits for LDS only.  Ahead of the tile requests, where the eight waves are still in
+    // step (the position and the pieces arrive together); behind them the waves are microseconds
+    // apart -- the load unit takes a CU's 128 KB of requests as fast as memory answers them --
+    // and a barrier there holds every wave's products until the last has all its requests out.
+            // A piece of the query or of the new K row, rotated.
+    [[maybe_unused]] auto rotate4 = [&](f4 x) {
+                if constexpr (NEOX) { // element e goes with e + D/2: the lane's piece is the first or the second of the pair, the other one 16 (8) lanes away
+                    const bool second = e0 >= D / 2;
+                    f4 y;
+    #pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        float lo, hi;
+                        if constexpr (D == 128) { // both halves of the pair land in both lanes
+                            const u32x2 s = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[e]), __float_as_uint(x[e]), false, false);
+                            lo = __uint_as_float(s.x);
+                            hi = __uint_as_float(s.y);
+                        } else {
+                            const int b = __float_as_int(x[e]);
+                            const float other = __int_as_float(__builtin_amdgcn_update_dpp(b, b, 0x128, 0xF, 0xF, false)); // row_ror:8
+                            lo = second ? other : x[e];
+                            hi = second ? x[e] : other;
+                        }
+                        rope_rotate(lo, hi, cs[e / 2][e % 2 * 2], cs[e / 2][e % 2 * 2 + 1]);
+                        y[e] = second ? hi : lo;
+                    }
+                    return y;
+                } else if constexpr (TABLE) {
+                    float x0 = x[0], x1 = x[1], x2 = x[2], x3 = x[3];
+                    rope_rotate(x0, x1, cs[0][0], cs[0][1]);
+                    rope_rotate(x2, x3, cs[0][2], cs[0][3]);
+                    return f4{x0, x1, x2, x3};
+                } else {
+                    return x;
+                }
+            };
+    if constexpr (LATE) {
+        float4 q_park = q_late;
+        // "Normal" pairs are neighbours, so the piece a wave fetched holds two whole pairs: with the caller's
+        // table of angles at hand the wave rotates just those before it parks the piece.  (Without a table the angles are a power,
+        // a sine and a cosine away.)
+        if (rot_early) {
+            if (lane < a.n_rot / 2) {
+                sh_cs[lane][0] = cs_given.x;
+                sh_cs[lane][1] = cs_given.y;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            const int e0 = q_e0, last = max(a.n_rot / 2 - 1, 0);
+            const float2 c0 = *reinterpret_cast<const float2*>(sh_cs[min(e0 / 2, last)]);
+            const float2 c1 = *reinterpret_cast<const float2*>(sh_cs[min(e0 / 2 + 1, last)]);
+            float x0 = q_park.x, x1 = q_park.y, y0 = q_park.z, y1 = q_park.w;
+            rope_rotate(x0, x1, c0.x, c0.y);
+            rope_rotate(y0, y1, c1.x, c1.y);
+            q_park.x = e0 < a.n_rot ? x0 : q_park.x;
+            q_park.y = e0 < a.n_rot ? x1 : q_park.y;
+            q_park.z = e0 + 2 < a.n_rot ? y0 : q_park.z;
+            q_park.w = e0 + 2 < a.n_rot ? y1 : q_park.w;
+        }
+        *reinterpret_cast<float4*>(qs + col * G::kQStride + q_e0) = q_park;
+    } else {
+        // The piece as operands: rotated, then its fp16 value and what that leaves off.
+        const f4 x = rotate4(q_share);
+        h4 hi, lo;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float xe = x[e] * qsign;
+            hi[e] = (_Float16)xe;
+            lo[e] = (_Float16)(xe - (float)hi[e]);
+        }
+        if (my_head < 16) {
+            unsigned char* const park = smem + G::kQOff + my_head * G::kQRowB + e0 * 2;
+            *reinterpret_cast<h4*>(park) = hi;
+            *reinterpret_cast<h4*>(park + G::kQPlaneB) = lo;
+        }
+    }
+    [[maybe_unused]] int own_wave = -1; // the wave of this workgroup whose tiles include the new row's, if any (not kRotateLate)
+    [[maybe_unused]] auto make_row = [&] {
+        // The new row: rotated and converted as the rotary kernel and the store kernel would, into LDS for the wave that
+        // owns it, which takes it instead of what its tile brings back, and into the cache (no other wave reads that row, so
+        // the order of this write and that read does not matter; one head group's workgroup writes it).
+        const f4 k = rotate4(k_raw);
+        h4 kh;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) kh[e] = (_Float16)k[e];
+        h8 vh;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) vh[e] = (_Float16)v_raw[e / 4][e % 4];
+        if (lane < kHeadLanes) *reinterpret_cast<h4*>(sh_krow_all[0] + e0) = kh;
+        if (lane < G::kChunksPerRow) *reinterpret_cast<h8*>(sh_vrow + lane * 8) = vh;
+        // (a wave's LDS writes are made in order: who sees the flag sees the row)
+        asm volatile("" ::: "memory");
+        *row_there = 1;
+        if (hg == 0) {
+            const size_t row_off = ((size_t)kvh * n_ctx + pos) * D;
+            if (lane < kHeadLanes) *reinterpret_cast<h4*>(const_cast<uint16_t*>(kc) + row_off + e0) = kh;
+            if (lane < G::kChunksPerRow) *reinterpret_cast<h8*>(const_cast<uint16_t*>(vc) + row_off + lane * 8) = vh;
+        }
+    };
+    if constexpr (STORE && !LATE) {
+        int last = own_tile; // where the last visible tile lies in a turn of all splits (a few turns at most)
+        while (last >= tile_step) last -= tile_step;
+        own_wave = store && last - id * wu < wu ? last - id * wu : -1; // (negative: another split's)
+        // By the last wave: behind the meeting where it has no tile of its own, while the owner's tile is on its way (the owner waits for the
+        // flag), and ahead of it where it has.
+        if (wave == kRowWave) {
+            if (own_wave >= 0 && wu == kWaves) make_row();
+            else *row_there = 0;
+        }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if constexpr (STORE && !LATE)
+        if (wave == kRowWave && own_wave >= 0 && wu < kWaves) make_row();
 
     // m_ref: reference maximum of the raw scores (before the scale); l_run: this lane's share of
     // the row sum; o: O^T accumulators, lane (col, grp) holds head_dim rows db*16 + grp*4 + i.
@@ -295,7 +419,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
         FA_STAMP(1);
         if constexpr (kProbeCutOff) { // (cut-off build: wait for the tile, keep every load alive, leave)
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            unsigned acc = __float_as_uint(q_share.x) ^ __float_as_uint(q_share.w);
+            unsigned acc = LATE ? __float_as_uint(q_late.x) ^ __float_as_uint(q_late.w) : __float_as_uint(q_share[0]) ^ __float_as_uint(q_share[3]);
 #pragma unroll
             for (int i = 0; i < 2 * G::kSteps; ++i) acc ^= kreg[i].x ^ kreg[i].y ^ kreg[i].z ^ kreg[i].w;
 #pragma unroll
@@ -304,51 +428,71 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
             if (acc != 0x9E3779BAu) return;
         }
         // (the query pieces met ahead of the tile requests; the operands are picked up while the first tile is on its way)
-        float qf[G::kSteps][8]; // this lane's 8 elements of every k-step: head_dim indices kk*32 + grp*8 + 0..7
+        h8 qhi[G::kSteps], qlo[G::kSteps];
+        [[maybe_unused]] u32x4 k_new16[G::kSteps], v_new16 = u32x4{0u, 0u, 0u, 0u};
+        [[maybe_unused]] bool owner = wave == own_wave; // (kRotateLate: further down)
+        if constexpr (!LATE) {
+            const unsigned char* const op = smem + G::kQOff + col * G::kQRowB + grp * 16;
 #pragma unroll
-        for (int kk = 0; kk < G::kSteps; ++kk) {
-            const float4 x0 = *reinterpret_cast<const float4*>(qs + col * G::kQStride + kk * 32 + grp * 8);
-            const float4 x1 = *reinterpret_cast<const float4*>(qs + col * G::kQStride + kk * 32 + grp * 8 + 4);
-            qf[kk][0] = x0.x; qf[kk][1] = x0.y; qf[kk][2] = x0.z; qf[kk][3] = x0.w;
-            qf[kk][4] = x1.x; qf[kk][5] = x1.y; qf[kk][6] = x1.z; qf[kk][7] = x1.w;
-        }
-        // (rotate + store) the rotation of this lane's 8 elements of every k-step, by the wave's table
-        // x0, x1: this lane's elements of k-steps kk and kk + kSteps/2 (head_dim indices kk*32 + grp*8 + e
-        // and the same + head_dim/2)
-        auto rotate2 = [&](float (&x0)[8], float (&x1)[8], int kk) {
-            if (a.neox) { // n_rot == D (checked by the host): element e pairs with e + D/2
+            for (int kk = 0; kk < G::kSteps; ++kk) {
+                qhi[kk] = *reinterpret_cast<const h8*>(op + kk * 64);
+                qlo[kk] = *reinterpret_cast<const h8*>(op + kk * 64 + G::kQPlaneB);
+            }
+            if constexpr (STORE) {
+                if (wave == own_wave) {
+                    while (*row_there == 0) {} // (the last wave sets it, whatever the others do)
+                    asm volatile("" ::: "memory");
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int i = kk * 32 + grp * 8 + e;
-                    rope_rotate(x0[e], x1[e], sh_cs[i][0], sh_cs[i][1]);
-                }
-            } else {      // elements 2i and 2i + 1, below n_rot
-                // No branch per pair: el0 differs from lane to lane, and a branch around each pair's table
-                // read makes the wave wait out sixteen LDS round trips one after the other (1.7 us of a
-                // Llama-3-8B launch).  Every lane reads an entry (its own, or the table's last), all reads
-                // go out together, and a pair past n_rot keeps its values by a select.
-                const int last = max(a.n_rot / 2 - 1, 0); // (n_rot = 0: nothing is rotated, entry 0 is read and not used)
-                float2 cs0[4], cs1[4];
-#pragma unroll
-                for (int e = 0; e < 8; e += 2) {
-                    const int el0 = kk * 32 + grp * 8 + e, el1 = el0 + D / 2;
-                    cs0[e / 2] = *reinterpret_cast<const float2*>(sh_cs[min(el0 / 2, last)]);
-                    cs1[e / 2] = *reinterpret_cast<const float2*>(sh_cs[min(el1 / 2, last)]);
-                }
-#pragma unroll
-                for (int e = 0; e < 8; e += 2) {
-                    const int el0 = kk * 32 + grp * 8 + e, el1 = el0 + D / 2;
-                    float a0 = x0[e], a1 = x0[e + 1], b0 = x1[e], b1 = x1[e + 1];
-                    rope_rotate(a0, a1, cs0[e / 2].x, cs0[e / 2].y);
-                    rope_rotate(b0, b1, cs1[e / 2].x, cs1[e / 2].y);
-                    x0[e] = el0 < a.n_rot ? a0 : x0[e];
-                    x0[e + 1] = el0 < a.n_rot ? a1 : x0[e + 1];
-                    x1[e] = el1 < a.n_rot ? b0 : x1[e];
-                    x1[e + 1] = el1 < a.n_rot ? b1 : x1[e + 1];
+                    for (int kk = 0; kk < G::kSteps; ++kk) k_new16[kk] = *reinterpret_cast<const u32x4*>(sh_krow_all[0] + (kk * 4 + grp) * 8);
+                    v_new16 = *reinterpret_cast<const u32x4*>(sh_vrow + (lane % G::kChunksPerRow) * 8);
                 }
             }
-        };
-        if constexpr (ROPE) {
+        } else {
+            const float qmul = valid ? qsign : 0.0f;
+            float qf[G::kSteps][8]; // this lane's 8 elements of every k-step: head_dim indices kk*32 + grp*8 + 0..7
+#pragma unroll
+            for (int kk = 0; kk < G::kSteps; ++kk) {
+                const float4 x0 = *reinterpret_cast<const float4*>(qs + col * G::kQStride + kk * 32 + grp * 8);
+                const float4 x1 = *reinterpret_cast<const float4*>(qs + col * G::kQStride + kk * 32 + grp * 8 + 4);
+                qf[kk][0] = x0.x; qf[kk][1] = x0.y; qf[kk][2] = x0.z; qf[kk][3] = x0.w;
+                qf[kk][4] = x1.x; qf[kk][5] = x1.y; qf[kk][6] = x1.z; qf[kk][7] = x1.w;
+            }
+            // (rotate + store) the rotation of this lane's 8 elements of every k-step, by the wave's table
+            // x0, x1: this lane's elements of k-steps kk and kk + kSteps/2 (head_dim indices kk*32 + grp*8 + e
+            // and the same + head_dim/2)
+            auto rotate2 = [&](float (&x0)[8], float (&x1)[8], int kk) {
+                if (a.neox) { // n_rot == D (checked by the host): element e pairs with e + D/2
+    #pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const int i = kk * 32 + grp * 8 + e;
+                        rope_rotate(x0[e], x1[e], sh_cs[i][0], sh_cs[i][1]);
+                    }
+                } else {      // elements 2i and 2i + 1, below n_rot
+                    // No branch per pair: el0 differs from lane to lane, and a branch around each pair's table
+                    // read makes the wave wait out sixteen LDS round trips one after the other (1.7 us of a
+                    // Llama-3-8B launch).  Every lane reads an entry (its own, or the table's last), all reads
+                    // go out together, and a pair past n_rot keeps its values by a select.
+                    const int last = max(a.n_rot / 2 - 1, 0); // (n_rot = 0: nothing is rotated, entry 0 is read and not used)
+                    float2 cs0[4], cs1[4];
+    #pragma unroll
+                    for (int e = 0; e < 8; e += 2) {
+                        const int el0 = kk * 32 + grp * 8 + e, el1 = el0 + D / 2;
+                        cs0[e / 2] = *reinterpret_cast<const float2*>(sh_cs[min(el0 / 2, last)]);
+                        cs1[e / 2] = *reinterpret_cast<const float2*>(sh_cs[min(el1 / 2, last)]);
+                    }
+    #pragma unroll
+                    for (int e = 0; e < 8; e += 2) {
+                        const int el0 = kk * 32 + grp * 8 + e, el1 = el0 + D / 2;
+                        float a0 = x0[e], a1 = x0[e + 1], b0 = x1[e], b1 = x1[e + 1];
+                        rope_rotate(a0, a1, cs0[e / 2].x, cs0[e / 2].y);
+                        rope_rotate(b0, b1, cs1[e / 2].x, cs1[e / 2].y);
+                        x0[e] = el0 < a.n_rot ? a0 : x0[e];
+                        x0[e + 1] = el0 < a.n_rot ? a1 : x0[e + 1];
+                        x1[e] = el1 < a.n_rot ? b0 : x1[e];
+                        x1[e + 1] = el1 < a.n_rot ? b1 : x1[e + 1];
+                    }
+                }
+            };
             // (cos, sin) of pair i at the raw position, as the rotary kernel forms them
             // A table per wave (head_dim <= 128: a wave's 64 lanes cover the pairs), so that no wave
             // waits here for the others: the waves of a workgroup get their loads out at very
@@ -374,35 +518,30 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
 #pragma unroll
                 for (int kk = 0; kk < G::kSteps / 2; ++kk) rotate2(qf[kk], qf[kk + G::kSteps / 2], kk);
             }
-        }
-        // ---- query heads -> B operands, fp16 hi + lo ----
-        h8 qhi[G::kSteps], qlo[G::kSteps];
+            // ---- query heads -> B operands, fp16 hi + lo ----
 #pragma unroll
-        for (int kk = 0; kk < G::kSteps; ++kk) {
-            const float* x = qf[kk];
+            for (int kk = 0; kk < G::kSteps; ++kk) {
+                const float* x = qf[kk];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float xe = x[e] * qmul;
-                qhi[kk][e] = (_Float16)xe;
-                qlo[kk][e] = (_Float16)(xe - (float)qhi[kk][e]);
+                for (int e = 0; e < 8; ++e) {
+                    const float xe = x[e] * qmul;
+                    qhi[kk][e] = (_Float16)xe;
+                    qlo[kk][e] = (_Float16)(xe - (float)qhi[kk][e]);
+                }
             }
         }
-
         __builtin_amdgcn_sched_barrier(0);
         FA_STAMP(2);
         const int v_rd = (grp * 4 + (col >> 2)) * G::kRowBV + (col & 3) * 8; // + h*16 rows, + db*32 bytes
 
-        // (store, rotate + store) The new row is made ready here, while the tiles travel, by the one wave whose tiles
+        // (kRotateLate) The new row is made ready here, while the tiles travel, by the one wave whose tiles
         // include the row's (the last visible tile: the wave's own last): converted -- and the K row rotated -- as the
         // store kernel and the rotary kernel would, the pieces this lane is to substitute and to write kept in
         // registers.  At that tile only the substitution and the two cache writes are left.  (Made ready at the tile
         // itself, as it used to be, the LDS round trips and the rotation sat between the arrival of the launch's last
         // tile and its products: 0.7 us of a Qwen2.5-1.5B launch pair at 32k.)  The row's loads went out ahead of the
         // tile requests, so waiting for them waits for no tile.
-        const int own_tile = n_tiles - 1;
-        [[maybe_unused]] bool owner = false;
-        [[maybe_unused]] u32x4 k_new16[G::kSteps], v_new16 = u32x4{0u, 0u, 0u, 0u};
-        if constexpr (STORE) {
+        if constexpr (LATE) {
 #pragma unroll
             for (int kk = 0; kk < G::kSteps; ++kk) k_new16[kk] = u32x4{0u, 0u, 0u, 0u};
             int last = tile_first; // this wave's last tile (a few steps at most)
@@ -424,7 +563,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
                     // rotating the 32 elements it will hold was 250 instructions, 0.6 us of the launch whose last tile is
                     // this wave's.)
                     float x[4] = {here(k_raw.x), here(k_raw.y), here(k_raw.z), here(k_raw.w)};
-                    if constexpr (ROPE) {
+                    {
                         const int e0 = (lane % (D / 4)) * 4;
                         if (a.neox) {
                             const bool second = e0 >= D / 2;
@@ -478,9 +617,10 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
                 }
             }
         }
-
-        for (; tile < n_tiles; tile += tile_step) {
-            const bool more = tile + tile_step < n_tiles;
+        // One tile; `more`: another follows, which is asked for as its registers become free.  (Two copies, with and without: under a
+        // condition in one, the compiler's waits at the loop's top are for K and V both, and the products start with V's arrival.)
+        auto attend = [&](auto morec) {
+            constexpr bool more = decltype(morec)::value;
             if constexpr (STORE) {
                 if (owner && tile == own_tile) { // the tile of the new row: into the operand registers
                     const int row = pos % kTile;
@@ -491,9 +631,6 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
                             for (int t = 0; t < 2; ++t) // (constant register indices: a computed one sends the array to scratch memory)
                                 if (row / 16 == t) kreg[t * G::kSteps + kk] = k_new16[kk];
                     }
-#pragma unroll
-                    for (int i = 0; i < G::kLoads; ++i)
-                        if ((i * 64 + lane) / G::kChunksPerRow == row) vreg[i] = v_new16;
                 }
             }
             // ---- S^T = K Q^T : rows = KV row (sub-tile t, row col), columns = query head ----
@@ -510,7 +647,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
                 }
             s[0] += s2[0];
             s[1] += s2[1];
-            if (more) fetch_k(tile + tile_step); // the operand registers are free again
+            if constexpr (more) fetch_k(tile + tile_step); // the operand registers are free again
             FA_STAMP(3);
 
             // ---- softmax weights; lane (col, grp) holds rows t*16 + grp*4 + i of its column ----
@@ -519,12 +656,13 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
             for (int t = 0; t < 2; ++t)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) v[t * 4 + i] = s[t][i];
-            if (tile * kTile + kTile > npos) { // the last tile: rows past the position do not exist
+            const int rows_left = npos - tile * kTile; // rows of this tile below the position (>= 32: all)
+            if (rows_left < kTile) { // the last tile: rows past the position do not exist
+                const int lim = rows_left - grp * 4;
 #pragma unroll
                 for (int t = 0; t < 2; ++t)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        if (tile * kTile + t * 16 + grp * 4 + i >= npos) v[t * 4 + i] = -INFINITY;
+                    for (int i = 0; i < 4; ++i) v[t * 4 + i] = t * 16 + i < lim ? v[t * 4 + i] : -INFINITY;
             }
             float mx = fmaxf(fmaxf(v[0], v[1]), v[2]);
             mx = fmaxf(fmaxf(mx, v[3]), v[4]);
@@ -532,7 +670,9 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
             mx = xor_max(fmaxf(mx, v[7]));
             // move the reference only when this tile's maximum is far above it (or it is unset)
             const bool move = (mx - m_ref) * c2 > kLazy || (m_ref == -INFINITY && mx > -INFINITY);
-            if (__builtin_amdgcn_ballot_w64(move) != 0) {
+            if (tile == tile_first) { // (nothing summed up yet)
+                m_ref = mx > -INFINITY ? mx : m_ref;
+            } else if (__builtin_amdgcn_ballot_w64(move) != 0) {
                 const float alpha = move ? fast_exp2((m_ref - mx) * c2) : 1.0f; // unset reference -> 0
                 if (move) m_ref = mx;
                 l_run *= alpha;
@@ -550,16 +690,23 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
                 pl[e] = (_Float16)(pe - (float)ph[e]);
             }
 
+            __builtin_amdgcn_sched_barrier(0); // (the weights are made while V is still on its way)
             // ---- V: registers -> this wave's LDS slice (K was needed first and arrives first) ----
-            const int rows_left = npos - tile * kTile; // rows of this tile below the position (>= 32: all)
+            auto park_v = [&](auto whole) {
 #pragma unroll
-            for (int i = 0; i < G::kLoads; ++i) {
-                const int c = i * 64 + lane;
-                // rows at or past the position may hold anything; their weights are zero, and 0 * NaN is not
-                const u32x4 x = (c / G::kChunksPerRow) < rows_left ? vreg[i] : u32x4{0u, 0u, 0u, 0u};
-                *reinterpret_cast<u32x4*>(vs + (c / G::kChunksPerRow) * G::kRowBV + (c % G::kChunksPerRow) * 16) = x;
-            }
-            if (more) fetch_v(tile + tile_step);
+                for (int i = 0; i < G::kLoads; ++i) {
+                    const int c = i * 64 + lane;
+                    // rows at or past the position may hold anything; their weights are zero, and 0 * NaN is not
+                    const u32x4 x = decltype(whole)::value || (c / G::kChunksPerRow) < rows_left ? vreg[i] : u32x4{0u, 0u, 0u, 0u};
+                    *reinterpret_cast<u32x4*>(vs + (c / G::kChunksPerRow) * G::kRowBV + (c % G::kChunksPerRow) * 16) = x;
+                }
+            };
+            if (rows_left < kTile) park_v(std::false_type());
+            else park_v(std::true_type());
+            if constexpr (STORE) // the new row, over what its tile brought back
+                if (owner && tile == own_tile && lane < G::kChunksPerRow)
+                    *reinterpret_cast<u32x4*>(vs + (pos % kTile) * G::kRowBV + lane * 16) = v_new16;
+            if constexpr (more) fetch_v(tile + tile_step);
             wave_lds_sync();
 
             // ---- O^T += V^T P : rows = head_dim index, columns = query head, k = the tile's 32 KV rows
@@ -572,14 +719,35 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
                 o[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, ph, o[db], 0, 0, 0);
                 o[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pl, o[db], 0, 0, 0);
             }
-            wave_lds_sync(); // the slice is overwritten at the top of the next iteration
-        }
+            if constexpr (more) wave_lds_sync(); // the slice is overwritten by the next tile
+        };
+        for (; tile + tile_step < n_tiles; tile += tile_step) attend(std::true_type());
+        attend(std::false_type());
     } else { // (marks for the timeline build)
         FA_STAMP(1);
         FA_STAMP(2);
     }
 
     FA_STAMP(4);
+    if (wu == 1) { // one wave has had a tile: nothing to merge
+        if (wave != 0) return;
+        FA_STAMP(5); // (nothing to hand over, nobody to wait for)
+        FA_STAMP(6);
+        const float l_tot = xor_sum(l_run);
+        const int head = kvh * r + hl;
+        if (!valid) return;
+        const float inv = n_splits > 1 ? 1.0f : l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
+        float* const po = n_splits > 1 ? part_o + ((size_t)id * n_head + head) * D : dst + (size_t)head * D; // (no splits: dst is the output)
+#pragma unroll
+        for (int db = 0; db < G::kDBlk; ++db) *reinterpret_cast<f4*>(po + db * 16 + grp * 4) = o[db] * inv;
+        if (n_splits > 1 && grp == 0) {
+            const size_t mi = (size_t)head * n_splits + id;
+            part_ml[mi * 2 + 0] = (m_ref == -INFINITY) ? -INFINITY : m_ref * c2;
+            part_ml[mi * 2 + 1] = l_tot;
+        }
+        FA_STAMP(7);
+        return;
+    }
     // ---- merge the waves through LDS ----
     float* const ml = reinterpret_cast<float*>(smem + G::kMlOff);
     float* const obuf = reinterpret_cast<float*>(smem + wave * G::kWaveB);
@@ -720,16 +888,22 @@ __global__ __launch_bounds__(512) void fa_decode_combine_kernel(const float* __r
 
 template <int D>
 hipError_t launch(const FaArgs& a, hipStream_t stream) {
-    if (a.n_splits > 0xffff || a.r > 0xffff || a.n_hgroups > 0xffff) return hipErrorInvalidValue;
+    if (a.n_splits > 0x7fff || a.r > 0xffff || a.n_hgroups > 0xffff) return hipErrorInvalidValue;
     constexpr int lds = DGeom<D>::kLdsB;
     const dim3 g(a.n_kv, a.n_hgroups, a.n_splits), b(kDecodeWaves * 64);
-    const unsigned splits_r = (unsigned)a.n_splits | (unsigned)a.r << 16;
+    const unsigned splits_r = (unsigned)a.n_splits | (a.qsign < 0.0f ? 0x8000u : 0u) | (unsigned)a.r << 16;
+    unsigned scale;
+    memcpy(&scale, &a.c, sizeof(scale));
+    const bool rotate = a.k_new && a.n_rot > 0, table = rotate && a.rope_angles && a.n_rot == D;
+    const uint64_t scale_heads = table ? arg_ptr(a.rope_angles) : arg_pair(scale, (unsigned)a.n_head);
     float* const dst = a.n_splits > 1 ? a.part_o : a.out;
-#define ORIN_FA_SPLIT_ARGS a.d_pos, a.q, a.kc, a.vc, a.n_ctx, splits_r, a.c * a.qsign, dst, a.n_head, a
-    if (a.k_new && a.n_rot > 0) hipLaunchKernelGGL((fa_decode_split_kernel<D, 2>), g, b, lds, stream, ORIN_FA_SPLIT_ARGS);
-    else if (a.k_new) hipLaunchKernelGGL((fa_decode_split_kernel<D, 1>), g, b, lds, stream, ORIN_FA_SPLIT_ARGS);
-    else hipLaunchKernelGGL((fa_decode_split_kernel<D, 0>), g, b, lds, stream, ORIN_FA_SPLIT_ARGS);
-#undef ORIN_FA_SPLIT_ARGS
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, g, b, lds, stream, a.d_pos, a.q, a.kc, a.vc, a.n_ctx, splits_r, scale_heads, dst, a); };
+    if (table && a.neox) go(fa_decode_split_kernel<D, kRotateNeox>);
+    else if (table) go(fa_decode_split_kernel<D, kRotate>);
+    else if (rotate) go(fa_decode_split_kernel<D, kRotateLate>);
+    else if (a.k_new) go(fa_decode_split_kernel<D, kStore>);
+    else go(fa_decode_split_kernel<D, kPlain>);
+
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess || a.n_splits == 1 || kProbeNoCombine) return e;
     const dim3 cgrid(a.n_head * (D / 64));
@@ -762,12 +936,15 @@ hipError_t allow_lds() {
 
 hipError_t decode_allow_lds() {
     hipError_t e;
-    if ((e = allow_lds<128, 0>()) != hipSuccess) return e;
-    if ((e = allow_lds<128, 1>()) != hipSuccess) return e;
-    if ((e = allow_lds<128, 2>()) != hipSuccess) return e;
-    if ((e = allow_lds<64, 0>()) != hipSuccess) return e;
-    if ((e = allow_lds<64, 1>()) != hipSuccess) return e;
-    return allow_lds<64, 2>();
+    auto all = [&](auto dc) {
+        constexpr int D = decltype(dc)::value;
+        if ((e = allow_lds<D, kPlain>()) != hipSuccess) return e;
+        if ((e = allow_lds<D, kStore>()) != hipSuccess) return e;
+        if ((e = allow_lds<D, kRotate>()) != hipSuccess) return e;
+        if ((e = allow_lds<D, kRotateNeox>()) != hipSuccess) return e;
+        return allow_lds<D, kRotateLate>();
+    };
+    return all(IntC<128>{}) != hipSuccess ? e : all(IntC<64>{});
 }
 
 hipError_t decode_stamps(long long* host, size_t n) {

@@ -328,6 +328,53 @@ def test_decode_rope_store_over_a_sweep_of_positions(fa, H, G, d, n_ctx, neox):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("H,G,d,n_ctx,neox,sign", [
+    (12, 2, 128, 4096, True, 1), (32, 8, 128, 16384, False, -1),   # (up to two turns of all splits)
+    (32, 2, 128, 2048, True, -1), (32, 2, 64, 2048, False, 1),     # sixteen heads: every wave has some of the query
+    (40, 2, 128, 8192, False, 1), (3, 3, 128, 200, True, 1),       # two head groups; one head a group, a cache of one split
+    (32, 8, 64, 32768, True, 1), (7, 1, 64, 1024, True, 1),
+])
+def test_decode_rope_store_with_a_table_over_runs_of_every_length(fa, H, G, d, n_ctx, neox, sign):
+    """With the caller's table of angles (8-byte aligned, no more), from one replayed graph: as many waves of a split with a tile as can
+    be, one to eight, the new row in the first of them, the last, and tiles of later turns; the four calls bit for bit."""
+    import torch
+    scale, theta = sign * float(1.0 / np.sqrt(d)), 1.0e6
+    rng = np.random.default_rng(H + n_ctx + d)
+    ka = torch.from_numpy(rng.standard_normal((G, n_ctx, d)).astype(np.float16).view(np.int16)).cuda()
+    va = torch.from_numpy(rng.standard_normal((G, n_ctx, d)).astype(np.float16).view(np.int16)).cuda()
+    kb, vb = ka.clone(), va.clone()
+    q, k_new, v_new = torch.zeros((H, d), device="cuda"), torch.zeros((G, d), device="cuda"), torch.zeros((G, d), device="cuda")
+    dpos = torch.zeros(1, dtype=torch.int32, device="cuda")
+    angles = torch.zeros((d // 2 + 1, 2), device="cuda")[1:]
+    out_a, out_b = torch.empty((H, d), device="cuda"), torch.empty((H, d), device="cuda")
+    rope_ind = fa.rope_neox_ind if neox else fa.rope_normal_ind
+    g = torch.cuda.CUDAGraph()
+    try:
+        with torch.cuda.graph(g):
+            fa.set_stream(torch.cuda.current_stream().cuda_stream)
+            fa.rope_angles_ind(angles, d, theta, dpos, None)
+            fa.flash_attention_decode_rope_store_ind(q, k_new, v_new, kb, vb, out_b, H, G, d, n_ctx, dpos, scale, d, theta, None, neox, angles)
+    finally:
+        fa.set_stream(torch.cuda.current_stream().cuda_stream)
+    turn = 32 * fa.lib().orin_fa_decode_splits(H, G, d, n_ctx)   # rows of a tile for every split
+    positions = sorted({p for w in range(1, 18) for p in (turn * w - 33, turn * w - 1, turn * w, turn * w + 70) if 0 <= p < n_ctx}
+                       | {0, 31, 32, n_ctx - 1, n_ctx, -1})
+    for pos in positions:
+        for t, k in ((q, 1.0), (k_new, 3.0), (v_new, 3.0)):
+            t.copy_(torch.from_numpy(rng.standard_normal(tuple(t.shape)).astype(np.float32) * k))
+        dpos.fill_(pos)
+        q_rot, k_rot = q.clone(), k_new.clone()
+        rope_ind(q_rot, H, d, d, theta, dpos, None)
+        rope_ind(k_rot, G, d, d, theta, dpos, None)
+        fa.kv_store_ind(ka, va, k_rot, v_new, G, d, n_ctx, dpos)
+        fa.flash_attention_decode_ind(q_rot, ka, va, out_a, H, G, d, n_ctx, dpos, scale)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(ka, kb) and torch.equal(va, vb), pos
+        assert torch.equal(out_a.view(torch.int32), out_b.view(torch.int32)), pos
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("H,G,d,n_ctx,n_past,batch,n_rot,neox,ff", [
     (12, 2, 128, 4096, 3584, 512, 128, True, False),   # Qwen2.5-1.5B chunk
     (32, 8, 128, 1024, 100, 300, 128, False, True),    # Llama-3 ("normal" pairing, frequency factors)
