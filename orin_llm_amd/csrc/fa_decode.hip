@@ -505,8 +505,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
                     float freq = rope_freq_of(a.freq, lane);
                     if (a.freq_factors) freq /= ff_given;
                     const float ang = (float)pos * freq;
-                    cs_given.x = cosf(ang);
-                    cs_given.y = sinf(ang);
+                    sincosf(ang, &cs_given.y, &cs_given.x);
                 }
                 sh_cs[lane][0] = cs_given.x;
                 sh_cs[lane][1] = cs_given.y;
