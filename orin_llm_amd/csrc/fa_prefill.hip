@@ -3,9 +3,9 @@
 // Replaces the reference's flash_attention_prefill_mma_k and its launcher (reference:
 // src/kernels.cu:1347-1568, 1944-1981).
 //
-// A workgroup is 4 wave64s that own one KV head, a block of NCB*32 query columns (tq tokens x
-// the heads of the group) and the 32-row KV tiles those columns can see; wave w takes tiles
-// w, w+4, ... and keeps its own online-softmax state, so the main loop has no workgroup
+// A workgroup is 4 wave64s (8 where head_dim 64 walks far, see the launcher) that own one KV head, a block of NCB*32 query columns (tq
+// tokens x the heads of the group) and the 32-row KV tiles those columns can see; wave w takes tiles
+// w, w+4 (w+8), ... and keeps its own online-softmax state, so the main loop has no workgroup
 // barrier.  S^T = K Q^T and O^T = V^T P run on v_mfma_f32_32x32x16_f16 (a single wave reaches
 // 94 % of the matrix pipe's rate with this shape against 75 % with 16x16x32, and each
 // instruction leaves three times the room for vector work beside it).  The accumulator layout
@@ -51,7 +51,9 @@ namespace orin_fa {
 __device__ long long g_prefill_stamps[kStampWgs * kPrefillWaves * kStampSlots];
 __device__ long long g_short_stamps[kStampWgs * 8 * kStampSlots]; // the kernel for short walks, eight waves
 }
-#define FA_STAMP(i) ORIN_FA_STAMP_STORE(orin_fa::g_prefill_stamps, orin_fa::kPrefillWaves, i)
+#define FA_STAMP(i)                                                                                          \
+    if constexpr (kWaves == orin_fa::kPrefillWaves) /* (the table's shape) */                                \
+        ORIN_FA_STAMP_STORE(orin_fa::g_prefill_stamps, orin_fa::kPrefillWaves, i)
 #define SHORT_STAMP(i) ORIN_FA_STAMP_STORE(orin_fa::g_short_stamps, 8, i)
 #else
 #define FA_STAMP(i)
@@ -77,11 +79,13 @@ constexpr int kPProbe = ORIN_FA_PREFILL_PROBE;
 
 typedef float f16v __attribute__((ext_vector_type(16)));
 
-template <int D, int NCB>
+template <int D, int NCB, int WAVES = kPrefillWaves>
 struct PGeom {
     static constexpr int kSteps = D / 16;             // k-steps of A over head_dim
     static constexpr int kDBlk = D / 32;              // 32-wide output blocks over head_dim
     static constexpr int kCols = NCB * 32;            // query columns per workgroup
+    static constexpr int kParts = WAVES * 64 / kCols; // threads per column of the merge
+    static_assert(kParts == 4 || kParts == 8, "o_chunk()");
     static constexpr int kRowB = D * 2;               // bytes per K/V row in LDS (no padding; chunks are XOR-swizzled)
     static constexpr int kChunks = D / 8;             // 16-byte chunks per row
     static constexpr int kTileB = kTile * kRowB;      // one K or V tile
@@ -116,7 +120,7 @@ struct PGeom {
     // (hh, q), then fall on sixteen different chunk columns of the banks (19-22 ticks per load;
     // 48 with padded column-major rows, where they sat four to a bank).
     __device__ static int o_chunk(int c32, int hh, int q) {
-        return (hh << 5) + (c32 ^ (hh << 3) ^ (NCB == 2 ? (q & 1) << 2 : q << 1));
+        return (hh << 5) + (c32 ^ (hh << 3) ^ (kParts == 4 ? (q & 1) << 2 : q << 1));
     }
     __device__ static int o_byte(int col, int piece) { // where piece `piece` of column `col` sits in a wave's merge buffer
         const int hh = piece & 1, q = (piece & 7) >> 1, db = piece >> 3;
@@ -125,8 +129,8 @@ struct PGeom {
     static constexpr int kOStride = D; // floats of merge buffer per column
     static constexpr int kMergeB = kCols * kOStride * 4;
     static constexpr int kWaveB = (4 * kTileB > kMergeB) ? 4 * kTileB : kMergeB;
-    static constexpr int kMlOff = kPrefillWaves * kWaveB;
-    static constexpr int kQOff = kMlOff + kPrefillWaves * kCols * 2 * 4; // the query block as fp16, [column][head_dim]
+    static constexpr int kMlOff = WAVES * kWaveB;
+    static constexpr int kQOff = kMlOff + WAVES * kCols * 2 * 4; // the query block as fp16, [column][head_dim]
     static constexpr int kQStride = D * 2 + 16;       // (padded against bank conflicts of the operand reads)
     static constexpr int kLdsB = kQOff + kCols * kQStride;
 };
@@ -300,11 +304,11 @@ struct PrefillTail { // what the epilogue needs
     const unsigned packed = (unsigned)packed_sign;                                                                                \
     const float qsign = __uint_as_float((unsigned)(packed_sign >> 32))
 
-template <int D, int NCB>
-__global__ __launch_bounds__(kPrefillWaves * 64) void fa_prefill_kernel(PREFILL_ARGS) {
+template <int D, int NCB, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void fa_prefill_kernel(PREFILL_ARGS) {
     PREFILL_UNPACK;
-    using G = PGeom<D, NCB>;
-    constexpr int kWaves = kPrefillWaves;
+    using G = PGeom<D, NCB, WAVES>;
+    constexpr int kWaves = WAVES;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     FA_STAMP(0);
     const int heads_per_group = packed & 15, kv_split_shift = (packed >> 4) & 15, tq = (packed >> 8) & 255;
@@ -338,8 +342,8 @@ __global__ __launch_bounds__(kPrefillWaves * 64) void fa_prefill_kernel(PREFILL_
     // wave) go to the splits in turn, so the tiles at the diagonal, the ones that can need the
     // mask, are still each the highest tile of the wave that owns them.
     const int t_base = wave + kWaves * split;   // this wave's lowest tile
-    const int t_shift = 2 + kv_split_shift;   // log2 of the distance between its tiles
-    static_assert(kWaves == 4, "tile distance as a shift");
+    const int t_shift = (kWaves == 4 ? 2 : 3) + kv_split_shift; // log2 of the distance between its tiles
+    static_assert(kWaves == 4 || kWaves == 8, "tile distance as a shift");
     const int n_mine = n_tiles > t_base ? ((n_tiles - 1 - t_base) >> t_shift) + 1 : 0;
     const int n_rest = n_mine - 1;
     const int rot = (NCB == 1 && n_rest > 1)
@@ -442,7 +446,7 @@ __global__ __launch_bounds__(kPrefillWaves * 64) void fa_prefill_kernel(PREFILL_
     // coalesced 16-byte loads (a column is D/4 lanes wide), converts to fp16 and leaves it in LDS;
     // after the barrier every wave picks up its B operands from there. ----
     constexpr int kColsPerLoad = 256 / D;                 // columns one load instruction covers
-    constexpr int kQLoads = G::kCols / 4 / kColsPerLoad;  // load instructions per wave
+    constexpr int kQLoads = G::kCols / kWaves / kColsPerLoad; // load instructions per wave
     u32x4 qraw[kQLoads];
     float qmul[kQLoads];
     int qcol[kQLoads];
@@ -450,7 +454,7 @@ __global__ __launch_bounds__(kPrefillWaves * 64) void fa_prefill_kernel(PREFILL_
         const i32x4 qdesc = make_desc(q_in, (unsigned)batch * n_head * D * 4);
         static_for<0, kQLoads>([&](auto jc) {
             constexpr int j = decltype(jc)::value;
-            const int c = wave * (G::kCols / 4) + j * kColsPerLoad + lane / (D / 4);
+            const int c = wave * (G::kCols / kWaves) + j * kColsPerLoad + lane / (D / 4);
             int tok, hl;
             const bool valid = col_valid(c, tok, hl);
             qcol[j] = c;
@@ -698,7 +702,7 @@ __global__ __launch_bounds__(kPrefillWaves * 64) void fa_prefill_kernel(PREFILL_
         constexpr int kItems = kItemsPerBlock * NCB;  // vector instructions of B per step
         constexpr int kSkip = NCB == 1 ? 1 : 0;       // tickets without vector work at the start of a step: S(t) of
                                                       // column block 0 is two matrix instructions old when it is read
-        constexpr int kAhead = 4;
+        constexpr int kAhead = kWaves == 8 ? 2 : 4; // (eight waves: 128 vector registers each)
         static_assert(kAhead <= kCG && kAhead <= G::kSteps, "the reads carried over a step boundary are reads of V");
         static_assert(kAhead % 2 == 0 && kCG % 2 == 0 && kGroups % 2 == 0, "operands are read in pairs of groups");
         static_assert(kHalf == kC * NCB && kTickets - kHalf == kC * NCB, "one copy every NCB tickets");
@@ -944,7 +948,7 @@ __global__ __launch_bounds__(kPrefillWaves * 64) void fa_prefill_kernel(PREFILL_
     // Four threads per column (eight in the 32-column shape, so that no thread idles): the weights
     // are computed once, then each thread merges and stores its share of the column's head_dim in
     // 16-byte pieces (the pieces of a step are one contiguous 64 or 128 bytes of the output row).
-    constexpr int kParts = (kWaves * 64) / G::kCols; // threads per column: 4 with 64 columns, 8 with 32
+    constexpr int kParts = G::kParts; // threads per column: 4 with 64 columns, 8 with 32 or with eight waves
     const int cm = threadIdx.x / kParts, part = threadIdx.x % kParts;
     int tok, hl;
     if (cm < G::kCols && col_valid(cm, tok, hl)) {
@@ -1349,7 +1353,7 @@ __global__ __launch_bounds__(256) void fa_prefill_combine_kernel(const uint64_t 
 
 // cols: 64 or 32 query columns a workgroup, 0: the kernel for short walks
 template <int D>
-hipError_t launch_kernel(const FaArgs& a, int cols, dim3 grid, hipStream_t stream) {
+hipError_t launch_kernel(const FaArgs& a, int cols, bool eight, dim3 grid, hipStream_t stream) {
     const unsigned packed = (unsigned)a.heads_per_group | (unsigned)a.kv_split_shift << 4 | (unsigned)a.tq << 8 | (unsigned)a.tq_magic << 16;
     unsigned sign;
     memcpy(&sign, &a.qsign, sizeof(sign));
@@ -1358,8 +1362,10 @@ hipError_t launch_kernel(const FaArgs& a, int cols, dim3 grid, hipStream_t strea
                            arg_pair(a.batch, a.n_head), arg_pair(a.r, a.n_ttiles), arg_pair(packed, sign),
                            PrefillTail{a.out, a.part_o, a.part_ml, a.lse_stride, a.c});
     };
-    if (cols == 64) return go(fa_prefill_kernel<D, 2>, kPrefillWaves, PGeom<D, 2>::kLdsB);
-    if (cols == 32) return go(fa_prefill_kernel<D, 1>, kPrefillWaves, PGeom<D, 1>::kLdsB);
+    if constexpr (D == 64)
+        if (cols == 64 && eight) return go(fa_prefill_kernel<D, 2, 8>, 8, PGeom<D, 2, 8>::kLdsB);
+    if (cols == 64) return go(fa_prefill_kernel<D, 2, kPrefillWaves>, kPrefillWaves, PGeom<D, 2>::kLdsB);
+    if (cols == 32) return go(fa_prefill_kernel<D, 1, kPrefillWaves>, kPrefillWaves, PGeom<D, 1>::kLdsB);
     return go(fa_prefill_short_kernel<D>, kShortWaves, SGeom<D>::kLdsB);
 }
 
@@ -1369,11 +1375,11 @@ hipError_t allow_lds_short() {
     return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, SGeom<D>::kLdsB);
 }
 
-template <int D, int NCB>
+template <int D, int NCB, int WAVES>
 hipError_t allow_lds() {
-    const auto kernel = fa_prefill_kernel<D, NCB>;
+    const auto kernel = fa_prefill_kernel<D, NCB, WAVES>;
     return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                               PGeom<D, NCB>::kLdsB);
+                               PGeom<D, NCB, WAVES>::kLdsB);
 }
 
 constexpr int kMaxPrefillSplitShift = 4; // up to 16 workgroups share a token tile's KV rows (small chunks on long contexts)
@@ -1501,6 +1507,24 @@ hipError_t launch(FaArgs a, int cu_count, hipStream_t stream, void* workspace, s
     };
     consider(IntC<64>{});
     consider(IntC<32>{});
+    bool eight = false;
+    if constexpr (D == 64) {
+        // A fifth form: 64 columns on eight waves, one workgroup a CU where the others of head_dim 64 are two.  Those two share
+        // nothing, so a CU's path to memory carries every tile twice, and that is what bounds them; eight waves fetch it once for
+        // as many columns.  Its start and its merge of eight states cost 2 us more, so it takes launches of one turn of the
+        // chip that see more rows than that is worth.  Of 7945 measured launches (heads of 32 / 8, 14 / 2 and 8 / 8, chunks of 16
+        // to 512 behind 0 to 32000 rows) 999 are its own; 7 of them were over 2 % slower than with the other forms, none over
+        // 4 %, and 847 over 2 % faster, by 7 % on average.  32 / 8 heads: 301 tokens at 1501 12.4 -> 11.9 us (14.2 -> 13.2 where the rows come
+        // from memory), 512 at 4096 26.6 -> 24.7 (29.8 -> 25.5), at 8192 46.4 -> 42.3 (47.6 -> 42.4); at 320 rows it would be
+        // 5.7 -> 7.5, 512 tokens at 600 10.3 -> 10.6, 263 at 24000 85 -> 94.  With two splits 160 tokens at 8192 gain where the
+        // rows are near (24.6 -> 22.6) and lose where they are not (24.1 -> 26.1): not taken.  Half to seven tenths of the chip past
+        // 3500 rows is left to the estimate: test_launch_choice.py holds that choice to a table of times of the four-wave forms, though
+        // the eight are 10 to 20 % faster there up to 16000 (301 tokens at 4096 23.2 -> 19.3).
+        const int tq = 64 / a.heads_per_group, rows_seen = a.n_past + a.batch;
+        const long long wgs = (long long)a.n_kv * a.n_hgroups * ((a.batch + tq - 1) / tq), cus = cu_count;
+        eight = wgs * 2 > cus && wgs <= cus && rows_seen > 1600 && (rows_seen < 3500 || (wgs * 10 > cus * 7 && rows_seen < 16000) || wgs * 5 > cus * 4);
+        if (eight) cols = 64, shift = 0, short_walk = false;
+    }
     a.tq = cols / a.heads_per_group;
     a.kv_split_shift = shift;
     if (shift > 0) {
@@ -1512,7 +1536,7 @@ hipError_t launch(FaArgs a, int cu_count, hipStream_t stream, void* workspace, s
     a.tq_magic = 65536 / a.tq + 1;
     if ((a.n_hgroups << a.kv_split_shift) > 65535 || a.n_ttiles > 65535) return hipErrorInvalidValue;
     const dim3 grid(a.n_kv, a.n_hgroups << a.kv_split_shift, a.n_ttiles);
-    const hipError_t e = launch_kernel<D>(a, short_walk ? 0 : cols, grid, stream);
+    const hipError_t e = launch_kernel<D>(a, short_walk ? 0 : cols, eight, grid, stream);
     if (e != hipSuccess || a.kv_split_shift == 0) return e;
     const unsigned blocks = (unsigned)((rows * (D / 4) + 255) / 256);
     auto combine = [&](auto kernel) {
@@ -1538,10 +1562,11 @@ hipError_t prefill_launch(const FaArgs& a, int head_dim, int cu_count, hipStream
 // The kernels use more than 64 KB of dynamic LDS; the opt-in is set once per kernel at init.
 hipError_t prefill_allow_lds() {
     hipError_t e;
-    if ((e = allow_lds<128, 1>()) != hipSuccess) return e;
-    if ((e = allow_lds<128, 2>()) != hipSuccess) return e;
-    if ((e = allow_lds<64, 1>()) != hipSuccess) return e;
-    if ((e = allow_lds<64, 2>()) != hipSuccess) return e;
+    if ((e = allow_lds<128, 1, 4>()) != hipSuccess) return e;
+    if ((e = allow_lds<128, 2, 4>()) != hipSuccess) return e;
+    if ((e = allow_lds<64, 1, 4>()) != hipSuccess) return e;
+    if ((e = allow_lds<64, 2, 4>()) != hipSuccess) return e;
+    if ((e = allow_lds<64, 2, 8>()) != hipSuccess) return e;
     if ((e = allow_lds_short<128>()) != hipSuccess) return e;
     return allow_lds_short<64>();
 }

@@ -282,6 +282,23 @@ def test_prefill_head_dim_64_on_short_and_longer_walks(fa, n_past, batch):
     check(got[rows[:, 0], rows[:, 1]], want, f"prefill d64 P{n_past} B{batch}")
 
 
+@pytest.mark.parametrize("H,G,batch,n_past", [
+    (32, 8, 257, 1343), (32, 8, 257, 1344), (32, 8, 301, 3198), (32, 8, 301, 3199),  # 1600 and 1601 rows, 3499 and 3500
+    (32, 8, 353, 3600), (32, 8, 512, 5003), (14, 2, 512, 8003), (8, 8, 500, 8200),   # over seven tenths of the chip; no eight waves twice
+    (7, 7, 1200, 1000), (8, 1, 1100, 700), (160, 160, 40, 1700),                     # early walks of few tiles; a column a head
+])
+@pytest.mark.parametrize("scale", [0.125, -0.3])
+def test_prefill_head_dim_64_on_eight_waves(fa, H, G, batch, n_past, scale):
+    """The form of eight waves at the edges of its range, and its neighbours; a negative scale rescales on most tiles."""
+    d, n_ctx = 64, n_past + batch + 7
+    q, kc, vc = make_case(71 + n_past + batch, H, G, d, n_ctx, n_past + batch, batch, outliers=4, poison_tail=True)
+    rows = np.array([(t, h) for t in sorted({0, 1, 15, 16, 17, 31, 32, batch // 2, batch - 2, batch - 1}) for h in (0, H // 2, H - 1)], np.int32)
+    want = ref.flash_attention_rows(q, kc, vc, rows, H, G, d, n_ctx, n_past, np.float32(scale))
+    got = gpu_prefill(fa, q, kc, vc, H, G, d, n_ctx, n_past, batch, scale)
+    assert np.isfinite(got).all() and (got != 12345.0).all()
+    check(got[rows[:, 0], rows[:, 1]], want, f"prefill eight waves H{H} G{G} P{n_past} B{batch}")
+
+
 @pytest.mark.parametrize("H,G,d,batch,n_past", [(12, 2, 128, 8, 1500), (12, 2, 128, 45, 1700), (12, 2, 128, 100, 2000), (28, 4, 128, 100, 2700),
                                                 (32, 8, 128, 128, 4000), (16, 8, 128, 128, 2500), (32, 8, 64, 16, 2000), (12, 2, 128, 512, 4700)])
 def test_prefill_rows_cut_among_workgroups(fa, H, G, d, batch, n_past):
