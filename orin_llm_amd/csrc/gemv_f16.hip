@@ -12,9 +12,14 @@
 //   * The matrices of a launch (q, k, v) are one sequence of batches, so that workgroups get equal shares of all of them.
 //     (As rows of the grid, two of three 1024-row matrices kept 512 workgroups each busy for two rows.)
 //   * The RMS norm is folded in as in gemv_mfma.hip: products of x w, the norm's scalar applied to the finished sums.
-// Llama-3-8B's shapes, per launch, before -> now: q, k, v 34.1 -> 11.2 us (50 MB), output projection 11.9 -> 8.0 (34 MB), gate/up
-// 47.7 -> 40.8 (235 MB, 5.75 TB/s: what a plain read reaches), down 25.0 -> 21.7 us (117 MB).
+// What a workgroup needs ahead of its first request is in registers when it starts, rows are addressed by descriptors in scalar registers, so
+// that nothing waits for a load but its use, and a launch of one matrix asks nothing of which one (kMulti).
+// Llama-3-8B's shapes, per launch, with gemv.hip's kernel -> now: q, k, v 34.1 -> 10.65 us (50 MB), output projection 11.9 -> 7.65 (34 MB),
+// gate/up 47.7 -> 37.0 (235 MB, 6.35 TB/s: what the fastest plain read of that size reaches), down 25.0 -> 20.5 us (117 MB, 5.7).
+// Rows beyond 16384 elements are the exception: 3584 of 18944 took 22.3 before the last change and take 22.9, the model's other launches 1 to 3 % less.
 #include "layer_common.hpp"
+
+#include <type_traits>
 
 namespace orin_fa {
 namespace {
@@ -22,21 +27,20 @@ namespace {
 constexpr int kRun = 512;      // elements of a row that a wave's load instruction covers
 constexpr int kMostRuns = 8;   // of a row, per wave
 
-struct F16Args {
-    GemvArgs g;
-    int batches[3]; // of each matrix
-};
-
 __device__ __forceinline__ void lds_meet() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // RUNS: runs of a row per wave.  RB: rows of a matrix in a batch.
-template <int RUNS, int RB, bool DUAL, int kWaves>
-__global__ __launch_bounds__(kWaves * 64) void gemv_f16_kernel(const F16Args a) {
+// What the first requests need comes in the leading arguments, in registers when a wave starts: the matrices (w1: of two that become
+// one product the second), the batches that end with the first matrix, with the second and with the last, and
+//   shape   n_in, 16 bits | rows of each matrix's last batch - 1, 4 bits each
+template <int RUNS, int RB, bool DUAL, int kWaves, bool kMulti>
+__global__ __launch_bounds__(kWaves * 64) void gemv_f16_kernel(const uint64_t w0, const uint64_t w1, const uint64_t w2, const float* x_in, const float* norm_w,
+                                                              const unsigned b01, const unsigned b012, const unsigned total, const unsigned shape, const GemvArgs a) {
     constexpr int M = DUAL ? 2 : 1, R = M * RB;
     __shared__ float sh_part[2][kWaves][R];
     __shared__ float sh_ss[kWaves];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int n_in = a.g.n_in;
+    const int n_in = (int)(shape & 0xffffu);
     const unsigned row_bytes = (unsigned)n_in * 2u;
 
     unsigned off[RUNS]; // of this lane's 16 bytes of each run; past the row's end: its last 16 bytes, whose products are discarded
@@ -46,24 +50,39 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_f16_kernel(const F16Args a) 
     // (the launcher's RUNS is the smallest that covers the row: only a wave's last run can reach past its end)
     const bool last_live = ((RUNS - 1) * kWaves + wave) * kRun + lane * 8 < n_in;
 
-    const int b01 = a.batches[0], b012 = b01 + a.batches[1], total = b012 + a.batches[2];
-    auto seg_of = [&](int b, int& row) {
-        const int s = b < b01 ? 0 : b < b012 ? 1 : 2;
-        row = (b - (s == 0 ? 0 : s == 1 ? b01 : b012)) * RB;
-        return s;
+    struct Batch {
+        int seg, row, rows;      // matrix, first row, rows of it
+        unsigned second, third;  // all ones where it is of the second matrix or behind it, of the third
+    };
+    auto past = [](unsigned b, unsigned limit) { return 0u - ((unsigned)(limit - b) >> 31); }; // all ones where b > limit (both below 2^31)
+    // (Captured by value: by reference the choices become loads from the stack.  And as masks of words: a comparison's outcome becomes a
+    // number by way of a vector register, and what follows from it then stays in those.)
+    auto batch_of = [b01, b012, total, shape, past](unsigned b) {
+        if constexpr (!kMulti) {
+            const unsigned last = past(b, total - 2u);
+            return Batch{0, (int)b * RB, RB == 1 ? 1 : (int)((shape >> 16 & 15u & last) | ((RB - 1u) & ~last)) + 1, 0u, 0u};
+        }
+        const unsigned second = past(b, b01 - 1u), third = past(b, b012 - 1u); // all ones or zero
+        const unsigned first = (b01 & second & ~third) | (b012 & third), end = (b01 & ~second) | (b012 & second & ~third) | (total & third);
+        const unsigned last = past(b, end - 2u), seg = (second & 1u) + (third & 1u);
+        return Batch{(int)seg, (int)(b - first) * RB, (int)((shape >> (16u + 4u * seg) & 15u & last) | ((RB - 1u) & ~last)) + 1, second, third};
     };
     h8 w[2][M][RB][RUNS];
-    auto request = [&](h8 (&r)[M][RB][RUNS], int b) {
-        int row;
-        const int s = seg_of(min(b, total - 1), row); // (past the end: the last batch once more; never used)
-        const GemvSeg& seg = a.g.seg[s];
+    auto request = [w0, w1, w2, total, row_bytes, &off, batch_of, past](h8 (&r)[M][RB][RUNS], unsigned b) {
+        b = min(b, total - 1); // (past the end: the last batch once more; never used)
+        const Batch t = batch_of(b);
+        const uint64_t second = (uint64_t)(int64_t)(int)t.second, third = (uint64_t)(int64_t)(int)t.third;
+        const uint64_t mine = !kMulti ? w0 : (w0 & ~second) | (w1 & second & ~third) | (w2 & third);
 #pragma unroll
         for (int m = 0; m < M; ++m)
 #pragma unroll
             for (int i = 0; i < RB; ++i) {
-                const unsigned char* const p = static_cast<const unsigned char*>(m ? a.g.w_up : seg.w) + (size_t)min(row + i, seg.n_out - 1) * row_bytes;
+                // (The row's address as a descriptor's base, in scalar registers: an address in vector registers takes some that loads
+                // under way return to, and the wait for them puts an end to two batches on their way.  A row that is not there is one of
+                // no bytes.)
+                const auto rsrc = make_rsrc(ptr_arg<const unsigned char>(m ? w1 : mine) + (size_t)(unsigned)(t.row + i) * row_bytes, i == 0 ? row_bytes : row_bytes & past((unsigned)t.rows, (unsigned)i));
 #pragma unroll
-                for (int j = 0; j < RUNS; ++j) r[m][i][j] = __builtin_nontemporal_load(reinterpret_cast<const h8*>(p + off[j]));
+                for (int j = 0; j < RUNS; ++j) r[m][i][j] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off[j], 0, 2)); // (streaming)
             }
     };
     // the activation's loads first (loads return in order), then the first batch
@@ -73,9 +92,9 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_f16_kernel(const F16Args a) 
 #pragma unroll
         for (int j = 0; j < RUNS; ++j) {
             const int e = (int)(off[j] >> 1);
-            *reinterpret_cast<float4*>(x[j]) = *reinterpret_cast<const float4*>(a.g.x + e);
-            *reinterpret_cast<float4*>(x[j] + 4) = *reinterpret_cast<const float4*>(a.g.x + e + 4);
-            const float* const nw = a.g.norm_w ? a.g.norm_w + e : a.g.x + e; // (always a load)
+            *reinterpret_cast<float4*>(x[j]) = *reinterpret_cast<const float4*>(x_in + e);
+            *reinterpret_cast<float4*>(x[j] + 4) = *reinterpret_cast<const float4*>(x_in + e + 4);
+            const float* const nw = norm_w ? norm_w + e : x_in + e; // (always a load)
             *reinterpret_cast<float4*>(g[j]) = *reinterpret_cast<const float4*>(nw);
             *reinterpret_cast<float4*>(g[j] + 4) = *reinterpret_cast<const float4*>(nw + 4);
         }
@@ -89,17 +108,17 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_f16_kernel(const F16Args a) 
             for (int i = 0; i < 8; ++i) {
                 const float v = live ? x[j][i] : 0.0f;
                 ss += v * v;
-                x[j][i] = a.g.norm_w ? v * g[j][i] : v;
+                x[j][i] = norm_w ? v * g[j][i] : v;
             }
         }
     }
-    const bool has_norm = a.g.norm_w != nullptr;
+    const bool has_norm = norm_w != nullptr;
     if (has_norm) {
         ss = wave_sum(ss);
         if (lane == 0) sh_ss[wave] = ss; // (read behind the first batch's barrier)
     }
     int set = 0;
-    auto finish = [&](const h8 (&r)[M][RB][RUNS], int b) {
+    auto finish = [&](const h8 (&r)[M][RB][RUNS], unsigned b) {
 #pragma unroll
         for (int m = 0; m < M; ++m)
 #pragma unroll
@@ -115,10 +134,10 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_f16_kernel(const F16Args a) 
                 if (lane == 0) sh_part[set][wave][m * RB + i] = acc;
             }
         lds_meet();
-        int row0;
-        const GemvSeg& seg = a.g.seg[seg_of(b, row0)];
-        const int row = row0 + (int)threadIdx.x;
-        if ((int)threadIdx.x < RB && row < seg.n_out) {
+        const Batch t = batch_of(b);
+        if ((int)threadIdx.x < t.rows) {
+            const GemvSeg& seg = a.seg[t.seg];
+            const int row = t.row + (int)threadIdx.x;
             float v[M];
 #pragma unroll
             for (int m = 0; m < M; ++m) {
@@ -130,39 +149,52 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_f16_kernel(const F16Args a) 
                 float s2 = 0.0f;
 #pragma unroll
                 for (int u = 0; u < kWaves; ++u) s2 += sh_ss[u];
-                const float rinv = 1.0f / sqrtf(s2 / (float)n_in + a.g.eps);
+                const float rinv = 1.0f / sqrtf(s2 / (float)n_in + a.eps);
 #pragma unroll
                 for (int m = 0; m < M; ++m) v[m] *= rinv;
             }
             float y = v[0];
             if constexpr (DUAL) y = y / (1.0f + expf(-y)) * v[1]; // SiLU(gate) * up
             if (seg.bias) y += seg.bias[row];
-            if (a.g.accumulate) atomicAdd(seg.y + row, y); // (one writer a row: a plain sum, without waiting for y)
+            if (a.accumulate) atomicAdd(seg.y + row, y); // (one writer a row: a plain sum, without waiting for y)
             else seg.y[row] = y;
         }
         set ^= 1; // (two sets: one barrier a batch)
     };
-    for (int b = blockIdx.x; b < total; b += 2 * (int)gridDim.x) {
-        request(w[1], b + (int)gridDim.x);
+    for (unsigned b = blockIdx.x; b < total; b += 2 * gridDim.x) {
+        request(w[1], b + gridDim.x);
         finish(w[0], b);
-        if (b + (int)gridDim.x >= total) break;
-        request(w[0], b + 2 * (int)gridDim.x);
-        finish(w[1], b + (int)gridDim.x);
+        if (b + gridDim.x >= total) break;
+        request(w[0], b + 2 * gridDim.x);
+        finish(w[1], b + gridDim.x);
     }
 }
 
 template <int RUNS, bool DUAL, int kWaves>
 hipError_t launch_as(const GemvArgs& g, int cu_count, hipStream_t stream) {
-    // rows in a batch: about 4 KB a wave on their way beside what is being multiplied out
-    constexpr int RB = RUNS * (DUAL ? 2 : 1) <= 2 ? 4 / (RUNS * (DUAL ? 2 : 1)) : 1;
-    // workgroups that are resident at once: longer shares of a row take more registers
-    constexpr int kPerCu = kWaves == 8 ? 1 : RUNS >= 5 ? 2 : 3;
-    F16Args a{};
-    a.g = g;
-    int total = 0;
-    for (int i = 0; i < g.n_seg; ++i) total += a.batches[i] = (g.seg[i].n_out + RB - 1) / RB;
-    const int wgs = min(total, cu_count * kPerCu);
-    hipLaunchKernelGGL((gemv_f16_kernel<RUNS, RB, DUAL, kWaves>), dim3(wgs), dim3(kWaves * 64), 0, stream, a);
+    // Rows in a batch and workgroups a CU: some 64 KB a CU on their way, in few workgroups -- each fetches the activation and the norm's weights
+    // for itself, 4 waves of 8 KB to 14 KB in each of two batches.  us a launch, three workgroups a CU with half the rows a batch
+    // (two, of long rows, with one) -> this: Llama-3-8B's q, k, v 11.5 -> 10.65, output 8.25 -> 7.65, gate/up 41.0 -> 37.0 (6.35 TB/s),
+    // down 21.8 -> 20.5, logits 158.5 -> 155.2 (6.8 TB/s); two workgroups a CU with these batches 11.35, 8.35, 37.6, 21.6, 160.5.
+    constexpr int M = DUAL ? 2 : 1, RB = RUNS * M <= 8 && RUNS <= 4 ? 8 / (RUNS * M) : DUAL ? 1 : 2;
+    static_assert(RB <= 16, "rows of a batch: four bits of `shape`");
+    constexpr int kPerCu = kWaves == 1 ? 4 : kWaves < 4 ? 2 : 1;
+    unsigned ends[3] = {}, total = 0, shape = (unsigned)g.n_in;
+    for (int i = 0; i < 3; ++i) {
+        if (i < g.n_seg) {
+            total += (unsigned)(g.seg[i].n_out + RB - 1) / RB;
+            shape |= (unsigned)((g.seg[i].n_out - 1) % RB) << (16 + 4 * i);
+        }
+        ends[i] = total;
+    }
+    const unsigned wgs = min(total, (unsigned)(cu_count * kPerCu));
+    auto go = [&](auto multi) {
+        constexpr bool kMulti = !DUAL && decltype(multi)::value;
+        hipLaunchKernelGGL((gemv_f16_kernel<RUNS, RB, DUAL, kWaves, kMulti>), dim3(wgs), dim3(kWaves * 64), 0, stream, arg_ptr(g.seg[0].w),
+                           arg_ptr(g.w_up ? g.w_up : g.seg[1].w), arg_ptr(g.seg[2].w), g.x, g.norm_w, ends[0], ends[1], ends[2], shape, g);
+    };
+    if (g.n_seg > 1) go(std::true_type());
+    else go(std::false_type());
     return hipGetLastError();
 }
 
@@ -173,7 +205,9 @@ hipError_t launch_runs(const GemvArgs& g, int cu_count, hipStream_t stream) {
 
 } // namespace
 
-// Four waves a workgroup up to rows of 16384 elements, eight beyond (at most 32768).
+// As many waves a workgroup as a row has runs, four from there on up to rows of 16384 elements, eight beyond (at most 32768).
+// (Rows of two and three runs by four waves, the others idle, and by two and three, two workgroups a CU: 151936 rows of 1024 45.4 -> 41.0 us,
+// 4096 rows 4.84 -> 4.31; 151936 rows of 1536 62.6 -> 60.1, two matrices of 8960 11.54 -> 11.32.)
 hipError_t gemv_f16_launch(const GemvArgs& g, int cu_count, hipStream_t stream) {
     const int runs = (g.n_in + kRun - 1) / kRun;
     if (runs > 4 * kMostRuns) {
@@ -185,8 +219,13 @@ hipError_t gemv_f16_launch(const GemvArgs& g, int cu_count, hipStream_t stream) 
         default: return hipErrorInvalidValue;
         }
     }
+    switch (runs) {
+    case 1: return launch_runs<1, 1>(g, cu_count, stream);
+    case 2: return launch_runs<1, 2>(g, cu_count, stream);
+    case 3: return launch_runs<1, 3>(g, cu_count, stream);
+    case 4: return launch_runs<1, 4>(g, cu_count, stream);
+    }
     switch ((runs + 3) / 4) {
-    case 1: return launch_runs<1, 4>(g, cu_count, stream);
     case 2: return launch_runs<2, 4>(g, cu_count, stream);
     case 3: return launch_runs<3, 4>(g, cu_count, stream);
     case 4: return launch_runs<4, 4>(g, cu_count, stream);

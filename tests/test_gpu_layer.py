@@ -461,6 +461,40 @@ def test_f16_rows_in_runs(ly, n_in):
         assert vec_err(got[:n], want) < TOL_OP, what
 
 
+@pytest.mark.parametrize("n_in, heights", [
+    (512, (8200, 9, 1)), (544, (8199, 1, 8)), (1024, (4103, 4105, 7)), (1056, (4104, 15, 4097)), (1536, (4097, 8, 8)),
+    (1568, (2049, 4111, 6)), (2048, (2055, 2056, 2057)), (2080, (1029, 5, 3)), (6176, (515, 2, 513)), (14336, (513, 1, 3)), (18944, (513, 2, 1)),
+])
+def test_f16_batches_of_several_turns(ly, n_in, heights):
+    """One to eight waves a workgroup, batches of one to eight rows that end inside a matrix, one and several turns of the chip:
+    three matrices as one launch, one alone, the pair."""
+    import torch
+
+    rs = lm.Stream(8800 + n_in)
+    rows = sum(heights)
+    # (a few different rows, in an order without a period: the oracle's time)
+    kinds = np.array(lm.make_tensor(rs, lm.F16, n_in, 61)[1]).view(np.uint8).reshape(61, -1)
+    order = np.random.default_rng(n_in).integers(0, 61, rows + heights[0])
+    dev = dev_bytes(np.ascontiguousarray(kinds).reshape(-1))
+    dw = dev.view(61, -1)[torch.from_numpy(order).cuda()].contiguous()
+    x, nw = rs.sym(n_in, 1.0), (1.0 + rs.sym(n_in, 0.3)).astype(np.float32)
+    xn, dx = ref.rms_norm(x, nw, 1e-5), _dev(x)
+    want = ref.gemv(lm.F16, kinds.reshape(-1), xn, n_in, 61)[order]
+    plain = ref.gemv(lm.F16, kinds.reshape(-1), x, n_in, 61)[order]
+    ends = np.cumsum((0,) + heights)
+    ys, y1, yg = [out_buf(n) for n in heights], out_buf(heights[0]), out_buf(heights[0])
+    ly.gemv_multi(lm.F16, [dw[e:] for e in ends[:3]], None, ys, list(heights), dx, _dev(nw), 1e-5, n_in)
+    ly.gemv(lm.F16, dw, dx, y1, n_in, heights[0])
+    ly.gemv_norm_gate_up_swiglu(lm.F16, dw, dw[rows:], dx, _dev(nw), 1e-5, yg, n_in, heights[0])
+    torch.cuda.synchronize()
+    checks = [(f"matrix {i}", y, want[ends[i]:ends[i + 1]], n) for i, (y, n) in enumerate(zip(ys, heights))]
+    checks += [("alone", y1, plain[:heights[0]], heights[0]), ("gate/up", yg, ref.swiglu(want[:heights[0]], want[rows:]), heights[0])]
+    for what, y, w, n in checks:
+        got = y.cpu().numpy()
+        assert (got[n:] == 12345.0).all(), f"{what}: rows past n_out were written"
+        assert vec_err(got[:n], w.astype(np.float64)) < TOL_OP, what
+
+
 @pytest.mark.parametrize("n_in", [32, 512, 1536, 2080, 3584, 16416])
 def test_f16_an_infinite_weight_anywhere_in_a_row(ly, n_in):
     """Lanes past a row's end fetch its last sixteen bytes: an infinity there must reach the sum once, as itself."""
