@@ -725,10 +725,10 @@ bool rows_enabled() {
     return on;
 }
 // Its workgroups per CU: three (staging is each wave's own business there, so a workgroup more costs little and
-// hides more of the others' waits); ORIN_GEMV_MFMA_WGS_PER_CU overrides as for the other kernel.
-int rows_wgs_per_cu(int given) {
+// hides more of the others' waits) or two (rows_two_a_cu()); ORIN_GEMV_MFMA_WGS_PER_CU overrides as for the other kernel.
+int rows_wgs_per_cu(int given, int usual) {
     static const bool env = getenv("ORIN_GEMV_MFMA_WGS_PER_CU") != nullptr;
-    return env ? given : 3;
+    return env ? given : usual;
 }
 
 // Tiles of a launch's matrices: 16 rows, or 8 of each of two.
@@ -877,6 +877,25 @@ bool launch_rows(const GemvArgs& a, int wgs, int shares, bool wide, int nb_wg, h
     }
 }
 
+// Two workgroups a CU instead of three for one matrix or pair that takes the chip several turns: each makes the digits of the whole row for
+// itself and fetches activation and norm weights, and the weights of two, two items a wave, are enough on their way.  Where a row's items come out
+// even among the four waves, or, of one matrix and of Q6_K, one short of it; with fewer the waves that have none leave too
+// little under way (1536 tiles of 9 to 12 blocks +2 to +4 %, 2048 +10 %; 18 and 20 blocks 0 to +6 %).  Q8_0, whose items are one block: pairs from
+// 12 blocks on (8 to 10: -2 to +5 %; one matrix: its items are chosen by turns, as measured with three).  us a launch, three -> two:
+//   two matrices of 14336 rows (7 tiles a CU)   of 16 blocks: Q4_K 14.67 -> 13.50, Q5_K 17.41 -> 15.96, Q6_K 20.24 -> 18.42, Q8_0 25.4 -> 23.9
+//     of 24: 20.2 -> 19.45, 23.8 -> 22.8, 28.3 -> 26.8, 36.8 -> 35.8; of 32: 25.4 -> 24.1, 30.0 -> 28.9, 40.6 -> 34.2, 47.1 -> 45.5
+//   of 18944 rows (9 1/4)   of 14 blocks: Q6_K 23.3 -> 22.9, Q8_0 30.2 -> 29.7 (Q4_K 16.4 -> 17.1, Q5_K 19.6 -> 20.5: not taken)
+//   one matrix of 152064 rows   of 14 blocks: 51.1 -> 49.5, 62.1 -> 60.9, 74.6 -> 73.6; of 16: 55.0 -> 53.8, 66.5 -> 65.8, 81.3 -> 80.3
+// Of 230 launches of 14 to 31 blocks a row, 4 to 31 tiles a CU, that take two, 190 are over 0.5 % faster, up to 19 (Q6_K from 30 blocks on, where three
+// do not fit), and four over 1.2 % slower (32000 rows of 22 blocks in Q4_K 19.9 -> 20.5, the others up to 1.7).
+template <int T>
+bool rows_two_a_cu(const GemvArgs& a, int tiles, int cu_count) {
+    const int nb = a.n_in / 256, last = (nb + 1) / 2 % 4;
+    if (a.n_seg != 1 || tiles <= 3 * cu_count || nb > 32) return false;
+    if (T == kQ8_0) return a.w_up && nb >= 12;
+    return nb >= 14 && (last == 0 || (last == 3 && (!a.w_up || T == kQ6_K)));
+}
+
 template <int T>
 hipError_t launch(const GemvArgs& a, int cu_count, hipStream_t stream) {
     int max_out = 0;
@@ -895,9 +914,9 @@ hipError_t launch(const GemvArgs& a, int cu_count, hipStream_t stream) {
     // second tile would have amortised the staging instead).
     const bool wide = ks == 1 && nb_row >= 16 && !a.w_up && (int)grid.x == (max_out + 15) / 16;
     {
-        const int per_cu = rows_wgs_per_cu(a.mfma_wgs_per_cu);
         g_rows_resident = cu_count * 3;
         const int tiles = rows_tiles(a);
+        const int per_cu = rows_wgs_per_cu(a.mfma_wgs_per_cu, rows_two_a_cu<T>(a, tiles, cu_count) ? 2 : 3);
         // One item a wave where a row is short enough: as many workgroups as there are tiles, for the chip to hand out, and
         // no second turn.  Of two matrices up to 8 blocks (Qwen2.5-1.5B's gate/up in Q4_K 6.5 -> 6.1 us; 16 blocks in workgroups
         // of eight waves: Llama-3-8B's 15.0 -> 17.4), in Q8_0 up to 6 (rows_small_waves(); 8 blocks: Llama-3.2-1B's 9.9 -> 10.2 us); of one
@@ -995,7 +1014,7 @@ hipError_t gemv_mfma_mixed_launch(GemvArgs a, int cu_count, hipStream_t stream) 
     bool rows = rows_enabled();
     for (int i = 0; i < a.n_seg; ++i) rows = rows && a.seg[i].n_out % 16 == 0 && a.seg[i].type != kQ8_0;
     if (rows) {
-        const int per_cu = rows_wgs_per_cu(a.mfma_wgs_per_cu), nb = a.n_in / 256;
+        const int per_cu = rows_wgs_per_cu(a.mfma_wgs_per_cu, 3), nb = a.n_in / 256;
         const int tiles = rows_tiles(a);
         const int wgs = per_cu > 0 ? min(tiles, cu_count * per_cu) : tiles;
         const bool wide_r = nb > 8 && wgs == tiles; // (as in launch() above)

@@ -520,6 +520,32 @@ def test_f16_an_infinite_weight_anywhere_in_a_row(ly, n_in):
         assert np.array_equal(got.cpu().numpy()[:len(spots)], want)
 
 
+@pytest.mark.parametrize("wtype, blocks", [(lm.Q4_K, 14), (lm.Q4_K, 15), (lm.Q5_K, 16), (lm.Q6_K, 14), (lm.Q6_K, 15), (lm.Q6_K, 30), (lm.Q4_K, 31), (lm.Q8_0, 12),
+                                           (lm.Q8_0, 15)])
+def test_two_workgroups_a_cu(ly, wtype, blocks):
+    """One matrix and a pair of 770 tiles, the first size at which two workgroups a CU take both, and of 1100."""
+    import torch
+
+    n_in, rs = blocks * 256, lm.Stream(6600 + blocks + wtype)
+    kinds = np.array(lm.make_tensor(rs, wtype, n_in, 61)[1]).view(np.uint8).reshape(61, -1)
+    order = np.random.default_rng(blocks).integers(0, 61, 2 * 1100 * 8)
+    dw = dev_bytes(np.ascontiguousarray(kinds[order]).reshape(-1)).view(len(order), -1)
+    x, nw = rs.sym(n_in, 1.0), (1.0 + rs.sym(n_in, 0.3)).astype(np.float32)
+    dx = _dev(x)
+    want = ref.gemv(wtype, kinds.reshape(-1), ref.rms_norm(x, nw, 1e-5), n_in, 61)[order]
+    plain = ref.gemv(wtype, kinds.reshape(-1), x, n_in, 61)[order]
+    for tiles in (770, 1100):
+        rows, half = tiles * 16, tiles * 8
+        y, yg = out_buf(rows), out_buf(half)
+        ly.gemv(wtype, dw, dx, y, n_in, rows)
+        ly.gemv_norm_gate_up_swiglu(wtype, dw, dw[half:], dx, _dev(nw), 1e-5, yg, n_in, half)
+        torch.cuda.synchronize()
+        for what, got, w, n in (("one", y, plain[:rows], rows), ("pair", yg, ref.swiglu(want[:half], want[half:rows]), half)):
+            got = got.cpu().numpy()
+            assert (got[n:] == 12345.0).all(), f"{what}: rows past n_out were written"
+            assert vec_err(got[:n], w.astype(np.float64)) < TOL_OP, (what, tiles)
+
+
 def test_rms_norm_rows_swiglu_and_in_place(ly):
     import torch
 

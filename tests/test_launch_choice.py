@@ -23,6 +23,25 @@ def test_q8_0_matrices_of_many_turns(blocks, item, n_out):
     assert rows_form(recorder().calls("orin_gemv", Q8_0, ptr(1), ptr(2), ptr(3), blocks * 256, n_out)) == (4, want)
 
 
+Q4_K, Q6_K = 12, 14
+
+
+@pytest.mark.parametrize("wtype, blocks, pair, two", [
+    (Q4_K, 16, True, True), (Q4_K, 15, True, True), (Q4_K, 24, False, True), (Q4_K, 14, False, True), (Q6_K, 14, True, True), (Q8_0, 12, True, True),
+    (Q4_K, 14, True, False), (Q4_K, 12, True, False), (Q4_K, 18, False, False), (Q6_K, 20, True, False), (Q8_0, 10, True, False), (Q8_0, 16, False, False),
+    (Q4_K, 33, True, False),
+])
+def test_workgroups_a_cu_of_many_turns(wtype, blocks, pair, two):
+    """Two where a row's items come out (nearly) even among four waves, where there are more tiles than three workgroups a CU."""
+    def workgroups(tiles):
+        n_in, rows = blocks * 256, tiles * (8 if pair else 16)
+        (one,) = (recorder().calls("orin_gemv_norm_gate_up_swiglu", wtype, ptr(1), ptr(2), ptr(3), ptr(4), 1e-5, ptr(5), n_in, rows) if pair
+                  else recorder().calls("orin_gemv", wtype, ptr(1), ptr(2), ptr(3), n_in, rows))
+        return one.grid[0]
+    assert workgroups(768) == 768
+    assert workgroups(770) == workgroups(5000) == (512 if two else 768)
+
+
 HEADS = {  # query heads, KV heads, head size
     "qwen1.5b": (12, 2, 128), "qwen7b": (28, 4, 128), "llama8b": (32, 8, 128), "llama1b": (32, 8, 64), "qwen3": (16, 8, 128),
 }
