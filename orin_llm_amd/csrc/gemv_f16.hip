@@ -16,7 +16,7 @@
 // that nothing waits for a load but its use, and a launch of one matrix asks nothing of which one (kMulti).
 // Llama-3-8B's shapes, per launch, with gemv.hip's kernel -> now: q, k, v 34.1 -> 10.65 us (50 MB), output projection 11.9 -> 7.65 (34 MB),
 // gate/up 47.7 -> 37.0 (235 MB, 6.35 TB/s: what the fastest plain read of that size reaches), down 25.0 -> 20.5 us (117 MB, 5.7).
-// Rows beyond 16384 elements are the exception: 3584 of 18944 took 22.3 before the last change and take 22.9, the model's other launches 1 to 3 % less.
+// Rows beyond 23040 elements are as fast as before the last change within 2 % either way.
 #include "layer_common.hpp"
 
 #include <type_traits>
@@ -176,7 +176,7 @@ hipError_t launch_as(const GemvArgs& g, int cu_count, hipStream_t stream) {
     // for itself, 4 waves of 8 KB to 14 KB in each of two batches.  us a launch, three workgroups a CU with half the rows a batch
     // (two, of long rows, with one) -> this: Llama-3-8B's q, k, v 11.5 -> 10.65, output 8.25 -> 7.65, gate/up 41.0 -> 37.0 (6.35 TB/s),
     // down 21.8 -> 20.5, logits 158.5 -> 155.2 (6.8 TB/s); two workgroups a CU with these batches 11.35, 8.35, 37.6, 21.6, 160.5.
-    constexpr int M = DUAL ? 2 : 1, RB = RUNS * M <= 8 && RUNS <= 4 ? 8 / (RUNS * M) : DUAL ? 1 : 2;
+    constexpr int M = DUAL ? 2 : 1, RB = kWaves > 4 ? (DUAL ? 1 : 2) : RUNS * M <= 8 && RUNS <= 4 ? 8 / (RUNS * M) : DUAL ? 1 : 2;
     static_assert(RB <= 16, "rows of a batch: four bits of `shape`");
     constexpr int kPerCu = kWaves == 1 ? 4 : kWaves < 4 ? 2 : 1;
     unsigned ends[3] = {}, total = 0, shape = (unsigned)g.n_in;
@@ -205,18 +205,27 @@ hipError_t launch_runs(const GemvArgs& g, int cu_count, hipStream_t stream) {
 
 } // namespace
 
-// As many waves a workgroup as a row has runs, four from there on up to rows of 16384 elements, eight beyond (at most 32768).
-// (Rows of two and three runs by four waves, the others idle, and by two and three, two workgroups a CU: 151936 rows of 1024 45.4 -> 41.0 us,
-// 4096 rows 4.84 -> 4.31; 151936 rows of 1536 62.6 -> 60.1, two matrices of 8960 11.54 -> 11.32.)
+// As many waves a workgroup as a row has runs, four from there on up to rows of 16384 elements, 11 to 15 with three runs each up to 23040, eight
+// beyond (at most 32768).  (Rows of two and three runs by four waves, the others idle, and by two and three, two workgroups a CU: 151936 rows of
+// 1024 45.4 -> 41.0 us, 4096 rows 4.84 -> 4.31; 151936 rows of 1536 62.6 -> 60.1, two matrices of 8960 11.54 -> 11.32.  3584 rows by eight waves and
+// by 11 to 15: of 16896 20.7 -> 19.7, of 22016 27.7 -> 26.6; from 24576 on eight are as fast or faster, 29.3 and 29.6.)
 hipError_t gemv_f16_launch(const GemvArgs& g, int cu_count, hipStream_t stream) {
     const int runs = (g.n_in + kRun - 1) / kRun;
-    if (runs > 4 * kMostRuns) {
+    if (runs > 45) {
         switch ((runs + 7) / 8) {
-        case 5: return launch_runs<5, 8>(g, cu_count, stream);
         case 6: return launch_runs<6, 8>(g, cu_count, stream);
         case 7: return launch_runs<7, 8>(g, cu_count, stream);
         case 8: return launch_runs<8, 8>(g, cu_count, stream);
         default: return hipErrorInvalidValue;
+        }
+    }
+    if (runs > 4 * kMostRuns) {
+        switch ((runs + 2) / 3) {
+        case 11: return launch_runs<3, 11>(g, cu_count, stream);
+        case 12: return launch_runs<3, 12>(g, cu_count, stream);
+        case 13: return launch_runs<3, 13>(g, cu_count, stream);
+        case 14: return launch_runs<3, 14>(g, cu_count, stream);
+        default: return launch_runs<3, 15>(g, cu_count, stream);
         }
     }
     switch (runs) {
