@@ -888,10 +888,11 @@ bool launch_rows(const GemvArgs& a, int wgs, int shares, bool wide, int nb_wg, h
 //   one matrix of 152064 rows   of 14 blocks: 51.1 -> 49.5, 62.1 -> 60.9, 74.6 -> 73.6; of 16: 55.0 -> 53.8, 66.5 -> 65.8, 81.3 -> 80.3
 // Of 230 launches of 14 to 31 blocks a row, 4 to 31 tiles a CU, that take two, 190 are over 0.5 % faster, up to 19 (Q6_K from 30 blocks on, where three
 // do not fit), and four over 1.2 % slower (32000 rows of 22 blocks in Q4_K 19.9 -> 20.5, the others up to 1.7).
+// (Not where two would take more turns than rows_head() has room for: the launch would leave this kernel.)
 template <int T>
 bool rows_two_a_cu(const GemvArgs& a, int tiles, int cu_count) {
     const int nb = a.n_in / 256, last = (nb + 1) / 2 % 4;
-    if (a.n_seg != 1 || tiles <= 3 * cu_count || nb > 32) return false;
+    if (a.n_seg != 1 || tiles <= 3 * cu_count || nb > 32 || tiles / (2 * cu_count) > (int)kMostRowsTurns) return false;
     if (T == kQ8_0) return a.w_up && nb >= 12;
     return nb >= 14 && (last == 0 || (last == 3 && (!a.w_up || T == kQ6_K)));
 }

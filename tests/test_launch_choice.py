@@ -42,6 +42,20 @@ def test_workgroups_a_cu_of_many_turns(wtype, blocks, pair, two):
     assert workgroups(770) == workgroups(5000) == (512 if two else 768)
 
 
+@pytest.mark.parametrize("wtype, blocks", [(Q4_K, 16), (Q4_K, 24), (Q6_K, 14), (Q6_K, 30), (Q8_0, 12)])
+@pytest.mark.parametrize("pair", [False, True])
+def test_the_tallest_matrices_stay_in_the_kernel_that_reads_long_runs(wtype, blocks, pair):
+    """A workgroup's turns are counted in six bits: what two workgroups a CU would take in more than 62 is three's."""
+    def one(tiles):
+        n_in, rows = blocks * 256, tiles * (8 if pair else 16)
+        (one,) = (recorder().calls("orin_gemv_norm_gate_up_swiglu", wtype, ptr(1), ptr(2), ptr(3), ptr(4), 1e-5, ptr(5), n_in, rows) if pair
+                  else recorder().calls("orin_gemv", wtype, ptr(1), ptr(2), ptr(3), n_in, rows))
+        return one.kernel, one.grid[0]
+    two = 768 if wtype == Q8_0 and not pair else 512
+    assert one(62 * 512 + 510) == ("gemv_rows_kernel", two)
+    assert one(63 * 512) == one(62 * 768 + 766) == ("gemv_rows_kernel", 768)
+
+
 HEADS = {  # query heads, KV heads, head size
     "qwen1.5b": (12, 2, 128), "qwen7b": (28, 4, 128), "llama8b": (32, 8, 128), "llama1b": (32, 8, 64), "qwen3": (16, 8, 128),
 }
