@@ -523,7 +523,7 @@ def test_f16_an_infinite_weight_anywhere_in_a_row(ly, n_in):
 @pytest.mark.parametrize("wtype, blocks", [(lm.Q4_K, 14), (lm.Q4_K, 15), (lm.Q5_K, 16), (lm.Q6_K, 14), (lm.Q6_K, 15), (lm.Q6_K, 30), (lm.Q4_K, 31), (lm.Q8_0, 12),
                                            (lm.Q8_0, 15)])
 def test_two_workgroups_a_cu(ly, wtype, blocks):
-    """One matrix and a pair of 770 tiles, the first size at which two workgroups a CU take both, and of 1100."""
+    """One matrix and a pair of 770 tiles, the first size at which two workgroups a CU take one of them, and of 1100, where they take both."""
     import torch
 
     n_in, rs = blocks * 256, lm.Stream(6600 + blocks + wtype)

@@ -23,7 +23,7 @@ def test_q8_0_matrices_of_many_turns(blocks, item, n_out):
     assert rows_form(recorder().calls("orin_gemv", Q8_0, ptr(1), ptr(2), ptr(3), blocks * 256, n_out)) == (4, want)
 
 
-Q4_K, Q6_K = 12, 14
+Q4_K, Q5_K, Q6_K = 12, 13, 14
 
 
 @pytest.mark.parametrize("wtype, blocks, pair, two", [
@@ -39,7 +39,26 @@ def test_workgroups_a_cu_of_many_turns(wtype, blocks, pair, two):
                   else recorder().calls("orin_gemv", wtype, ptr(1), ptr(2), ptr(3), n_in, rows))
         return one.grid[0]
     assert workgroups(768) == 768
-    assert workgroups(770) == workgroups(5000) == (512 if two else 768)
+    few = two and not (pair and blocks <= 16 and wtype != Q8_0)  # (up to four tiles a CU such pairs are 1 to 6 % slower by two)
+    assert workgroups(770) == workgroups(1024) == (512 if few else 768)
+    assert workgroups(1026) == workgroups(5000) == (512 if two else 768)
+
+
+@pytest.mark.parametrize("wtype, blocks, pair, three", [
+    (Q4_K, 22, False, (6, 8, 10)), (Q4_K, 24, True, (6, 8, 10)), (Q5_K, 23, False, (6, 8, 10)), (Q4_K, 32, False, (8, 10)), (Q5_K, 32, True, (8, 10)),
+    (Q4_K, 16, True, (4, 8, 10)), (Q5_K, 15, True, (4, 8, 10)), (Q4_K, 16, False, ()), (Q5_K, 14, False, ()), (Q6_K, 24, False, (6,)), (Q6_K, 22, True, (6,)),
+    (Q6_K, 16, True, (4,)), (Q6_K, 30, False, ()), (Q8_0, 12, True, ()), (Q8_0, 16, True, (4,)), (Q8_0, 24, True, ()),
+])
+def test_two_workgroups_a_cu_only_where_they_were_measured_faster(wtype, blocks, pair, three):
+    """Tiles a CU, rounded up, at which three workgroups a CU were measured faster: 2055 launches of 784 to 8000 tiles."""
+    def workgroups(tiles):
+        n_in, rows = blocks * 256, tiles * (8 if pair else 16)
+        (one,) = (recorder().calls("orin_gemv_norm_gate_up_swiglu", wtype, ptr(1), ptr(2), ptr(3), ptr(4), 1e-5, ptr(5), n_in, rows) if pair
+                  else recorder().calls("orin_gemv", wtype, ptr(1), ptr(2), ptr(3), n_in, rows))
+        return one.grid[0]
+    for per_cu in (4, 5, 6, 7, 8, 9, 10, 11, 12, 20):
+        want = 768 if per_cu in three else 512
+        assert workgroups(256 * per_cu - 254) == workgroups(256 * per_cu) == want, per_cu
 
 
 @pytest.mark.parametrize("wtype, blocks", [(Q4_K, 16), (Q4_K, 24), (Q6_K, 14), (Q6_K, 30), (Q8_0, 12)])
