@@ -16,7 +16,6 @@
 // that nothing waits for a load but its use, and a launch of one matrix asks nothing of which one (kMulti).
 // Llama-3-8B's shapes, per launch, with gemv.hip's kernel -> now: q, k, v 34.1 -> 10.65 us (50 MB), output projection 11.9 -> 7.65 (34 MB),
 // gate/up 47.7 -> 37.0 (235 MB, 6.35 TB/s: what the fastest plain read of that size reaches), down 25.0 -> 20.5 us (117 MB, 5.7).
-// Rows beyond 23040 elements are as fast as before the last change within 2 % either way.
 #include "layer_common.hpp"
 
 #include <type_traits>
@@ -172,15 +171,11 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_f16_kernel(const uint64_t w0
     }
 }
 
-template <int RUNS, bool DUAL, int kWaves>
-hipError_t launch_as(const GemvArgs& g, int cu_count, hipStream_t stream) {
-    // Rows in a batch and workgroups a CU: some 64 KB a CU on their way, in few workgroups -- each fetches the activation and the norm's weights
-    // for itself, 4 waves of 8 KB to 14 KB in each of two batches.  us a launch, three workgroups a CU with half the rows a batch
-    // (two, of long rows, with one) -> this: Llama-3-8B's q, k, v 11.5 -> 10.65, output 8.25 -> 7.65, gate/up 41.0 -> 37.0 (6.35 TB/s),
-    // down 21.8 -> 20.5, logits 158.5 -> 155.2 (6.8 TB/s); two workgroups a CU with these batches 11.35, 8.35, 37.6, 21.6, 160.5.
-    constexpr int M = DUAL ? 2 : 1, RB = kWaves > 4 ? (DUAL ? 1 : 2) : RUNS * M <= 8 && RUNS <= 4 ? 8 / (RUNS * M) : DUAL ? 1 : 2;
+template <int RUNS, bool DUAL, int kWaves, int RB>
+hipError_t launch_batches(const GemvArgs& g, int cu_count, hipStream_t stream) {
     static_assert(RB <= 16, "rows of a batch: four bits of `shape`");
-    constexpr int kPerCu = kWaves == 1 ? 4 : kWaves < 4 ? 2 : 1;
+    constexpr int R = (DUAL ? 2 : 1) * RB;
+    const unsigned cus = (unsigned)cu_count, row_bytes = (unsigned)g.n_in * 2u;
     unsigned ends[3] = {}, total = 0, shape = (unsigned)g.n_in;
     for (int i = 0; i < 3; ++i) {
         if (i < g.n_seg) {
@@ -189,15 +184,46 @@ hipError_t launch_as(const GemvArgs& g, int cu_count, hipStream_t stream) {
         }
         ends[i] = total;
     }
-    const unsigned wgs = min(total, (unsigned)(cu_count * kPerCu));
-    auto go = [&](auto multi) {
-        constexpr bool kMulti = !DUAL && decltype(multi)::value;
+    // Workgroups a CU (four waves): one, or two where the two batches of one are short of 64 KB, its waves' last runs being partly idle, and
+    // two turns of the chip do not take all batches; of several matrices up to 64 KB; and with rows of up to 2048 elements, eight rows a
+    // batch, where one more batch a CU is a long turn: of several matrices, and of pairs up to four turns.  us a launch, one -> two: of
+    // 5120 elements 5120 rows 11.6 -> 10.25, q, k, v of 5120, 1280 and 1280 17.8 -> 14.75, pairs of 4096 17.3 -> 16.0, but 768 rows alone
+    // 3.75 -> 4.1; of 3072 elements q, k, v of 4096, 1024 and 1024 9.25 -> 8.6, but 2048 rows alone 4.3 -> 4.55; of 4096 elements 4096
+    // rows 7.35 -> 7.55; of 2048 elements q, k, v of 2048, 512 and 512 5.2 -> 4.95, pairs of 1536 5.15 -> 4.9, but of 6144 10.65 -> 11.0.
+    const unsigned under_way = 2u * R * row_bytes;
+    const bool multi = g.n_seg > 1;
+    bool two = false;
+    if constexpr (kWaves == 4)
+        two = RUNS == 1 ? multi || (DUAL && total < 4 * cus) : total > 2 * cus && under_way <= (multi ? 64u : 48u) * 1024u;
+    const unsigned wgs = min(total, cus * (kWaves == 1 ? 4u : kWaves < 4 || two ? 2u : 1u));
+    auto go = [&](auto multic) {
+        constexpr bool kMulti = !DUAL && decltype(multic)::value;
         hipLaunchKernelGGL((gemv_f16_kernel<RUNS, RB, DUAL, kWaves, kMulti>), dim3(wgs), dim3(kWaves * 64), 0, stream, arg_ptr(g.seg[0].w),
                            arg_ptr(g.w_up ? g.w_up : g.seg[1].w), arg_ptr(g.seg[2].w), g.x, g.norm_w, ends[0], ends[1], ends[2], shape, g);
     };
-    if (g.n_seg > 1) go(std::true_type());
+    if (multi) go(std::true_type());
     else go(std::false_type());
     return hipGetLastError();
+}
+
+template <int RUNS, bool DUAL, int kWaves>
+hipError_t launch_as(const GemvArgs& g, int cu_count, hipStream_t stream) {
+    // Rows in a batch: some 64 KB a CU on their way, in few workgroups -- each fetches the activation and the norm's weights
+    // for itself, 4 waves of 5 KB to 16 KB in each of two batches.  us a launch, three workgroups a CU with half the rows a batch
+    // (two, of long rows, with one) -> this: Llama-3-8B's q, k, v 11.5 -> 10.65, output 8.25 -> 7.65, gate/up 41.0 -> 37.0 (6.35 TB/s),
+    // down 21.8 -> 20.5, logits 158.5 -> 155.2 (6.8 TB/s); two workgroups a CU with these batches 11.35, 8.35, 37.6, 21.6, 160.5.
+    // Eight waves, whose rows are over 45 KB: one (two: 28672 elements, 4096 rows 35.4 -> 36.5 us, q, k, v of 4096, 1024 and 1024 51.65 ->
+    // 53.5, 640 rows 8.65 -> 10.3).  11 to 15: two, but up to three rows a CU one, which is less for the busiest CU (18944 elements, 640 rows
+    // by two 7.95, by one 7.05 us, 128 rows 5.3 and 4.4, 1024 rows 8.9 both; q, k, v of 4096, 1024 and 1024 35.25 and 39.5).
+    constexpr int M = DUAL ? 2 : 1;
+    if constexpr (kWaves > 8 && !DUAL) {
+        long long rows = 0;
+        for (int i = 0; i < g.n_seg; ++i) rows += g.seg[i].n_out;
+        return rows <= 3 * cu_count ? launch_batches<RUNS, DUAL, kWaves, 1>(g, cu_count, stream) : launch_batches<RUNS, DUAL, kWaves, 2>(g, cu_count, stream);
+    } else {
+        constexpr int RB = kWaves > 4 ? 1 : RUNS * M <= 8 && RUNS <= 4 ? 8 / (RUNS * M) : DUAL ? 1 : 2;
+        return launch_batches<RUNS, DUAL, kWaves, RB>(g, cu_count, stream);
+    }
 }
 
 template <int RUNS, int kWaves>

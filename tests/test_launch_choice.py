@@ -1,5 +1,7 @@
 """Which kernel the launchers take for a shape, read from the launches themselves (recorder.py): the rules over sizes that
 no other test would allocate."""
+import ctypes
+
 import pytest
 
 from recorder import ptr, recorder
@@ -73,6 +75,30 @@ def test_the_tallest_matrices_stay_in_the_kernel_that_reads_long_runs(wtype, blo
     two = 768 if wtype == Q8_0 and not pair else 512
     assert one(62 * 512 + 510) == ("gemv_rows_kernel", two)
     assert one(63 * 512) == one(62 * 768 + 766) == ("gemv_rows_kernel", 768)
+
+
+F16 = 1
+
+
+@pytest.mark.parametrize("n_in, heights, pair, want", [  # (waves, rows a batch, workgroups on 256 CUs)
+    (5120, (768,), False, (4, 2, 256)), (5120, (1024,), False, (4, 2, 256)), (5120, (1026,), False, (4, 2, 512)), (5120, (5120, 1280, 1280), False, (4, 2, 512)),
+    (5120, (512,), True, (4, 1, 256)), (5120, (513,), True, (4, 1, 512)), (3072, (2048,), False, (4, 4, 256)), (3072, (4096, 1024, 1024), False, (4, 4, 512)),
+    (3104, (4096,), False, (4, 4, 256)), (3584, (4096, 512, 512), False, (4, 4, 512)), (4096, (4096,), False, (4, 4, 256)), (6144, (4096,), False, (4, 2, 512)),
+    (2048, (2048, 512, 512), False, (4, 8, 384)), (2048, (8192,), False, (4, 8, 256)), (2048, (1536,), True, (4, 4, 384)), (2048, (8192,), True, (4, 4, 256)),
+    (28672, (4096,), False, (8, 1, 256)), (28672, (4096,), True, (8, 1, 256)), (18944, (768,), False, (13, 1, 256)), (18944, (769,), False, (13, 2, 256)),
+    (18944, (384, 96, 96), False, (13, 1, 256)), (18944, (640, 160, 160), False, (13, 2, 256)), (18944, (512,), True, (13, 1, 256)),
+    (1024, (8192,), False, (2, 8, 512)), (512, (16384,), False, (1, 8, 1024)), (14336, (4096,), False, (4, 2, 256)),
+])
+def test_f16_batches_and_workgroups(n_in, heights, pair, want):
+    """Bytes on their way at once and rows of the busiest CU, as measured: both sides of the lines."""
+    calls = recorder().calls
+    if pair:
+        (one,) = calls("orin_gemv_norm_gate_up_swiglu", F16, ptr(1), ptr(2), ptr(3), ptr(4), 1e-5, ptr(5), n_in, heights[0])
+    else:
+        n, p = len(heights), ctypes.c_void_p * len(heights)
+        (one,) = calls("orin_gemv_multi", F16, n, p(*map(ptr, range(1, 1 + n))), p(*[None] * n), p(*map(ptr, range(4, 4 + n))), (ctypes.c_int * n)(*heights), ptr(7), ptr(8), 1e-5, n_in, 0)
+    assert one.kernel == "gemv_f16_kernel"
+    assert (int(one.params[3]), int(one.params[1]), one.grid[0]) == want and one.block == 64 * want[0]
 
 
 HEADS = {  # query heads, KV heads, head size
