@@ -690,6 +690,12 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
             }
 
             __builtin_amdgcn_sched_barrier(0); // (the weights are made while V is still on its way)
+            // head_dim 64 and kRotateLate: the next tile's K is waited for here, ahead of the request for its V.  Without the wait a wave has both on
+            // their way nearly all the time, and in caches of a power of two of rows many KV heads at the same row, walked together, fall
+            // on the same memory channels.  us a launch pair, rotate + store + attend, with table, without -> with the wait: 32 KV heads of 64, 8192 rows 20.2 ->
+            // 18.6 (8232 rows: 15.2 both), 16 of them 12.75 -> 12.0; without a table, head_dim 128, 28 / 4 heads at 32000 of 32768 16.1 -> 15.2,
+            // 32 / 32 at 4000 of 4096 16.1 -> 15.3.  With a table, head_dim 128 is the faster without: 28 / 4 heads 15.2, 15.4.
+            if constexpr (more && (D == 64 || LATE)) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             // ---- V: registers -> this wave's LDS slice (K was needed first and arrives first) ----
             auto park_v = [&](auto whole) {
 #pragma unroll
