@@ -43,6 +43,7 @@
 // fa_prefill_combine_kernel merges them into `out`.
 #include "fa_common.hpp"
 
+#include <limits.h>
 #include <string.h>
 
 // Stage marks: wall-clock stamps in the timeline build, nothing otherwise (fa_common.hpp).
@@ -1512,17 +1513,26 @@ hipError_t launch(FaArgs a, int cu_count, hipStream_t stream, void* workspace, s
         // A fifth form: 64 columns on eight waves, one workgroup a CU where the others of head_dim 64 are two.  Those two share
         // nothing, so a CU's path to memory carries every tile twice, and that is what bounds them; eight waves fetch it once for
         // as many columns.  Its start and its merge of eight states cost 2 us more, so it takes launches of one turn of the
-        // chip that see more rows than that is worth.  Of 7945 measured launches (heads of 32 / 8, 14 / 2 and 8 / 8, chunks of 16
-        // to 512 behind 0 to 32000 rows) 999 are its own; 7 of them were over 2 % slower than with the other forms, none over
-        // 4 %, and 847 over 2 % faster, by 7 % on average.  32 / 8 heads: 301 tokens at 1501 12.4 -> 11.9 us (14.2 -> 13.2 where the rows come
-        // from memory), 512 at 4096 26.6 -> 24.7 (29.8 -> 25.5), at 8192 46.4 -> 42.3 (47.6 -> 42.4); at 320 rows it would be
-        // 5.7 -> 7.5, 512 tokens at 600 10.3 -> 10.6, 263 at 24000 85 -> 94.  With two splits 160 tokens at 8192 gain where the
-        // rows are near (24.6 -> 22.6) and lose where they are not (24.1 -> 26.1): not taken.  Half to seven tenths of the chip past
-        // 3500 rows is left to the estimate: test_launch_choice.py holds that choice to a table of times of the four-wave forms, though
-        // the eight are 10 to 20 % faster there up to 16000 (301 tokens at 4096 23.2 -> 19.3).
-        const int tq = 64 / a.heads_per_group, rows_seen = a.n_past + a.batch;
-        const long long wgs = (long long)a.n_kv * a.n_hgroups * ((a.batch + tq - 1) / tq), cus = cu_count;
-        eight = wgs * 2 > cus && wgs <= cus && rows_seen > 1600 && (rows_seen < 3500 || (wgs * 10 > cus * 7 && rows_seen < 16000) || wgs * 5 > cus * 4);
+        // chip whose first token already sees more rows than that is worth (and a tile for every wave several times over).  us,
+        // rows in the caches / from memory, the estimate's choice -> eight, 32 / 8 heads:
+        //   301 tokens at 1501 12.7 / 14.5 -> 12.3 / 13.4, at 4096 23.8 / 23.9 -> 20.1 / 22.5; 512 at 1800 16.0 / 16.8 -> 15.5 / 16.3, at 4500
+        //   28.3 / 31.4 -> 27.1 / 26.3, at 24000 114 / 109 -> 112 / 108; not behind 1300 rows or fewer: 512 at 420 10.0 / 10.3 -> 10.2 / 11.3,
+        //   8 / 1 heads, 1700 tokens at 0 11.7 / 12.2 -> 12.0 / 12.7, 1 / 1, 8256 tokens at 0 24.1 / 23.4 -> 29.5 / 30.4
+        // Deep walks of a part of the chip are faster by it only while the caches have the rows: fewer CUs ask memory for them than with
+        // KV splits (280 at 8000 36.5 / 34.5 -> 31.3 / 36.1, 300 at 24000 86 / 84 -> 94 / 99), sooner with more KV heads (40 / 40, 320 tokens
+        // at 9680 51.2 / 45.3 -> 49.8 / 51.7).  Hence the limits below.  And not where 32 columns are a workgroup a CU: 20 / 5 heads, 407 tokens
+        // at 1563, 255 of them, 12.2 / 11.8, 130 of eight waves 13.8 / 13.4.
+        // Of 1561 measured launches of its own (18 head shapes, up to 2688 tokens behind 1300 to 26800 rows), each both ways in turn, three are over 2 % slower
+        // with rows in the caches and eight with rows from memory, at most 3, none in both; 7.7 % and 8.4 % faster on average.  With two splits 160
+        // tokens at 8192 gain where the rows are near (24.6 -> 22.6) and lose where they are not (24.1 -> 26.1): not taken.
+        auto wgs_of = [&](int c) { const int tq = c / a.heads_per_group; return (long long)a.n_kv * a.n_hgroups * ((a.batch + tq - 1) / tq); };
+        const long long wgs = wgs_of(64), cus = cu_count;
+        const bool few_heads = a.n_kv <= 8; // (an XCD streams one of them)
+        int limit; // of rows, by the part of the chip that has a workgroup
+        if (wgs * 10 > cus * 9) limit = few_heads ? INT_MAX : 16000;
+        else if (wgs * 5 > cus * 4) limit = few_heads ? 16000 : 8000;
+        else limit = !few_heads ? 4000 : wgs * 10 > cus * 7 ? 10000 : 7000;
+        eight = wgs * 2 > cus && wgs_of(32) > cus && wgs <= cus && a.n_past > 1300 && a.n_past + a.batch < limit;
         if (eight) cols = 64, shift = 0, short_walk = false;
     }
     a.tq = cols / a.heads_per_group;

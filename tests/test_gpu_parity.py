@@ -283,9 +283,11 @@ def test_prefill_head_dim_64_on_short_and_longer_walks(fa, n_past, batch):
 
 
 @pytest.mark.parametrize("H,G,batch,n_past", [
-    (32, 8, 257, 1343), (32, 8, 257, 1344), (32, 8, 301, 3198), (32, 8, 301, 3199),  # 1600 and 1601 rows, 3499 and 3500
+    (32, 8, 257, 1343), (32, 8, 257, 1344), (32, 8, 301, 3198), (32, 8, 301, 3199),
     (32, 8, 353, 3600), (32, 8, 512, 5003), (14, 2, 512, 8003), (8, 8, 500, 8200),   # over seven tenths of the chip; no eight waves twice
-    (7, 7, 1200, 1000), (8, 1, 1100, 700), (160, 160, 40, 1700),                     # early walks of few tiles; a column a head
+    (7, 7, 1200, 1000), (8, 1, 1100, 700), (160, 160, 40, 1700),                     # early walks of few tiles, by four waves; a column a head
+    (32, 8, 257, 1300), (32, 8, 257, 1301), (32, 8, 353, 1300), (32, 8, 353, 1301),  # by four waves and by eight
+    (32, 8, 257, 6742), (32, 8, 257, 6743), (32, 8, 512, 15487), (7, 7, 1600, 1700), (8, 1, 2000, 1301),
 ])
 @pytest.mark.parametrize("scale", [0.125, -0.3])
 def test_prefill_head_dim_64_on_eight_waves(fa, H, G, batch, n_past, scale):

@@ -107,14 +107,15 @@ HEADS = {  # query heads, KV heads, head size
 
 
 def form_of(h, g, d, past, tokens, in_place=False):
-    """"short", or the query columns of a workgroup, with the number of KV splits where there are any: "64x4"."""
+    """"short", or the query columns of a workgroup, with the number of KV splits where there are any ("64x4") or its waves where they are not four ("64w8")."""
     attend, *combine = recorder().calls("orin_fa_prefill", ptr(1), ptr(2), ptr(3), ptr(1 if in_place else 4), h, g, d, 32768 + 512, past, tokens, float(d ** -0.5))
     splits = attend.grid[1] // -(-h // g // 8)  # (heads of a group in eights)
     assert (splits > 1) == bool(combine)
     if attend.kernel == "fa_prefill_short_kernel":
         return "short"
-    cols = 32 * int(attend.params[1])
-    return f"{cols}x{splits}" if splits > 1 else f"{cols}"
+    cols, waves = 32 * int(attend.params[1]), int(attend.params[2])
+    assert attend.block == 64 * waves
+    return f"{cols}x{splits}" if splits > 1 else f"{cols}" if waves == 4 else f"{cols}w{waves}"
 
 
 def prefill_form(model, past, tokens):
@@ -161,7 +162,7 @@ def test_a_partial_turn_costs_what_its_short_walks_take(model, past, tokens, us)
     assert taken <= 1.02 * min(map(sum, us.values()))
 
 
-# (us a launch, caches as they are between replays)
+# (us a launch of the forms of four waves, caches as they are between replays)
 HEADS_OF_64 = [
     ("llama1b", 1501, 301, {"32": 11.9, "64": 11.9}),
     ("llama1b", 3584, 280, {"32": 20.7, "64x2": 22.5, "64": 24.0}),
@@ -179,7 +180,59 @@ HEADS_OF_64 = [
 
 @pytest.mark.parametrize("model, past, tokens, us", HEADS_OF_64)
 def test_forms_of_head_dim_64_at_depth(model, past, tokens, us):
-    assert us[prefill_form(model, past, tokens)] <= 1.1 * min(us.values())
+    form = prefill_form(model, past, tokens)
+    if form == "64w8":
+        assert (model, past, tokens) in [row[:3] for row in EIGHT_WAVES]
+    else:
+        assert us[form] <= 1.1 * min(us.values())
+
+
+# (pairs as above: rows in the caches, and caches emptied; all forms in one session)
+EIGHT_WAVES = [
+    ("llama1b", 1501, 301, {"32": (12.8, 13.6), "64": (12.6, 14.9), "64x2": (16.7, 15.8), "64w8": (12.3, 13.4)}),
+    ("llama1b", 3584, 280, {"32": (21.1, 21.3), "64": (19.8, 25.3), "64x2": (22.6, 22.4), "64w8": (18.4, 20.3)}),
+    ("llama1b", 4500, 260, {"32": (24.3, 25.4), "64": (22.9, 30.5), "64x2": (25.2, 24.8), "64w8": (21.3, 24.4)}),
+    ("llama1b", 4500, 301, {"32": (25.4, 26.0), "64": (23.2, 30.4), "64x2": (26.2, 25.5), "64w8": (21.4, 24.4)}),
+    ("llama1b", 5500, 260, {"32": (28.7, 28.6), "64": (26.1, 36.1), "64x2": (28.3, 27.7), "64w8": (23.9, 27.5)}),
+    ("llama1b", 8000, 280, {"32": (39.3, 38.5), "64": (35.1, 48.9), "64x2": (36.6, 35.0), "64w8": (31.3, 36.1)}),
+    ("llama1b", 8000, 330, {"32": (41.3, 40.8), "64": (35.6, 48.7), "64x2": (38.4, 35.9), "64w8": (33.1, 36.2)}),
+    ("llama1b", 900, 420, {"32": (11.2, 11.8), "64": (11.2, 11.5), "64x2": (16.7, 15.7), "64w8": (11.3, 12.1)}),
+    ("llama1b", 420, 512, {"32": (9.8, 10.7), "64": (9.8, 10.4), "64x2": (16.4, 15.1), "64w8": (10.2, 11.3)}),
+    ("llama1b", 4500, 512, {"32": (32.4, 31.8), "64": (28.1, 31.8), "64x2": (32.1, 30.3), "64w8": (27.1, 26.3)}),
+    ("llama1b", 3584, 512, {"32": (27.3, 27.5), "64": (23.9, 26.5), "64x2": (28.5, 25.7), "64w8": (23.4, 22.5)}),
+    ("llama1b", 4096, 301, {"32": (23.6, 24.3), "64": (21.8, 28.3), "64x2": (25.0, 24.0), "64w8": (20.1, 22.5)}),
+    ("llama1b", 1300, 512, {"32": (14.5, 15.1), "64": (13.5, 14.1), "64x2": (19.6, 18.1), "64w8": (13.4, 14.5)}),
+    ("llama1b", 1800, 512, {"32": (17.4, 17.9), "64": (16.2, 17.1), "64x2": (21.5, 20.3), "64w8": (15.5, 16.3)}),
+    ("llama1b", 6500, 280, {"32": (33.0, 33.2), "64": (29.8, 41.2), "64x2": (32.0, 31.3), "64w8": (26.9, 31.1)}),
+    ("llama1b", 7200, 280, {"32": (35.7, 36.5), "64": (32.4, 44.9), "64x2": (33.9, 33.1), "64w8": (29.1, 33.9)}),
+    ("llama1b", 9500, 400, {"32": (51.5, 50.7), "64": (43.6, 56.3), "64x2": (45.7, 42.3), "64w8": (41.4, 42.4)}),
+    ("llama1b", 14000, 400, {"32": (72.2, 72.3), "64": (61.5, 80.9), "64x2": (61.8, 58.6), "64w8": (57.4, 61.2)}),
+    ("llama1b", 14000, 512, {"32": (85.5, 85.4), "64": (72.1, 81.8), "64x2": (71.8, 68.6), "64w8": (68.3, 64.6)}),
+    ("llama1b", 18000, 512, {"32": (114.7, 114.8), "64": (102.0, 103.9), "64x2": (89.4, 86.5), "64w8": (85.6, 82.5)}),
+    ("llama1b", 24000, 300, {"32": (127.0, 126.9), "64": (129.7, 135.5), "64x2": (87.2, 84.2), "64w8": (93.6, 98.7)}),
+    ("llama1b", 24000, 512, {"32": (161.0, 154.2), "64": (137.0, 136.3), "64x2": (114.5, 109.8), "64w8": (111.9, 107.6)}),
+]
+
+
+@pytest.mark.parametrize("model, past, tokens, us", EIGHT_WAVES)
+def test_eight_waves_only_where_rows_from_memory_do_not_make_them_slower(model, past, tokens, us):
+    """A part of the chip, deep in a context, is 14 % faster by eight waves while the caches have the rows and as much slower where they do not:
+    the choice holds for rows from memory within 4 %, which costs 7.2 % of the sum at most (330 tokens at 8000)."""
+    taken = us[prefill_form(model, past, tokens)]
+    assert taken[1] <= 1.04 * min(cold for _, cold in us.values())
+    assert sum(taken) <= 1.08 * min(map(sum, us.values()))
+
+
+@pytest.mark.parametrize("h, g, past, tokens, taken", [  # (heads of 64; by the heads, 16 to 64 tokens a workgroup)
+    (32, 8, 1300, 272, False), (32, 8, 1301, 272, True), (32, 8, 1301, 256, False), (32, 8, 1300, 360, False), (32, 8, 1301, 360, True),
+    (32, 8, 6720, 279, True), (32, 8, 6721, 279, False), (32, 8, 9639, 360, True), (32, 8, 9640, 360, False), (32, 8, 15584, 415, True), (32, 8, 15585, 415, False),
+    (32, 8, 30000, 480, True), (32, 8, 30000, 513, False), (16, 16, 3360, 639, True), (16, 16, 3361, 639, False), (16, 16, 7167, 832, True), (16, 16, 7168, 832, False),
+    (16, 16, 15039, 960, True), (16, 16, 15040, 960, False), (20, 5, 1563, 407, False), (20, 5, 1563, 410, True), (1, 1, 0, 8256, False), (2, 1, 0, 8192, False),
+    (8, 1, 0, 2048, False), (8, 1, 1300, 2048, False), (8, 1, 1301, 2048, True),
+])
+def test_the_lines_of_the_form_of_eight_waves(h, g, past, tokens, taken):
+    """Behind so few rows that some wave of some workgroup would have no tile, or one, it is never taken."""
+    assert (form_of(h, g, 64, past, tokens) == "64w8") == taken
 
 
 FEW_TOKENS_DEEP = [
@@ -203,7 +256,7 @@ def parameters(test):
     for mark in test.pytestmark:
         if mark.name == "parametrize":
             names = [n.strip() for n in mark.args[0].split(",")]
-            out = [{**o, **dict(zip(names, v))} for o in out for v in mark.args[1]]
+            out = [{**o, **dict(zip(names, v if len(names) > 1 else [v]))} for o in out for v in mark.args[1]]
     return out
 
 
@@ -219,6 +272,10 @@ def test_the_parity_tests_reach_every_form():
     assert forms(t.test_prefill_short_chunks, 64) | forms(t.test_prefill_kv_splits, 64) >= {"short", "32x4", "32x16", "64x4", "64x8"}
     assert forms(t.test_prefill_in_place, 128, True) >= {"short", "32x2", "32x4", "32x16", "64x2", "64x8"}
     assert forms(t.test_prefill_in_place, 64, True) >= {"short", "32x4"}
+    eight = {(p["H"], p["G"], p["n_past"], p["batch"]) for p in parameters(t.test_prefill_head_dim_64_on_eight_waves)
+             if form_of(p["H"], p["G"], 64, p["n_past"], p["batch"]) == "64w8"}
+    assert eight == {(32, 8, 1301, 257), (32, 8, 1301, 353), (32, 8, 1343, 257), (32, 8, 1344, 257), (32, 8, 3198, 301), (32, 8, 3199, 301), (32, 8, 3600, 353),
+                     (32, 8, 5003, 512), (32, 8, 6742, 257), (32, 8, 15487, 512), (7, 7, 1700, 1600), (8, 1, 1301, 2000), (160, 160, 1700, 40)}
     for p in parameters(t.test_short_walks_keep_infinities_and_nans_where_they_belong):
         assert form_of(p["H"], p["G"], p["d"], p["n_past"], p["batch"]) == "short", p
 
