@@ -886,20 +886,21 @@ bool launch_rows(const GemvArgs& a, int wgs, int shares, bool wide, int nb_wg, h
 //     of 24: 20.2 -> 19.45, 23.8 -> 22.8, 28.3 -> 26.8, 36.8 -> 35.8; of 32: 25.4 -> 24.1, 30.0 -> 28.9, 40.6 -> 34.2, 47.1 -> 45.5
 //   of 18944 rows (9 1/4)   of 14 blocks: Q6_K 23.3 -> 22.9, Q8_0 30.2 -> 29.7 (Q4_K 16.4 -> 17.1, Q5_K 19.6 -> 20.5: not taken)
 //   one matrix of 152064 rows   of 14 blocks: 51.1 -> 49.5, 62.1 -> 60.9, 74.6 -> 73.6; of 16: 55.0 -> 53.8, 66.5 -> 65.8, 81.3 -> 80.3
-// Tiles a CU, rounded up, at which three are the faster: four where a pair's rows have 16 blocks or fewer (800 tiles of 16 blocks: Q4_K 9.1 three,
-// 9.5 two; one matrix of them 9.2, 8.6), six where they have 21 to 24 (1300 tiles of 24: 16.2, 16.9; 1552 to 1744, seven a CU, 1 to 7 % faster by
-// two), and, in Q4_K and Q5_K, eight and ten of either (2000 tiles: pairs of 16 blocks 14.7, 15.3, one of 22 20.1, 20.5; 2064 to 2256 3 to
-// 6 % faster by two).  Of 2055 launches, 784 to 8000 tiles of 12 to 32 blocks, that takes two for 1735, of which 1574 are over 0.5 % faster, up
-// to 19 (Q6_K from 29 blocks on, where three do not fit), and six over 1.2 % slower, at most 2 (Q8_0 pairs of 12 blocks, 1040 and 1104 tiles);
-// of 410 others that it takes two for, at sizes drawn apart, 336 and three, at most 2.2.
+// Tiles a CU, rounded up, at which three are the faster: four where a pair's rows have 16 blocks or fewer (800 tiles of 16 blocks in Q4_K by three
+// 9.1, by two 9.5; one matrix of them 9.2, 8.6); and, in Q4_K and Q5_K, six where they have 21 to 24 (1300 tiles of 24: 16.2, 16.9; 1552 to 1744,
+// seven a CU, 1 to 7 % faster by two; of Q6_K only pairs of 22 and 24), eight where they have more than 16 or are a pair's (2000 tiles: pairs of
+// 16 blocks 14.7, 15.3, one of 22 20.1, 20.5; 2064 to 2256 3 to 6 % faster by two), ten likewise up to 24.  Of 2055 launches, 784 to 8000 tiles of 12
+// to 32 blocks, two were over 1.2 % slower at 127, up to 6 %; of 420 that the lines leave to three, each timed both ways in turn, three are over
+// 1.2 % faster at 153, up to 5 %, and slower at 23, up to 2, most of those since taken by two.
 // (Not where two would take more turns than rows_head() has room for: the launch would leave this kernel.)
 template <int T>
 bool rows_two_a_cu(const GemvArgs& a, int tiles, int cu_count) {
     const int nb = a.n_in / 256, last = (nb + 1) / 2 % 4, per_cu = (tiles + cu_count - 1) / cu_count;
     if (a.n_seg != 1 || tiles <= 3 * cu_count || nb > 32 || tiles / (2 * cu_count) > (int)kMostRowsTurns) return false;
     if (T == kQ8_0) return a.w_up && nb >= 12 && (nb != 16 || per_cu > 4);
-    if ((a.w_up && nb <= 16 && per_cu <= 4) || (nb > 16 && nb <= 24 && per_cu == 6)) return false;
-    if ((T == kQ4_K || T == kQ5_K) && (a.w_up || nb > 16) && (per_cu == 8 || per_cu == 10)) return false;
+    if (a.w_up && nb <= 16 && per_cu <= 4) return false;
+    if (per_cu == 6 && nb > 16 && nb <= 24 && (T != kQ6_K || (a.w_up && nb % 2 == 0))) return false;
+    if (T != kQ6_K && (a.w_up || nb > 16) && (per_cu == 8 || (per_cu == 10 && nb <= 24))) return false;
     return nb >= 14 && (last == 0 || (last == 3 && (!a.w_up || T == kQ6_K)));
 }
 

@@ -47,12 +47,12 @@ def test_workgroups_a_cu_of_many_turns(wtype, blocks, pair, two):
 
 
 @pytest.mark.parametrize("wtype, blocks, pair, three", [
-    (Q4_K, 22, False, (6, 8, 10)), (Q4_K, 24, True, (6, 8, 10)), (Q5_K, 23, False, (6, 8, 10)), (Q4_K, 32, False, (8, 10)), (Q5_K, 32, True, (8, 10)),
-    (Q4_K, 16, True, (4, 8, 10)), (Q5_K, 15, True, (4, 8, 10)), (Q4_K, 16, False, ()), (Q5_K, 14, False, ()), (Q6_K, 24, False, (6,)), (Q6_K, 22, True, (6,)),
-    (Q6_K, 16, True, (4,)), (Q6_K, 30, False, ()), (Q8_0, 12, True, ()), (Q8_0, 16, True, (4,)), (Q8_0, 24, True, ()),
+    (Q4_K, 22, False, (6, 8, 10)), (Q4_K, 24, True, (6, 8, 10)), (Q5_K, 23, False, (6, 8, 10)), (Q4_K, 32, False, (8,)), (Q5_K, 32, True, (8,)),
+    (Q4_K, 16, True, (4, 8, 10)), (Q5_K, 15, True, (4, 8, 10)), (Q4_K, 16, False, ()), (Q5_K, 14, False, ()), (Q6_K, 24, False, ()), (Q6_K, 22, True, (6,)),
+    (Q6_K, 23, True, ()), (Q6_K, 16, True, (4,)), (Q6_K, 30, False, ()), (Q8_0, 12, True, ()), (Q8_0, 16, True, (4,)), (Q8_0, 24, True, ()),
 ])
 def test_two_workgroups_a_cu_only_where_they_were_measured_faster(wtype, blocks, pair, three):
-    """Tiles a CU, rounded up, at which three workgroups a CU were measured faster: 2055 launches of 784 to 8000 tiles."""
+    """Tiles a CU, rounded up, at which three workgroups a CU were measured faster: 2475 launches of 784 to 8000 tiles."""
     def workgroups(tiles):
         n_in, rows = blocks * 256, tiles * (8 if pair else 16)
         (one,) = (recorder().calls("orin_gemv_norm_gate_up_swiglu", wtype, ptr(1), ptr(2), ptr(3), ptr(4), 1e-5, ptr(5), n_in, rows) if pair
