@@ -78,7 +78,6 @@ struct DGeom {
     static_assert(2 * kQPlaneB >= 16 * kQStride * 4, "either form");
 };
 
-typedef float f4_a8 __attribute__((ext_vector_type(4), aligned(8))); // (a table of angles is 8-byte aligned)
 // 16 bytes a lane through a descriptor (base, byte count): zeros, and no access, at kNowhere.
 constexpr int kNowhere = 0x7ffffff8;
 __device__ __forceinline__ f4 load16(const float* base, unsigned bytes, int off) {
@@ -108,7 +107,9 @@ enum : int { kPlain = 0, kStore = 1, kRotate = 2, kRotateNeox = 3, kRotateLate =
 //     of its own, so that every wait is for what is used next.
 // Rotate + store + attend, us a launch pair, caches emptied between replays, before -> now: Qwen2.5-1.5B at 200 of 4096 7.6 -> 6.5, at 4095 7.9 ->
 // 7.0, at 32767 of 32768 11.7 -> 11.2; Llama-3-8B at 1000 of 8192 7.75 -> 6.8, at 8191 11.5 -> 11.1; Qwen2.5-7B at 16001 of 32768 12.3 ->
-// 11.2; Llama-3.2-1B at 1777 of 8192 7.1 -> 6.6.  Plain decode 6.2 -> 6.05, 6.75 -> 6.6, 10.7 -> 10.9, 6.7 -> 6.5, 11.3 -> 11.25, 11.25 -> 11.15, 6.3 -> 6.2.
+// 11.2; Llama-3.2-1B at 1777 of 8192 7.1 -> 6.6.  Plain decode 6.2 -> 6.05, 6.75 -> 6.6, the same within 2 % at 32767, 6.7 -> 6.5, 11.3 -> 11.25, 11.25 ->
+// 11.15, 6.3 -> 6.2.  Without a table (every layer with rows of its own) 6.9 -> 6.5, 7.6 -> 7.3, 11.5 -> 11.35; "normal" pairs 7.55 -> 6.8,
+// 11.75 -> 11.3; 12.0 -> 11.75; 6.7 -> 6.25.
 template <int D, int MODE>
 __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
     // What the first loads need comes first, as scalars: the leading kernel arguments are handed
@@ -287,42 +288,42 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
     [[maybe_unused]] auto* const row_there = (__attribute__((address_space(3))) volatile int*)&sh_row_there;
     float (*const sh_cs)[2] = sh_cs_all[LATE ? wave : 0];
     const bool rot_early = LATE && !a.neox && a.rope_angles != nullptr; // (the query is rotated piece by piece before it is parked)
+    // A piece of the query or of the new K row, rotated.
+    [[maybe_unused]] auto rotate4 = [&](f4 x) {
+        if constexpr (NEOX) { // element e goes with e + D/2: the lane's piece is the first or the second of the pair, the other one 16 (8) lanes away
+            const bool second = e0 >= D / 2;
+            f4 y;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float lo, hi;
+                if constexpr (D == 128) { // both halves of the pair land in both lanes
+                    const u32x2 s = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[e]), __float_as_uint(x[e]), false, false);
+                    lo = __uint_as_float(s.x);
+                    hi = __uint_as_float(s.y);
+                } else {
+                    const int b = __float_as_int(x[e]);
+                    const float other = __int_as_float(__builtin_amdgcn_update_dpp(b, b, 0x128, 0xF, 0xF, false)); // row_ror:8
+                    lo = second ? other : x[e];
+                    hi = second ? x[e] : other;
+                }
+                rope_rotate(lo, hi, cs[e / 2][e % 2 * 2], cs[e / 2][e % 2 * 2 + 1]);
+                y[e] = second ? hi : lo;
+            }
+            return y;
+        } else if constexpr (TABLE) {
+            float x0 = x[0], x1 = x[1], x2 = x[2], x3 = x[3];
+            rope_rotate(x0, x1, cs[0][0], cs[0][1]);
+            rope_rotate(x2, x3, cs[0][2], cs[0][3]);
+            return f4{x0, x1, x2, x3};
+        } else {
+            return x;
+        }
+    };
     // The query pieces meet in LDS: each wave parks the piece it fetched, then a barrier that
     // waits for LDS only.  Ahead of the tile requests, where the eight waves are still in
     // step (the position and the pieces arrive together); behind them the waves are microseconds
     // apart -- the load unit takes a CU's 128 KB of requests as fast as memory answers them --
     // and a barrier there holds every wave's products until the last has all its requests out.
-            // A piece of the query or of the new K row, rotated.
-    [[maybe_unused]] auto rotate4 = [&](f4 x) {
-                if constexpr (NEOX) { // element e goes with e + D/2: the lane's piece is the first or the second of the pair, the other one 16 (8) lanes away
-                    const bool second = e0 >= D / 2;
-                    f4 y;
-    #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        float lo, hi;
-                        if constexpr (D == 128) { // both halves of the pair land in both lanes
-                            const u32x2 s = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[e]), __float_as_uint(x[e]), false, false);
-                            lo = __uint_as_float(s.x);
-                            hi = __uint_as_float(s.y);
-                        } else {
-                            const int b = __float_as_int(x[e]);
-                            const float other = __int_as_float(__builtin_amdgcn_update_dpp(b, b, 0x128, 0xF, 0xF, false)); // row_ror:8
-                            lo = second ? other : x[e];
-                            hi = second ? x[e] : other;
-                        }
-                        rope_rotate(lo, hi, cs[e / 2][e % 2 * 2], cs[e / 2][e % 2 * 2 + 1]);
-                        y[e] = second ? hi : lo;
-                    }
-                    return y;
-                } else if constexpr (TABLE) {
-                    float x0 = x[0], x1 = x[1], x2 = x[2], x3 = x[3];
-                    rope_rotate(x0, x1, cs[0][0], cs[0][1]);
-                    rope_rotate(x2, x3, cs[0][2], cs[0][3]);
-                    return f4{x0, x1, x2, x3};
-                } else {
-                    return x;
-                }
-            };
     if constexpr (LATE) {
         float4 q_park = q_late;
         // "Normal" pairs are neighbours, so the piece a wave fetched holds two whole pairs: with the caller's
@@ -462,7 +463,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
             // and the same + head_dim/2)
             auto rotate2 = [&](float (&x0)[8], float (&x1)[8], int kk) {
                 if (a.neox) { // n_rot == D (checked by the host): element e pairs with e + D/2
-    #pragma unroll
+#pragma unroll
                     for (int e = 0; e < 8; ++e) {
                         const int i = kk * 32 + grp * 8 + e;
                         rope_rotate(x0[e], x1[e], sh_cs[i][0], sh_cs[i][1]);
@@ -474,13 +475,13 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void fa_decode_split_kernel(
                     // go out together, and a pair past n_rot keeps its values by a select.
                     const int last = max(a.n_rot / 2 - 1, 0); // (n_rot = 0: nothing is rotated, entry 0 is read and not used)
                     float2 cs0[4], cs1[4];
-    #pragma unroll
+#pragma unroll
                     for (int e = 0; e < 8; e += 2) {
                         const int el0 = kk * 32 + grp * 8 + e, el1 = el0 + D / 2;
                         cs0[e / 2] = *reinterpret_cast<const float2*>(sh_cs[min(el0 / 2, last)]);
                         cs1[e / 2] = *reinterpret_cast<const float2*>(sh_cs[min(el1 / 2, last)]);
                     }
-    #pragma unroll
+#pragma unroll
                     for (int e = 0; e < 8; e += 2) {
                         const int el0 = kk * 32 + grp * 8 + e, el1 = el0 + D / 2;
                         float a0 = x0[e], a1 = x0[e + 1], b0 = x1[e], b1 = x1[e + 1];

@@ -53,7 +53,7 @@ __device__ long long g_prefill_stamps[kStampWgs * kPrefillWaves * kStampSlots];
 __device__ long long g_short_stamps[kStampWgs * 8 * kStampSlots]; // the kernel for short walks, eight waves
 }
 #define FA_STAMP(i)                                                                                          \
-    if constexpr (kWaves == orin_fa::kPrefillWaves) /* (the table's shape) */                                \
+    if constexpr (kWaves == orin_fa::kPrefillWaves) /* (the table's shape; eight waves leave no marks) */    \
         ORIN_FA_STAMP_STORE(orin_fa::g_prefill_stamps, orin_fa::kPrefillWaves, i)
 #define SHORT_STAMP(i) ORIN_FA_STAMP_STORE(orin_fa::g_short_stamps, 8, i)
 #else
@@ -946,7 +946,7 @@ __global__ __launch_bounds__(WAVES * 64) void fa_prefill_kernel(PREFILL_ARGS) {
     __syncthreads();
     FA_STAMP(7);
 
-    // Four threads per column (eight in the 32-column shape, so that no thread idles): the weights
+    // Four threads per column (eight with 32 columns or with eight waves, so that no thread idles): the weights
     // are computed once, then each thread merges and stores its share of the column's head_dim in
     // 16-byte pieces (the pieces of a step are one contiguous 64 or 128 bytes of the output row).
     constexpr int kParts = G::kParts; // threads per column: 4 with 64 columns, 8 with 32 or with eight waves

@@ -18,7 +18,8 @@
 // operation in fp32.  Sine and cosine are the accurate library versions (full range
 // reduction), not the fast hardware approximations the reference's GPU path uses.  They are taken
 // together: one range reduction (100 instructions where the angle is large) instead of two, the same
-// bits as sinf and cosf give for every one of the 2^32 floats.  Back to back in a graph, rotary and
+// bits as sinf and cosf give (all 2^32 floats compared once, with the compiler that check_toolchain() in
+// build.py asks for).  Back to back in a graph, rotary and
 // cache rows of 512 tokens, apart -> together: 12 + 2 heads of 128 2.87 -> 2.82 us, 32 + 8 heads
 // 4.75 -> 4.59, 28 + 4 heads 4.04 -> 3.94; 301 tokens of 32 + 8 heads of 64 3.12 -> 3.07.
 #include "fa_common.hpp"
