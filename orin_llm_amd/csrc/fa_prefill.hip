@@ -1510,11 +1510,12 @@ hipError_t launch(FaArgs a, int cu_count, hipStream_t stream, void* workspace, s
     consider(IntC<32>{});
     bool eight = false;
     if constexpr (D == 64) {
-        // A fifth form: 64 columns on eight waves, one workgroup a CU where the others of head_dim 64 are two.  Those two share
-        // nothing, so a CU's path to memory carries every tile twice, and that is what bounds them; eight waves fetch it once for
-        // as many columns.  Its start and its merge of eight states cost 2 us more, so it takes launches of one turn of the
-        // chip whose first token already sees more rows than that is worth (and a tile for every wave several times over).  us,
-        // rows in the caches / from memory, the estimate's choice -> eight, 32 / 8 heads:
+        // A fifth form: 64 columns on eight waves, one workgroup a CU.  Up to a workgroup a CU the form of four waves has one there as well,
+        // a wave a SIMD that nothing else runs beside: with two the same bytes and products take fewer cycles (512 tokens at 4096 49.8 k ->
+        // 43.6 k, 4.8 M and 5.0 M look-ups in the L1s).  Against 32 columns, two workgroups a CU, it has half the look-ups (301 tokens at 4096 5.5 M -> 2.9 M), and
+        // against two KV splits no partial results to merge.  Its start and its merge of eight states cost 2 us more, so it takes launches of
+        // one turn of the chip whose first token already sees more rows than that is worth (and a tile for every wave several times over).
+        // us, rows in the caches / from memory, the estimate's choice -> eight, 32 / 8 heads:
         //   301 tokens at 1501 12.7 / 14.5 -> 12.3 / 13.4, at 4096 23.8 / 23.9 -> 20.1 / 22.5; 512 at 1800 16.0 / 16.8 -> 15.5 / 16.3, at 4500
         //   28.3 / 31.4 -> 27.1 / 26.3, at 24000 114 / 109 -> 112 / 108; not behind 1300 rows or fewer: 512 at 420 10.0 / 10.3 -> 10.2 / 11.3,
         //   8 / 1 heads, 1700 tokens at 0 11.7 / 12.2 -> 12.0 / 12.7, 1 / 1, 8256 tokens at 0 24.1 / 23.4 -> 29.5 / 30.4
