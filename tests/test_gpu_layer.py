@@ -464,10 +464,11 @@ def test_f16_rows_in_runs(ly, n_in):
 @pytest.mark.parametrize("n_in, heights", [
     (512, (8200, 9, 1)), (544, (8199, 1, 8)), (1024, (4103, 4105, 7)), (1056, (4104, 15, 4097)), (1536, (4097, 8, 8)),
     (1568, (2049, 4111, 6)), (2048, (2055, 2056, 2057)), (2080, (1029, 5, 3)), (6176, (515, 2, 513)), (14336, (513, 1, 3)), (17440, (515, 1, 2)), (18944, (513, 2, 1)), (23040, (514, 3, 1)), (23072, (513, 1, 2)),
+    (3072, (4103, 7, 9)), (5120, (2055, 9, 1)), (5152, (1025, 1, 2)), (17440, (771, 1, 2)), (18944, (1031, 2, 1)), (28672, (257, 2, 1)),
 ])
 def test_f16_batches_of_several_turns(ly, n_in, heights):
-    """One to four, eight and 11 to 15 waves a workgroup, batches of one to eight rows that end inside a matrix, one and several turns of the chip:
-    three matrices as one launch, one alone, the pair."""
+    """One to four, eight and 11 to 15 waves a workgroup, one and two workgroups a CU, batches of one to eight rows that end inside a matrix, one and
+    several turns of the chip: three matrices as one launch, one alone, the pair."""
     import torch
 
     rs = lm.Stream(8800 + n_in)
