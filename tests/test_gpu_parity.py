@@ -457,6 +457,7 @@ def test_cfg2_full_stack_28_layers(fa):
     (12, 2, 128, 4096, 550, 4),      # ... with a second and a third tile a wave
     (32, 8, 64, 4096, 20, 70),       # ... at head_dim 64
     (12, 2, 128, 16384, 8000, 100),  # eight splits of 64 columns
+    (32, 8, 64, 4096, 2900, 301),    # eight waves, no splits
 ])
 def test_prefill_in_place(fa, H, G, d, n_ctx, n_past, batch):
     """out = q: a split's log-sum-exps must not land in query rows that another split of the tile has still to read."""
